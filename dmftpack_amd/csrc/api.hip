@@ -116,7 +116,7 @@ extern "C" int dmftgpu_destroy(dmftgpu_handle h)
     h->prep.release();
     h->stat.release();
     h->static_cache.release();
-    h->fused.release();
+    h->tail_dev.release();
     h->cot.release();
     h->core.release();
     delete h;
@@ -205,6 +205,17 @@ static int check_lattice(dmftgpu_handle h, const dmftgpu_lattice* L)
     return DMFTGPU_OK;
 }
 
+// Frequency points of the density sums for the moments in h->mom
+static int set_points(dmftgpu_handle h)
+{
+    const dmftgpu_lattice& L = h->lat;
+    const int nw_tot = L.n_freq * L.high_freq, n_tail = (int)h->tail.size() / 2;
+    h->n_plan = n_tail ? L.n_freq + n_tail : nw_tot;
+    HIPCHK(dg::launch_freq_points(h->mom, L.n_corr, L.n_freq, nw_tot, n_tail, (const double*)h->tail_dev.ptr, L.beta,
+                                  h->pt_n, h->pt_w, h->pt_wt, h->stream));
+    return DMFTGPU_OK;
+}
+
 extern "C" int dmftgpu_prepare(dmftgpu_handle h, const dmftgpu_lattice* L, const double* Hk, const double* moments)
 {
     (void)hipGetLastError();  // drop an error left by an earlier failed call
@@ -226,6 +237,8 @@ extern "C" int dmftgpu_prepare(dmftgpu_handle h, const dmftgpu_lattice* L, const
     const bool lane_kernels = dg::schur_supported(n, nc) && dg::schur_multi_supported(nc);
     size_t o_kd = cv.take<cd>(lane_kernels ? (size_t)nk * dg::schur_kdata_size(n, nc) + dg::kKdataPadBytes / sizeof(cd)
                                           : 1);
+    const size_t nw_tot = (size_t)L->n_freq * L->high_freq;
+    size_t o_pt = cv.take<double>(2 * nw_tot + 1);
     hipError_t e;
     char* base = (char*)h->prep.get(cv.off, &e);
     if (!base) return fail(h, DMFTGPU_ERR_HIP, "prepare alloc %zu bytes: %s", cv.off, hipGetErrorString(e));
@@ -236,6 +249,9 @@ extern "C" int dmftgpu_prepare(dmftgpu_handle h, const dmftgpu_lattice* L, const
     h->Vd = (cd*)(base + o_Vd);
     h->W = (cd*)(base + o_W);
     h->kdata = lane_kernels ? (cd*)(base + o_kd) : nullptr;
+    h->pt_w = (double*)(base + o_pt);
+    h->pt_wt = h->pt_w + nw_tot;
+    h->pt_n = (int*)(h->pt_wt + nw_tot);
     HIPCHK(hipMemcpyAsync(h->mom, moments, sizeof(cd) * 4 * nc * nc, hipMemcpyDefault, h->stream));
     // static part: eig(H(k) + P m0 P^H)   (GreenFtn.cpp:197-215)
     HIPCHK(dg::launch_herm_eig(h->Hk, n, 0, n, h->mom, nc, h->ev, h->U, nk, h->stream));
@@ -249,6 +265,19 @@ extern "C" int dmftgpu_prepare(dmftgpu_handle h, const dmftgpu_lattice* L, const
         if (lane_kernels) HIPCHK(dg::launch_schur_kdata(h->Hk, h->W, h->ed, n, nc, nk, h->kdata, h->stream));
         h->schur_ready = true;
     }
+    // (after the launches above: the host forms the rule while they run)
+    if (h->tail_nf != L->n_freq || h->tail_tot != (int)nw_tot) {
+        h->tail_nf = 0;  // valid again once the copy below is in place
+        h->tail = dg::freq_tail(L->n_freq, (int)nw_tot);
+        if (!h->tail.empty()) {
+            void* t = h->tail_dev.get(h->tail.size() * sizeof(double), &e);
+            if (!t) return fail(h, DMFTGPU_ERR_HIP, "frequency rule: %s", hipGetErrorString(e));
+            HIPCHK(hipMemcpyAsync(t, h->tail.data(), h->tail.size() * sizeof(double), hipMemcpyHostToDevice, h->stream));
+        }
+        h->tail_nf = L->n_freq;
+        h->tail_tot = (int)nw_tot;
+    }
+    if ((rc = set_points(h))) return rc;
     h->core_n_orb = 0;  // Kohn-Sham bands belong to the previous H(k)
     h->prepared = true;
     ++h->prep_gen;
@@ -267,6 +296,7 @@ extern "C" int dmftgpu_update_moments(dmftgpu_handle h, const double* moments)
     const int n = h->lat.n, nc = h->lat.n_corr, nk = h->lat.n_k;
     HIPCHK(hipMemcpyAsync(h->mom, moments, sizeof(cd) * 4 * nc * nc, hipMemcpyDefault, h->stream));
     HIPCHK(dg::launch_herm_eig(h->Hk, n, 0, n, h->mom, nc, h->ev, h->U, nk, h->stream));
+    if (int rc = set_points(h)) return rc;
     ++h->prep_gen;
     return DMFTGPU_OK;
 }
@@ -447,6 +477,8 @@ bool method_ok(dmftgpu_handle h, int method, int* rc)
 //   Sbsum [n_freq][m2] and musum [n_freq] (VJP).
 struct Sums {
     cd *Gsum = nullptr, *tr = nullptr, *tr2 = nullptr, *Sb = nullptr, *mu = nullptr;
+    const int* pt_n = nullptr;      // the frequency points the sums were taken at (LatArgs)
+    const double* pt_wt = nullptr;
 };
 
 // Real-axis frequency grid z_n = e0 + n de + i eta, n < n_e (retarded_GreenFtn2).
@@ -462,13 +494,16 @@ struct PerK {
     cd* tr;
 };
 
-// fused_tr2 (one-matrix-per-lane Schur only): the [chunks][nw_tot] tr G^2 partials
-// shared by a forward that fills them beyond n_freq and the adjoint that follows
-// (dmftgpu_gloc_loss_grad), which fills the rest and reduces them.
+// frequency points a launch covers (grid planning): every frequency for the plain
+// method, the point table for the Schur methods on the Matsubara axis
+int plan_points(dmftgpu_handle h, int method, const RealAxis* ra)
+{
+    return ra ? ra->n_e : method == DMFTGPU_PLAIN_F64 ? h->lat.n_freq * h->lat.high_freq : h->n_plan;
+}
+
 int run_lattice(dmftgpu_handle h, int method, int mode, const double* sigma, double mu, const double* gbar,
                 double nbar, char* ws, size_t& off, Sums& S, bool want_trace = false, const RealAxis* ra = nullptr,
-                const PerK* pk = nullptr, cd* fused_tr2 = nullptr, int fused_chunks = 0, int max_chunks = 0,
-                size_t cap = SIZE_MAX)
+                const PerK* pk = nullptr, int max_chunks = 0, size_t cap = SIZE_MAX)
 {
     const dmftgpu_lattice& L = h->lat;
     const int n = L.n, nc = L.n_corr, nk = L.n_k, m2 = nc * nc;
@@ -478,14 +513,12 @@ int run_lattice(dmftgpu_handle h, int method, int mode, const double* sigma, dou
     if (method == DMFTGPU_PLAIN_F64) slots = dg::plain_slots(n, mode);
     else slots = dg::schur_slots(nc, mode, method == DMFTGPU_SCHUR_F32R, h->schur_layout == 1 || (ra && mode != dg::MODE_FWD));
     const bool cols = h->schur_layout == 1 || (ra && mode != dg::MODE_FWD);
-    Plan P = pk ? Plan{nk, 1} : make_plan(nk, nw_tot, slots, lattice_target(h, method, nc, cols, nk, nw_tot, slots));
+    const int nw_plan = plan_points(h, method, ra);
+    Plan P = pk ? Plan{nk, 1} : make_plan(nk, nw_plan, slots, lattice_target(h, method, nc, cols, nk, nw_plan, slots));
     if (max_chunks > 0 && P.n_chunks > max_chunks) {  // partial sums held to a fixed scratch size
         const int kpc = (nk + max_chunks - 1) / max_chunks;
         P = Plan{(nk + kpc - 1) / kpc, kpc};
     }
-    if (fused_tr2 && P.n_chunks != fused_chunks)  // both halves of a fused pair must chunk k alike
-        return fail(h, DMFTGPU_ERR_STATE, "fused partials laid out for %d k chunks, this call uses %d", fused_chunks,
-                    P.n_chunks);
     dg::LatArgs a{};
     a.Hk = h->Hk;
     a.sigma = (const cd*)sigma;
@@ -512,6 +545,12 @@ int run_lattice(dmftgpu_handle h, int method, int mode, const double* sigma, dou
     a.kdata = h->kdata;
     a.refine = h->refine_steps;
     a.want_trace = want_trace ? 1 : 0;
+    if (method != DMFTGPU_PLAIN_F64 && !ra) {
+        a.pt_n = h->pt_n;
+        a.pt_w = h->pt_w;
+        a.pt_wt = h->pt_wt;
+        a.n_plan = h->n_plan;
+    }
     auto take = [&](size_t bytes) {
         char* p = ws + off;
         off += (bytes + 255) / 256 * 256;
@@ -525,8 +564,7 @@ int run_lattice(dmftgpu_handle h, int method, int mode, const double* sigma, dou
         a.pTr = (cd*)take(C * nw_tot * sizeof(cd));
         if (mode == dg::MODE_FWD) a.pG = (cd*)take(C * nw_tot * m2 * sizeof(cd));
     }
-    if (fused_tr2) a.pTr2 = fused_tr2;
-    else if (mode != dg::MODE_FWD) a.pTr2 = (cd*)take(C * nw_tot * sizeof(cd));
+    if (mode != dg::MODE_FWD) a.pTr2 = (cd*)take(C * nw_tot * sizeof(cd));
     if (mode == dg::MODE_VJP) {
         a.pSb = (cd*)take(C * n_freq * m2 * sizeof(cd));
         a.pMu = (cd*)take(C * n_freq * sizeof(cd));
@@ -549,18 +587,20 @@ int run_lattice(dmftgpu_handle h, int method, int mode, const double* sigma, dou
     } else {
         // schur_wg 0: each launch at its default width (launch_lattice_schur)
         HIPCHK(dg::launch_lattice_schur(a, mode, method == DMFTGPU_SCHUR_F32R, h->stream, h->schur_wg,
-                                        h->schur_layout == 1, fused_tr2 != nullptr));
+                                        h->schur_layout == 1));
     }
     if (h->timing) {
         HIPCHK(hipEventRecord(h->ev1[mode], h->stream));
         h->ev_used[mode] = true;
     }
     if (pk) return DMFTGPU_OK;
-    HIPCHK(dg::launch_reduce_chunks(a.pTr, P.n_chunks, nw_tot, S.tr, h->stream));
+    S.pt_n = a.pt_n;
+    S.pt_wt = a.pt_wt;
+    HIPCHK(dg::launch_reduce_chunks(a.pTr, P.n_chunks, nw_tot, S.tr, h->stream, a.pt_n));
     if (mode == dg::MODE_FWD) {
-        HIPCHK(dg::launch_reduce_chunks(a.pG, P.n_chunks, (size_t)nw_tot * m2, S.Gsum, h->stream));
+        HIPCHK(dg::launch_reduce_chunks(a.pG, P.n_chunks, (size_t)nw_tot * m2, S.Gsum, h->stream, a.pt_n, m2));
     } else {
-        HIPCHK(dg::launch_reduce_chunks(a.pTr2, P.n_chunks, nw_tot, S.tr2, h->stream));
+        HIPCHK(dg::launch_reduce_chunks(a.pTr2, P.n_chunks, nw_tot, S.tr2, h->stream, a.pt_n));
     }
     if (mode == dg::MODE_VJP) {
         HIPCHK(dg::launch_reduce_chunks(a.pSb, P.n_chunks, (size_t)n_freq * m2, S.Sb, h->stream));
@@ -578,9 +618,10 @@ size_t lattice_ws_bytes(dmftgpu_handle h, int method, int mode, const RealAxis* 
     int slots = method == DMFTGPU_PLAIN_F64 ? dg::plain_slots(L.n, mode)
                                             : dg::schur_slots(nc, mode, method == DMFTGPU_SCHUR_F32R,
                                                               h->schur_layout == 1 || (ra && mode != dg::MODE_FWD));
-    Plan P = make_plan(L.n_k, (int)nw_tot, slots,
-                       lattice_target(h, method, nc, h->schur_layout == 1 || (ra && mode != dg::MODE_FWD), L.n_k,
-                                      (int)nw_tot, slots));
+    const int nw_plan = plan_points(h, method, ra);
+    Plan P = make_plan(L.n_k, nw_plan, slots,
+                       lattice_target(h, method, nc, h->schur_layout == 1 || (ra && mode != dg::MODE_FWD), L.n_k, nw_plan,
+                                      slots));
     size_t C = P.n_chunks + 1;  // +1 for the reduced copy
     size_t b = (C + 1) * nw_tot * 16 * (2 + (size_t)m2) + C * n_freq * 16 * (m2 + 1) + 64 * 256;
     return b;
@@ -595,8 +636,7 @@ namespace {
 // the handle's workspaces (the static part then keeps no cache); the k
 // chunking is reduced until the partial sums fit.
 int forward_impl(dmftgpu_handle h, int method, const double* sigma, double mu, double* gloc, double* gloc_hf,
-                 double* num_matrix, double* n_total, cd* fused_tr2, int fused_chunks, char* ext_ws = nullptr,
-                 size_t ext_cap = 0)
+                 double* num_matrix, double* n_total, char* ext_ws = nullptr, size_t ext_cap = 0)
 {
     const dmftgpu_lattice& L = h->lat;
     const int nc = L.n_corr, m2 = nc * nc;
@@ -636,9 +676,10 @@ int forward_impl(dmftgpu_handle h, int method, const double* sigma, double mu, d
     int rc = run_static(h, mu, st, sts, ws, off, ext_ws != nullptr, nullptr, cap);
     if (rc) return rc;
     rc = run_lattice(h, method, dg::MODE_FWD, sigma, mu, nullptr, 0.0, ws, off, S, n_total != nullptr, nullptr,
-                     nullptr, fused_tr2, fused_chunks, max_chunks, cap);
+                     nullptr, max_chunks, cap);
     if (rc) return rc;
-    HIPCHK(dg::launch_freq_totals(S.Gsum, m2, nc, S.tr, nullptr, nw_tot, nullptr, 0, tot, h->stream));
+    HIPCHK(dg::launch_freq_totals(S.Gsum, m2, nc, S.tr, nullptr, nw_tot, nullptr, 0, tot, h->stream, S.pt_n,
+                                  S.pt_wt));
     const double inv_nk = 1.0 / (double)L.n_k_global;
     HIPCHK(dg::launch_gloc_finalize(S.Gsum, L.n_freq, nc, L.n_cluster, inv_nk, (cd*)gloc, h->stream));
     if (gloc_hf)
@@ -680,7 +721,7 @@ extern "C" int dmftgpu_greenftn_w(dmftgpu_handle h, int method, const double* si
         return fail(h, DMFTGPU_ERR_UNSUPPORTED, "Schur method needs n_corr <= 16 (n=%d, n_corr=%d)", h->lat.n, h->lat.n_corr);
     if (!sigma || !gloc || !num_matrix) return fail(h, DMFTGPU_ERR_ARG, "sigma, gloc and num_matrix are required");
     if (!std::isfinite(mu)) return fail(h, DMFTGPU_ERR_ARG, "mu is not finite");
-    return forward_impl(h, method, sigma, mu, gloc, gloc_hf, num_matrix, n_total, nullptr, 0);
+    return forward_impl(h, method, sigma, mu, gloc, gloc_hf, num_matrix, n_total);
 }
 
 // dmftgpu_greenftn_w without device allocation: every scratch buffer is carved
@@ -697,7 +738,7 @@ extern "C" int dmftgpu_greenftn_w_noalloc(dmftgpu_handle h, int method, const do
     if (!sigma || !gloc || !num_matrix) return fail(h, DMFTGPU_ERR_ARG, "sigma, gloc and num_matrix are required");
     if (!std::isfinite(mu)) return fail(h, DMFTGPU_ERR_ARG, "mu is not finite");
     if (!h->scratch) return fail(h, DMFTGPU_ERR_HIP, "no-alloc scratch unavailable on device %d", h->device);
-    return forward_impl(h, method, sigma, mu, gloc, gloc_hf, num_matrix, n_total, nullptr, 0, (char*)h->scratch,
+    return forward_impl(h, method, sigma, mu, gloc, gloc_hf, num_matrix, n_total, (char*)h->scratch,
                         dgi::kNoAllocScratchBytes);
 }
 
@@ -788,7 +829,7 @@ static int density_impl(dmftgpu_handle h, int method, const double* sigma, doubl
     off += 256;
     rc = run_static(h, mu, st, sts, ws, off);
     if (rc) return rc;
-    HIPCHK(dg::launch_freq_totals(nullptr, m2, nc, S.tr, S.tr2, nw_tot, nullptr, 0, tot, h->stream));
+    HIPCHK(dg::launch_freq_totals(nullptr, m2, nc, S.tr, S.tr2, nw_tot, nullptr, 0, tot, h->stream, S.pt_n, S.pt_wt));
     std::vector<cd> htot(m2 + 3);
     double hsts[2];
     HIPCHK(hipMemcpyAsync(htot.data(), tot, sizeof(cd) * (m2 + 3), hipMemcpyDeviceToHost, h->stream));
@@ -864,7 +905,7 @@ extern "C" int dmftgpu_adjust_mu(dmftgpu_handle h, int method, const double* sig
 namespace {
 
 int vjp_impl(dmftgpu_handle h, int method, const double* sigma, double mu, const double* gloc_bar, double n_bar,
-             double* sigma_bar, double* mu_bar, cd* fused_tr2, int fused_chunks)
+             double* sigma_bar, double* mu_bar)
 {
     const dmftgpu_lattice& L = h->lat;
     const int nc = L.n_corr, m2 = nc * nc;
@@ -875,8 +916,7 @@ int vjp_impl(dmftgpu_handle h, int method, const double* sigma, double mu, const
     if (!ws) return fail(h, DMFTGPU_ERR_HIP, "workspace %zu bytes: %s", need, hipGetErrorString(e));
     size_t off = 0;
     Sums S;
-    int rc = run_lattice(h, method, dg::MODE_VJP, sigma, mu, gloc_bar, n_bar, ws, off, S, false, nullptr, nullptr,
-                         fused_tr2, fused_chunks);
+    int rc = run_lattice(h, method, dg::MODE_VJP, sigma, mu, gloc_bar, n_bar, ws, off, S);
     if (rc) return rc;
     cd* tot = (cd*)(ws + off);
     off += ((size_t)(m2 + 3) * sizeof(cd) + 255) / 256 * 256;
@@ -888,8 +928,8 @@ int vjp_impl(dmftgpu_handle h, int method, const double* sigma, double mu, const
     if (rc) return rc;
     const double inv_nk = 1.0 / (double)L.n_k_global;
     HIPCHK(dg::launch_scale(S.Sb, (size_t)L.n_freq * m2, inv_nk, (cd*)sigma_bar, h->stream));
-    // (tr G itself is not needed here; after a fused forward only its first N_freq entries are formed)
-    HIPCHK(dg::launch_freq_totals(nullptr, m2, nc, nullptr, S.tr2, nw_tot, S.mu, L.n_freq, tot, h->stream));
+    HIPCHK(dg::launch_freq_totals(nullptr, m2, nc, nullptr, S.tr2, nw_tot, S.mu, L.n_freq, tot, h->stream, S.pt_n,
+                                  S.pt_wt));
     std::vector<cd> htot(m2 + 3);
     double hsts[2];
     HIPCHK(hipMemcpyAsync(htot.data(), tot, sizeof(cd) * (m2 + 3), hipMemcpyDeviceToHost, h->stream));
@@ -914,7 +954,7 @@ extern "C" int dmftgpu_gloc_vjp(dmftgpu_handle h, int method, const double* sigm
     if (!method_ok(h, method, &rc)) return rc;
     if (!sigma || !gloc_bar || !sigma_bar) return fail(h, DMFTGPU_ERR_ARG, "sigma, gloc_bar and sigma_bar are required");
     if (!std::isfinite(mu) || !std::isfinite(n_bar)) return fail(h, DMFTGPU_ERR_ARG, "mu or n_bar is not finite");
-    return vjp_impl(h, method, sigma, mu, gloc_bar, n_bar, sigma_bar, mu_bar, nullptr, 0);
+    return vjp_impl(h, method, sigma, mu, gloc_bar, n_bar, sigma_bar, mu_bar);
 }
 
 // Jacobian-vector product of (G_loc, N) in (Sigma(iw_n), n < N_freq; mu), moments
@@ -954,7 +994,8 @@ static int jvp_impl(dmftgpu_handle h, int method, const double* sigma, double mu
     if (rc) return rc;
     const double inv_nk = 1.0 / (double)L.n_k_global;
     HIPCHK(dg::launch_adjoint_stack(S.Sb, (size_t)L.n_freq, nc, inv_nk, (cd*)dgloc, h->stream));
-    HIPCHK(dg::launch_freq_totals(nullptr, m2, nc, nullptr, S.tr2, nw_tot, S.mu, L.n_freq, tot, h->stream));
+    HIPCHK(dg::launch_freq_totals(nullptr, m2, nc, nullptr, S.tr2, nw_tot, S.mu, L.n_freq, tot, h->stream, S.pt_n,
+                                  S.pt_wt));
     cd htot[32 * 32 + 3];
     double hsts[2];
     HIPCHK(hipMemcpyAsync(htot, tot, sizeof(cd) * (m2 + 3), hipMemcpyDeviceToHost, h->stream));
@@ -980,9 +1021,7 @@ extern "C" int dmftgpu_gloc_jvp(dmftgpu_handle h, int method, const double* sigm
 }
 
 // Loss L = sum_{n<N_freq} ||G_loc(iw_n) - G_tgt(iw_n)||_F^2 + (N - N_tgt)^2 and its
-// gradient: forward, cotangents on the device, adjoint.  On the one-matrix-per-lane
-// Schur path the forward also forms tr G^2 beyond N_freq (fused), so the adjoint
-// only covers the first N_freq frequencies.
+// gradient: forward, cotangents on the device, adjoint.
 extern "C" int dmftgpu_gloc_loss_grad(dmftgpu_handle h, int method, const double* sigma, double mu,
                                       const double* gloc_target, double n_target, double* gloc, double* num_matrix,
                                       double* n_total, double* loss, double* sigma_bar, double* mu_bar)
@@ -996,19 +1035,9 @@ extern "C" int dmftgpu_gloc_loss_grad(dmftgpu_handle h, int method, const double
     if (!std::isfinite(mu) || !std::isfinite(n_target)) return fail(h, DMFTGPU_ERR_ARG, "mu or n_target is not finite");
     const dmftgpu_lattice& L = h->lat;
     const int nc = L.n_corr, m2 = nc * nc;
-    const int nw_tot = L.n_freq * L.high_freq;
     hipError_t e;
-    cd* ftr2 = nullptr;
-    int fchunks = 0;
-    if (method != DMFTGPU_PLAIN_F64 && dg::schur_can_fuse(nc, h->schur_layout == 1, false) && nw_tot > L.n_freq) {
-        const int slots = dg::schur_slots(nc, dg::MODE_FWD, method == DMFTGPU_SCHUR_F32R, false);
-        const Plan P = make_plan(L.n_k, nw_tot, slots, lattice_target(h, method, nc, false, L.n_k, nw_tot, slots));
-        fchunks = P.n_chunks;
-        ftr2 = (cd*)h->fused.get((size_t)P.n_chunks * nw_tot * sizeof(cd), &e);
-        if (!ftr2) return fail(h, DMFTGPU_ERR_HIP, "fused partials: %s", hipGetErrorString(e));
-    }
     double N = 0.0;
-    rc = forward_impl(h, method, sigma, mu, gloc, nullptr, num_matrix, &N, ftr2, fchunks);
+    rc = forward_impl(h, method, sigma, mu, gloc, nullptr, num_matrix, &N);
     if (rc) return rc;
     // cotangents: gbar = 2 (G_loc - G_tgt) on the returned (cluster-block-diagonal)
     // entries, 0 on the inter-cluster ones, which the output fixes at zero
@@ -1018,7 +1047,7 @@ extern "C" int dmftgpu_gloc_loss_grad(dmftgpu_handle h, int method, const double
     HIPCHK(dg::launch_loss_cotangent((const cd*)gloc, (const cd*)gloc_target, L.n_freq, nc, nc / L.n_cluster, gbar, dloss,
                                      h->stream));
     const double nbar = 2.0 * (N - n_target);
-    rc = vjp_impl(h, method, sigma, mu, (const double*)gbar, nbar, sigma_bar, mu_bar, ftr2, fchunks);
+    rc = vjp_impl(h, method, sigma, mu, (const double*)gbar, nbar, sigma_bar, mu_bar);
     if (rc) return rc;
     if (n_total) *n_total = N;
     if (loss) {
@@ -1071,6 +1100,9 @@ extern "C" int dmftgpu_density_matrix(dmftgpu_handle h, const double* sigma, dou
     a.kdata = h->kdata;
     if (block) {
         a.pSigAll = sig_all;
+        a.pt_n = h->pt_n;
+        a.pt_w = h->pt_w;
+        a.pt_wt = h->pt_wt;
         HIPCHK(dg::launch_sigma_all(a, h->stream));
         HIPCHK(dg::launch_density_matrix_lr(a, h->W, h->Vd, h->ed, h->U, wt, (cd*)dens, h->stream));
     } else {

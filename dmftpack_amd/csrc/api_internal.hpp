@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <string>
+#include <vector>
 
 #include "../../include/dmftgpu.h"
 #include "dev_common.hpp"
@@ -44,6 +45,14 @@ struct dmftgpu_handle_s {
     dg::cd* Vd = nullptr;    // [nk][nd][nd]
     dg::cd* W = nullptr;     // [nk][nc][nd] H_cd V_d
     dg::cd* kdata = nullptr; // [nk][H_cc | P_d pairs | e_d] of the one-matrix-per-lane Schur kernels
+    // frequency points of the density sums (freq_points.hip): the rule beyond n_freq for
+    // the last (n_freq, high_freq n_freq), and the table for the bound moments
+    int tail_nf = 0, tail_tot = 0;
+    std::vector<double> tail;  // [x..., weight...]
+    dgi::Workspace tail_dev;
+    int n_plan = 0;            // points of the table when the rule applies
+    int* pt_n = nullptr;
+    double *pt_w = nullptr, *pt_wt = nullptr;
     int target_wg = 0;       // work items per lattice launch (k chunking); 0: lattice_target's default
     // static-part totals for the last mu (valid until the next prepare)
     unsigned prep_gen = 0, static_gen = ~0u;
@@ -78,7 +87,6 @@ struct dmftgpu_handle_s {
     double* core_eps = nullptr;
     unsigned char* core_out = nullptr;
     dgi::Workspace core;
-    dgi::Workspace fused;    // tr G^2 partials shared by a fused forward and its adjoint
     dgi::Workspace cot;      // loss cotangents gbar [n_freq][nc][nc] + the loss sum
     // optional kernel timing (dmftgpu_enable_timing): events around the main
     // lattice kernel of each mode (FWD, DENS, VJP)

@@ -85,6 +85,10 @@ struct Sys {
     cd *trF, *Gsum, *trV, *tr2, *Sb, *musum;
     // chosen plans
     int chunks_f, kpc_f, chunks_v, kpc_v;
+    // frequency points of the density sums (freq_points.hip)
+    int n_plan, n_tail;
+    double *tail, *pt_w, *pt_wt;
+    int* pt_n;
 };
 
 // per-mode slots of a group: 0 forward, 1 adjoint
@@ -92,7 +96,7 @@ inline int slot(int mode) { return mode == MODE_VJP ? 1 : 0; }
 
 struct Group {
     int nc;
-    bool cols = false;  // n_c > 6: column-per-lane kernels, one work list over every frequency
+    bool cols = false;  // n_c > 6: column-per-lane kernels
     std::vector<int> systems;
     int wg[2] = {64, 64};
     double target[2] = {0, 0};
@@ -100,15 +104,6 @@ struct Group {
     LatArgs* dargs[2] = {nullptr, nullptr};
     int4* ditems[2] = {nullptr, nullptr};
     int n_items[2] = {0, 0};
-    // frequencies n >= N_freq: the forward accumulates the Hermitian part of G_cc
-    // (MODE_FWD_HERM), the adjoint only needs tr G, tr G^2 (density kernel); with
-    // an adjoint in the step both happen in the forward (MODE_DENS_HERM, writing
-    // the adjoint's tr G^2 partials, same k chunking) and the adjoint has no
-    // upper work list
-    int mode_hi[2] = {MODE_FWD_HERM, MODE_DENS};
-    LatArgs* dargs_hi[2] = {nullptr, nullptr};
-    int4* ditems_hi[2] = {nullptr, nullptr};
-    int n_items_hi[2] = {0, 0};
     int max_nd = 0;
 };
 
@@ -175,6 +170,9 @@ LatArgs make_args(const dmftgpu_batch_s* b, const Sys& s, int mode, int chunks, 
     a.kdata = s.kdata;
     a.refine = b->h->refine_steps;
     a.pSigAll = s.sig_all;
+    a.pt_n = s.pt_n;
+    a.pt_w = s.pt_w;
+    a.pt_wt = s.pt_wt;
     if (mode == MODE_FWD) {
         a.pTr = s.pTrF;
         a.pG = s.pG;
@@ -194,8 +192,8 @@ LatArgs make_args(const dmftgpu_batch_s* b, const Sys& s, int mode, int chunks, 
 int build_group(dmftgpu_batch_s* b, Group& g, int mode, int wg, double target)
 {
     dmftgpu_handle h = b->h;
-    std::vector<LatArgs> args, args_hi;
-    std::vector<int4> items, items_hi;
+    std::vector<LatArgs> args;
+    std::vector<int4> items, spare;
     for (size_t q = 0; q < g.systems.size(); ++q) {
         Sys& s = b->sys[g.systems[q]];
         int kpc;
@@ -208,33 +206,19 @@ int build_group(dmftgpu_batch_s* b, Group& g, int mode, int wg, double target)
             s.kpc_v = kpc;
         }
         LatArgs a = make_args(b, s, mode, chunks, kpc);
-        const bool split = s.nw_tot > s.nf && !g.cols;
-        if (split) {  // [0, nf) forward / adjoint, [nf, nw_tot) see Group::mode_hi
-            LatArgs hi = a;
-            a.nw_end = s.nf;
-            hi.nw_begin = s.nf;
-            if (mode == MODE_FWD && b->vjp) hi.pTr2 = s.pTr2;  // fused: the adjoint's partials
-            args_hi.push_back(hi);
-        } else {
-            args_hi.push_back(a);  // unused placeholder keeps the system index
-        }
         args.push_back(a);
-        // (the k-pair form covers 64 frequencies per item; the upper launch runs at 64)
+        // (the k-pair form covers 64 frequencies per item)
         const int wf = wg == dg::SCHUR_WG_KPAIR ? 64 : wg;
         const int per_tile = g.cols ? dg::schur_slots(s.nc, mode, b->method == DMFTGPU_SCHUR_F32R, true) : wf;
-        const int nwt = ((split ? s.nf : s.nw_tot) + per_tile - 1) / per_tile;
+        // tiles past the planned frequency points have work only when the moments rule the
+        // Gauss points out: listed last, so that the striding stays even without them
+        const int nwt = (s.nw_tot + per_tile - 1) / per_tile, nwp = (s.n_plan + per_tile - 1) / per_tile;
         for (int c = 0; c < chunks; ++c)
-            for (int t = 0; t < nwt; ++t) items.push_back(int4{(int)q, t, c, 0});
-        if (split && !(mode == MODE_VJP && b->vjp)) {  // fused adjoint: the forward did these
-            const int nwh = (s.nw_tot - s.nf + wf - 1) / wf;
-            for (int c = 0; c < chunks; ++c)
-                for (int t = 0; t < nwh; ++t) items_hi.push_back(int4{(int)q, t, c, 0});
-        }
+            for (int t = 0; t < nwt; ++t) (t < nwp ? items : spare).push_back(int4{(int)q, t, c, 0});
     }
-    g.mode_hi[0] = b->vjp ? MODE_DENS_HERM : MODE_FWD_HERM;
     // interleave systems so neighbouring workgroups mix large and small items
     std::stable_sort(items.begin(), items.end(), [](const int4& x, const int4& y) { return x.z < y.z; });
-    std::stable_sort(items_hi.begin(), items_hi.end(), [](const int4& x, const int4& y) { return x.z < y.z; });
+    items.insert(items.end(), spare.begin(), spare.end());
     if (!g.dargs[slot(mode)]) {
         void* p = nullptr;
         HIPCHK(hipMalloc(&p, sizeof(LatArgs) * args.size()));
@@ -250,22 +234,6 @@ int build_group(dmftgpu_batch_s* b, Group& g, int mode, int wg, double target)
     g.target[slot(mode)] = target;
     HIPCHK(hipMemcpy(g.dargs[slot(mode)], args.data(), sizeof(LatArgs) * args.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(g.ditems[slot(mode)], items.data(), sizeof(int4) * items.size(), hipMemcpyHostToDevice));
-    const int sl = slot(mode);
-    g.n_items_hi[sl] = (int)items_hi.size();
-    if (!g.dargs_hi[sl]) {
-        void* p = nullptr;
-        HIPCHK(hipMalloc(&p, sizeof(LatArgs) * args_hi.size()));
-        b->extra.push_back(p);
-        g.dargs_hi[sl] = (LatArgs*)p;
-    }
-    HIPCHK(hipMemcpy(g.dargs_hi[sl], args_hi.data(), sizeof(LatArgs) * args_hi.size(), hipMemcpyHostToDevice));
-    if (!items_hi.empty()) {
-        void* p = nullptr;
-        HIPCHK(hipMalloc(&p, sizeof(int4) * items_hi.size()));
-        b->extra.push_back(p);
-        g.ditems_hi[sl] = (int4*)p;
-        HIPCHK(hipMemcpy(g.ditems_hi[sl], items_hi.data(), sizeof(int4) * items_hi.size(), hipMemcpyHostToDevice));
-    }
     return DMFTGPU_OK;
 }
 
@@ -283,20 +251,11 @@ int launch_group(dmftgpu_batch_s* b, Group& g, int mode)
     m.n_items = g.n_items[slot(mode)];
     m.grid = std::min(g.n_items[slot(mode)], 256 * 16);
     m.max_nd = g.max_nd;
-    if (g.cols) {  // every frequency in the one list (no upper-half work list)
+    if (g.cols) {
         HIPCHK(dg::launch_lattice_schur_cols_multi(proto, mode, fp32, h->stream, m));
         return DMFTGPU_OK;
     }
     HIPCHK(dg::launch_lattice_schur_multi(proto, mode, fp32, h->stream, g.wg[slot(mode)], m));
-    if (g.n_items_hi[slot(mode)] > 0) {
-        SchurMulti mh = m;
-        mh.args = g.dargs_hi[slot(mode)];
-        mh.items = g.ditems_hi[slot(mode)];
-        mh.n_items = g.n_items_hi[slot(mode)];
-        mh.grid = std::min(mh.n_items, 256 * 16);
-        const int wg_hi = g.wg[slot(mode)] == dg::SCHUR_WG_KPAIR ? 64 : g.wg[slot(mode)];
-        HIPCHK(dg::launch_lattice_schur_multi(proto, g.mode_hi[slot(mode)], fp32, h->stream, wg_hi, mh));
-    }
     return DMFTGPU_OK;
 }
 
@@ -306,6 +265,8 @@ int issue_prepare(dmftgpu_batch_s* b)
     dmftgpu_handle h = b->h;
     for (Sys& s : b->sys) {
         HIPCHK(hipMemcpyAsync(s.mom, s.d.moments, sizeof(cd) * 4 * s.m2, hipMemcpyDeviceToDevice, h->stream));
+        HIPCHK(dg::launch_freq_points(s.mom, s.nc, s.nf, s.nw_tot, s.n_tail, s.tail, s.d.lat.beta, s.pt_n, s.pt_w, s.pt_wt,
+                                      h->stream));
         HIPCHK(dg::launch_herm_eig((const cd*)s.d.Hk, s.n, 0, s.n, s.mom, s.nc, s.ev, s.U, s.nk, h->stream));
         if (s.nd > 0) {
             HIPCHK(dg::launch_herm_eig((const cd*)s.d.Hk, s.n, s.nc, s.nd, nullptr, 0, s.ed, s.Vd, s.nk, h->stream));
@@ -351,9 +312,10 @@ int issue_step(dmftgpu_batch_s* b)
     }
     for (Sys& s : b->sys) {
         const double inv_nk = 1.0 / (double)s.d.lat.n_k_global;
-        HIPCHK(dg::launch_reduce_chunks(s.pTrF, s.chunks_f, s.nw_tot, s.trF, h->stream));
-        HIPCHK(dg::launch_reduce_chunks(s.pG, s.chunks_f, (size_t)s.nw_tot * s.m2, s.Gsum, h->stream));
-        HIPCHK(dg::launch_freq_totals(s.Gsum, s.m2, s.nc, s.trF, nullptr, s.nw_tot, nullptr, 0, s.tot_f, h->stream));
+        HIPCHK(dg::launch_reduce_chunks(s.pTrF, s.chunks_f, s.nw_tot, s.trF, h->stream, s.pt_n));
+        HIPCHK(dg::launch_reduce_chunks(s.pG, s.chunks_f, (size_t)s.nw_tot * s.m2, s.Gsum, h->stream, s.pt_n, s.m2));
+        HIPCHK(dg::launch_freq_totals(s.Gsum, s.m2, s.nc, s.trF, nullptr, s.nw_tot, nullptr, 0, s.tot_f, h->stream, s.pt_n,
+                                      s.pt_wt));
         HIPCHK(dg::launch_gloc_finalize(s.Gsum, s.nf, s.nc, s.d.lat.n_cluster, inv_nk, (cd*)s.d.gloc, h->stream));
         hipLaunchKernelGGL(k_fin_fwd, dim3(1), dim3(1024), 0, h->stream, s.tot_f, s.st, s.sts, s.m2, s.d.lat.beta,
                            inv_nk, (cd*)s.d.num_matrix, s.d.n_total);
@@ -373,12 +335,13 @@ int issue_step(dmftgpu_batch_s* b)
     }
     for (Sys& s : b->sys) {
         const double inv_nk = 1.0 / (double)s.d.lat.n_k_global;
-        HIPCHK(dg::launch_reduce_chunks(s.pTrV, s.chunks_v, s.nw_tot, s.trV, h->stream));
-        HIPCHK(dg::launch_reduce_chunks(s.pTr2, s.chunks_v, s.nw_tot, s.tr2, h->stream));
+        HIPCHK(dg::launch_reduce_chunks(s.pTrV, s.chunks_v, s.nw_tot, s.trV, h->stream, s.pt_n));
+        HIPCHK(dg::launch_reduce_chunks(s.pTr2, s.chunks_v, s.nw_tot, s.tr2, h->stream, s.pt_n));
         HIPCHK(dg::launch_reduce_chunks(s.pSb, s.chunks_v, (size_t)s.nf * s.m2, s.Sb, h->stream));
         HIPCHK(dg::launch_reduce_chunks(s.pMu, s.chunks_v, s.nf, s.musum, h->stream));
         HIPCHK(dg::launch_scale(s.Sb, (size_t)s.nf * s.m2, inv_nk, (cd*)s.d.sigma_bar, h->stream));
-        HIPCHK(dg::launch_freq_totals(nullptr, s.m2, s.nc, s.trV, s.tr2, s.nw_tot, s.musum, s.nf, s.tot_v, h->stream));
+        HIPCHK(dg::launch_freq_totals(nullptr, s.m2, s.nc, s.trV, s.tr2, s.nw_tot, s.musum, s.nf, s.tot_v, h->stream,
+                                      s.pt_n, s.pt_wt));
         hipLaunchKernelGGL(k_fin_vjp, dim3(1), dim3(1), 0, h->stream, s.tot_v, s.sts, s.m2, s.d.lat.beta, inv_nk,
                            s.nbar, s.d.mu_bar);
         HIPCHK(hipGetLastError());
@@ -437,71 +400,6 @@ int tune_group(dmftgpu_batch_s* b, Group& g, int mode)
     return build_group(b, g, mode, bw, bt);
 }
 
-// Forward and adjoint of a fused step share the k chunking (the forward writes the
-// adjoint's tr G^2 partials beyond N_freq), so one target is chosen for both: per
-// target the best workgroup width of each, the target with the least sum.
-int tune_group_pair(dmftgpu_batch_s* b, Group& g)
-{
-    dmftgpu_handle h = b->h;
-    const int wgs[3] = {64, 128, dg::SCHUR_WG_KPAIR};
-    const double targets[4] = {6.25e4, 2.5e5, 1.0e6, 4.0e6};
-    struct Events {  // destroyed on every return path
-        hipEvent_t e0 = nullptr, e1 = nullptr;
-        ~Events()
-        {
-            if (e0) (void)hipEventDestroy(e0);
-            if (e1) (void)hipEventDestroy(e1);
-        }
-    } ev;
-    HIPCHK(hipEventCreate(&ev.e0));
-    HIPCHK(hipEventCreate(&ev.e1));
-    double best_sum = 1e300, best_ms[2] = {0, 0};
-    int best_wg[2] = {64, 64};
-    double best_t = targets[2];
-    for (double t : targets) {
-        double ms_mode[2];
-        int wg_mode[2];
-        for (int mode : {MODE_FWD, MODE_VJP}) {
-            double bm = 1e300;
-            int bw = 64;
-            for (int wg : wgs) {
-                if (g.cols && wg != 64) continue;  // one width: a wavefront per workgroup
-                if (wg == dg::SCHUR_WG_KPAIR && !kpair_ok(b, g, mode)) continue;
-                int rc = build_group(b, g, mode, wg, t);
-                if (rc) return rc;
-                rc = launch_group(b, g, mode);  // warm-up
-                if (rc) return rc;
-                HIPCHK(hipEventRecord(ev.e0, h->stream));
-                rc = launch_group(b, g, mode);
-                if (rc) return rc;
-                HIPCHK(hipEventRecord(ev.e1, h->stream));
-                HIPCHK(hipEventSynchronize(ev.e1));
-                float ms = 0.f;
-                HIPCHK(hipEventElapsedTime(&ms, ev.e0, ev.e1));
-                if (ms < bm) {
-                    bm = ms;
-                    bw = wg;
-                }
-            }
-            ms_mode[slot(mode)] = bm;
-            wg_mode[slot(mode)] = bw;
-        }
-        if (ms_mode[0] + ms_mode[1] < best_sum) {
-            best_sum = ms_mode[0] + ms_mode[1];
-            best_t = t;
-            for (int q = 0; q < 2; ++q) {
-                best_ms[q] = ms_mode[q];
-                best_wg[q] = wg_mode[q];
-            }
-        }
-    }
-    g.ms[0] = best_ms[0];
-    g.ms[1] = best_ms[1];
-    int rc = build_group(b, g, MODE_FWD, best_wg[0], best_t);
-    if (rc) return rc;
-    return build_group(b, g, MODE_VJP, best_wg[1], best_t);
-}
-
 }  // namespace
 
 static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system* systems, int method, int flags);
@@ -544,6 +442,7 @@ static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system
     b->flags = flags;
     b->sys.resize(count);
     std::map<int, int> gidx;
+    std::vector<std::vector<double>> tails(count);  // frequency rules (freq_points.hip)
     size_t total = 0;
     for (int i = 0; i < count; ++i) {
         Sys& s = b->sys[i];
@@ -567,6 +466,9 @@ static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system
         s.nf = L.n_freq;
         s.nw_tot = L.n_freq * L.high_freq;
         s.m2 = s.nc * s.nc;
+        tails[i] = dg::freq_tail(s.nf, s.nw_tot);
+        s.n_tail = (int)tails[i].size() / 2;
+        s.n_plan = s.n_tail ? s.nf + s.n_tail : s.nw_tot;
         s.max_chunks = std::max(1, std::min(s.nk, 128));
         s.st_kpc = (s.nk + 255) / 256;
         s.st_chunks = (s.nk + s.st_kpc - 1) / s.st_kpc;
@@ -602,6 +504,7 @@ static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system
         t += rnd(16 * C * s.nf * s.m2) + rnd(16 * C * s.nf);
         t += 3 * rnd(16 * (size_t)s.nw_tot) + rnd(16 * (size_t)s.nw_tot * s.m2) + rnd(16 * (size_t)s.nf * s.m2) +
              rnd(16 * (size_t)s.nf);
+        t += rnd(8 * tails[i].size()) + 2 * rnd(8 * (size_t)s.nw_tot) + rnd(4);
         need[i] = t;
         total += t;
     }
@@ -649,7 +552,14 @@ static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system
         s.Gsum = (cd*)take(16 * (size_t)s.nw_tot * s.m2);
         s.Sb = (cd*)take(16 * (size_t)s.nf * s.m2);
         s.musum = (cd*)take(16 * (size_t)s.nf);
+        s.tail = (double*)take(8 * tails[i].size());
+        s.pt_w = (double*)take(8 * (size_t)s.nw_tot);
+        s.pt_wt = (double*)take(8 * (size_t)s.nw_tot);
+        s.pt_n = (int*)take(4);
+        if (s.n_tail)
+            HIPCHK(hipMemcpyAsync(s.tail, tails[i].data(), 8 * tails[i].size(), hipMemcpyHostToDevice, h->stream));
     }
+    HIPCHK(hipStreamSynchronize(h->stream));  // the rules are host temporaries
     int rc = issue_prepare(b);
     if (!rc) rc = issue_sigma_tables(b);
     if (rc) return rc;
@@ -674,7 +584,8 @@ static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system
             if (!rc) rc = issue_step(b);
             if (!rc && hipStreamSynchronize(h->stream) != hipSuccess) rc = fail(h, DMFTGPU_ERR_HIP, "tuning step");
             for (Group& g : b->groups)
-                if (!rc) rc = tune_group_pair(b, g);
+                for (int mode : {MODE_FWD, MODE_VJP})
+                    if (!rc) rc = tune_group(b, g, mode);
         }
         if (rc) return rc;
     }

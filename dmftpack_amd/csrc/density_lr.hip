@@ -50,7 +50,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NC <= 5 ? 2 
     // G_cc of the pass's frequencies, [w][i + b NC]; after the frequency loop
     // the same memory holds two 16 x 16 column-major work matrices
     __shared__ cd lds[PW * M2 > 512 ? PW * M2 : 512];
-    __shared__ double sW[PW];  // the pass's Matsubara frequencies
+    __shared__ double sW[PW], sWt[PW];  // the pass's frequencies and their weights
     cd* sG = lds;
     cd* sA = lds;
     cd* sB = lds + 256;
@@ -74,13 +74,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NC <= 5 ? 2 
 
     dv4 P1 = {0.0, 0.0, 0.0, 0.0}, P2 = P1, P3 = P1;
     cd gsum = cd{0.0, 0.0};
-    for (int w0 = 0; w0 < a.nw_tot; w0 += PW) {
+    const int npts = n_points(a);
+    for (int w0 = 0; w0 < npts; w0 += PW) {
         // ---- phase 1: G_cc of frequency w0 + lane (lane < PW)
         {
             const int nw = w0 + lane;
-            const bool wv = nw < a.nw_tot && lane < PW;
-            const int nwc = wv ? nw : a.nw_tot - 1;
-            const double w = matsubara(nwc, a.beta);
+            const bool wv = nw < npts && lane < PW;
+            const int nwc = wv ? nw : npts - 1;
+            const double w = a.pt_w ? a.pt_w[nwc] : matsubara(nwc, a.beta);
             const cd* sig = a.pSigAll + (size_t)nwc * M2;  // Sigma, moment tail beyond n_freq
             // sum_d g_d P_d = R + i J accumulated as in the Schur kernels:
             // G[a][b] = R_ab, G[b][a] = J_ab (a < b), G[a][a] = (R_aa, J_aa)
@@ -125,11 +126,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NC <= 5 ? 2 
                 }
             gj_inverse<NC>(G);
             if (lane < PW) {
+                // weight of the frequency in the sum (freq_points.hip): on G_cc here, which
+                // enters the product once, and on g_d in gsum
+                const double wt = wv ? (a.pt_wt ? a.pt_wt[nwc] : 1.0) : 0.0;
                 sW[lane] = w;
+                sWt[lane] = wt;
 #pragma unroll
                 for (int b = 0; b < NC; ++b)
 #pragma unroll
-                    for (int i = 0; i < NC; ++i) sG[lane * M2 + i + b * NC] = wv ? G[i][b] : cd{0.0, 0.0};
+                    for (int i = 0; i < NC; ++i) sG[lane * M2 + i + b * NC] = wv ? cscale(G[i][b], wt) : cd{0.0, 0.0};
             }
         }
         wave_sync();
@@ -141,7 +146,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NC <= 5 ? 2 
 #pragma unroll 1
         for (int t = 0; t < PW / 4; ++t) {
             const int wl = 4 * t + s;
-            const bool v2 = w0 + wl < a.nw_tot;
+            const bool v2 = w0 + wl < npts;
             const double w2 = sW[wl];
             const cd* Gs = sG + wl * M2;
             const double x = mu - e_j;
@@ -149,7 +154,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NC <= 5 ? 2 
             const double md = (jd && v2) ? 1.0 : 0.0;  // lane of a d column, valid frequency
             const double m1 = (j < NC && v2) ? 1.0 : 0.0;  // lane of a c column, valid frequency
             const cd g = cd{md * x * rr, -md * w2 * rr};
-            gsum = cadd(gsum, g);
+            gsum = cd{fma(sWt[wl], g.x, gsum.x), fma(sWt[wl], g.y, gsum.y)};
             const int jc = j < NC ? j : 0;
 #pragma unroll
             for (int q = 0; q < NC; ++q) {

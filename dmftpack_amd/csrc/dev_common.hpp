@@ -105,15 +105,14 @@ __device__ __forceinline__ void lds_add(cd* p, cd v)
 // Matsubara frequency w_n = pi(2n+1)/beta (GreenFtn.cpp:219).
 __device__ __forceinline__ double matsubara(int n, double beta) { return kPi * (2.0 * n + 1.0) / beta; }
 
-// Sigma(iw_n) element (i,j) for frequency index nw: SelfE_w for nw < n_freq,
+// Sigma(iw) element (i,j) for frequency point nw at w: SelfE_w for nw < n_freq,
 // otherwise the moment expansion m0 + m1/iw + m2/iw^2 + m3/iw^3
 // (GreenFtn.cpp:224-240).  Column-major nc x nc.
-__device__ __forceinline__ cd sigma_elem(const cd* __restrict__ sigma, const cd* __restrict__ mom, int nc, int n_freq,
-                                         double beta, int nw, int i, int j)
+__device__ __forceinline__ cd sigma_elem_at(const cd* __restrict__ sigma, const cd* __restrict__ mom, int nc,
+                                            int n_freq, double w, int nw, int i, int j)
 {
     const int e = i + j * nc;
     if (nw < n_freq) return sigma[(size_t)nw * nc * nc + e];
-    const double w = matsubara(nw, beta);
     // 1/iw = -i/w, 1/iw^2 = -1/w^2, 1/iw^3 = i/w^3
     const double r1 = 1.0 / w, r2 = r1 * r1, r3 = r2 * r1;
     const size_t m2 = (size_t)nc * nc;
@@ -123,6 +122,11 @@ __device__ __forceinline__ cd sigma_elem(const cd* __restrict__ sigma, const cd*
     v = cadd(v, cd{-mm2.x * r2, -mm2.y * r2});
     v = cadd(v, cd{-m3.y * r3, m3.x * r3});
     return v;
+}
+__device__ __forceinline__ cd sigma_elem(const cd* __restrict__ sigma, const cd* __restrict__ mom, int nc, int n_freq,
+                                         double beta, int nw, int i, int j)
+{
+    return sigma_elem_at(sigma, mom, nc, n_freq, matsubara(nw, beta), nw, i, j);
 }
 
 }  // namespace dg

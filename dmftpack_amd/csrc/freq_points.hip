@@ -1,0 +1,188 @@
+// Frequency points of the density sums (NumMatrix, N, dN/dmu, densityMatDFT).
+//
+// GreenFtn_w and GiwToNele sum over high_freq * N_freq Matsubara frequencies, and
+// beyond N_freq Sigma is its moment expansion (GreenFtn.cpp:224-240), so there the
+// summand f(w) (entries of G_cc, tr G, tr G^2) is an analytic function of w.  Its
+// sum over a run of frequencies w_a..w_b with w_b <= 2 w_a is taken by the Gauss
+// rule of the discrete measure itself: 16 points and positive weights that
+// integrate every polynomial in u = 1/w of degree <= 31 over that set exactly.
+//
+// Error: f is analytic where A(w) = (iw + mu) - H - P Sigma(w) P^H is invertible.
+// On the Bernstein ellipse rho = 4.5 around [1/w_b, 1/w_a] both Re w and |w| are
+// >= 0.746 w_a =: r, and the Hermitian part of -iA is >= r - s there, with s a bound
+// of |Sigma - Herm m0| (H and mu drop out: H is Hermitian).  k_freq_points takes
+// the rule only if s <= r/2, from the moments' Frobenius norms; then
+// |G| <= 2/r on the ellipse and the rule is off by <= 4.3 |f| rho^-32 < 1e-20 of
+// the sum, far below the rounding of adding the terms one by one.  Otherwise (short
+// grids at low temperature, moments that are not finite) every frequency is a point
+// with weight 1, as it is for a run of at most kGaussMin frequencies.
+//
+// What it gives: the kernels solve N_freq + 16 frequencies instead of 2 N_freq.
+// The plain method keeps every frequency (the reference's algorithm as it stands).
+#include <cmath>
+#include <vector>
+
+#include "lattice_kernels.hpp"
+
+namespace dg {
+
+namespace {
+
+// Gauss rule of the measure with unit mass at each t_n = 1/(2n+1), n0 <= n < n1:
+// x[i] = 1/node (a real-valued "2n+1"), w[i] its weight.  Stieltjes recurrence, then
+// implicit QL on the 16 x 16 Jacobi matrix (first eigenvector row only).  The sums over
+// the measure take 8 partial sums, which vectorise: 83 us of host time at 2048
+// frequencies, in dmftgpu_prepare under the eigensolvers; node and weight errors of a
+// few 1e-16.
+void gauss_rule(int n0, int n1, double* x, double* w)
+{
+    constexpr int m = kGaussPoints, V = 8;
+    const int len = n1 - n0, lv = (len + V - 1) / V * V;
+    const double hi = 1.0 / (2.0 * n0 + 1.0), lo = 1.0 / (2.0 * (n1 - 1) + 1.0);
+    std::vector<double> s(lv, 0.0), p0(lv, 0.0), p1(lv, 0.0);
+    for (int i = 0; i < len; ++i) {
+        // (2 t - lo - hi)/(hi - lo) as differences of t, which do not cancel at the ends
+        const double t = 1.0 / (2.0 * (n0 + i) + 1.0);
+        s[i] = ((t - lo) - (hi - t)) / (hi - lo);
+        p1[i] = 1.0 / std::sqrt((double)len);
+    }
+    double d[m], e[m], z[m], beta = 0.0;
+    for (int k = 0; k < m; ++k) {
+        double sa[V] = {}, sn[V] = {};
+        for (int i = 0; i < lv; i += V)
+            for (int v = 0; v < V; ++v) sa[v] += s[i + v] * p1[i + v] * p1[i + v];
+        const double al = ((sa[0] + sa[1]) + (sa[2] + sa[3])) + ((sa[4] + sa[5]) + (sa[6] + sa[7]));
+        for (int i = 0; i < lv; i += V)
+            for (int v = 0; v < V; ++v) {
+                const double q = (s[i + v] - al) * p1[i + v] - beta * p0[i + v];
+                p0[i + v] = p1[i + v];
+                p1[i + v] = q;
+                sn[v] += q * q;
+            }
+        beta = std::sqrt(((sn[0] + sn[1]) + (sn[2] + sn[3])) + ((sn[4] + sn[5]) + (sn[6] + sn[7])));
+        for (int i = 0; i < lv; ++i) p1[i] /= beta;
+        d[k] = al;
+        e[k] = beta;
+        z[k] = k == 0 ? 1.0 : 0.0;
+    }
+    e[m - 1] = 0.0;
+    for (int l = 0; l < m; ++l) {  // implicit QL, Wilkinson shift
+        for (int it = 0; it < 60; ++it) {
+            int q = l;
+            for (; q < m - 1; ++q)
+                if (std::fabs(e[q]) <= 1e-17 * (std::fabs(d[q]) + std::fabs(d[q + 1]))) break;
+            if (q == l) break;
+            double g = (d[l + 1] - d[l]) / (2.0 * e[l]);
+            double r = std::hypot(g, 1.0);
+            g = d[q] - d[l] + e[l] / (g + (g >= 0.0 ? r : -r));
+            double sn = 1.0, cs = 1.0, p = 0.0;
+            int i = q - 1;
+            for (; i >= l; --i) {
+                double f = sn * e[i];
+                const double b = cs * e[i];
+                r = std::hypot(f, g);
+                e[i + 1] = r;
+                if (r == 0.0) {
+                    d[i + 1] -= p;
+                    e[q] = 0.0;
+                    break;
+                }
+                sn = f / r;
+                cs = g / r;
+                g = d[i + 1] - p;
+                r = (d[i] - g) * sn + 2.0 * cs * b;
+                p = sn * r;
+                d[i + 1] = g + p;
+                g = cs * r - b;
+                f = z[i + 1];
+                z[i + 1] = sn * z[i] + cs * f;
+                z[i] = cs * z[i] - sn * f;
+            }
+            if (r == 0.0 && i >= l) continue;
+            d[l] -= p;
+            e[l] = g;
+            e[q] = 0.0;
+        }
+    }
+    double zz = 0.0;
+    for (int i = 0; i < m; ++i) zz += z[i] * z[i];
+    for (int i = 0; i < m; ++i) {
+        x[i] = 2.0 / (d[i] * (hi - lo) + hi + lo);
+        w[i] = z[i] * z[i] / zz * len;
+    }
+}
+
+// The point table: the first n_freq Matsubara frequencies, then the Gauss points
+// (rule) or the remaining frequencies.  One workgroup; n_pts, pt_w, pt_wt as in LatArgs.
+__global__ __launch_bounds__(256) void k_freq_points(const cd* __restrict__ mom, int nc, int n_freq, int nw_tot,
+                                                     int n_tail, const double* __restrict__ tail, double beta,
+                                                     int* __restrict__ n_pts, double* __restrict__ pt_w,
+                                                     double* __restrict__ pt_wt)
+{
+    __shared__ double red[4][256];
+    const int m2 = nc * nc, t0 = threadIdx.x;
+    double nrm[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int e = t0; e < m2; e += 256) {
+        const cd a = mom[e], b = mom[e / nc + (e % nc) * nc];
+        const double ax = 0.5 * (a.x - b.x), ay = 0.5 * (a.y + b.y);  // anti-Hermitian part of m0
+        nrm[0] += ax * ax + ay * ay;
+        for (int q = 1; q < 4; ++q) {
+            const cd m = mom[(size_t)q * m2 + e];
+            nrm[q] += m.x * m.x + m.y * m.y;
+        }
+    }
+    for (int q = 0; q < 4; ++q) red[q][t0] = nrm[q];
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if (t0 < o)
+            for (int q = 0; q < 4; ++q) red[q][t0] += red[q][t0 + o];
+        __syncthreads();
+    }
+    const double r = 0.746 * matsubara(n_freq, beta), ir = 1.0 / r;
+    const double s = sqrt(red[0][0]) + ir * (sqrt(red[1][0]) + ir * (sqrt(red[2][0]) + ir * sqrt(red[3][0])));
+    const bool rule = n_tail > 0 && s <= 0.5 * r;  // false for NaN
+    const int np = rule ? n_freq + n_tail : nw_tot;
+    if (t0 == 0) *n_pts = np;
+    for (int i = t0; i < np; i += 256) {
+        const bool node = rule && i >= n_freq;
+        pt_w[i] = node ? kPi * tail[i - n_freq] / beta : matsubara(i, beta);
+        pt_wt[i] = node ? tail[n_tail + i - n_freq] : 1.0;
+    }
+}
+
+}  // namespace
+
+std::vector<double> freq_tail(int n_freq, int nw_tot)
+{
+    std::vector<double> x, w;
+    bool any = false;
+    for (int a = n_freq; a < nw_tot;) {
+        // w_b <= 2 w_a holds up to n = 2a; runs of at most kGaussMin are listed as they are
+        const int b = nw_tot - a <= a ? nw_tot : 2 * a;
+        if (b - a > kGaussMin) {
+            x.resize(x.size() + kGaussPoints);
+            w.resize(w.size() + kGaussPoints);
+            gauss_rule(a, b, x.data() + x.size() - kGaussPoints, w.data() + w.size() - kGaussPoints);
+            any = true;
+        } else {
+            for (int n = a; n < b; ++n) {
+                x.push_back(2.0 * n + 1.0);
+                w.push_back(1.0);
+            }
+        }
+        a = b;
+    }
+    if (!any) return {};
+    x.insert(x.end(), w.begin(), w.end());
+    return x;
+}
+
+hipError_t launch_freq_points(const cd* mom, int nc, int n_freq, int nw_tot, int n_tail, const double* tail,
+                              double beta, int* n_pts, double* pt_w, double* pt_wt, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_freq_points, dim3(1), dim3(256), 0, s, mom, nc, n_freq, nw_tot, n_tail, tail, beta, n_pts,
+                       pt_w, pt_wt);
+    return hipGetLastError();
+}
+
+}  // namespace dg

@@ -250,21 +250,24 @@ constexpr int kRedX = 32, kRedY = 8;
 
 template <class T>
 __global__ __launch_bounds__(kRedX* kRedY) void k_reduce_chunks(const T* __restrict__ part, int n_chunks, size_t len,
-                                                                 T* __restrict__ out)
+                                                                 T* __restrict__ out, const int* __restrict__ n_pts,
+                                                                 int per)
 {
     __shared__ T red[kRedY][kRedX];
+    const size_t lim = n_pts ? (size_t)*n_pts * per : len;
+    if ((size_t)blockIdx.x * kRedX >= lim) return;
     const int tx = threadIdx.x % kRedX, ty = threadIdx.x / kRedX;
     const size_t i = (size_t)blockIdx.x * kRedX + tx;
     const int c0 = (int)((long long)n_chunks * ty / kRedY);
     const int c1 = (int)((long long)n_chunks * (ty + 1) / kRedY);
     T acc{};
-    if (i < len) {
+    if (i < lim) {
 #pragma unroll 4
         for (int c = c0; c < c1; ++c) acc = radd(acc, part[(size_t)c * len + i]);
     }
     red[ty][tx] = acc;
     __syncthreads();
-    if (ty == 0 && i < len) {
+    if (ty == 0 && i < lim) {
         T sum = red[0][tx];
         for (int y = 1; y < kRedY; ++y) sum = radd(sum, red[y][tx]);
         out[i] = sum;
@@ -272,17 +275,19 @@ __global__ __launch_bounds__(kRedX* kRedY) void k_reduce_chunks(const T* __restr
 }
 
 template <class T>
-static hipError_t launch_reduce(const T* part, int n_chunks, size_t len, T* out, hipStream_t s)
+static hipError_t launch_reduce(const T* part, int n_chunks, size_t len, T* out, hipStream_t s,
+                                const int* n_pts = nullptr, int per = 1)
 {
     if (len == 0) return hipSuccess;
     hipLaunchKernelGGL(k_reduce_chunks<T>, dim3((unsigned)((len + kRedX - 1) / kRedX)), dim3(kRedX * kRedY), 0, s,
-                       part, n_chunks, len, out);
+                       part, n_chunks, len, out, n_pts, per);
     return hipGetLastError();
 }
 
-hipError_t launch_reduce_chunks(const cd* part, int n_chunks, size_t len, cd* out, hipStream_t s)
+hipError_t launch_reduce_chunks(const cd* part, int n_chunks, size_t len, cd* out, hipStream_t s, const int* n_pts,
+                                int per)
 {
-    return launch_reduce(part, n_chunks, len, out, s);
+    return launch_reduce(part, n_chunks, len, out, s, n_pts, per);
 }
 
 hipError_t launch_reduce_chunks_d(const double* part, int n_chunks, size_t len, double* out, hipStream_t s)
@@ -295,26 +300,30 @@ hipError_t launch_reduce_chunks_d(const double* part, int n_chunks, size_t len, 
 // m2+2 -> sum Re mu.  Fixed-order block reduction.
 __global__ __launch_bounds__(256) void k_freq_totals(const cd* __restrict__ G, int m2, int nc,
                                                      const cd* __restrict__ tr, const cd* __restrict__ tr2, int nw_tot,
-                                                     const cd* __restrict__ mu, int n_mu, cd* __restrict__ out)
+                                                     const cd* __restrict__ mu, int n_mu, cd* __restrict__ out,
+                                                     const int* __restrict__ n_pts, const double* __restrict__ pt_wt)
 {
     __shared__ double rx[256], ry[256];
     const int q = blockIdx.x;
     double ax = 0.0, ay = 0.0;
+    if (n_pts) nw_tot = *n_pts;
+    auto wt = [&](int nw) { return pt_wt ? pt_wt[nw] : 1.0; };
     if (q < m2) {
         if (G) {
             const int i = q % nc, j = q / nc, et = j + i * nc;
             for (int nw = threadIdx.x; nw < nw_tot; nw += 256) {
                 const cd g = G[(size_t)nw * m2 + q], gt = G[(size_t)nw * m2 + et];
-                ax += g.x + gt.x;
-                ay += g.y - gt.y;
+                const double f = wt(nw);
+                ax = fma(f, g.x + gt.x, ax);
+                ay = fma(f, g.y - gt.y, ay);
             }
         }
     } else if (q == m2) {
         if (tr)
-            for (int nw = threadIdx.x; nw < nw_tot; nw += 256) ax += 2.0 * tr[nw].x;
+            for (int nw = threadIdx.x; nw < nw_tot; nw += 256) ax = fma(2.0 * wt(nw), tr[nw].x, ax);
     } else if (q == m2 + 1) {
         if (tr2)
-            for (int nw = threadIdx.x; nw < nw_tot; nw += 256) ax += 2.0 * tr2[nw].x;
+            for (int nw = threadIdx.x; nw < nw_tot; nw += 256) ax = fma(2.0 * wt(nw), tr2[nw].x, ax);
     } else {
         if (mu)
             for (int nw = threadIdx.x; nw < n_mu; nw += 256) ax += mu[nw].x;
@@ -333,9 +342,10 @@ __global__ __launch_bounds__(256) void k_freq_totals(const cd* __restrict__ G, i
 }
 
 hipError_t launch_freq_totals(const cd* G, int m2, int nc, const cd* tr, const cd* tr2, int nw_tot, const cd* mu,
-                              int n_mu, cd* out, hipStream_t s)
+                              int n_mu, cd* out, hipStream_t s, const int* n_pts, const double* pt_wt)
 {
-    hipLaunchKernelGGL(k_freq_totals, dim3(m2 + 3), dim3(256), 0, s, G, m2, nc, tr, tr2, nw_tot, mu, n_mu, out);
+    hipLaunchKernelGGL(k_freq_totals, dim3(m2 + 3), dim3(256), 0, s, G, m2, nc, tr, tr2, nw_tot, mu, n_mu, out, n_pts,
+                       pt_wt);
     return hipGetLastError();
 }
 

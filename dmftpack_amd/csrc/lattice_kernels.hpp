@@ -3,19 +3,13 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <vector>
+
 #include "dev_common.hpp"
 
 namespace dg {
 
 enum LatMode { MODE_FWD = 0, MODE_DENS = 1, MODE_VJP = 2 };
-// One-matrix-per-lane kernels only: the forward over frequencies n >= N_freq,
-// whose G_cc enters NumMatrix alone (through G + G^H), accumulates the
-// Hermitian part (G + G^H)/2 (n_c^2 reals instead of n_c^2 complex).
-constexpr int MODE_FWD_HERM = 3;
-// The same Hermitian-part forward fused with the density terms (tr G^2): when an
-// adjoint follows at the same (Sigma, mu), the frequencies beyond N_freq are done
-// once, in the forward, instead of once there and once in the adjoint.
-constexpr int MODE_DENS_HERM = 4;
 // One-matrix-per-lane kernels only: the forward on the real axis (retarded_GreenFtn2),
 // frequency point nw being z = e0 + nw de + i eta (freq_point)
 constexpr int MODE_FWD_REAL = 5;
@@ -144,10 +138,30 @@ struct LatArgs {
     double e0, de, eta;
     // per-k blocks of the one-matrix-per-lane Schur kernels [nk][schur_kdata_size]
     const cd* kdata;
-    // one-matrix-per-lane Schur kernels: frequency range [nw_begin, nw_end) of
-    // this launch (nw_end = 0: up to nw_tot); partial sums keep the nw_tot stride
-    int nw_begin, nw_end;
+    // Frequency points of the density sums (freq_points.hip; Schur methods on the
+    // Matsubara axis): *pt_n points, frequency pt_w[nw] with weight pt_wt[nw] in the
+    // frequency sums, the first n_freq being the Matsubara ones.  Null: the nw_tot
+    // Matsubara (or real-axis) points, weight 1.  Arrays keep the nw_tot stride.
+    const int* pt_n;
+    const double* pt_w;
+    const double* pt_wt;
+    int n_plan;  // points the host plans for (*pt_n is n_plan or nw_tot); 0: nw_tot
 };
+
+// Grid of a lattice launch over tiles of fw points: (tiles of the planned points,
+// k chunks, layers), layer z holding tiles x + gridDim.x z.  Layers z > 0 have work
+// only when the moments rule the planned points out and return at once otherwise.  As
+// the slowest index they come after all work: interleaved with it (a plain grid over
+// nw_tot) they left half the CUs idle, workgroups being dealt to the shader engines
+// in turn (adjoint at n_c = 5, 33 of 64 tiles: 29.9 ms against 15.4 ms in layers).
+inline dim3 lattice_grid(const LatArgs& a, int fw)
+{
+    const int tp = ((a.n_plan ? a.n_plan : a.nw_tot) + fw - 1) / fw, tt = (a.nw_tot + fw - 1) / fw;
+    return dim3(tp, a.n_chunks, (tt + tp - 1) / tp);
+}
+__device__ __forceinline__ int lattice_tile() { return blockIdx.x + gridDim.x * blockIdx.z; }
+
+__device__ __forceinline__ int n_points(const LatArgs& a) { return a.pt_n ? *a.pt_n : a.nw_tot; }
 
 // (real shift added to mu, imaginary part) of frequency point nw
 __device__ __forceinline__ void freq_point(const LatArgs& a, int nw, double& mu, double& w)
@@ -157,9 +171,22 @@ __device__ __forceinline__ void freq_point(const LatArgs& a, int nw, double& mu,
         w = a.eta;
     } else {
         mu = a.mu;
-        w = matsubara(nw, a.beta);
+        w = a.pt_w ? a.pt_w[nw] : matsubara(nw, a.beta);
     }
 }
+
+// Gauss rule of the density sums beyond n_freq (freq_points.hip): points per run of
+// frequencies, and the longest run that is summed as it is.  A launch covers the
+// points in tiles of 64 (or 6) lanes, so a run of 32 costs what the rule costs.
+constexpr int kGaussPoints = 16;
+constexpr int kGaussMin = 32;
+// The rule for n_freq <= n < nw_tot: [x..., weight...] with frequency pi x / beta, or
+// empty where no run is long enough.  Depends on the two counts only.
+std::vector<double> freq_tail(int n_freq, int nw_tot);
+// Point table (pt_n, pt_w, pt_wt of LatArgs; pt_w and pt_wt hold nw_tot entries) from
+// the tail rule (n_tail points, device copy) and Sigma's tail moments
+hipError_t launch_freq_points(const cd* mom, int nc, int n_freq, int nw_tot, int n_tail, const double* tail,
+                              double beta, int* n_pts, double* pt_w, double* pt_wt, hipStream_t s);
 
 // plain FP64 full inverse; returns 0 or a HIP error
 hipError_t launch_lattice_plain(const LatArgs& a, int mode, hipStream_t s, int* wtile_out);
@@ -173,21 +200,16 @@ hipError_t launch_density_matrix_lr(const LatArgs& a, const cd* W, const cd* Vd,
 
 // Schur complement (FP64 or FP32 + refinement); wg = workgroup width of the
 // one-matrix-per-lane kernels: 64 or 128 frequencies, or 0 for the default of
-// each launch (the FP32R forward over the first n_freq frequencies in
-// SCHUR_WG_KPAIR form, the adjoint at 128, the others at 64); cols selects the
-// column-per-lane kernels for n_c <= 6 (always used above 6)
-// fused (one-matrix-per-lane kernels, schur_can_fuse): a forward that also
-// writes tr G^2 (a.pTr2) beyond n_freq, and the adjoint at the same (Sigma, mu)
-// that then covers the first n_freq frequencies only (same k chunking).
+// each launch (the FP32R forward at n_c >= 5 in SCHUR_WG_KPAIR form, the adjoint at
+// 128, the others at 64); cols selects the column-per-lane kernels for n_c <= 6
+// (always used above 6)
 // wg value of the FP32R forward kernel (n_c >= 5) as two wavefronts over 64
 // frequencies, each walking every other k of the chunk into shared LDS
 // accumulators (half the LDS per wavefront of the 64-lane form); its work items
 // cover 64 frequencies
 constexpr int SCHUR_WG_KPAIR = 1;
-hipError_t launch_lattice_schur(const LatArgs& a, int mode, bool fp32, hipStream_t s, int wg = 64, bool cols = false,
-                                bool fused = false);
-bool schur_can_fuse(int nc, bool cols, bool real_axis);
-// Sigma expanded over all nw_tot frequencies into a.pSigAll
+hipError_t launch_lattice_schur(const LatArgs& a, int mode, bool fp32, hipStream_t s, int wg = 64, bool cols = false);
+// Sigma expanded over all frequency points into a.pSigAll
 hipError_t launch_sigma_all(const LatArgs& a, hipStream_t s);
 // Persistent launch over a work list of several lattices sharing n_c (and mode,
 // precision, refinement): args [systems] in device memory, items {system,
@@ -269,7 +291,9 @@ hipError_t launch_gloc_hf(const double* ev, const cd* U, int n, int nc, int nk, 
                           double inv_nkg, int n_cluster, cd* out, hipStream_t s);
 
 // Deterministic reductions over chunks: out[i] = sum_c part[c*len + i]
-hipError_t launch_reduce_chunks(const cd* part, int n_chunks, size_t len, cd* out, hipStream_t s);
+// (n_pts, optional: only the first *n_pts * per entries of each chunk are summed)
+hipError_t launch_reduce_chunks(const cd* part, int n_chunks, size_t len, cd* out, hipStream_t s,
+                                const int* n_pts = nullptr, int per = 1);
 hipError_t launch_reduce_chunks_d(const double* part, int n_chunks, size_t len, double* out, hipStream_t s);
 
 // Final reductions over frequency: for FWD/DENS/VJP totals.
@@ -277,9 +301,11 @@ hipError_t launch_reduce_chunks_d(const double* part, int n_chunks, size_t len, 
 //   sumTr    = sum_nw 2 Re tr[nw]
 //   sumTr2   = sum_nw 2 Re tr2[nw]                          if tr2 != null
 //   sumMu    = sum_nw Re mu[nw] over n_mu entries           if mu != null
-// out layout: [m2 complex] [3 doubles as complex .x]
+// out layout: [m2 complex] [3 doubles as complex .x].  With n_pts the sums run over
+// *n_pts points, each term weighted by pt_wt[nw].
 hipError_t launch_freq_totals(const cd* G, int m2, int nc, const cd* tr, const cd* tr2, int nw_tot, const cd* mu,
-                              int n_mu, cd* out, hipStream_t s);
+                              int n_mu, cd* out, hipStream_t s, const int* n_pts = nullptr,
+                              const double* pt_wt = nullptr);
 
 // gloc[nw][e] = Gsum[nw][e] * scale for nw < n_freq, zero outside cluster blocks
 hipError_t launch_gloc_finalize(const cd* Gsum, int n_freq, int nc, int n_cluster, double scale, cd* gloc,

@@ -37,38 +37,34 @@ static hipError_t dispatch_nc(const LatArgs& a, int mode, bool fp32, const cd* s
     }
 }
 
-// Sigma at every frequency of the density sum (moment tail beyond n_freq)
-__global__ void k_sigma_all(const cd* __restrict__ sigma, const cd* __restrict__ mom, int nc, int n_freq, int nw_tot,
-                            double beta, cd* __restrict__ out)
+// Sigma at every frequency point of the density sum (moment tail beyond n_freq)
+__global__ void k_sigma_all(LatArgs a)
 {
-    const int m2 = nc * nc;
+    const int m2 = a.nc * a.nc;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nw_tot * m2) return;
     const int nw = t / m2, e = t % m2;
-    out[t] = sigma_elem(sigma, mom, nc, n_freq, beta, nw, e % nc, e / nc);
+    if (nw >= n_points(a)) return;
+    const double w = a.pt_w ? a.pt_w[nw] : matsubara(nw, a.beta);
+    a.pSigAll[t] = sigma_elem_at(a.sigma, a.mom, a.nc, a.n_freq, w, nw, e % a.nc, e / a.nc);
 }
 
 hipError_t launch_sigma_all(const LatArgs& a, hipStream_t s)
 {
     const int m2 = a.nc * a.nc;
-    hipLaunchKernelGGL(k_sigma_all, dim3((a.nw_tot * m2 + 255) / 256), dim3(256), 0, s, a.sigma, a.mom, a.nc, a.n_freq,
-                       a.nw_tot, a.beta, a.pSigAll);
+    hipLaunchKernelGGL(k_sigma_all, dim3((a.nw_tot * m2 + 255) / 256), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
-bool schur_can_fuse(int nc, bool cols, bool real_axis) { return nc >= 1 && nc <= 6 && !cols && !real_axis; }
-
-hipError_t launch_lattice_schur(const LatArgs& a, int mode, bool fp32, hipStream_t s, int wg, bool cols, bool fused)
+hipError_t launch_lattice_schur(const LatArgs& a, int mode, bool fp32, hipStream_t s, int wg, bool cols)
 {
-    if (fused && !schur_can_fuse(a.nc, cols, a.real_axis)) return hipErrorInvalidValue;
     // wg = 0: the adjoint call at 128 frequencies per workgroup (its one wavefront
     // per SIMD gains from a second sharing each per-k scalar fill), the FP32R
-    // forward over the first n_freq frequencies at n_c >= 5 as two wavefronts
-    // splitting the k walk over 64 frequencies (its LDS accumulators, n_c^2 x 1 KB
-    // per 64 frequencies, then allow the 8 wavefronts per CU that its registers
-    // allow, against 6 at n_c = 5 and 4 at n_c = 6), the other launches at 64
+    // forward at n_c >= 5 as two wavefronts splitting the k walk over 64 frequencies
+    // (its LDS accumulators, n_c^2 x 1 KB per 64 frequencies, then allow the 8
+    // wavefronts per CU that its registers allow, against 6 at n_c = 5 and 4 at
+    // n_c = 6), the other launches at 64
     const int wg_call = wg ? wg : mode == MODE_VJP ? 128 : 64;
-    const int wg_lo = wg ? wg : mode == MODE_FWD && fp32 && a.nc >= 5 ? SCHUR_WG_KPAIR : wg_call;
+    const int wg_fwd = wg ? wg : mode == MODE_FWD && fp32 && a.nc >= 5 ? SCHUR_WG_KPAIR : wg_call;
     hipError_t e = launch_sigma_all(a, s);
     if (e != hipSuccess) return e;
     if (a.real_axis && mode == MODE_FWD && a.nc <= 6 && !cols)
@@ -84,28 +80,7 @@ hipError_t launch_lattice_schur(const LatArgs& a, int mode, bool fp32, hipStream
             default: return launch_cols_16(a, mode, fp32, a.pSigAll, s);
         }
     }
-    if (mode == MODE_FWD && a.nw_tot > a.n_freq) {
-        // Frequencies beyond n_freq enter NumMatrix (and N) only: the Hermitian
-        // part of G_cc is accumulated there, half the accumulators.
-        LatArgs lo = a, hi = a;
-        lo.nw_end = a.n_freq;
-        hi.nw_begin = a.n_freq;
-        e = dispatch_nc(lo, MODE_FWD, fp32, a.pSigAll, s, wg_lo, nullptr);
-        if (e != hipSuccess) return e;
-        // fused: the adjoint that follows needs tr G^2 there too (a.pTr2)
-        return dispatch_nc(hi, fused ? MODE_DENS_HERM : MODE_FWD_HERM, fp32, a.pSigAll, s, wg_call, nullptr);
-    }
-    if (mode == MODE_VJP && a.nw_tot > a.n_freq) {
-        // Frequencies beyond n_freq contribute only tr G and tr G^2 (dN/dmu):
-        // the density kernel does that at twice the occupancy of the adjoint.
-        LatArgs lo = a, hi = a;
-        lo.nw_end = a.n_freq;
-        hi.nw_begin = a.n_freq;
-        e = dispatch_nc(lo, MODE_VJP, fp32, a.pSigAll, s, wg_call, nullptr);
-        if (e != hipSuccess || fused) return e;  // fused: the forward wrote tr G^2 beyond n_freq
-        return dispatch_nc(hi, MODE_DENS, fp32, a.pSigAll, s, wg_call, nullptr);
-    }
-    return dispatch_nc(a, mode, fp32, a.pSigAll, s, wg_lo, nullptr);
+    return dispatch_nc(a, mode, fp32, a.pSigAll, s, wg_fwd, nullptr);
 }
 
 hipError_t launch_lattice_schur_multi(const LatArgs& proto, int mode, bool fp32, hipStream_t s, int wg,

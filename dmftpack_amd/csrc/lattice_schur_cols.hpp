@@ -92,9 +92,11 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
     cd* MA = gsh + 32;
     cd* MB = MA + N * N;
     cd* GB = MB + N * N;
+    const int npts = n_points(a);
+    if (wtile * SLOTS >= npts) return;  // tile past the last frequency point
     const int nw = wtile * SLOTS + wave * SPW + (active ? sl : 0);
-    const bool wvalid = active && nw < a.nw_tot;
-    const int nwc = nw < a.nw_tot ? nw : a.nw_tot - 1;
+    const bool wvalid = active && nw < npts;
+    const int nwc = nw < npts ? nw : npts - 1;
     const int k0 = chunk * a.k_per_chunk;
     const int k1 = min(a.nk, k0 + a.k_per_chunk);
     double mu, w;
@@ -398,7 +400,7 @@ template <int N, int MODE, int PREC, bool TRACE>
 __global__ __launch_bounds__(cols_wg(MODE, PREC)) void k_lattice_schur_cols(LatArgs a, const cd* __restrict__ sig_all)
 {
     extern __shared__ cd lds[];
-    cols_item<N, MODE, PREC, TRACE>(a, sig_all, blockIdx.x, blockIdx.y, lds);
+    cols_item<N, MODE, PREC, TRACE>(a, sig_all, lattice_tile(), blockIdx.y, lds);
 }
 
 // Persistent form over a work list spanning several lattices with n_c in this
@@ -437,7 +439,7 @@ hipError_t launch_cols_k(const LatArgs& a, const cd* sig_all, hipStream_t s, con
     hipError_t e = hipFuncSetAttribute((const void*)k_lattice_schur_cols<N, MODE, PREC, TRACE>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
     if (e != hipSuccess) return e;
-    dim3 grid((a.nw_tot + SLOTS - 1) / SLOTS, a.n_chunks);
+    const dim3 grid = lattice_grid(a, SLOTS);
     hipLaunchKernelGGL((k_lattice_schur_cols<N, MODE, PREC, TRACE>), grid, dim3(cols_wg(MODE, PREC)), shm, s, a,
                        sig_all);
     return hipGetLastError();

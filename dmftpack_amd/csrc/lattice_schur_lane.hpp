@@ -167,24 +167,25 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
     using BD = kconst_double;
     constexpr int NP = NC * (NC + 1) / 2;
     constexpr int M2 = NC * NC;
-    constexpr bool HERM = MODE == MODE_FWD_HERM || MODE == MODE_DENS_HERM;
-    constexpr bool FWDLIKE = MODE == MODE_FWD || MODE == MODE_FWD_HERM || MODE == MODE_FWD_REAL;
+    constexpr bool FWDLIKE = MODE == MODE_FWD || MODE == MODE_FWD_REAL;
     // accumulators that do not fit next to the working matrices live in LDS
-    constexpr bool ACC_LDS = (MODE == MODE_VJP) || (MODE == MODE_DENS_HERM) || (FWDLIKE && F32R);
+    constexpr bool ACC_LDS = (MODE == MODE_VJP) || (FWDLIKE && F32R);
     constexpr int FW = WG / KS;       // frequencies per workgroup
     static_assert(KS == 1 || (KS == 2 && MODE == MODE_FWD && ACC_LDS && FW % 64 == 0),
                   "k pairs: LDS-accumulating forward, whole wavefronts per part");
     const int nd = a.n - NC;
     const int bs = kblock_size<NC>(nd);
     cd* sAcc = lds;                   // [M2][FW] complex, frequency-contiguous
-    double* sAccH = (double*)lds;     // HERM: [M2][FW] reals
     cd* sTr = lds + M2 * FW;          // KS > 1: [FW] sums of the tr G shares
     const int lane = KS == 1 ? (int)threadIdx.x : (int)threadIdx.x % FW;  // this lane's frequency in the tile
     // which k of every KS: wave-uniform (FW is a multiple of 64), so that the k
     // walk and the per-k block addresses stay scalar
     const int part = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / FW);
-    const int nw_hi = a.nw_end ? a.nw_end : a.nw_tot;
-    const int nw = a.nw_begin + wtile * FW + lane;
+    const int nw_hi = n_points(a);
+    const int nw = wtile * FW + lane;
+    // a wavefront past the last point has no work (KS > 1: both parts of a
+    // workgroup hold the same frequencies, so they leave together)
+    if (__builtin_amdgcn_readfirstlane(nw) >= nw_hi) return;
     const bool wvalid = nw < nw_hi;
     const int nwc = wvalid ? nw : nw_hi - 1;  // clamp for loads
     const int k0 = chunk * a.k_per_chunk;
@@ -194,7 +195,7 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
     if constexpr (MODE == MODE_FWD_REAL) {
         freq_point(a, nwc, mu, w);
     } else {
-        w = matsubara(nwc, a.beta);
+        w = a.pt_w ? a.pt_w[nwc] : matsubara(nwc, a.beta);
         mu = a.mu;
     }
     const bool vjp_here = (MODE == MODE_VJP) && wvalid && nw < a.n_freq;
@@ -203,18 +204,8 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
     // nbar: host value, or (batched adjoint) a device scalar written by an earlier kernel
     const double cn = 2.0 * (a.nbar_dev ? *a.nbar_dev : a.nbar) / a.beta;
 
-    cd acc[ACC_LDS || HERM ? 1 : NC][ACC_LDS || HERM ? 1 : NC];
-    // HERM: sums of Re G_ii and, for i < j, of (G_ij + G_ji).x, (G_ij - G_ji).y,
-    // in the order (j ascending, i <= j ascending)
-    double accH[HERM && !ACC_LDS ? M2 : 1];
-    if (HERM) {
-        if (ACC_LDS) {
-            for (int e = 0; e < M2; ++e) sAccH[e * FW + lane] = 0.0;
-        } else {
-#pragma unroll
-            for (int e = 0; e < (HERM && !ACC_LDS ? M2 : 1); ++e) accH[e] = 0.0;
-        }
-    } else if (ACC_LDS) {
+    cd acc[ACC_LDS ? 1 : NC][ACC_LDS ? 1 : NC];
+    if (ACC_LDS) {
         // (KS > 1: every part clears the same entries, before the barrier below)
         for (int e = 0; e < M2; ++e) sAcc[e * FW + lane] = cd{0.0, 0.0};
         if constexpr (KS > 1) {
@@ -395,27 +386,8 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
             }
         }
 
-        if constexpr (HERM) {  // Hermitian-part accumulation (before G is folded below)
-            int q = 0;
-#pragma unroll
-            for (int j = 0; j < NC; ++j)
-#pragma unroll
-                for (int i = 0; i <= j; ++i) {
-                    const double h0 = i == j ? G[i][i].x : G[i][j].x + G[j][i].x;
-                    const double h1 = G[i][j].y - G[j][i].y;
-                    if (ACC_LDS) {
-                        lds_add(&sAccH[q * FW + lane], h0);
-                        if (i != j) lds_add(&sAccH[(q + 1) * FW + lane], h1);
-                    } else {
-                        accH[q] += h0;
-                        if (i != j) accH[q + 1] += h1;
-                    }
-                    q += i == j ? 1 : 2;
-                }
-        }
         if (FWDLIKE) {
-            if constexpr (HERM) {
-            } else if (ACC_LDS) {
+            if constexpr (ACC_LDS) {
                 auto add_g = [&]() {
 #pragma unroll
                     for (int j = 0; j < NC; ++j)
@@ -434,9 +406,9 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                 }
             } else {
 #pragma unroll
-                for (int i = 0; i < (ACC_LDS || HERM ? 1 : NC); ++i)
+                for (int i = 0; i < (ACC_LDS ? 1 : NC); ++i)
 #pragma unroll
-                    for (int j = 0; j < (ACC_LDS || HERM ? 1 : NC); ++j) acc[i][j] = cadd(acc[i][j], G[i][j]);
+                    for (int j = 0; j < (ACC_LDS ? 1 : NC); ++j) acc[i][j] = cadd(acc[i][j], G[i][j]);
             }
             if (TRACE) {  // tr G = sum_d g_d + tr G_cc + sum_d g_d^2 M_d
                 cd t = cd{0.0, 0.0};
@@ -648,36 +620,15 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
     }
     if (!wvalid) return;
     const size_t ch = chunk;
-    if (HERM) {
-        // (G + G^H)/2 in full layout: NumMatrix sums G_ij + conj(G_ji) over frequencies
-        a.pTr[ch * a.nw_tot + nw] = trA;
-        if (MODE == MODE_DENS_HERM) a.pTr2[ch * a.nw_tot + nw] = tr2A;
-        cd* out = a.pG + (ch * a.nw_tot + nw) * M2;
-        int q = 0;
-#pragma unroll
-        for (int j = 0; j < NC; ++j)
-#pragma unroll
-            for (int i = 0; i <= j; ++i) {
-                const double h0 = ACC_LDS ? sAccH[q * FW + lane] : accH[q];
-                if (i == j) {
-                    out[i + i * NC] = cd{h0, 0.0};
-                    q += 1;
-                } else {
-                    const double h1 = ACC_LDS ? sAccH[(q + 1) * FW + lane] : accH[q + 1];
-                    out[i + j * NC] = cd{0.5 * h0, 0.5 * h1};
-                    out[j + i * NC] = cd{0.5 * h0, -0.5 * h1};
-                    q += 2;
-                }
-            }
-    } else if (MODE == MODE_FWD || MODE == MODE_FWD_REAL) {
+    if (MODE == MODE_FWD || MODE == MODE_FWD_REAL) {
         a.pTr[ch * a.nw_tot + nw] = trA;
         if (ACC_LDS) {
             for (int e = 0; e < M2; ++e) a.pG[(ch * a.nw_tot + nw) * M2 + e] = sAcc[e * FW + lane];
         } else {
 #pragma unroll
-            for (int i = 0; i < (ACC_LDS || HERM ? 1 : NC); ++i)
+            for (int i = 0; i < (ACC_LDS ? 1 : NC); ++i)
 #pragma unroll
-                for (int j = 0; j < (ACC_LDS || HERM ? 1 : NC); ++j)
+                for (int j = 0; j < (ACC_LDS ? 1 : NC); ++j)
                     a.pG[(ch * a.nw_tot + nw) * M2 + i + j * NC] = acc[i][j];
         }
     } else {
@@ -701,7 +652,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(schur_waves<
 void k_lattice_schur(LatArgs a, const cd* __restrict__ sig_all)
 {
     extern __shared__ cd lds[];
-    schur_item<NC, MODE, F32R, WG, TRACE, REFINE, KS>(a, sig_all, blockIdx.x, blockIdx.y, lds);
+    schur_item<NC, MODE, F32R, WG, TRACE, REFINE, KS>(a, sig_all, lattice_tile(), blockIdx.y, lds);
 }
 
 // Persistent form over a work list spanning several lattices of the same n_c:
@@ -725,8 +676,6 @@ void k_lattice_schur_multi(const LatArgs* __restrict__ args,
 template <int NC, int MODE, bool F32R, int WG, int KS = 1>
 constexpr size_t schur_shm()
 {
-    if constexpr (MODE == MODE_FWD_HERM) return F32R ? sizeof(double) * (size_t)NC * NC * WG : 0;
-    if constexpr (MODE == MODE_DENS_HERM) return sizeof(double) * (size_t)NC * NC * WG;
     constexpr bool ACC_LDS = (MODE == MODE_VJP) || ((MODE == MODE_FWD || MODE == MODE_FWD_REAL) && F32R);
     // KS > 1: one accumulator set per frequency, plus the tr G sums
     return ACC_LDS ? sizeof(cd) * (size_t)(NC * NC + (KS > 1 ? 1 : 0)) * (WG / KS) : 0;
@@ -745,8 +694,7 @@ hipError_t launch_nc_w(const LatArgs& a, const cd* sig_all, hipStream_t s, const
         return hipGetLastError();
     }
     constexpr int FW = WG / KS;  // frequencies per workgroup
-    const int span = (a.nw_end ? a.nw_end : a.nw_tot) - a.nw_begin;
-    dim3 grid((span + FW - 1) / FW, a.n_chunks);
+    const dim3 grid = lattice_grid(a, FW);
     hipError_t e = hipFuncSetAttribute((const void*)k_lattice_schur<NC, MODE, F32R, WG, TRACE, REFINE, KS>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
     if (e != hipSuccess) return e;
@@ -792,13 +740,6 @@ hipError_t launch_lane_nc(const LatArgs& a, int mode, bool fp32, const cd* sig_a
         return fp32 ? launch_nc<NC, MODE_FWD, true, false>(a, sig_all, s, wg, m)
                     : launch_nc<NC, MODE_FWD, false, false>(a, sig_all, s, wg, m);
     }
-    if (mode == MODE_FWD_HERM) {
-        if (a.want_trace)
-            return fp32 ? launch_nc<NC, MODE_FWD_HERM, true, true>(a, sig_all, s, wg, m)
-                        : launch_nc<NC, MODE_FWD_HERM, false, true>(a, sig_all, s, wg, m);
-        return fp32 ? launch_nc<NC, MODE_FWD_HERM, true, false>(a, sig_all, s, wg, m)
-                    : launch_nc<NC, MODE_FWD_HERM, false, false>(a, sig_all, s, wg, m);
-    }
     if (mode == MODE_FWD_REAL) {
         if (a.want_trace)
             return fp32 ? launch_nc<NC, MODE_FWD_REAL, true, true>(a, sig_all, s, wg, m)
@@ -809,9 +750,6 @@ hipError_t launch_lane_nc(const LatArgs& a, int mode, bool fp32, const cd* sig_a
     if (mode == MODE_DENS)
         return fp32 ? launch_nc<NC, MODE_DENS, true, false>(a, sig_all, s, wg, m)
                     : launch_nc<NC, MODE_DENS, false, false>(a, sig_all, s, wg, m);
-    if (mode == MODE_DENS_HERM)
-        return fp32 ? launch_nc<NC, MODE_DENS_HERM, true, false>(a, sig_all, s, wg, m)
-                    : launch_nc<NC, MODE_DENS_HERM, false, false>(a, sig_all, s, wg, m);
     return fp32 ? launch_nc<NC, MODE_VJP, true, false>(a, sig_all, s, wg, m)
                 : launch_nc<NC, MODE_VJP, false, false>(a, sig_all, s, wg, m);
 }

@@ -44,7 +44,10 @@ extern "C" {
 #define DMFTGPU_ERR_NUMERIC 4     /* non-finite result, failed bracketing */
 #define DMFTGPU_ERR_UNSUPPORTED 5 /* size or option this build does not handle */
 
-/* Methods for the per-(k, iw) solve. */
+/* Methods for the per-(k, iw) solve.  The Schur methods take the density sums beyond
+ * n_freq (where Sigma is its moment expansion) by a Gauss rule of that sum, 16 points per
+ * octave and exact to rounding, whenever the moments guarantee it; the plain method
+ * solves every frequency. */
 #define DMFTGPU_PLAIN_F64 0  /* full n x n inverse per (k,iw) in FP64 (GreenFtn.cpp:261) */
 #define DMFTGPU_SCHUR_F64 1  /* Schur complement on the correlated block, FP64 */
 #define DMFTGPU_SCHUR_F32R 2 /* Schur complement, FP32 solve + FP64-residual refinement */
@@ -78,9 +81,9 @@ const char* dmftgpu_version(void);
                                            32768 for the one-matrix-per-lane Schur kernels, keeping >= 64 k per
                                            chunk and >= 8192 items; 8192 for the others) */
 #define DMFTGPU_OPT_SCHUR_WG 3          /* frequencies per workgroup of the Schur kernels (64 or 128; default 0 =
-                                           the adjoint at 128, the FP32R forward over the first N_freq
-                                           frequencies at n_corr >= 5 as two wavefronts over 64 frequencies
-                                           splitting the k walk, the others at 64) */
+                                           the adjoint at 128, the FP32R forward at n_corr >= 5 as two
+                                           wavefronts over 64 frequencies splitting the k walk, the others
+                                           at 64) */
 #define DMFTGPU_OPT_SCHUR_LAYOUT 4      /* n_c <= 6: 0 = one (k,iw) matrix per lane (default), 1 = one column
                                            per lane (always used for n_c > 6) */
 #define DMFTGPU_OPT_UPFOLD_CHUNK 5      /* k points per chunk of dmftgpu_upfold_density (0 = as many as 512 MiB of
@@ -227,8 +230,7 @@ int dmftgpu_gloc_jvp(dmftgpu_handle h, int method, const double* sigma, double m
  *   n_total, loss, mu_bar          HOST outputs (each may be NULL)
  *   sigma_bar [n_freq][nc][nc]     out, dL/dRe + i dL/dIm (as dmftgpu_gloc_vjp)
  * Equal to dmftgpu_greenftn_w, the cotangents 2 (G_loc - G_tgt) and 2 (N - n_target),
- * and dmftgpu_gloc_vjp; on the one-matrix-per-lane Schur path the forward also forms
- * tr G^2 beyond N_freq, which the adjoint then skips.  No reference counterpart. */
+ * and dmftgpu_gloc_vjp.  No reference counterpart. */
 int dmftgpu_gloc_loss_grad(dmftgpu_handle h, int method, const double* sigma, double mu, const double* gloc_target,
                            double n_target, double* gloc, double* num_matrix, double* n_total, double* loss,
                            double* sigma_bar, double* mu_bar);
