@@ -111,6 +111,7 @@ extern "C" int dmftgpu_destroy(dmftgpu_handle h)
         if (h->ev1[m]) (void)hipEventDestroy(h->ev1[m]);
     }
     h->ft.release();
+    h->czt.release();
     for (auto& m : h->mom_cache) m.buf.release();
     h->ws.release();
     h->prep.release();
@@ -128,6 +129,7 @@ extern "C" int dmftgpu_set_stream(dmftgpu_handle h, void* stream)
     (void)hipGetLastError();  // drop an error left by an earlier failed call
     if (!h) return DMFTGPU_ERR_ARG;
     h->stream = (hipStream_t)stream;
+    h->czt_n = 0;  // formed on the previous stream
     return DMFTGPU_OK;
 }
 

@@ -67,6 +67,8 @@ struct dmftgpu_handle_s {
     dgi::Workspace prep;     // prepare-time data
     dgi::Workspace ws;       // per-call scratch
     dgi::Workspace ft;       // Fourier-transform scratch
+    dgi::Workspace czt;      // chirp-z tables (ft_czt.hpp) of the last n_tau
+    int czt_n = 0;
     // moment fit: basis table + inverted normal matrices per (n_freq, beta, branch);
     // kMomCache grids are kept (a DMFT iteration alternates the Sigma-like and
     // G-like fits), the least recently used one is formed again

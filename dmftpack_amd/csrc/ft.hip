@@ -6,21 +6,22 @@
 //
 // GPU work: the sliding-window least-squares fits (one thread per window start
 // and matrix element, summing in the reference's ascending order), the window
-// averages, the batched positivity tests, and both transforms as tiled complex
-// matrix products over frequency (tau) with the twiddles computed from the
-// same FP64 phase w*tau the reference uses.  The tail of FourierTransform_tau
-// does not depend on tau, so it is subtracted once per frequency, not once
-// per (tau, frequency) as in the reference loop (:55-61).
+// averages, the batched positivity tests, and both transforms: on the uniform tau grid as
+// chirp-z transforms (ft_czt.hip), at arbitrary tau values as a dense complex product.  The
+// tail of FourierTransform_tau does not depend on tau, so it is subtracted once per
+// frequency, not once per (tau, frequency) as in the reference loop (:55-61).
 // Host work: the small d x d set-up (square roots, inverses, eigenbases) and
 // the sequential selection / patch logic, restated from the reference.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
 
 #include "../../include/dmftgpu.h"
 #include "api_internal.hpp"
+#include "ft_czt.hpp"
 #include "host_linalg.hpp"
 #include "lattice_kernels.hpp"
 
@@ -386,111 +387,84 @@ __global__ void k_mom_final(const cd* __restrict__ mt, int d, int range, int gre
 // ---------------------------------------------------------------------------
 // iw -> tau
 // ---------------------------------------------------------------------------
-// D_i = F_i - tail_i,  tail_i = 1/2 sum_h A_h diag(1/(i w_i - e_h)) A_h^H   (:55-61)
-__global__ void k_ft_subtract_tail(const cd* __restrict__ fw, int d, int n_freq, double beta,
-                                   const cd* __restrict__ A1, const double* __restrict__ e1,
-                                   const cd* __restrict__ A2, const double* __restrict__ e2, cd* __restrict__ D)
+// Tiles of 16 rows (frequency or tau) x 16 elements, 256 threads: reads and writes of
+// either order move 256-byte runs, the transpose going through LDS.
+constexpr int kTile = 16;
+
+// D_i = F_i - tail_i,  tail_i = 1/2 sum_h A_h diag(1/(i w_i - e_h)) A_h^H   (:55-61), written to
+// D[i*si + e*se].  The d factors 1/(i w_i - e_h) of a row and the d products
+// A_h(a,l) conj(A_h(b,l)) of an element are formed once per tile.
+__global__ __launch_bounds__(256) void k_ft_subtract_tail(const cd* __restrict__ fw, int d, int n_freq, double beta,
+                                                          const cd* __restrict__ A1, const double* __restrict__ e1,
+                                                          const cd* __restrict__ A2, const double* __restrict__ e2,
+                                                          cd* __restrict__ D, size_t si, size_t se,
+                                                          int* __restrict__ bad)
 {
-    const int m2 = d * d;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)n_freq * m2) return;
-    const int i = (int)(t / m2), e = (int)(t % m2), a = e % d, b = e / d;
-    const double w = (kPi / beta) + i * ((2 * kPi) / beta);
-    cd tail = cd{0, 0};
-    for (int l = 0; l < d; ++l) {
-        const cd g1 = crcp(cd{-e1[l], w});
-        const cd g2 = crcp(cd{-e2[l], w});
-        tail = cfma(cmulc(A1[a + l * d], A1[b + l * d]), g1, tail);
-        tail = cfma(cmulc(A2[a + l * d], A2[b + l * d]), g2, tail);
+    __shared__ cd sg[2][kTile][33], sp[2][kTile][33], st[kTile][kTile + 1];
+    const int m2 = d * d, i0 = blockIdx.x * kTile, f0 = blockIdx.y * kTile;
+    if (bad && i0 == 0 && f0 == 0 && threadIdx.x == 0) *bad = 0;  // for the definiteness test that follows
+    for (int t = threadIdx.x; t < kTile * d; t += 256) {
+        const int r = t / d, l = t % d;
+        const double w = (kPi / beta) + (i0 + r) * ((2 * kPi) / beta);
+        sg[0][r][l] = crcp(cd{-e1[l], w});
+        sg[1][r][l] = crcp(cd{-e2[l], w});
+        const int e = min(f0 + r, m2 - 1), a = e % d, b = e / d;
+        sp[0][r][l] = cmulc(A1[a + l * d], A1[b + l * d]);
+        sp[1][r][l] = cmulc(A2[a + l * d], A2[b + l * d]);
     }
-    D[t] = csub(fw[t], cscale(tail, 0.5));
+    __syncthreads();
+    {
+        const int q = threadIdx.x % kTile, r = threadIdx.x / kTile, i = i0 + r, e = f0 + q;
+        cd v = cd{0.0, 0.0};
+        if (i < n_freq && e < m2) {
+            cd tail = cd{0.0, 0.0};
+            for (int l = 0; l < d; ++l) {
+                tail = cfma(sp[0][q][l], sg[0][r][l], tail);
+                tail = cfma(sp[1][q][l], sg[1][r][l], tail);
+            }
+            v = csub(fw[(size_t)i * m2 + e], cscale(tail, 0.5));
+        }
+        st[r][q] = v;
+    }
+    __syncthreads();
+    const bool rows = si < se;  // consecutive threads along the faster index of D
+    const int r = rows ? threadIdx.x % kTile : threadIdx.x / kTile, q = rows ? threadIdx.x / kTile : threadIdx.x % kTile;
+    if (i0 + r < n_freq && f0 + q < m2) D[(i0 + r) * si + (f0 + q) * se] = st[r][q];
 }
 
-// out[j][e] = sum_i coef(j,i) in[i][e]  (NIN = 1)  or  sum_i ca in0 + cb in1 (NIN = 2)
-// workgroup: TJ consecutive rows j, all elements; inputs staged in LDS TI rows at a time.
-// Phase recurrence of the matrix-core transform (k_dft_mfma, iw -> tau): a lane
-// walks its row j through i, i + 4, i + 8, ...; the phase factor at i + 4 is the
-// one at i times a per-row constant, and every 16th step it is formed again
-// exactly from the FP64 phase, so the rounding of the products stays at ~1e-15.
-struct PhaseWalk {
-    cd p;   // phase factor at the current i
-    cd m4;  // factor from i to i + 4
-};
-
-struct CoefW2Tau {
-    static constexpr bool PHASE_ROW = false;
-    static constexpr bool WALK = true;  // coefficients by the phase recurrence in k_dft_mfma
-    double beta, w0, dw, tstep;
-    const double* taus;  // explicit tau values (FourierTransform_tau), or null for tau_j = j*tstep
-    __device__ void operator()(int j, int i, cd* c) const
+// ---------------------------------------------------------------------------
+// The sum over frequencies at arbitrary tau values (FourierTransform_tau called with its
+// own points): out[j][e] = sum_i exp(-i w_i tau_j) in[i][e], a dense complex product.  The
+// uniform grids take the chirp-z form (ft_czt.hip).
+// ---------------------------------------------------------------------------
+struct TauPoints {
+    double w0, dw;
+    const double* taus;
+    __device__ cd operator()(int j, int i) const  // exp(-i w_i tau_j), the reference's FP64 w*tau
     {
-        const double w = w0 + i * dw;
-        const double tau = taus ? taus[j] : j * tstep;
-        double s, co;
-        sincos(w * tau, &s, &co);
-        c[0] = cd{co, -s};  // exp(-i w tau)
-    }
-    __device__ void walk_start(int j, int i, PhaseWalk& st) const
-    {
-        const double tau = taus ? taus[j] : j * tstep;
-        double s, co;
-        sincos((w0 + i * dw) * tau, &s, &co);
-        st.p = cd{co, -s};
-        sincos(4.0 * dw * tau, &s, &co);
-        st.m4 = cd{co, -s};
-    }
-    __device__ void walk_coef(const PhaseWalk& st, int, int, cd* c) const { c[0] = st.p; }
-};
-
-struct CoefTau2W {
-    // the phases exp(i w_n tau_t) of a tile's rows are formed once per (n, t)
-    // (k_dft stages them in LDS); segment t takes those at t and t + 1
-    static constexpr bool PHASE_ROW = true;
-    double beta, dt;
-    __device__ cd phase(int n, int t) const
-    {
-        const double wn = (2 * n + 1) * kPi / beta;
-        const double tau = t * dt;
         double s, c;
-        sincos(tau * wn, &s, &c);
-        return cd{c, s};
+        sincos((w0 + i * dw) * taus[j], &s, &c);
+        return cd{c, -s};
     }
-    // The coefficients take differences of neighbouring phase factors, which cancel
-    // at low frequency, so every phase is formed exactly (no recurrence): rounding
-    // in them would be amplified by 1/(w dt).
-    static constexpr bool WALK = false;
-    __device__ void operator()(int n, int t, cd* c) const { from_phases(n, t, phase(n, t), phase(n, t + 1), c); }
-    __device__ void walk_start(int, int, PhaseWalk&) const {}
-    __device__ void walk_coef(const PhaseWalk&, int n, int t, cd* c) const { (*this)(n, t, c); }
-    __device__ void from_phases(int n, int t, cd e0, cd e1, cd* c) const
+    __device__ cd step4(int j) const  // from i to i + 4
     {
-        const double wn = (2 * n + 1) * kPi / beta;
-        const double tau0 = t * dt, tau1 = (t + 1) * dt;
-        const double s0 = e0.y, c0 = e0.x, s1 = e1.y, c1 = e1.x;
-        const cd pI = cd{c1 - c0, s1 - s0};
-        const cd pI2 = cd{tau1 * c1 - tau0 * c0, tau1 * s1 - tau0 * s0};
-        // ca = pI/w^2 + pI2/(i w) ; cb = pI/(i w);  1/(i w) = -i/w
-        const double r = 1.0 / wn;
-        const cd a1 = cscale(pI, r * r);
-        const cd a2 = cd{pI2.y * r, -pI2.x * r};
-        c[0] = cadd(a1, a2);
-        c[1] = cd{pI.y * r, -pI.x * r};
+        double s, c;
+        sincos(4.0 * dw * taus[j], &s, &c);
+        return cd{c, -s};
     }
 };
 
-// out[j][e] = sum_i coef(j, i) in[i][e] over this workgroup's share of i:
-// blockIdx.y selects the i range [y*ichunk, min(ni, (y+1)*ichunk)); with more
-// than one range the results are partial sums, out + y*nj*m2, which
-// k_dft_sum_parts adds in range order.
-template <class Coef, int NIN, int OPT>
+// VALU form, any m2: a workgroup takes TJ consecutive rows j and all elements over its share
+// of i, [y*ichunk, min(ni, (y+1)*ichunk)), inputs staged in LDS TI rows at a time; with more
+// than one range the results are partial sums, out + y*nj*m2, which k_dft_sum_parts adds in
+// range order.
+template <int OPT>
 __global__ __launch_bounds__(256) void k_dft(int nj, int ni, int m2, int TJ, int TI, int ichunk,
-                                             const cd* __restrict__ in0, const cd* __restrict__ in1,
-                                             cd* __restrict__ out, Coef coef)
+                                             const cd* __restrict__ in, cd* __restrict__ out, TauPoints coef)
 {
     extern __shared__ cd sm[];
-    cd* sc = sm;                        // [NIN][TJ][TI]
-    cd* sx = sm + NIN * TJ * TI;        // [NIN][TI][m2]
-    cd* sp = sx + NIN * TI * m2;        // PHASE_ROW: [TJ][TI + 1]
+    cd* sc = sm;            // [TJ][TI]
+    cd* sx = sm + TJ * TI;  // [TI][m2]
     const int j0 = blockIdx.x * TJ;
     const int ib = blockIdx.y * ichunk;
     const int ie = min(ni, ib + ichunk);
@@ -501,30 +475,11 @@ __global__ __launch_bounds__(256) void k_dft(int nj, int ni, int m2, int TJ, int
     for (int q = 0; q < OPT; ++q) acc[q] = cd{0, 0};
     for (int i0 = ib; i0 < ie; i0 += TI) {
         __syncthreads();
-        if constexpr (Coef::PHASE_ROW) {
-            for (int t = threadIdx.x; t < TJ * (TI + 1); t += 256) {
-                const int jj = t / (TI + 1), ii = t % (TI + 1);
-                sp[t] = (j0 + jj < nj && i0 + ii <= ie) ? coef.phase(j0 + jj, i0 + ii) : cd{0, 0};
-            }
-            __syncthreads();
-        }
         for (int t = threadIdx.x; t < TJ * TI; t += 256) {
             const int jj = t / TI, ii = t % TI;
-            cd c[2] = {cd{0, 0}, cd{0, 0}};
-            if (j0 + jj < nj && i0 + ii < ie) {
-                if constexpr (Coef::PHASE_ROW)
-                    coef.from_phases(j0 + jj, i0 + ii, sp[jj * (TI + 1) + ii], sp[jj * (TI + 1) + ii + 1], c);
-                else
-                    coef(j0 + jj, i0 + ii, c);
-            }
-            for (int q = 0; q < NIN; ++q) sc[(q * TJ + jj) * TI + ii] = c[q];
+            sc[t] = (j0 + jj < nj && i0 + ii < ie) ? coef(j0 + jj, i0 + ii) : cd{0, 0};
         }
-        for (int t = threadIdx.x; t < TI * m2; t += 256) {
-            const int ii = t / m2, e = t % m2;
-            const bool ok = i0 + ii < ie;
-            sx[ii * m2 + e] = ok ? in0[(size_t)(i0 + ii) * m2 + e] : cd{0, 0};
-            if (NIN == 2) sx[(TI + ii) * m2 + e] = ok ? in1[(size_t)(i0 + ii) * m2 + e] : cd{0, 0};
-        }
+        for (int t = threadIdx.x; t < TI * m2; t += 256) sx[t] = i0 + t / m2 < ie ? in[(size_t)i0 * m2 + t] : cd{0, 0};
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < OPT; ++q) {
@@ -532,10 +487,7 @@ __global__ __launch_bounds__(256) void k_dft(int nj, int ni, int m2, int TJ, int
             if (o >= nout) break;
             const int jj = o / m2, e = o % m2;
             cd s = acc[q];
-            for (int ii = 0; ii < TI; ++ii) {
-                s = cfma(sc[jj * TI + ii], sx[ii * m2 + e], s);
-                if (NIN == 2) s = cfma(sc[(TJ + jj) * TI + ii], sx[(TI + ii) * m2 + e], s);
-            }
+            for (int ii = 0; ii < TI; ++ii) s = cfma(sc[jj * TI + ii], sx[ii * m2 + e], s);
             acc[q] = s;
         }
     }
@@ -548,45 +500,132 @@ __global__ __launch_bounds__(256) void k_dft(int nj, int ni, int m2, int TJ, int
     }
 }
 
-// G(tau_j) = Herm[ (X + X^H)/beta + 1/2 sum_h A_h diag(-1/(e^{e tau} + e^{e (tau-beta)})) A_h^H ]   (:62-90)
-__global__ void k_ft_finish(const cd* __restrict__ X, int d, int ntau1, double beta, double tstep,
-                            const double* __restrict__ taus, const cd* __restrict__ A1,
-                            const double* __restrict__ e1, const cd* __restrict__ A2, const double* __restrict__ e2,
-                            cd* __restrict__ out)
+// G(tau_j) = Herm[ (X + X^H)/beta + 1/2 sum_h A_h diag(-1/(e^{e tau} + e^{e (tau-beta)})) A_h^H ]   (:62-90),
+// X_j(e) = sum_q X[q*sq + j*sj + e*se] over nq partial sums; with wrap, X_{n_tau} = -X_0 (the
+// phase there is e^{-i pi (2n+1)}).  The upper triangle of the tail is the conjugate of the
+// lower one, so the result is Hermitian to the last bit.  The 2d exponential factors of a tau
+// are formed once per tile (they were 4d exponentials per element: 81 -> 12 us at d = 10,
+// N_tau = 8192).
+struct FtSums {
+    const cd* X;
+    int nq;
+    size_t sq, sj, se;
+    int wrap;  // n_tau, or -1
+};
+
+__global__ __launch_bounds__(256) void k_ft_finish(FtSums x, int d, int ntau1, double beta, double tstep,
+                                                   const double* __restrict__ taus, const cd* __restrict__ A1,
+                                                   const double* __restrict__ e1, const cd* __restrict__ A2,
+                                                   const double* __restrict__ e2, cd* __restrict__ out)
 {
-    const int m2 = d * d;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)ntau1 * m2) return;
-    const int j = (int)(t / m2), e = (int)(t % m2), a = e % d, b = e / d;
-    const double tau = taus ? taus[j] : j * tstep;
-    const cd* Xj = X + (size_t)j * m2;
-    auto elem = [&](int p, int q) {
-        cd v = cadd(Xj[p + q * d], cconj(Xj[q + p * d]));
-        v = cscale(v, 1.0 / beta);
-        cd s = cd{0, 0};
-        for (int l = 0; l < d; ++l) {
-            const double g1 = -1.0 / (exp(e1[l] * tau) + exp(e1[l] * (tau - beta)));
-            const double g2 = -1.0 / (exp(e2[l] * tau) + exp(e2[l] * (tau - beta)));
-            s = cadd(s, cscale(cmulc(A1[p + l * d], A1[q + l * d]), g1));
-            s = cadd(s, cscale(cmulc(A2[p + l * d], A2[q + l * d]), g2));
+    __shared__ double sg[2][kTile][33];
+    __shared__ cd sp[2][kTile][33], st[kTile][kTile + 1];
+    const int m2 = d * d, j0 = blockIdx.x * kTile, f0 = blockIdx.y * kTile;
+    for (int t = threadIdx.x; t < kTile * d; t += 256) {
+        const int r = t / d, l = t % d;
+        const int j = min(j0 + r, ntau1 - 1);
+        const double tau = taus ? taus[j] : j * tstep;
+        sg[0][r][l] = -1.0 / (exp(e1[l] * tau) + exp(e1[l] * (tau - beta)));
+        sg[1][r][l] = -1.0 / (exp(e2[l] * tau) + exp(e2[l] * (tau - beta)));
+        const int e = min(f0 + r, m2 - 1), a = e % d, b = e / d, hi = max(a, b), lo = min(a, b);
+        sp[0][r][l] = cmulc(A1[hi + l * d], A1[lo + l * d]);
+        sp[1][r][l] = cmulc(A2[hi + l * d], A2[lo + l * d]);
+    }
+    __syncthreads();
+    {
+        const bool rows = x.sj < x.se;
+        const int r = rows ? threadIdx.x % kTile : threadIdx.x / kTile;
+        const int q = rows ? threadIdx.x / kTile : threadIdx.x % kTile;
+        const int j = j0 + r, e = f0 + q;
+        cd v = cd{0.0, 0.0};
+        if (j < ntau1 && e < m2) {
+            const int a = e % d, b = e / d;
+            const bool wr = j == x.wrap;
+            const cd* p = x.X + (wr ? 0 : j) * x.sj;
+            cd xab = cd{0.0, 0.0}, xba = cd{0.0, 0.0};
+            for (int y = 0; y < x.nq; ++y) {
+                xab = cadd(xab, p[y * x.sq + (size_t)e * x.se]);
+                xba = cadd(xba, p[y * x.sq + (size_t)(b + a * d) * x.se]);
+            }
+            v = cscale(cadd(xab, cconj(xba)), (wr ? -1.0 : 1.0) / beta);
+            cd s = cd{0.0, 0.0};
+            for (int l = 0; l < d; ++l) {
+                s = cadd(s, cscale(sp[0][q][l], sg[0][r][l]));
+                s = cadd(s, cscale(sp[1][q][l], sg[1][r][l]));
+            }
+            v = cadd(v, cscale(a >= b ? s : cconj(s), 0.5));
+            if (a == b) v.y = 0.0;
         }
-        return cadd(v, cscale(s, 0.5));
-    };
-    const cd gab = elem(a, b), gba = elem(b, a);
-    out[t] = cscale(cadd(gab, cconj(gba)), 0.5);
+        st[r][q] = v;
+    }
+    __syncthreads();
+    const int r = threadIdx.x / kTile, q = threadIdx.x % kTile;
+    if (j0 + r < ntau1 && f0 + q < m2) out[(size_t)(j0 + r) * m2 + f0 + q] = st[r][q];
 }
 
-// FT_t_to_w segment slopes (:531-536)
-__global__ void k_ft_segments(const cd* __restrict__ gt, int m2, int nseg, double dt, cd* __restrict__ at,
-                              cd* __restrict__ bt)
+// G(tau_t), t = 1..n_tau-1, as [e][t] with a zero at t = 0 (the chirp-z input of tau -> iw);
+// clears the counter of the definiteness test that follows
+__global__ __launch_bounds__(256) void k_ft_gather_tau(const cd* __restrict__ gt, int m2, int n_tau,
+                                                       cd* __restrict__ out, int* __restrict__ bad)
 {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)nseg * m2) return;
-    const int s = (int)(t / m2);
-    const double tau0 = s * dt, tau1 = (s + 1) * dt;
-    const cd a = cscale(csub(gt[t + m2], gt[t]), 1.0 / (tau1 - tau0));
-    at[t] = a;
-    bt[t] = cadd(cscale(cneg(a), tau0), gt[t]);
+    __shared__ cd st[kTile][kTile + 1];
+    const int i0 = blockIdx.x * kTile, f0 = blockIdx.y * kTile;
+    if (i0 == 0 && f0 == 0 && threadIdx.x == 0) *bad = 0;
+    int r = threadIdx.x / kTile, q = threadIdx.x % kTile;
+    st[r][q] = (i0 + r > 0 && i0 + r < n_tau && f0 + q < m2) ? gt[(size_t)(i0 + r) * m2 + f0 + q] : cd{0.0, 0.0};
+    __syncthreads();
+    r = threadIdx.x % kTile;
+    q = threadIdx.x / kTile;
+    if (i0 + r < n_tau && f0 + q < m2) out[(size_t)(f0 + q) * n_tau + i0 + r] = st[r][q];
+}
+
+// FT_t_to_w (:531-547) from the plain sums S = sum_{0<t<n_tau} e^{i w tau_t} G(tau_t): the
+// integral of the piecewise linear interpolant is, with theta = w dt and
+// alpha = int_0^1 (1-u) e^{i theta u} du,
+//   dt [ (sin(theta/2)/(theta/2))^2 S + alpha G(0) - conj(alpha) G(beta) ]
+// (e^{i w beta} = -1).  alpha by its Taylor series below theta = 1, where the closed form
+// cancels.
+__global__ __launch_bounds__(256) void k_ft_w_finish(const cd* __restrict__ parts, int nq, const cd* __restrict__ gt,
+                                                     int m2, int n_freq, int n_tau, double dt, cd* __restrict__ fw)
+{
+    __shared__ cd st[kTile][kTile + 1], sa[kTile];
+    __shared__ double sw[kTile];
+    const int n0 = blockIdx.x * kTile, f0 = blockIdx.y * kTile;
+    if (threadIdx.x < kTile) {
+        const double th = kPi * (2.0 * (n0 + (int)threadIdx.x) + 1.0) / n_tau;
+        const double h = sin(0.5 * th) / (0.5 * th);
+        cd al;
+        if (th < 1.0) {
+            const double t2 = th * th;
+            double x = 0.0, y = 0.0;
+            for (int p = 9; p >= 0; --p) {  // x = sum (-1)^p th^2p/(2p+2)!,  y = sum (-1)^p th^2p/(2p+3)!
+                x = 1.0 - t2 * x / ((2.0 * p + 3.0) * (2.0 * p + 4.0));
+                y = 1.0 - t2 * y / ((2.0 * p + 4.0) * (2.0 * p + 5.0));
+            }
+            al = cd{0.5 * x, th * y / 6.0};
+        } else {
+            double s, c;
+            sincos(th, &s, &c);
+            al = cd{(1.0 - c) / (th * th), (th - s) / (th * th)};
+        }
+        sa[threadIdx.x] = cscale(al, dt);
+        sw[threadIdx.x] = h * h * dt;
+    }
+    {
+        const int r = threadIdx.x % kTile, q = threadIdx.x / kTile;
+        cd v = cd{0.0, 0.0};
+        if (n0 + r < n_freq && f0 + q < m2)
+            for (int y = 0; y < nq; ++y) v = cadd(v, parts[((size_t)y * m2 + f0 + q) * n_freq + n0 + r]);
+        st[r][q] = v;
+    }
+    __syncthreads();
+    const int r = threadIdx.x / kTile, q = threadIdx.x % kTile, e = f0 + q;
+    if (n0 + r < n_freq && e < m2) {
+        cd v = cscale(st[r][q], sw[r]);
+        v = cfma(sa[r], gt[e], v);
+        v = csub(v, cmulc(gt[(size_t)n_tau * m2 + e], sa[r]));
+        fw[(size_t)(n0 + r) * m2 + e] = v;
+    }
 }
 
 // (F - F^H)/(2i), for the causality test of FT_t_to_w (:552)
@@ -602,80 +641,6 @@ __global__ void k_antiherm(const cd* __restrict__ f, int d, int count, cd* __res
     out[t] = cd{0.5 * dlt.y, -0.5 * dlt.x};  // dlt / (2i)
 }
 
-// Register-tiled form for m2 <= 256 (used for tau -> iw, two inputs per i):
-// thread (jg, e), jg < jgroups, keeps output
-// element e of the rj consecutive rows jg*rj .. jg*rj + rj - 1, so one read of
-// in[i][e] from LDS serves rj complex FMAs and the coefficient reads are the
-// same address across the lanes of a row group (broadcast).  Tiles, i ranges
-// and the order of the sum over i are those of k_dft.
-template <class Coef, int NIN, int RJ>
-__global__ __launch_bounds__(256) void k_dft_rt(int nj, int ni, int m2, int TJ, int TI, int ichunk, int jgroups,
-                                                int rj, const cd* __restrict__ in0, const cd* __restrict__ in1,
-                                                cd* __restrict__ out, Coef coef)
-{
-    extern __shared__ cd sm[];
-    cd* sc = sm;                        // [NIN][TJ][TI]
-    cd* sx = sm + NIN * TJ * TI;        // [NIN][TI][m2]
-    cd* sp = sx + NIN * TI * m2;        // PHASE_ROW: [TJ][TI + 1]
-    const int j0 = blockIdx.x * TJ;
-    const int ib = blockIdx.y * ichunk;
-    const int ie = min(ni, ib + ichunk);
-    out += (size_t)blockIdx.y * nj * m2;
-    const int e = threadIdx.x % m2, jg = threadIdx.x / m2;
-    const bool act = jg < jgroups;
-    cd acc[RJ];
-#pragma unroll
-    for (int r = 0; r < RJ; ++r) acc[r] = cd{0, 0};
-    for (int i0 = ib; i0 < ie; i0 += TI) {
-        __syncthreads();
-        if constexpr (Coef::PHASE_ROW) {
-            for (int t = threadIdx.x; t < TJ * (TI + 1); t += 256) {
-                const int jj = t / (TI + 1), ii = t % (TI + 1);
-                sp[t] = (j0 + jj < nj && i0 + ii <= ie) ? coef.phase(j0 + jj, i0 + ii) : cd{0, 0};
-            }
-            __syncthreads();
-        }
-        for (int t = threadIdx.x; t < TJ * TI; t += 256) {
-            const int jj = t / TI, ii = t % TI;
-            cd c[2] = {cd{0, 0}, cd{0, 0}};
-            if (j0 + jj < nj && i0 + ii < ie) {
-                if constexpr (Coef::PHASE_ROW)
-                    coef.from_phases(j0 + jj, i0 + ii, sp[jj * (TI + 1) + ii], sp[jj * (TI + 1) + ii + 1], c);
-                else
-                    coef(j0 + jj, i0 + ii, c);
-            }
-            for (int q = 0; q < NIN; ++q) sc[(q * TJ + jj) * TI + ii] = c[q];
-        }
-        for (int t = threadIdx.x; t < TI * m2; t += 256) {
-            const int ii = t / m2, ee = t % m2;
-            const bool ok = i0 + ii < ie;
-            sx[ii * m2 + ee] = ok ? in0[(size_t)(i0 + ii) * m2 + ee] : cd{0, 0};
-            if (NIN == 2) sx[(TI + ii) * m2 + ee] = ok ? in1[(size_t)(i0 + ii) * m2 + ee] : cd{0, 0};
-        }
-        __syncthreads();
-        if (act) {
-            const int jr = jg * rj;
-            for (int ii = 0; ii < TI; ++ii) {
-                const cd x0 = sx[ii * m2 + e];
-                const cd x1 = NIN == 2 ? sx[(TI + ii) * m2 + e] : cd{0, 0};
-#pragma unroll
-                for (int r = 0; r < RJ; ++r) {
-                    if (r < rj) {
-                        acc[r] = cfma(sc[(jr + r) * TI + ii], x0, acc[r]);
-                        if (NIN == 2) acc[r] = cfma(sc[(TJ + jr + r) * TI + ii], x1, acc[r]);
-                    }
-                }
-            }
-        }
-    }
-    if (!act) return;
-#pragma unroll
-    for (int r = 0; r < RJ; ++r) {
-        const int jj = jg * rj + r;
-        if (r < rj && j0 + jj < nj) out[(size_t)(j0 + jj) * m2 + e] = acc[r];
-    }
-}
-
 // parts[y][j][e] -> out[j][e], y ascending
 __global__ void k_dft_sum_parts(const cd* __restrict__ parts, int nparts, size_t count, cd* __restrict__ out)
 {
@@ -686,21 +651,19 @@ __global__ void k_dft_sum_parts(const cd* __restrict__ parts, int nparts, size_t
     out[t] = s;
 }
 
-// The same transform on the matrix cores (FP64 MFMA), for m2 <= 16 * NE:
-// out[j][e] = sum_i sum_q coef_q(j, i) in_q[i][e] as complex products split
-// into real v_mfma_f64_16x16x4 (D = A B + D, A 16 x 4, B 4 x 16).  A wavefront
-// owns 16 consecutive rows j and every e tile (NE tiles of 16 elements), so
-// each coefficient it forms serves NE tiles.  Per step of 4 summed indices,
-// lane l = r + 16 k forms coef(j0 + r, i0 + k), the A operand's (r, k) entry
-// (by the phase recurrence of PhaseWalk),
-// and loads in[i0 + k][16 t + r], the B operand's (k, r) entry of tile t; the
-// accumulator of tile t holds out[j0 + c][16 t + r'] at lane r' + 16 (c % 4),
-// register c / 4.  blockIdx.y selects the range of i, as in k_dft.
+// The same sum on the matrix cores (FP64 MFMA), for m2 <= 16 * NE: complex products split
+// into real v_mfma_f64_16x16x4 (D = A B + D, A 16 x 4, B 4 x 16).  A wavefront owns 16
+// consecutive rows j and every e tile (NE tiles of 16 elements), so each phase factor it
+// forms serves NE tiles.  Per step of 4 summed indices, lane l = r + 16 k holds the factor
+// (j0 + r, i0 + k), the A operand's (r, k) entry, walked along i by a per-row constant and
+// formed again exactly every 16th step (rounding ~1e-15), and loads in[i0 + k][16 t + r], the
+// B operand's (k, r) entry of tile t; the accumulator of tile t holds out[j0 + c][16 t + r'] at
+// lane r' + 16 (c % 4), register c / 4.  blockIdx.y selects the range of i, as in k_dft.
 typedef double dmfma4 __attribute__((ext_vector_type(4)));
 
-template <class Coef, int NIN, int NE>
-__global__ __launch_bounds__(256) void k_dft_mfma(int nj, int ni, int m2, int ichunk, const cd* __restrict__ in0,
-                                                  const cd* __restrict__ in1, cd* __restrict__ out, Coef coef)
+template <int NE>
+__global__ __launch_bounds__(256) void k_dft_mfma(int nj, int ni, int m2, int ichunk, const cd* __restrict__ in,
+                                                  cd* __restrict__ out, TauPoints coef)
 {
     const int lane = threadIdx.x & 63;
     const int r = lane & 15, k = lane >> 4;
@@ -716,35 +679,29 @@ __global__ __launch_bounds__(256) void k_dft_mfma(int nj, int ni, int m2, int ic
     }
     const int j = j0 + r;
     const bool jok = j < nj;
-    PhaseWalk st{};
+    const cd m4 = coef.step4(jok ? j : 0);
+    cd p = cd{0, 0};
     for (int i0 = ib, step = 0; i0 < ie; i0 += 4, ++step) {
         const int i = i0 + k;
-        if constexpr (Coef::WALK) {
-            if ((step & 15) == 0) coef.walk_start(jok ? j : 0, i, st);
-            else st.p = cmul(st.p, st.m4);
+        if ((step & 15) == 0) p = coef(jok ? j : 0, i);
+        else p = cmul(p, m4);
+        const cd c = (i < ie && jok) ? p : cd{0, 0};
+        cd b[NE];
+#pragma unroll
+        for (int t = 0; t < NE; ++t) {
+            const int e = 16 * t + r;
+            b[t] = (i < ie && e < m2) ? in[(size_t)i * m2 + e] : cd{0, 0};
         }
-        cd c[2] = {cd{0, 0}, cd{0, 0}};
-        if (i < ie && jok) coef.walk_coef(st, j, i, c);
+        // four passes over the tiles: consecutive MFMAs update different accumulators
+        const double ar = c.x, ai = c.y;
 #pragma unroll
-        for (int q = 0; q < NIN; ++q) {
-            const cd* in = q == 0 ? in0 : in1;
-            cd b[NE];
+        for (int t = 0; t < NE; ++t) accR[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, b[t].x, accR[t], 0, 0, 0);
 #pragma unroll
-            for (int t = 0; t < NE; ++t) {
-                const int e = 16 * t + r;
-                b[t] = (i < ie && e < m2) ? in[(size_t)i * m2 + e] : cd{0, 0};
-            }
-            // four passes over the tiles: consecutive MFMAs update different accumulators
-            const double ar = c[q].x, ai = c[q].y;
+        for (int t = 0; t < NE; ++t) accI[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, b[t].y, accI[t], 0, 0, 0);
 #pragma unroll
-            for (int t = 0; t < NE; ++t) accR[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, b[t].x, accR[t], 0, 0, 0);
+        for (int t = 0; t < NE; ++t) accR[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai, b[t].y, accR[t], 0, 0, 0);
 #pragma unroll
-            for (int t = 0; t < NE; ++t) accI[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, b[t].y, accI[t], 0, 0, 0);
-#pragma unroll
-            for (int t = 0; t < NE; ++t) accR[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-ai, b[t].y, accR[t], 0, 0, 0);
-#pragma unroll
-            for (int t = 0; t < NE; ++t) accI[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, b[t].x, accI[t], 0, 0, 0);
-        }
+        for (int t = 0; t < NE; ++t) accI[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, b[t].x, accI[t], 0, 0, 0);
     }
 #pragma unroll
     for (int t = 0; t < NE; ++t) {
@@ -759,134 +716,61 @@ __global__ __launch_bounds__(256) void k_dft_mfma(int nj, int ni, int m2, int ic
 }
 
 struct DftShape {
-    int TJ, TI, ks, ichunk, jgroups, rj;  // jgroups > 0: the register-tiled kernel
+    int TJ, TI, ks, ichunk;
+    bool mfma;
 };
 
-// Tiles of the transform and the split of the summed index i over
-// workgroups: enough workgroups to fill the device (about 1024) when the
-// output alone gives fewer.
-// The matrix-core form (k_dft_mfma) for m2 <= 128: rows in tiles of 64 per
-// workgroup (16 per wavefront), the summed index split so that the launch has
-// about 4096 wavefronts (4 per SIMD), in multiples of 4.
-constexpr int kDftMfmaMaxM2 = 128;
-
-inline DftShape dft_shape_mfma(int nj, int ni)
+// Tiles of the dense sum and the split of the summed index i over workgroups: about 1024
+// workgroups.  m2 <= 128 on the matrix cores, rows in tiles of 64 per workgroup (16 per
+// wavefront), i split in multiples of 4.
+inline DftShape dft_shape(int nj, int ni, int m2)
 {
     DftShape d{};
-    d.TJ = 64;
-    d.TI = 4;
-    const int gx = (nj + d.TJ - 1) / d.TJ;
-    const int steps = (ni + 3) / 4;
-    int ks = (1024 + gx - 1) / gx;
-    if (ks > steps) ks = steps;
-    if (ks > 32) ks = 32;
-    if (ks < 1) ks = 1;
-    d.ichunk = (steps + ks - 1) / ks * 4;
-    d.ks = (ni + d.ichunk - 1) / d.ichunk;
-    d.jgroups = -1;
-    return d;
-}
-
-inline DftShape dft_shape(int nj, int ni, int m2, int nin, bool phase_row)
-{
-    if (m2 <= kDftMfmaMaxM2) return dft_shape_mfma(nj, ni);
-    DftShape d;
-    if (m2 <= 256 && nin == 2) {  // register-tiled (tau -> iw; measured slower for iw -> tau): TJ = jgroups * rj rows
-        d.jgroups = 256 / m2;
-        d.rj = 256 / d.jgroups;
-        if (d.rj > 8) d.rj = 8;
-        d.TJ = d.jgroups * d.rj;
-        d.TI = 3072 / (nin * (d.TJ + m2) + (phase_row ? d.TJ + 1 : 0));
-        if (d.TI > 32) d.TI = 32;
-        if (d.TI < 1) d.TI = 1;
+    d.mfma = m2 <= 128;
+    if (d.mfma) {
+        d.TJ = 64;
+        d.TI = 4;
     } else {
-        d.jgroups = 0;
-        d.rj = 0;
-        d.TJ = 2048 / m2;
-        if (d.TJ > 32) d.TJ = 32;
-        if (d.TJ < 1) d.TJ = 1;
-        d.TI = 2048 / (m2 * nin);
-        if (d.TI > 32) d.TI = 32;
-        if (d.TI < 1) d.TI = 1;
+        d.TJ = std::max(1, std::min(32, 2048 / m2));
+        d.TI = std::max(1, std::min(32, 2048 / m2));
     }
     const int gx = (nj + d.TJ - 1) / d.TJ;
-    const int itiles = (ni + d.TI - 1) / d.TI;
-    int ks = (1024 + gx - 1) / gx;
-    if (ks > itiles) ks = itiles;
-    if (ks > 16) ks = 16;
-    if (ks < 1) ks = 1;
-    const int per = (itiles + ks - 1) / ks;
-    d.ichunk = per * d.TI;
+    const int steps = (ni + d.TI - 1) / d.TI;
+    const int ks = std::max(1, std::min({(1024 + gx - 1) / gx, steps, d.mfma ? 32 : 16}));
+    d.ichunk = (steps + ks - 1) / ks * d.TI;
     d.ks = (ni + d.ichunk - 1) / d.ichunk;
     return d;
 }
 
-// scratch (in cd) the split transform needs for its partial sums
-inline size_t dft_part_count(int nj, int ni, int m2, int nin, bool phase_row)
+// scratch (in cd) the split sum needs for its partial sums
+inline size_t dft_part_count(int nj, int ni, int m2)
 {
-    const DftShape d = dft_shape(nj, ni, m2, nin, phase_row);
+    const DftShape d = dft_shape(nj, ni, m2);
     return d.ks > 1 ? (size_t)d.ks * nj * m2 : 0;
 }
 
-template <class Coef, int NIN>
-hipError_t launch_dft(int nj, int ni, int m2, const cd* in0, const cd* in1, cd* out, Coef coef, cd* parts,
-                      hipStream_t s)
+hipError_t launch_dft(int nj, int ni, int m2, const cd* in, cd* out, TauPoints coef, cd* parts, hipStream_t s)
 {
-    const DftShape d = dft_shape(nj, ni, m2, NIN, Coef::PHASE_ROW);
-    if (d.jgroups < 0) {  // matrix cores
-        if (d.ks > 1 && !parts) return hipErrorInvalidValue;
-        cd* dstm = d.ks > 1 ? parts : out;
-        dim3 gridm((nj + d.TJ - 1) / d.TJ, d.ks);
-#define M_(NE)                                                                                                    \
-    if (m2 <= 16 * NE) {                                                                                          \
-        hipLaunchKernelGGL((k_dft_mfma<Coef, NIN, NE>), gridm, dim3(256), 0, s, nj, ni, m2, d.ichunk, in0, in1, dstm, \
-                           coef);                                                                                 \
-    } else
+    const DftShape d = dft_shape(nj, ni, m2);
+    if (d.ks > 1 && !parts) return hipErrorInvalidValue;
+    cd* dst = d.ks > 1 ? parts : out;
+    const dim3 grid((nj + d.TJ - 1) / d.TJ, d.ks);
+    if (d.mfma) {
+#define M_(NE)                                                                                                          if (m2 <= 16 * NE) {                                                                                                    hipLaunchKernelGGL((k_dft_mfma<NE>), grid, dim3(256), 0, s, nj, ni, m2, d.ichunk, in, dst, coef);               } else
         M_(1) M_(2) M_(4) M_(6) M_(7) M_(8) return hipErrorInvalidValue;
 #undef M_
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess || d.ks == 1) return e;
-        const size_t cnt = (size_t)nj * m2;
-        hipLaunchKernelGGL(k_dft_sum_parts, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, parts, d.ks, cnt, out);
-        return hipGetLastError();
-    }
-    const int TJ = d.TJ, TI = d.TI;
-    const int opt = (TJ * m2 + 255) / 256;
-    size_t shm = sizeof(cd) * ((size_t)NIN * TJ * TI + (size_t)NIN * TI * m2 +
-                               (Coef::PHASE_ROW ? (size_t)TJ * (TI + 1) : 0));
-    dim3 grid((nj + TJ - 1) / TJ, d.ks);
-    cd* dst = d.ks > 1 ? parts : out;
-    if (d.ks > 1 && !parts) return hipErrorInvalidValue;
-    if (d.jgroups > 0) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_dft_rt<Coef, NIN, 8>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((k_dft_rt<Coef, NIN, 8>), grid, dim3(256), shm, s, nj, ni, m2, TJ, TI, d.ichunk, d.jgroups,
-                           d.rj, in0, in1, dst, coef);
-        e = hipGetLastError();
-        if (e != hipSuccess || d.ks == 1) return e;
-        const size_t cnt = (size_t)nj * m2;
-        hipLaunchKernelGGL(k_dft_sum_parts, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, parts, d.ks, cnt, out);
-        return hipGetLastError();
-    }
-#define L_(O)                                                                                                     \
-    {                                                                                                             \
-        hipError_t e = hipFuncSetAttribute((const void*)k_dft<Coef, NIN, O>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                           (int)shm);                                                             \
-        if (e != hipSuccess) return e;                                                                            \
-        hipLaunchKernelGGL((k_dft<Coef, NIN, O>), grid, dim3(256), shm, s, nj, ni, m2, TJ, TI, d.ichunk, in0, in1,  \
-                           dst, coef);                                                                            \
-        e = hipGetLastError();                                                                                    \
-        if (e != hipSuccess || d.ks == 1) return e;                                                               \
-        const size_t cnt = (size_t)nj * m2;                                                                       \
-        hipLaunchKernelGGL(k_dft_sum_parts, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, parts, d.ks, cnt, out); \
-        return hipGetLastError();                                                                                 \
-    }
-    if (opt <= 1) L_(1)
-    if (opt <= 2) L_(2)
-    if (opt <= 4) L_(4)
-    L_(8)
+    } else {
+        const int opt = (d.TJ * m2 + 255) / 256;
+        const size_t shm = sizeof(cd) * ((size_t)d.TJ * d.TI + (size_t)d.TI * m2);
+#define L_(O)                                                                                                            {                                                                                                                        hipError_t e = hipFuncSetAttribute((const void*)k_dft<O>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);         if (e != hipSuccess) return e;                                                                                       hipLaunchKernelGGL((k_dft<O>), grid, dim3(256), shm, s, nj, ni, m2, d.TJ, d.TI, d.ichunk, in, dst, coef);        }
+        if (opt <= 4) L_(4) else L_(8)
 #undef L_
+    }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || d.ks == 1) return e;
+    const size_t cnt = (size_t)nj * m2;
+    hipLaunchKernelGGL(k_dft_sum_parts, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, parts, d.ks, cnt, out);
+    return hipGetLastError();
 }
 
 unsigned nblk(size_t n) { return (unsigned)((n + 255) / 256); }
@@ -1028,16 +912,20 @@ static void tail_setup(int d, const std::vector<hl::cx>& m1, const std::vector<h
 {
     using namespace hl;
     Mat V = zeros(d), H1 = zeros(d), H2 = zeros(d);
-    if (min_eig(d, m1) > 0) {
-        V = herm_func(d, m1, [](double x) { return std::sqrt(x > 0 ? x : 0.0); });
+    std::vector<double> w;
+    Mat Q;
+    eigh(d, m1, w, Q);
+    if (w[0] > 0) {
+        V = herm_func(d, w, Q, [](double x) { return std::sqrt(x > 0 ? x : 0.0); });
         Mat Vi, ViH;
         inverse(d, V, Vi);
         inverse(d, adj(d, V), ViH);
         Mat M2 = mul(d, mul(d, ViH, lin(m2, 2.0, m2, 0.0)), Vi);
         Mat M3 = mul(d, mul(d, ViH, lin(m3, 2.0, m3, 0.0)), Vi);
         Mat X = lin(M3, 0.5, mul(d, M2, M2), -0.25);
-        if (min_eig(d, X) > 0) {
-            Mat sq = herm_func(d, X, [](double x) { return std::sqrt(x > 0 ? x : 0.0); });
+        eigh(d, X, w, Q);
+        if (w[0] > 0) {
+            Mat sq = herm_func(d, w, Q, [](double x) { return std::sqrt(x > 0 ? x : 0.0); });
             H1 = lin(M2, 0.5, sq, 1.0);
         } else {
             H1 = lin(M2, 0.5, M2, 0.0);
@@ -1050,6 +938,44 @@ static void tail_setup(int d, const std::vector<hl::cx>& m1, const std::vector<h
     A1 = mul(d, VH, U);
     eigh(d, H2, e2, U);
     A2 = mul(d, VH, U);
+}
+
+// The two-pole tail on the device, one copy
+struct TailDev {
+    const cd *A1, *A2;
+    const double *e1, *e2;
+};
+
+static TailDev tail_upload(dmftgpu_handle h, int d, const std::vector<hl::cx>& A1, const std::vector<double>& e1,
+                           const std::vector<hl::cx>& A2, const std::vector<double>& e2, Carve& cv, int* rc)
+{
+    const int m2 = d * d;
+    std::vector<double> host((size_t)4 * m2 + 2 * d);
+    std::memcpy(host.data(), A1.data(), sizeof(cd) * m2);
+    std::memcpy(host.data() + 2 * m2, A2.data(), sizeof(cd) * m2);
+    std::memcpy(host.data() + 4 * m2, e1.data(), sizeof(double) * d);
+    std::memcpy(host.data() + 4 * m2 + d, e2.data(), sizeof(double) * d);
+    double* dev = cv.take<double>(host.size());
+    const hipError_t e = hipMemcpyAsync(dev, host.data(), sizeof(double) * host.size(), hipMemcpyHostToDevice, h->stream);
+    if (e != hipSuccess) *rc = fail(h, DMFTGPU_ERR_HIP, "tail upload: %s", hipGetErrorString(e));
+    return TailDev{(const cd*)dev, (const cd*)(dev + 2 * m2), dev + 4 * m2, dev + 4 * m2 + d};
+}
+
+// Tables of the chirp-z form for n_tau, kept in the handle for the last n_tau
+static const cd* czt_tables(dmftgpu_handle h, int n_tau, int* rc)
+{
+    hipError_t e;
+    if (h->czt_n != n_tau) {
+        h->czt_n = 0;
+        cd* t = (cd*)h->czt.get(dg::czt_table_count(n_tau) * sizeof(cd), &e);
+        if (t) e = dg::launch_czt_tables(n_tau, t, h->stream);
+        if (e != hipSuccess) {
+            *rc = fail(h, DMFTGPU_ERR_HIP, "transform tables: %s", hipGetErrorString(e));
+            return nullptr;
+        }
+        h->czt_n = n_tau;
+    }
+    return (const cd*)h->czt.ptr;
 }
 
 extern "C" int dmftgpu_ft_w2tau(dmftgpu_handle h, int d, int n_freq, int n_tau, double beta, const double* fw,
@@ -1070,41 +996,48 @@ extern "C" int dmftgpu_ft_w2tau(dmftgpu_handle h, int d, int n_freq, int n_tau, 
     std::vector<hl::cx> A1, A2;
     std::vector<double> e1, e2;
     tail_setup(d, m1, mm2, m3, A1, e1, A2, e2);
-    const size_t npart = dft_part_count(ntau1, n_freq, m2, 1, CoefW2Tau::PHASE_ROW);
-    size_t need = (size_t)n_freq * m2 * 16 + (size_t)ntau1 * m2 * 16 + 4 * (size_t)m2 * 16 + 4 * (size_t)d * 8 +
+    const dg::CztPlan cp = dg::czt_plan(n_tau, n_freq, n_tau);
+    const size_t npart = (size_t)cp.in_tiles * m2 * n_tau;
+    size_t need = (size_t)n_freq * m2 * 16 + 4 * (size_t)m2 * 16 + 4 * (size_t)d * 8 +
                   (size_t)ntau1 * d * 8 + npart * 16 + 16 * 256;
     int rc = 0;
     char* base = ft_ws(h, need, &rc);
     if (!base) return rc;
     Carve cv{base};
     cd* D = cv.take<cd>((size_t)n_freq * m2);
-    cd* X = cv.take<cd>((size_t)ntau1 * m2);
-    cd* parts = npart ? cv.take<cd>(npart) : nullptr;
-    cd* dA1 = cv.take<cd>(m2);
-    cd* dA2 = cv.take<cd>(m2);
-    double* de1 = cv.take<double>(d);
-    double* de2 = cv.take<double>(d);
+    cd* parts = cv.take<cd>(npart);
+    const TailDev tl = tail_upload(h, d, A1, e1, A2, e2, cv, &rc);
+    if (rc) return rc;
     double* wmin = cv.take<double>((size_t)ntau1 * d);
-    HIPCHK(hipMemcpyAsync(dA1, A1.data(), sizeof(cd) * m2, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dA2, A2.data(), sizeof(cd) * m2, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(de1, e1.data(), sizeof(double) * d, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(de2, e2.data(), sizeof(double) * d, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_ft_subtract_tail, dim3(nblk((size_t)n_freq * m2)), dim3(256), 0, s, (const cd*)fw, d, n_freq,
-                       beta, dA1, de1, dA2, de2, D);
+    int* bad = cv.take<int>(1);
+    const dim3 gf((n_freq + kTile - 1) / kTile, (m2 + kTile - 1) / kTile);
+    const cd* tab = czt_tables(h, n_tau, &rc);
+    if (!tab) return rc;
+    hipLaunchKernelGGL(k_ft_subtract_tail, gf, dim3(256), 0, s, (const cd*)fw, d, n_freq, beta, tl.A1, tl.e1, tl.A2, tl.e2,
+                       D, (size_t)1, (size_t)n_freq, bad);
     HIPCHK(hipGetLastError());
-    CoefW2Tau cw{beta, kPi / beta, (2 * kPi) / beta, beta / n_tau, nullptr};
-    HIPCHK((launch_dft<CoefW2Tau, 1>(ntau1, n_freq, m2, D, nullptr, X, cw, parts, s)));
+    HIPCHK(dg::launch_czt(cp, false, m2, tab, D, parts, s));
+    const FtSums xs{parts, cp.in_tiles, (size_t)m2 * n_tau, 1, (size_t)n_tau, n_tau};
     cd* out = (cd*)gtau;
-    hipLaunchKernelGGL(k_ft_finish, dim3(nblk((size_t)ntau1 * m2)), dim3(256), 0, s, X, d, ntau1, beta, beta / n_tau,
-                       (const double*)nullptr, dA1, de1, dA2, de2, out);
+    hipLaunchKernelGGL(k_ft_finish, dim3((ntau1 + kTile - 1) / kTile, (m2 + kTile - 1) / kTile), dim3(256), 0, s, xs, d,
+                       ntau1, beta, beta / n_tau, (const double*)nullptr, tl.A1, tl.e1, tl.A2, tl.e2, out);
     HIPCHK(hipGetLastError());
-    // causality patch (:145-175): min eigenvalue of every G(tau_j)
-    HIPCHK(dg::launch_herm_eig(out, d, 0, d, nullptr, 0, wmin, nullptr, ntau1, s));
-    std::vector<double> hw((size_t)ntau1 * d);
-    HIPCHK(hipMemcpyAsync(hw.data(), wmin, sizeof(double) * hw.size(), hipMemcpyDeviceToHost, s));
+    // causality patch (:145-175): it acts where the largest eigenvalue test fails, i.e. where
+    // G(tau_j) is not negative definite.  -G(tau_j) - 1e-13 tr I positive definite for every j
+    // settles that there is nothing to do; otherwise the eigenvalues decide
+    HIPCHK(dg::launch_not_posdef(out, d, ntau1, false, bad, s));
+    int hbad = 0;
+    HIPCHK(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
+    std::vector<double> hw;
     bool any = false;
-    for (int t = 0; t <= n_tau; ++t) any |= hw[(size_t)t * d] >= 0;
+    if (hbad) {
+        HIPCHK(dg::launch_herm_eig(out, d, 0, d, nullptr, 0, wmin, nullptr, ntau1, s));
+        hw.resize((size_t)ntau1 * d);
+        HIPCHK(hipMemcpyAsync(hw.data(), wmin, sizeof(double) * hw.size(), hipMemcpyDeviceToHost, s));
+        HIPCHK(hipStreamSynchronize(s));
+        for (int t = 0; t <= n_tau; ++t) any |= hw[(size_t)t * d] >= 0;
+    }
     int check = 0;
     if (any) {  // rare path: restate the reference loop on the host
         std::vector<hl::cx> g((size_t)ntau1 * m2);
@@ -1151,22 +1084,38 @@ extern "C" int dmftgpu_ft_tau2w(dmftgpu_handle h, int d, int n_freq, int n_tau, 
     const int m2 = d * d;
     const double dt = beta / n_tau;
     hipStream_t s = h->stream;
-    const size_t npart = dft_part_count(n_freq, n_tau, m2, 2, CoefTau2W::PHASE_ROW);
-    size_t need = 2 * (size_t)n_tau * m2 * 16 + (size_t)n_freq * m2 * 16 + (size_t)n_freq * d * 8 + npart * 16 + 8 * 256;
+    const dg::CztPlan cp = dg::czt_plan(n_tau, n_tau, n_freq);
+    const size_t npart = (size_t)cp.in_tiles * m2 * n_freq;
+    size_t need = (size_t)n_tau * m2 * 16 + (size_t)n_freq * m2 * 16 + (size_t)n_freq * d * 8 + npart * 16 + 9 * 256;
     int rc = 0;
     char* base = ft_ws(h, need, &rc);
     if (!base) return rc;
     Carve cv{base};
-    cd* at = cv.take<cd>((size_t)n_tau * m2);
-    cd* bt = cv.take<cd>((size_t)n_tau * m2);
+    cd* gin = cv.take<cd>((size_t)n_tau * m2);
     cd* ah = cv.take<cd>((size_t)n_freq * m2);
     double* wmax = cv.take<double>((size_t)n_freq * d);
-    cd* parts = npart ? cv.take<cd>(npart) : nullptr;
-    hipLaunchKernelGGL(k_ft_segments, dim3(nblk((size_t)n_tau * m2)), dim3(256), 0, s, (const cd*)gtau, m2, n_tau, dt,
-                       at, bt);
+    int* bad = cv.take<int>(1);
+    cd* parts = cv.take<cd>(npart);
+    const cd* tab = czt_tables(h, n_tau, &rc);
+    if (!tab) return rc;
+    hipLaunchKernelGGL(k_ft_gather_tau, dim3((n_tau + kTile - 1) / kTile, (m2 + kTile - 1) / kTile), dim3(256), 0, s,
+                       (const cd*)gtau, m2, n_tau, gin, bad);
     HIPCHK(hipGetLastError());
-    CoefTau2W ct{beta, dt};
-    HIPCHK((launch_dft<CoefTau2W, 2>(n_freq, n_tau, m2, at, bt, (cd*)fw, ct, parts, s)));
+    HIPCHK(dg::launch_czt(cp, true, m2, tab, gin, parts, s));
+    hipLaunchKernelGGL(k_ft_w_finish, dim3((n_freq + kTile - 1) / kTile, (m2 + kTile - 1) / kTile), dim3(256), 0, s, parts,
+                       cp.in_tiles, (const cd*)gtau, m2, n_freq, n_tau, dt, (cd*)fw);
+    HIPCHK(hipGetLastError());
+    // causality test (:551-558): a frequency violates it where (F - F^H)/2i has a positive
+    // eigenvalue.  Negative definite by a margin at every frequency: no violation; otherwise
+    // the eigenvalues are counted
+    HIPCHK(dg::launch_not_posdef((const cd*)fw, d, n_freq, true, bad, s));
+    int hbad = 0;
+    HIPCHK(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    if (!hbad) {
+        if (violations) *violations = 0;
+        return DMFTGPU_OK;
+    }
     hipLaunchKernelGGL(k_antiherm, dim3(nblk((size_t)n_freq * m2)), dim3(256), 0, s, (const cd*)fw, d, n_freq, ah);
     HIPCHK(hipGetLastError());
     HIPCHK(dg::launch_herm_eig(ah, d, 0, d, nullptr, 0, wmax, nullptr, n_freq, s));
@@ -1200,7 +1149,7 @@ extern "C" int dmftgpu_ft_w2tau_points(dmftgpu_handle h, int d, int n_freq, doub
     std::vector<hl::cx> A1, A2;
     std::vector<double> e1, e2;
     tail_setup(d, m1, mm2, m3, A1, e1, A2, e2);
-    const size_t npart = dft_part_count(n_points, n_freq, m2, 1, CoefW2Tau::PHASE_ROW);
+    const size_t npart = dft_part_count(n_points, n_freq, m2);
     size_t need = (size_t)n_freq * m2 * 16 + (size_t)n_points * m2 * 16 + 4 * (size_t)m2 * 16 + 4 * (size_t)d * 8 +
                   (size_t)n_points * 8 + npart * 16 + 16 * 256;
     int rc = 0;
@@ -1210,23 +1159,17 @@ extern "C" int dmftgpu_ft_w2tau_points(dmftgpu_handle h, int d, int n_freq, doub
     cd* D = cv.take<cd>((size_t)n_freq * m2);
     cd* X = cv.take<cd>((size_t)n_points * m2);
     cd* parts = npart ? cv.take<cd>(npart) : nullptr;
-    cd* dA1 = cv.take<cd>(m2);
-    cd* dA2 = cv.take<cd>(m2);
-    double* de1 = cv.take<double>(d);
-    double* de2 = cv.take<double>(d);
+    const TailDev tl = tail_upload(h, d, A1, e1, A2, e2, cv, &rc);
+    if (rc) return rc;
     double* dtau = cv.take<double>(n_points);
-    HIPCHK(hipMemcpyAsync(dA1, A1.data(), sizeof(cd) * m2, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(dA2, A2.data(), sizeof(cd) * m2, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(de1, e1.data(), sizeof(double) * d, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(de2, e2.data(), sizeof(double) * d, hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(dtau, taus_host, sizeof(double) * n_points, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_ft_subtract_tail, dim3(nblk((size_t)n_freq * m2)), dim3(256), 0, s, (const cd*)fw, d, n_freq,
-                       beta, dA1, de1, dA2, de2, D);
+    hipLaunchKernelGGL(k_ft_subtract_tail, dim3((n_freq + kTile - 1) / kTile, (m2 + kTile - 1) / kTile), dim3(256), 0, s,
+                       (const cd*)fw, d, n_freq, beta, tl.A1, tl.e1, tl.A2, tl.e2, D, (size_t)m2, (size_t)1, (int*)nullptr);
     HIPCHK(hipGetLastError());
-    CoefW2Tau cw{beta, kPi / beta, (2 * kPi) / beta, 0.0, dtau};
-    HIPCHK((launch_dft<CoefW2Tau, 1>(n_points, n_freq, m2, D, nullptr, X, cw, parts, s)));
-    hipLaunchKernelGGL(k_ft_finish, dim3(nblk((size_t)n_points * m2)), dim3(256), 0, s, X, d, n_points, beta, 0.0,
-                       (const double*)dtau, dA1, de1, dA2, de2, (cd*)out);
+    HIPCHK(launch_dft(n_points, n_freq, m2, D, X, TauPoints{kPi / beta, (2 * kPi) / beta, dtau}, parts, s));
+    hipLaunchKernelGGL(k_ft_finish, dim3((n_points + kTile - 1) / kTile, (m2 + kTile - 1) / kTile), dim3(256), 0, s,
+                       FtSums{X, 1, 0, (size_t)m2, 1, -1}, d, n_points, beta, 0.0, (const double*)dtau, tl.A1, tl.e1, tl.A2,
+                       tl.e2, (cd*)out);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(s));
     return DMFTGPU_OK;

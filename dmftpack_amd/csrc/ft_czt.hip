@@ -1,0 +1,296 @@
+// The sums of FourierTransform_tau (FourierTransform.cpp:46-90) and FT_t_to_w (:531-547)
+// on the uniform tau grid as chirp-z transforms.
+//
+// With tau_j = j beta/N and w_n = pi (2n+1)/beta the phase w_n tau_j is pi (2n+1) j / N,
+// an integer multiple of pi/N: both sums are transforms by e^{-+ 2 pi i n j/N} with an
+// extra factor e^{-+ i pi j/N}, for any N and any number of frequencies.  Writing
+// 2ab = a^2 + b^2 - (b-a)^2 turns a tile of 2048 inputs x 2048 outputs into a
+// convolution with the chirp e^{i pi k^2/N}, done by FFTs of length 4096; the tile's
+// offsets only add phases that are linear in a or in b.  The phases are exact: integer
+// multiples reduced mod 2N, looked up in one table of e^{i pi m/N}.
+//
+// Cost: 2 FFTs per tile and matrix element instead of 2048^2 products.  At d = 10, N_freq =
+// 4096, N_tau = 8192 the kernel takes 64 us (iw -> tau) and 67 us (tau -> iw) where the dense sums
+// on FP64 MFMA took 739 and 1197 us; down to one tile (N_freq = 64) the whole call is no slower
+// either, so there is no dense form on the uniform grid.  Errors against 64-bit sums with
+// exact phases fall too (2.6e-14 -> 4e-15 at that size): the dense form rounded w tau.
+//
+// The FFT: 256 threads hold 16 elements each (element t + 256 r in register r), three
+// radix-16 passes with two exchanges through LDS (68 KB with one pad element in 16, so
+// that the strided stores of the first pass spread over the banks; two workgroups per
+// CU).  Input and output order are the same, so the product with the chirp's spectrum and
+// the second FFT follow in registers.
+#include "ft_czt.hpp"
+
+namespace dg {
+
+namespace {
+
+__device__ __forceinline__ cd mul_mi(cd a) { return cd{a.y, -a.x}; }  // -i a
+
+// x[0..3] -> DFT of length 4, e^{-2 pi i jk/4}
+__device__ __forceinline__ void dft4(cd& a, cd& b, cd& c, cd& d)
+{
+    const cd s0 = cadd(a, c), s1 = csub(a, c), s2 = cadd(b, d), s3 = mul_mi(csub(b, d));
+    a = cadd(s0, s2);
+    b = cadd(s1, s3);
+    c = csub(s0, s2);
+    d = csub(s1, s3);
+}
+
+// v -> DFT of length 16, natural order
+__device__ __forceinline__ void dft16(cd (&v)[16])
+{
+    constexpr double C1 = 0.92387953251128675613, S1 = 0.38268343236508977173, R = 0.70710678118654752440;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dft4(v[i], v[i + 4], v[i + 8], v[i + 12]);
+    // twiddles e^{-2 pi i i k/16}, row k = element i + 4k
+    v[5] = cmul(v[5], cd{C1, -S1});
+    v[6] = cmul(v[6], cd{R, -R});
+    v[7] = cmul(v[7], cd{S1, -C1});
+    v[9] = cmul(v[9], cd{R, -R});
+    v[10] = mul_mi(v[10]);
+    v[11] = cmul(v[11], cd{-R, -R});
+    v[13] = cmul(v[13], cd{S1, -C1});
+    v[14] = cmul(v[14], cd{-R, -R});
+    v[15] = cmul(v[15], cd{-C1, S1});
+    cd o[16];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        cd a = v[4 * k], b = v[4 * k + 1], c = v[4 * k + 2], d = v[4 * k + 3];
+        dft4(a, b, c, d);
+        o[k] = a;
+        o[k + 4] = b;
+        o[k + 8] = c;
+        o[k + 12] = d;
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = o[r];
+}
+
+__device__ __forceinline__ int pad(int i) { return i + (i >> 4); }
+constexpr int kFftLds = kCztM + kCztM / 16;
+
+// FFT of length 4096 of the elements t + 256 r (thread t, register r), same order out
+__device__ void fft4096(cd (&v)[16], cd* sm, const cd* __restrict__ tw, int t)
+{
+    dft16(v);
+    __syncthreads();  // sm is free again
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sm[pad(16 * t + r)] = v[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = sm[pad(t + 256 * r)];
+    const int k1 = t & 15;
+#pragma unroll
+    for (int r = 1; r < 16; ++r) v[r] = cmul(v[r], tw[16 * r * k1]);
+    dft16(v);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sm[pad((t >> 4) * 256 + k1 + 16 * r)] = v[r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = sm[pad(t + 256 * r)];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) v[r] = cmul(v[r], tw[r * t]);
+    dft16(v);
+}
+
+// m mod 2N for 0 <= m < 2^52
+__device__ __forceinline__ int mod2n(long long m, int n2, double inv)
+{
+    int r = (int)(m - (long long)n2 * (long long)((double)m * inv));
+    if (r < 0) r += n2;
+    return r >= n2 ? r - n2 : r;
+}
+
+__global__ __launch_bounds__(256) void k_czt_phases(int n_tau, cd* __restrict__ tab)
+{
+    const int t = blockIdx.x * 256 + threadIdx.x, n2 = 2 * n_tau;
+    double s, c;
+    if (t < n2) {
+        sincospi((double)t / n_tau, &s, &c);
+        tab[t] = cd{c, s};
+    } else if (t < n2 + kCztM) {
+        sincospi((double)(t - n2) / (kCztM / 2), &s, &c);
+        tab[t] = cd{c, -s};
+    }
+}
+
+// spectrum of the chirp e^{i pi k^2/N}, k = -2048..2047 at k mod 4096, with the 1/4096 of
+// the inverse FFT
+__global__ __launch_bounds__(256) void k_czt_filter(int n_tau, cd* __restrict__ tab)
+{
+    extern __shared__ cd sm[];
+    const int t = threadIdx.x, n2 = 2 * n_tau;
+    const cd* tw = tab + n2;
+    const double inv = 1.0 / n2;
+    cd v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int i = t + 256 * r, k = i < kCztM / 2 ? i : kCztM - i;
+        v[r] = tab[mod2n((long long)k * k, n2, inv)];
+    }
+    fft4096(v, sm, tw, t);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) tab[n2 + kCztM + t + 256 * r] = cscale(v[r], 1.0 / kCztM);
+}
+
+// One tile: inputs a0..a0+2047 of element e, outputs b0..b0+2047 (grid: element, output
+// tile, input tile).  Phase -+ pi (2f+1) t/N with (f, t) = (input, output) for iw -> tau and
+// (output, input) for tau -> iw; the + sign by conjugating input and output.
+template <bool TO_W>
+__global__ __launch_bounds__(256) void k_czt(CztPlan p, int m2, const cd* __restrict__ tab, const cd* __restrict__ in,
+                                             cd* __restrict__ parts)
+{
+    extern __shared__ cd sm[];
+    const int t = threadIdx.x, e = blockIdx.x, n2 = 2 * p.n_tau;
+    const long long b0 = (long long)blockIdx.y * kCztTile, a0 = (long long)blockIdx.z * kCztTile;
+    const cd *tw = tab + n2, *filt = tw + kCztM;
+    const double inv = 1.0 / n2;
+    const cd* x = in + (size_t)e * p.ld_in + a0;
+    const int na = min(kCztTile, p.n_in - (int)a0), nb = min(kCztTile, p.n_out - (int)b0);
+    cd v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int a = t + 256 * r;
+        v[r] = cd{0.0, 0.0};
+        if (r < 8 && a < na) {
+            cd g = x[a];
+            if (TO_W) g.y = -g.y;
+            // 2 a b0 + a^2, and the half step (2f+1) t: + t for the tau index on the input side
+            const long long m = 2 * (long long)a * b0 + (long long)a * a + (TO_W ? a0 + a : 0);
+            v[r] = cmulc(g, tab[mod2n(m, n2, inv)]);
+        }
+    }
+    fft4096(v, sm, tw, t);
+    // inverse FFT as conj(FFT(conj(.)))
+#pragma unroll
+    for (int r = 0; r < 16; ++r) v[r] = cconj(cmul(v[r], filt[t + 256 * r]));
+    fft4096(v, sm, tw, t);
+    cd* y = parts + ((size_t)blockIdx.z * m2 + e) * p.ld_out + b0;
+    const long long ab = mod2n(2 * a0 * b0, n2, inv);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+        const int b = t + 256 * r;
+        if (b < nb) {
+            const long long m = ab + 2 * (long long)b * a0 + (long long)b * b + (TO_W ? 0 : b0 + b);
+            const cd w = cmulc(cconj(v[r]), tab[mod2n(m, n2, inv)]);
+            y[b] = TO_W ? cconj(w) : w;
+        }
+    }
+}
+
+// Definiteness of M_b = -X_b, or of -(X_b - X_b^H)/2i (ANTI), by the pivots of its elimination: a
+// slot of N lanes per matrix, lane c holds column c, the pivot column is read from its lane.
+// M_b counts as positive definite only by a margin of 1e-13 of its trace (>= its largest
+// eigenvalue), a hundred times the rounding of an eigenvalue.
+template <int N, bool ANTI>
+__global__ __launch_bounds__(64) void k_not_posdef(const cd* __restrict__ X, int d, int count, int* __restrict__ bad)
+{
+    const int lane = threadIdx.x, c = lane % N, sl = lane / N;
+    const int b = blockIdx.x * (64 / N) + sl;
+    const bool live = b < count && c < d;
+    const cd* M = X + (size_t)(b < count ? b : count - 1) * d * d;
+    cd col[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        cd v = cd{i == c ? 1.0 : 0.0, 0.0};
+        if (live && i < d) {
+            if (ANTI) {  // -(x - conj(y))/2i
+                const cd x = M[i + c * d], y = M[c + i * d];
+                v = cd{-0.5 * (x.y + y.y), 0.5 * (x.x - y.x)};
+            } else {  // Hermitian to the last bit: the lower triangle
+                const cd m = i >= c ? M[i + c * d] : cconj(M[c + i * d]);
+                v = cd{-m.x, i == c ? 0.0 : -m.y};
+            }
+        }
+        col[i] = v;
+    }
+    double tr = 0.0;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        if (i == c && live) tr = col[i].x;
+#pragma unroll
+    for (int o = N / 2; o > 0; o >>= 1) tr += __shfl_xor(tr, o, N);
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+        if (i == c && live) col[i].x -= 1e-13 * tr;
+    bool ok = true;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        if (j < d) {
+            const double p = __shfl(col[j].x, j, N);
+            ok = ok && p > 0.0 && p < 1e300;  // false for NaN and infinities
+            const cd f = cscale(col[j], 1.0 / p);  // A_jc / p
+#pragma unroll
+            for (int i = j + 1; i < N; ++i) {
+                if (i >= d) continue;
+                const cd l = cd{__shfl(col[i].x, j, N), __shfl(col[i].y, j, N)};
+                col[i] = cfms(l, f, col[i]);
+            }
+        }
+    }
+    if (live && c == 0 && !ok) atomicAdd(bad, 1);
+}
+
+}  // namespace
+
+hipError_t launch_czt_tables(int n_tau, cd* tab, hipStream_t s)
+{
+    const int total = 2 * n_tau + kCztM;
+    hipLaunchKernelGGL(k_czt_phases, dim3((total + 255) / 256), dim3(256), 0, s, n_tau, tab);
+    const int shm = (int)(sizeof(cd) * kFftLds);
+    hipError_t e = hipFuncSetAttribute((const void*)k_czt_filter, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_czt_filter, dim3(1), dim3(256), shm, s, n_tau, tab);
+    return hipGetLastError();
+}
+
+CztPlan czt_plan(int n_tau, int n_in, int n_out)
+{
+    CztPlan p;
+    p.n_tau = n_tau;
+    p.n_in = n_in;
+    p.n_out = n_out;
+    p.in_tiles = (n_in + kCztTile - 1) / kCztTile;
+    p.out_tiles = (n_out + kCztTile - 1) / kCztTile;
+    p.ld_in = n_in;
+    p.ld_out = n_out;
+    return p;
+}
+
+hipError_t launch_czt(const CztPlan& p, bool to_w, int m2, const cd* tab, const cd* in, cd* parts, hipStream_t s)
+{
+    const int shm = (int)(sizeof(cd) * kFftLds);
+    const dim3 grid(m2, p.out_tiles, p.in_tiles);
+    hipError_t e;
+    if (to_w) {
+        e = hipFuncSetAttribute((const void*)k_czt<true>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL((k_czt<true>), grid, dim3(256), shm, s, p, m2, tab, in, parts);
+    } else {
+        e = hipFuncSetAttribute((const void*)k_czt<false>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL((k_czt<false>), grid, dim3(256), shm, s, p, m2, tab, in, parts);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_not_posdef(const cd* X, int d, int count, bool anti, int* bad, hipStream_t s)
+{
+#define P_(N)                                                                                                       \
+    {                                                                                                               \
+        const dim3 grid((count + 64 / N - 1) / (64 / N));                                                           \
+        if (anti) hipLaunchKernelGGL((k_not_posdef<N, true>), grid, dim3(64), 0, s, X, d, count, bad);              \
+        else hipLaunchKernelGGL((k_not_posdef<N, false>), grid, dim3(64), 0, s, X, d, count, bad);                  \
+        return hipGetLastError();                                                                                   \
+    }
+    if (d <= 4) P_(4)
+    if (d <= 8) P_(8)
+    if (d <= 16) P_(16)
+    P_(32)
+#undef P_
+}
+
+}  // namespace dg
