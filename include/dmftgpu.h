@@ -327,7 +327,8 @@ int dmftgpu_hyb_delta(dmftgpu_handle h, int nc, int n_freq, double beta, double 
  *   hop_idx [n_hop][5]  HOST int: R1 R2 R3 i j (0-based orbitals i, j < n)
  *   hop     [n_hop]     HOST complex t
  *   kphase  [n_k][3]    k_x a_x, k_y a_y, k_z a_z
- *   Hk      [n_k][n][n] output; hops of one element are summed in list order. */
+ *   Hk      [n_k][n][n] output; hops of one element are summed in list order, or, in lists
+ *           dense in (R, i, j), in the order in which the R vectors first appear. */
 int dmftgpu_hk_from_hr(dmftgpu_handle h, int n, int n_hop, const int* hop_idx, const double* hop, int n_k,
                        const double* kphase, double* Hk);
 
