@@ -7,15 +7,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <array>
 #include <cstdlib>
 #include <cmath>
-#include <map>
 #include <vector>
 
 #include "../../include/dmftgpu.h"
 #include "api_internal.hpp"
 #include "gj.hpp"
+#include "r_index.hpp"
 
 using dg::cd;
 using namespace dgi;
@@ -205,43 +204,6 @@ __global__ __launch_bounds__(256) void k_hk_dense(const cd* __restrict__ T, int 
 #pragma unroll
     for (int q = 0; q < KD; ++q)
         if (kt + q < nk) Hk[(size_t)(kt + q) * nn + e] = acc[q];
-}
-
-// Index of each hop's R among the distinct ones (in order of first appearance)
-struct RIndex {
-    std::vector<int4> R;
-    std::vector<int> of;  // per hop
-};
-
-RIndex index_r(int n_hop, const int* hop_idx)
-{
-    RIndex x;
-    x.of.resize(n_hop);
-    long long lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-    for (int q = 0; q < n_hop; ++q)
-        for (int c = 0; c < 3; ++c) {
-            lo[c] = std::min<long long>(lo[c], hop_idx[5 * q + c]);
-            hi[c] = std::max<long long>(hi[c], hop_idx[5 * q + c]);
-        }
-    const long long e0 = hi[0] - lo[0] + 1, e1 = hi[1] - lo[1] + 1, e2 = hi[2] - lo[2] + 1;
-    const bool grid = e0 < 65536 && e1 < 65536 && e2 < 65536 && e0 * e1 < 65536 && e0 * e1 * e2 < 65536;
-    std::vector<int> at(grid ? e0 * e1 * e2 : 0, -1);
-    std::map<std::array<int, 3>, int> far;  // scattered R vectors
-    int last = -1;
-    for (int q = 0; q < n_hop; ++q) {
-        const int* v = hop_idx + 5 * q;
-        if (last < 0 || x.R[last].x != v[0] || x.R[last].y != v[1] || x.R[last].z != v[2]) {
-            int* slot = grid ? &at[((v[0] - lo[0]) * e1 + (v[1] - lo[1])) * e2 + (v[2] - lo[2])]
-                             : &far.emplace(std::array<int, 3>{v[0], v[1], v[2]}, -1).first->second;
-            if (*slot < 0) {
-                *slot = (int)x.R.size();
-                x.R.push_back(int4{v[0], v[1], v[2], 0});
-            }
-            last = *slot;
-        }
-        x.of[q] = last;
-    }
-    return x;
 }
 
 }  // namespace

@@ -10,11 +10,12 @@
 //   DDir = S^{-1} D,  DD = S^{-1} D S^{-1}     (:49-50)
 // then dmr[x][r] = sum_k Y_x(k)(i0, m0) exp(+i kphase_k . R) / n_k_global, (:67-86).
 //
-// All of it is O(n_orb^3) per k next to the lattice path's O(n^3) per (k, iw),
-// so the kernels are plain: a batched square complex GEMM with 16x16 LDS
-// tiles, an in-place Gauss-Jordan inverse with partial pivoting (one
-// workgroup per matrix, the matrix in global memory), a gather that builds K,
-// and a k -> R sum that stages a tile of k values in LDS and gives every
+// Up to n_orb = 32 one kernel takes a k point from its inputs to D, DDir and DD
+// (upfold_small.hip).  Above that the kernels are plain: a batched square complex
+// GEMM with 16x16 LDS tiles, an in-place Gauss-Jordan inverse with partial
+// pivoting (one workgroup per matrix) and a gather that builds K.  The R sums of
+// lists dense in (R, element) are one sum per distinct R and element
+// (upfold_small.hip); others stage a tile of k values in LDS and give every
 // thread one R of one matrix element.  k is processed in chunks that bound the
 // scratch.
 #include <hip/hip_runtime.h>
@@ -26,6 +27,8 @@
 
 #include "../../include/dmftgpu.h"
 #include "api_internal.hpp"
+#include "r_index.hpp"
+#include "upfold_small.hpp"
 
 using dg::cd;
 using namespace dgi;
@@ -421,47 +424,59 @@ extern "C" int dmftgpu_upfold_density(dmftgpu_handle h, int n, int n_orb, int n_
         return fail(h, DMFTGPU_ERR_ARG, "null argument");
     if (n_r > 0 && (!r_idx || !dmr)) return fail(h, DMFTGPU_ERR_ARG, "n_r > 0 needs r_idx and dmr");
     if (n_r == 0 && !dm_k) return fail(h, DMFTGPU_ERR_ARG, "nothing to compute: n_r = 0 and dm_k = NULL");
-    // FromValToKS -> band-to-window map, checked: each k's window bands are distinct
-    std::vector<int> inv((size_t)n_k * n_orb, -1);
-    for (int k = 0; k < n_k; ++k)
+    const bool small = n_orb <= dg::kUpfoldSmall;
+    // FromValToKS -> band-to-window map, checked: each k's window bands are distinct (the
+    // fused kernel takes FromValToKS itself)
+    std::vector<int> inv(small ? 0 : (size_t)n_k * n_orb, -1);
+    for (int k = 0; k < n_k; ++k) {
+        unsigned seen = 0;
         for (int i = 0; i < n; ++i) {
             const int b = val_to_ks[(size_t)k * n + i];
             if (b == -1) continue;  // a padded band (NBAND[k] < n): no KS band
             if (b < 0 || b >= n_orb) return fail(h, DMFTGPU_ERR_ARG, "val_to_ks[%d][%d]=%d outside 0..%d", k, i, b, n_orb - 1);
-            if (inv[(size_t)k * n_orb + b] >= 0)
+            if (small ? (seen >> b & 1u) != 0 : inv[(size_t)k * n_orb + b] >= 0)
                 return fail(h, DMFTGPU_ERR_ARG, "val_to_ks[%d] names band %d twice", k, b);
-            inv[(size_t)k * n_orb + b] = i;
+            if (small) seen |= 1u << b;
+            else inv[(size_t)k * n_orb + b] = i;
         }
+    }
     // R list grouped by matrix element (stable), work items of <= 256 R
     const size_t oo = (size_t)n_orb * n_orb, nn = (size_t)n * n;
-    std::vector<int> order(n_r);
     for (int r = 0; r < n_r; ++r) {
         const int i0 = r_idx[5 * (size_t)r + 3], m0 = r_idx[5 * (size_t)r + 4];
         if (i0 < 0 || i0 >= n_orb || m0 < 0 || m0 >= n_orb)
             return fail(h, DMFTGPU_ERR_ARG, "r_idx[%d]: orbital pair (%d,%d) outside 0..%d", r, i0, m0, n_orb - 1);
-        order[r] = r;
     }
+    // at least half of all (R, element) pairs listed: a sum per distinct R and element, then a
+    // gather (below that the unlisted sums cost more than the per-entry phases)
+    const RIndex ri = index_r(n_r, r_idx);
+    const int n_rv = (int)ri.R.size();
+    const int nx = overlap ? 3 : 1;
+    const bool dense = n_r > 0 && (double)n_rv * oo <= 2.0 * n_r && (size_t)dg::rs_pad(n_rv) * nx <= 65535;
+    std::vector<int> order(dense ? 0 : n_r);
+    for (size_t r = 0; r < order.size(); ++r) order[r] = (int)r;
+    const int n_ent = (int)order.size();  // entries of the per-entry R sums (0 for dense lists)
     auto elem = [&](int r) { return (size_t)r_idx[5 * (size_t)r + 3] + (size_t)r_idx[5 * (size_t)r + 4] * n_orb; };
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return elem(a) < elem(b); });
-    std::vector<int> rs(4 * (size_t)std::max(n_r, 1), 0);
+    std::vector<int> rs(4 * (size_t)std::max(n_ent, 1), 0);
     std::vector<RItem> items;
-    for (int q = 0; q < n_r;) {
+    for (int q = 0; q < n_ent;) {
         const size_t e = elem(order[q]);
         int q1 = q;
-        while (q1 < n_r && elem(order[q1]) == e) ++q1;
+        while (q1 < n_ent && elem(order[q1]) == e) ++q1;
         for (int a = q; a < q1; a += 256) items.push_back(RItem{(int)e, a, std::min(q1, a + 256), 0});
         q = q1;
     }
     // the axes kernel's items: runs of <= 256 entries over <= DMR_EM elements
     std::vector<RItemE> items_e;
-    std::vector<int> ielem, eslot(std::max(n_r, 1), 0);
+    std::vector<int> ielem, eslot(std::max(n_ent, 1), 0);
     {
         RItemE cur{0, 0, 0, 0};
         bool open = false;
-        for (int q = 0; q < n_r;) {
+        for (int q = 0; q < n_ent;) {
             const size_t e = elem(order[q]);
             int q1 = q;
-            while (q1 < n_r && elem(order[q1]) == e) ++q1;
+            while (q1 < n_ent && elem(order[q1]) == e) ++q1;
             for (int a = q; a < q1;) {
                 if (!open || cur.q1 - cur.q0 == 256 || cur.ne == DMR_EM) {
                     if (open) items_e.push_back(cur);
@@ -482,59 +497,91 @@ extern "C" int dmftgpu_upfold_density(dmftgpu_handle h, int n, int n_orb, int n_
     int rmax = 0;  // the R sums take the per-axis phase tables when |R_a| <= 16
     for (int r = 0; r < n_r; ++r)
         for (int c = 0; c < 3; ++c) rmax = std::max(rmax, std::abs(r_idx[5 * (size_t)r + c]));
-    const bool axes = n_r > 0 && rmax <= 16;
+    const bool axes = n_ent > 0 && rmax <= 16;
     const int nrr = 2 * rmax + 1;
     const int kt = std::max(16, std::min(256, (48 * 1024 / (int)sizeof(cd)) / (3 * DMR_EM + 3 * nrr)));
     // k segments of the R sums: about 1024 workgroups per launch, each segment >= 2 tiles
     const int nseg_max = axes ? std::max(1, std::min(16, (1024 + (int)items_e.size() - 1) / (int)items_e.size())) : 1;
-    for (int q = 0; q < n_r; ++q) {
+    for (int q = 0; q < n_ent; ++q) {
         const int r = order[q];
         rs[4 * (size_t)q] = r_idx[5 * (size_t)r];
         rs[4 * (size_t)q + 1] = r_idx[5 * (size_t)r + 1];
         rs[4 * (size_t)q + 2] = r_idx[5 * (size_t)r + 2];
         rs[4 * (size_t)q + 3] = r;
     }
-    // scratch: maps + per-chunk W1, W2, E (+ D) [oo], T1, M [nn] and the axis phases per k
-    const size_t per_k = (4 * oo + 2 * nn + (axes ? 3 * (size_t)nrr : 0)) * sizeof(cd);
+    std::vector<int2> of(dense ? n_r : 0);  // (R, element) of every entry
+    for (size_t r = 0; r < of.size(); ++r) of[r] = int2{ri.of[r], (int)elem((int)r)};
+    // scratch: maps + per chunk of k the matrices and the R sums' phases.  Fused: D, DDir, DD;
+    // otherwise W1, W2, E, D [oo] and T1, M [nn]
+    const size_t n_pad = dense ? dg::rs_pad(n_rv) : 0;
+    const size_t per_k = ((small ? (overlap ? 3 : 1) * oo : 4 * oo + 2 * nn) + (axes ? 3 * (size_t)nrr : 0) + n_pad) *
+                         sizeof(cd);
     size_t kc_cap = std::min<size_t>({(size_t)n_k, UPF_CHUNK_BYTES / per_k, 65535});
     if (h->upfold_chunk > 0) kc_cap = std::min<size_t>(kc_cap, (size_t)h->upfold_chunk);
     const int kc_max = (int)std::max<size_t>(1, kc_cap);
-    const size_t b_inv = align256(inv.size() * sizeof(int));
-    const size_t b_rs = align256(rs.size() * sizeof(int));
-    const size_t b_items = align256(std::max<size_t>(items.size(), 1) * sizeof(RItem));
-    const size_t b_items_e = align256(std::max<size_t>(items_e.size(), 1) * sizeof(RItemE));
-    const size_t b_ielem = align256(std::max<size_t>(ielem.size(), 1) * sizeof(int));
-    const size_t b_eslot = align256(eslot.size() * sizeof(int));
-    const size_t b_part = axes ? align256((size_t)nseg_max * 3 * n_r * sizeof(cd)) : 0;
-    const size_t b_lists = b_items + b_items_e + b_ielem + b_eslot + b_part;
-    const size_t b_flag = 256;
-    const size_t b_chunk = align256(per_k * kc_max);
+    // dense R sums: k segments for about 4096 wavefronts, of at least 16 k, 128 MiB of partial sums
+    int rseg_max = 1;
+    if (dense) {
+        const size_t waves = (oo + 63) / 64 * (n_pad / dg::kRsTile) * nx, bytes = (size_t)nx * n_rv * oo * sizeof(cd);
+        rseg_max = (int)std::max<size_t>(1, std::min<size_t>({4096 / waves + 1, (size_t)kc_max / 16, ((size_t)128 << 20) / bytes}));
+    }
+    size_t total = 0;
+    auto region = [&](size_t bytes) {
+        const size_t o = total;
+        total += align256(std::max<size_t>(bytes, 1));
+        return o;
+    };
+    const size_t o_inv = region((small ? (size_t)n_k * n : inv.size()) * sizeof(int));
+    const size_t o_rs = region(rs.size() * sizeof(int));
+    const size_t o_items = region(items.size() * sizeof(RItem));
+    const size_t o_items_e = region(items_e.size() * sizeof(RItemE));
+    const size_t o_ielem = region(ielem.size() * sizeof(int));
+    const size_t o_eslot = region(eslot.size() * sizeof(int));
+    const size_t o_rv = region((size_t)n_rv * sizeof(int4));
+    const size_t o_of = region(of.size() * sizeof(int2));
+    const size_t o_part = region(axes ? (size_t)nseg_max * 3 * n_ent * sizeof(cd)
+                                      : dense ? (size_t)rseg_max * nx * n_rv * oo * sizeof(cd) : 0);
+    const size_t o_flag = region(sizeof(int));
+    const size_t o_chunk = region(per_k * kc_max);
     hipError_t e;
-    char* base = (char*)h->ws.get(b_inv + b_rs + b_lists + b_flag + b_chunk, &e);
+    char* base = (char*)h->ws.get(total, &e);
     if (!base) return fail(h, DMFTGPU_ERR_HIP, "workspace: %s", hipGetErrorString(e));
-    int* d_inv = (int*)base;
-    int4* d_rs = (int4*)(base + b_inv);
-    RItem* d_items = (RItem*)(base + b_inv + b_rs);
-    RItemE* d_items_e = (RItemE*)(base + b_inv + b_rs + b_items);
-    int* d_ielem = (int*)(base + b_inv + b_rs + b_items + b_items_e);
-    int* d_eslot = (int*)(base + b_inv + b_rs + b_items + b_items_e + b_ielem);
-    cd* d_part = (cd*)(base + b_inv + b_rs + b_items + b_items_e + b_ielem + b_eslot);
-    int* d_flag = (int*)(base + b_inv + b_rs + b_lists);
-    cd* W1 = (cd*)(base + b_inv + b_rs + b_lists + b_flag);
-    cd* W2 = W1 + oo * kc_max;
-    cd* Eb = W2 + oo * kc_max;
+    int* d_inv = (int*)(base + o_inv);  // small: FromValToKS
+    int4* d_rs = (int4*)(base + o_rs);
+    RItem* d_items = (RItem*)(base + o_items);
+    RItemE* d_items_e = (RItemE*)(base + o_items_e);
+    int* d_ielem = (int*)(base + o_ielem);
+    int* d_eslot = (int*)(base + o_eslot);
+    int4* d_rv = (int4*)(base + o_rv);
+    int2* d_of = (int2*)(base + o_of);
+    cd* d_part = (cd*)(base + o_part);
+    int* d_flag = (int*)(base + o_flag);
+    cd* W1 = (cd*)(base + o_chunk);  // small: D
+    cd* W2 = W1 + oo * kc_max;       // small: DDir
+    cd* Eb = W2 + oo * kc_max;       // small: DD
     cd* Dw = Eb + oo * kc_max;
     cd* T1 = Dw + oo * kc_max;
     cd* Mb = T1 + nn * kc_max;
-    cd* Ptab = Mb + nn * kc_max;  // axes: [kc][3][2 rmax + 1]
+    // phases after the matrices: axes [kc][3][2 rmax + 1], dense [kc][n_pad]
+    cd* Ptab = small ? W1 + (overlap ? 3 : 1) * oo * kc_max : Mb + nn * kc_max;
     hipStream_t s = h->stream;
-    HIPCHK(hipMemcpyAsync(d_inv, inv.data(), inv.size() * sizeof(int), hipMemcpyHostToDevice, s));
+    auto put = [&](void* dst, const void* src, size_t bytes) {
+        return bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s) : hipSuccess;
+    };
+    if (small) HIPCHK(put(d_inv, val_to_ks, (size_t)n_k * n * sizeof(int)));
+    else HIPCHK(put(d_inv, inv.data(), inv.size() * sizeof(int)));
+    if (n_ent > 0) {
+        HIPCHK(put(d_rs, rs.data(), rs.size() * sizeof(int)));
+        HIPCHK(put(d_items, items.data(), items.size() * sizeof(RItem)));
+        HIPCHK(put(d_items_e, items_e.data(), items_e.size() * sizeof(RItemE)));
+        HIPCHK(put(d_ielem, ielem.data(), ielem.size() * sizeof(int)));
+        HIPCHK(put(d_eslot, eslot.data(), eslot.size() * sizeof(int)));
+    }
+    if (dense) {
+        HIPCHK(put(d_rv, ri.R.data(), (size_t)n_rv * sizeof(int4)));
+        HIPCHK(put(d_of, of.data(), of.size() * sizeof(int2)));
+    }
     if (n_r > 0) {
-        HIPCHK(hipMemcpyAsync(d_rs, rs.data(), rs.size() * sizeof(int), hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemcpyAsync(d_items, items.data(), items.size() * sizeof(RItem), hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemcpyAsync(d_items_e, items_e.data(), items_e.size() * sizeof(RItemE), hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemcpyAsync(d_ielem, ielem.data(), ielem.size() * sizeof(int), hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemcpyAsync(d_eslot, eslot.data(), eslot.size() * sizeof(int), hipMemcpyHostToDevice, s));
         const size_t cnt = 3 * (size_t)n_r;
         hipLaunchKernelGGL(k_zero, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, (cd*)dmr, cnt);
         HIPCHK(hipGetLastError());
@@ -547,31 +594,45 @@ extern "C" int dmftgpu_upfold_density(dmftgpu_handle h, int n, int n_orb, int n_
     for (int k0 = 0; k0 < n_k; k0 += kc_max) {
         const int kc = std::min(kc_max, n_k - k0);
         const size_t ko = (size_t)k0 * oo, kn = (size_t)k0 * nn;
-        cd* D = dm_k ? (cd*)dm_k + ko : Dw;
-        // E = (T^{-1})^H K_o
-        HIPCHK(hipMemcpyAsync(W1, Tm + ko, oo * kc * sizeof(cd), hipMemcpyDeviceToDevice, s));
-        HIPCHK(gj_inverse(n_orb, kc, W1, d_flag, s));
-        HIPCHK((zgemm_sq<true, false>(n_orb, kc, W1, Ko + ko, Eb, s)));
-        // M = C^H (X C)
-        HIPCHK((zgemm_sq<false, false>(n, kc, X + kn, Cb + kn, T1, s)));
-        HIPCHK((zgemm_sq<true, false>(n, kc, Cb + kn, T1, Mb, s)));
-        // K, then D = (E K) E^H
-        const size_t tot = oo * kc;
-        hipLaunchKernelGGL(k_upfold_assemble, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, Mb,
-                           ks_energy + (size_t)k0 * n_orb, d_inv + (size_t)k0 * n_orb, n, n_orb, kc, beta, mu, W1);
-        HIPCHK(hipGetLastError());
-        HIPCHK((zgemm_sq<false, false>(n_orb, kc, Eb, W1, W2, s)));
-        HIPCHK((zgemm_sq<false, true>(n_orb, kc, W2, Eb, D, s)));
+        cd* D = dm_k ? (cd*)dm_k + ko : small ? W1 : Dw;
         const cd *DD = D, *DDir = D;
-        if (Sm) {  // DDir = S^{-1} D (W2), DD = DDir S^{-1} (Eb)
-            HIPCHK(hipMemcpyAsync(W1, Sm + ko, oo * kc * sizeof(cd), hipMemcpyDeviceToDevice, s));
+        if (small) {
+            const dg::UpfoldArgs ua{n, n_orb, kc, beta, mu, X + kn, Cb + kn, Tm + ko, Ko + ko, Sm ? Sm + ko : nullptr,
+                                    ks_energy + (size_t)k0 * n_orb, d_inv + (size_t)k0 * n, D, W2, Eb, d_flag};
+            HIPCHK(dg::launch_upfold_small(ua, s));
+        } else {
+            // E = (T^{-1})^H K_o
+            HIPCHK(hipMemcpyAsync(W1, Tm + ko, oo * kc * sizeof(cd), hipMemcpyDeviceToDevice, s));
             HIPCHK(gj_inverse(n_orb, kc, W1, d_flag, s));
-            HIPCHK((zgemm_sq<false, false>(n_orb, kc, W1, D, W2, s)));
-            HIPCHK((zgemm_sq<false, false>(n_orb, kc, W2, W1, Eb, s)));
+            HIPCHK((zgemm_sq<true, false>(n_orb, kc, W1, Ko + ko, Eb, s)));
+            // M = C^H (X C)
+            HIPCHK((zgemm_sq<false, false>(n, kc, X + kn, Cb + kn, T1, s)));
+            HIPCHK((zgemm_sq<true, false>(n, kc, Cb + kn, T1, Mb, s)));
+            // K, then D = (E K) E^H
+            const size_t tot = oo * kc;
+            hipLaunchKernelGGL(k_upfold_assemble, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, Mb,
+                               ks_energy + (size_t)k0 * n_orb, d_inv + (size_t)k0 * n_orb, n, n_orb, kc, beta, mu, W1);
+            HIPCHK(hipGetLastError());
+            HIPCHK((zgemm_sq<false, false>(n_orb, kc, Eb, W1, W2, s)));
+            HIPCHK((zgemm_sq<false, true>(n_orb, kc, W2, Eb, D, s)));
+            if (Sm) {  // DDir = S^{-1} D (W2), DD = DDir S^{-1} (Eb)
+                HIPCHK(hipMemcpyAsync(W1, Sm + ko, oo * kc * sizeof(cd), hipMemcpyDeviceToDevice, s));
+                HIPCHK(gj_inverse(n_orb, kc, W1, d_flag, s));
+                HIPCHK((zgemm_sq<false, false>(n_orb, kc, W1, D, W2, s)));
+                HIPCHK((zgemm_sq<false, false>(n_orb, kc, W2, W1, Eb, s)));
+            }
+        }
+        if (Sm) {
             DDir = W2;
             DD = Eb;
         }
-        if (axes) {
+        if (dense) {
+            const int nseg = std::max(1, std::min(rseg_max, kc / 16));
+            const cd* const Y[3] = {DD, DDir, D};
+            HIPCHK(dg::launch_r_phases(d_rv, n_rv, kphase + 3 * (size_t)k0, kc, Ptab, s));
+            HIPCHK(dg::launch_r_sums(Y, nx, (int)oo, kc, n_rv, Ptab, nseg, d_part, s));
+            HIPCHK(dg::launch_r_scatter(d_part, nseg, nx, n_rv, (int)oo, d_of, n_r, inv_nk, (cd*)dmr, s));
+        } else if (axes) {
             const size_t np = (size_t)kc * 3 * nrr;
             hipLaunchKernelGGL(k_axis_phases, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, s,
                                kphase + 3 * (size_t)k0, kc, rmax, Ptab);
