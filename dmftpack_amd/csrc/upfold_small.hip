@@ -12,7 +12,10 @@
 //     there serves two rows' products.
 //   * The products E = T^-H K_o, X C, C^H (X C), E K, (E K) E^H, S^-1 D, (S^-1 D) S^-1 on FP64
 //     MFMA (v_mfma_f64_16x16x4, complex as four real products), a wavefront taking 16 rows.
-// What bounds it at n_orb = 28: see the figures at launch_upfold_small.
+// At n_orb = 28, 32^3 k it takes 2.3 ms (the batched kernels: 5.2 ms): 39 KB of LDS per k leave
+// two wavefronts per SIMD, whose vector work (7200 instructions) and MFMAs (0.18 of the SIMD
+// cycles) share the SIMD, with a third of the time waiting on LDS, barriers and loads.  The
+// pivot search by shuffles of (|a|^2, row) pairs and divisions in the copy loops cost 2.7 ms.
 #include "upfold_small.hpp"
 
 #include <algorithm>
@@ -22,6 +25,20 @@ namespace dg {
 namespace {
 
 typedef double dv4 __attribute__((ext_vector_type(4)));
+
+template <int CTRL>
+__device__ __forceinline__ unsigned dpp_row(unsigned x)
+{
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false);
+}
+
+// 0 for rows out of the search; otherwise > 0, ordered by |a|^2 (NaN as 0)
+__device__ __forceinline__ unsigned pivot_key(cd a, int row, bool in)
+{
+    const double m = fma(a.x, a.x, a.y * a.y);
+    const unsigned hi = m >= 0.0 ? (unsigned)__double2hiint(m) : 0u;
+    return in ? ((hi >> 5) << 6) | 32u | (31u - row) : 0u;
+}
 
 // In-register inverse of the n x n matrix in a[s][c] = A(r + 16 s, 8 g + c) (zero outside), lane
 // r + 16 g.  buf: 64 cd + 32 int of this wavefront's LDS.  On return row s of the lane is row
@@ -38,31 +55,17 @@ __device__ void gj_wave(cd (&a)[2][8], int n, cd* buf, int* pbuf, int lane, int 
         for (int jj = 0; jj < 8; ++jj) {
             const int j = 8 * jg + jj;
             if (j < n) {
-                // pivot: largest modulus of column j over the rows not used yet
-                const double m0 = (jr[0] < 0 && r < n) ? fma(a[0][jj].x, a[0][jj].x, a[0][jj].y * a[0][jj].y) : -1.0;
-                const double m1 = (jr[1] < 0 && r + 16 < n) ? fma(a[1][jj].x, a[1][jj].x, a[1][jj].y * a[1][jj].y) : -1.0;
-                double best = m0 >= 0.0 ? m0 : -1.0;  // (NaN is never a pivot)
-                int bi = r;
-                if (m1 > best) {
-                    best = m1;
-                    bi = r + 16;
-                }
-#pragma unroll
-                for (int o = 8; o > 0; o >>= 1) {
-                    const double ob = __shfl_xor(best, o);
-                    const int oi = __shfl_xor(bi, o);
-                    if (ob > best || (ob == best && oi < bi)) {
-                        best = ob;
-                        bi = oi;
-                    }
-                }
-                // the lanes of group jg hold column j
-                const int p = __builtin_amdgcn_readlane(bi, 16 * jg);
-                const bool okp = __builtin_amdgcn_readlane((int)(best > 0.0), 16 * jg) != 0;
-                if (lane == 0) {
-                    pbuf[j] = p;
-                    if (!okp) *singular = 1;
-                }
+                // pivot: the row with the largest modulus of column j among those not used yet, to
+                // 15 bits (the high word of |a|^2 with the row number in its low bits), so that the
+                // search is four DPP maxima; the lanes of group jg hold column j
+                unsigned key = pivot_key(a[0][jj], r, jr[0] < 0 && r < n);
+                key = max(key, pivot_key(a[1][jj], r + 16, jr[1] < 0 && r + 16 < n));
+                key = max(key, dpp_row<0xB1>(key));   // quad_perm 1 0 3 2
+                key = max(key, dpp_row<0x4E>(key));   // quad_perm 2 3 0 1
+                key = max(key, dpp_row<0x141>(key));  // row_half_mirror
+                key = max(key, dpp_row<0x140>(key));  // row_mirror
+                const int p = 31 - (__builtin_amdgcn_readlane((int)key, 16 * jg) & 31);
+                if (lane == 0) pbuf[j] = p;
                 const bool mine = r == (p & 15);
                 if (mine) {
                     if (p < 16) {
@@ -83,7 +86,14 @@ __device__ void gj_wave(cd (&a)[2][8], int n, cd* buf, int* pbuf, int lane, int 
                 cd t[8];
 #pragma unroll
                 for (int c = 0; c < 8; ++c) t[c] = row[8 * g + c];
-                const cd rp = okp ? crcp(d) : cd{0.0, 0.0};
+                const double q = fma(d.x, d.x, d.y * d.y);
+                const bool okp = q > 0.0;  // false for NaN
+                if (lane == 0 && !okp) *singular = 1;
+                cd rp = cd{0.0, 0.0};
+                if (okp) {
+                    const double iq = q > 1e-280 && q < 1e280 ? rcp_pos(q) : 1.0 / q;
+                    rp = cd{d.x * iq, -d.y * iq};
+                }
 #pragma unroll
                 for (int c = 0; c < 8; ++c) t[c] = cmul(t[c], rp);
                 if (g == jg) {  // column j of the inverse takes the place of column j
@@ -159,31 +169,43 @@ __device__ __forceinline__ void zprod(Prod& p, const cd* A, const cd* B, int n, 
         p.im[t] = p.re[t];
     }
     if (16 * wave >= n) return;
-    const int i = min(16 * wave + r, n - 1);
     const bool two = n > 16;
-    for (int l0 = 0; l0 < n; l0 += 4) {
-        const int l = min(l0 + q, n - 1);
-        const double m = l0 + q < n ? 1.0 : 0.0;
-        cd a = HA ? cconj(A[l + i * ld]) : A[i + l * ld];
-        a = cscale(a, m);
-        cd b[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int j = min(16 * t + r, n - 1);
-            b[t] = HB ? cconj(B[j + l * ld]) : B[l + j * ld];
+    const int i = min(16 * wave + r, n - 1), j0 = min(r, n - 1), j1 = min(16 + r, n - 1);
+    // operands of summed index l at pa + l * sa, pb0 + l * sb, pb1 + l * sb
+    const int sa = HA ? 1 : ld, sb = HB ? ld : 1;
+    const cd* pa = A + (HA ? i * ld : i);
+    const cd* pb0 = B + (HB ? j0 : j0 * ld);
+    const cd* pb1 = B + (HB ? j1 : j1 * ld);
+    auto step = [&](cd a, cd b0, cd b1) {
+        if (HA) a.y = -a.y;
+        if (HB) {
+            b0.y = -b0.y;
+            b1.y = -b1.y;
         }
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-            if (t == 0 || two) {
-                p.re[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b[t].x, p.re[t], 0, 0, 0);
-                p.im[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b[t].y, p.im[t], 0, 0, 0);
-            }
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-            if (t == 0 || two) {
-                p.re[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, b[t].y, p.re[t], 0, 0, 0);
-                p.im[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b[t].x, p.im[t], 0, 0, 0);
-            }
+        p.re[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b0.x, p.re[0], 0, 0, 0);
+        p.im[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b0.y, p.im[0], 0, 0, 0);
+        if (two) {
+            p.re[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b1.x, p.re[1], 0, 0, 0);
+            p.im[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b1.y, p.im[1], 0, 0, 0);
+        }
+        p.re[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, b0.y, p.re[0], 0, 0, 0);
+        p.im[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b0.x, p.im[0], 0, 0, 0);
+        if (two) {
+            p.re[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, b1.y, p.re[1], 0, 0, 0);
+            p.im[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b1.x, p.im[1], 0, 0, 0);
+        }
+    };
+    int l0 = 0;
+#pragma unroll 2
+    for (; l0 + 4 <= n; l0 += 4) {
+        const int l = l0 + q;
+        step(pa[l * sa], pb0[l * sb], pb1[l * sb]);
+    }
+    if (l0 < n) {
+        const int l = min(l0 + q, n - 1);
+        cd a = pa[l * sa];
+        if (l0 + q >= n) a = cd{0.0, 0.0};
+        step(a, pb0[l * sb], pb1[l * sb]);
     }
 }
 
@@ -201,13 +223,18 @@ __device__ __forceinline__ void each(const Prod& p, int n, int wave, int lane, F
         }
 }
 
+// n x n matrix between global memory and LDS: lane = row, four columns at a time
 __device__ __forceinline__ void load_lds(cd* M, int ld, const cd* __restrict__ g, int n, int tid)
 {
-    for (int e = tid; e < n * n; e += 128) M[e % n + (e / n) * ld] = g[e];
+    const int i = tid & 31;
+    if (i < n)
+        for (int c = tid >> 5; c < n; c += 4) M[i + c * ld] = g[i + c * n];
 }
 __device__ __forceinline__ void store_lds(const cd* M, int ld, cd* __restrict__ g, int n, int tid)
 {
-    for (int e = tid; e < n * n; e += 128) g[e] = M[e % n + (e / n) * ld];
+    const int i = tid & 31;
+    if (i < n)
+        for (int c = tid >> 5; c < n; c += 4) g[i + c * n] = M[i + c * ld];
 }
 
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) void k_upfold_small(UpfoldArgs u)
