@@ -148,50 +148,61 @@ __global__ void k_mom_kinv(int range, int green, double* __restrict__ kinv)
 // design matrix contributes sum_b Kinv[a][b] Re_b and the Im row
 // sum_b Kinv[a][b] Im_b (the rows' zero entries left out), each taken times
 // its half of g and added, Re row first, in ascending frequency order.
-__global__ void k_mom_fit(const cd* __restrict__ fw, int d, int n_freq, int range, const double4* __restrict__ tab,
-                          int green, const double* __restrict__ kinv, cd* __restrict__ mt)
+// One thread per (moment, window, element): the sum is a serial chain, so the time is
+// that of the longest window, and the loads of kFitAhead frequencies are issued together
+// ahead of their use.  With one thread per (window, element) and loads at their use, d = 5
+// and N_freq = 1000 took 275 us (660 cycles a frequency, most of it load latency); this
+// form 220 us (bound by its L1 loads).
+constexpr int kFitAhead = 8;
+
+template <bool GREEN>
+__global__ __launch_bounds__(256) void k_mom_fit(const cd* __restrict__ fw, int d, int n_freq, int range,
+                                                 const double4* __restrict__ tab, const double* __restrict__ kinv,
+                                                 cd* __restrict__ mt)
 {
 #pragma clang fp contract(off)
-    const int m2 = d * d;
+    const int m2 = d * d, a = blockIdx.y;
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (size_t)range * m2) return;
     const int w = (int)(t / m2), e = (int)(t % m2);
     const int al = e % d, be = e / d;
-    const int nm = green ? 2 : 4;
-    const double* X = kinv + (size_t)w * 16;  // Kinv(a, b) at X[a + 4 b]
-    double xk[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) xk[a][b] = X[a + 4 * b];
-    cd s[4] = {cd{0, 0}, cd{0, 0}, cd{0, 0}, cd{0, 0}};
-    for (int wn = w; wn < n_freq; ++wn) {
-        const double4 c = tab[wn];
-        const cd fab = fw[(size_t)wn * m2 + al + be * d];
-        const cd fba = fw[(size_t)wn * m2 + be + al * d];
+    const double* X = kinv + (size_t)w * 16 + a;  // Kinv(a, b) at X[4 b]
+    const double x0 = X[0], x1 = X[4], x2 = GREEN ? 0.0 : X[8], x3 = GREEN ? 0.0 : X[12];
+    const cd* fa = fw + al + (size_t)be * d;
+    const cd* fb = fw + be + (size_t)al * d;
+    cd s = cd{0, 0};
+    auto add = [&](double4 c, cd fab, cd fba) {
         // Re = (F_ab + conj(F_ba))/2 ; Im = (F_ab - conj(F_ba))/(2i)
         const cd re = cd{0.5 * (fab.x + fba.x), 0.5 * (fab.y - fba.y)};
         cd im = cd{0.5 * (fab.y + fba.y), -0.5 * (fab.x - fba.x)};
-        if (!green) {
+        double kr, ki;
+        if (!GREEN) {
             // Re row [1, 0, -1/z^2, 0], Im row [0, -1/z, 0, 1/z^3]   (:227-230)
-#pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                const double kr = fma(xk[a][2], c.y, xk[a][0]);
-                const double ki = fma(xk[a][3], c.z, xk[a][1] * c.x);
-                s[a] = cadd(s[a], cd{fma(ki, im.x, kr * re.x), fma(ki, im.y, kr * re.y)});
-            }
+            kr = fma(x2, c.y, x0);
+            ki = fma(x3, c.z, x1 * c.x);
         } else {
             // Re row [-1/z^2, 0], Im row [0, 1/z^3]   (:366-367)
             if (al == be) im.x += c.w;  // (:373)
-#pragma unroll
-            for (int a = 0; a < 2; ++a) {
-                const double kr = xk[a][0] * c.y;
-                const double ki = xk[a][1] * c.z;
-                s[a] = cadd(s[a], cd{fma(ki, im.x, kr * re.x), fma(ki, im.y, kr * re.y)});
-            }
+            kr = x0 * c.y;
+            ki = x1 * c.z;
         }
+        s = cadd(s, cd{fma(ki, im.x, kr * re.x), fma(ki, im.y, kr * re.y)});
+    };
+    int wn = w;
+    for (; wn + kFitAhead <= n_freq; wn += kFitAhead) {
+        double4 c[kFitAhead];
+        cd p[kFitAhead], q[kFitAhead];
+#pragma unroll
+        for (int u = 0; u < kFitAhead; ++u) {
+            c[u] = tab[wn + u];
+            p[u] = fa[(size_t)(wn + u) * m2];
+            q[u] = fb[(size_t)(wn + u) * m2];
+        }
+#pragma unroll
+        for (int u = 0; u < kFitAhead; ++u) add(c[u], p[u], q[u]);
     }
-    for (int a = 0; a < nm; ++a) mt[((size_t)a * range + w) * m2 + e] = s[a];
+    for (; wn < n_freq; ++wn) add(tab[wn], fa[(size_t)wn * m2], fb[(size_t)wn * m2]);
+    mt[((size_t)a * range + w) * m2 + e] = s;
 }
 
 // trace[a][w] = sum_alpha Re mt[a][w][alpha alpha]     (:244-247)
@@ -215,7 +226,9 @@ __global__ void k_mom_avg(const cd* __restrict__ mt, int m2, int range, int nm, 
     const int c = (int)((t / m2) % ncent);
     const int a = (int)(t / ((size_t)m2 * ncent));
     cd s = cd{0, 0};
-    for (int iw = c; iw <= c + 2 * Nv; ++iw) s = cadd(s, mt[((size_t)a * range + iw) * m2 + e]);
+    const cd* m = mt + ((size_t)a * range + c) * m2 + e;
+#pragma unroll 8
+    for (int iw = 0; iw <= 2 * Nv; ++iw) s = cadd(s, m[(size_t)iw * m2]);
     const double cnt = 2 * Nv + 1;
     avg[t] = cd{s.x / cnt, s.y / cnt};
 }
@@ -223,64 +236,63 @@ __global__ void k_mom_avg(const cd* __restrict__ mt, int m2, int range, int nm, 
 // positivity matrix per window centre:
 //   non-G: T = Vi m3 Vi - (Vi m2 Vi)^2, Vi = (m1)^{-1/2}   (:298-308)
 //   G    : T = m1 - m0^2                                   (:423-424)
-// (w1, U1) = eig(m1avg) for the non-G branch.  scratch: 3 d*d per centre
-// (Vi, P2 = Vi m2 Vi, tmp).  One thread per (centre, entry); the non-G branch
-// runs as five launches (stage 0: Vi, 1: tmp = Vi m2, 2: P2 = tmp Vi,
-// 3: tmp = Vi m3, 4: T = tmp Vi - P2 P2), stage -1 is the G branch.  A centre
-// whose m1 is not positive gets T = -1 (the window is rejected anyway).
-__global__ void k_mom_posmat(const cd* __restrict__ avg, int d, int ncent, int stage, const double* __restrict__ w1,
-                             const cd* __restrict__ U1, cd* __restrict__ T, cd* __restrict__ scr)
+// (w1, U1) = eig(m1avg) for the non-G branch.  One wavefront per centre, the products
+// one after the other in LDS (Vi, tmp, P2), an entry's sum in the order of its inner index.  A
+// centre whose m1 is not positive gets T = -1 (the window is rejected anyway).
+__global__ __launch_bounds__(64) void k_mom_posmat(const cd* __restrict__ avg, int d, int ncent, int green,
+                                                   const double* __restrict__ w1, const cd* __restrict__ U1,
+                                                   cd* __restrict__ T)
 {
-    const int m2 = d * d;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)ncent * m2) return;
-    const int c = (int)(t / m2), e = (int)(t % m2), i = e % d, j = e / d;
+    extern __shared__ cd pm[];
+    const int m2 = d * d, c = blockIdx.x, t = threadIdx.x;
     auto A = [&](int a) { return avg + ((size_t)a * ncent + c) * m2; };
     cd* out = T + (size_t)c * m2;
-    if (stage < 0) {
+    if (green) {
         const cd* m0 = A(0);
-        cd s = A(1)[e];
-        for (int l = 0; l < d; ++l) s = cfms(m0[i + l * d], m0[l + j * d], s);
-        out[e] = s;
+        for (int e = t; e < m2; e += 64) {
+            cd s = A(1)[e];
+            for (int l = 0; l < d; ++l) s = cfms(m0[e % d + l * d], m0[l + (e / d) * d], s);
+            out[e] = s;
+        }
         return;
     }
     const double* w = w1 + (size_t)c * d;
     if (!(w[0] > 0.0)) {
-        if (stage == 4) out[e] = cd{-1.0, 0.0};
+        for (int e = t; e < m2; e += 64) out[e] = cd{-1.0, 0.0};
         return;
     }
-    cd* Vi = scr + (size_t)c * 3 * m2;
-    cd* P2 = Vi + m2;
-    cd* tmp = P2 + m2;
-    cd s = cd{0, 0};
-    switch (stage) {
-    case 0: {
-        const cd* U = U1 + (size_t)c * m2;
-        for (int l = 0; l < d; ++l) s = cadd(s, cscale(cmulc(U[i + l * d], U[j + l * d]), 1.0 / sqrt(w[l])));
+    cd *Vi = pm, *tmp = pm + m2, *P2 = pm + 2 * m2, *mq = pm + 3 * m2;
+    const cd* U = U1 + (size_t)c * m2;
+    for (int e = t; e < m2; e += 64) mq[e] = U[e];
+    wave_sync();
+    for (int e = t; e < m2; e += 64) {
+        const int i = e % d, j = e / d;
+        cd s = cd{0, 0};
+        for (int l = 0; l < d; ++l) s = cadd(s, cscale(cmulc(mq[i + l * d], mq[j + l * d]), 1.0 / sqrt(w[l])));
         Vi[e] = s;
-        break;
     }
-    case 1: {
-        const cd* m2a = A(2);
-        for (int l = 0; l < d; ++l) s = cfma(Vi[i + l * d], m2a[l + j * d], s);
-        tmp[e] = s;
-        break;
-    }
-    case 2:
-        for (int l = 0; l < d; ++l) s = cfma(tmp[i + l * d], Vi[l + j * d], s);
-        P2[e] = s;
-        break;
-    case 3: {
-        const cd* m3a = A(3);
-        for (int l = 0; l < d; ++l) s = cfma(Vi[i + l * d], m3a[l + j * d], s);
-        tmp[e] = s;
-        break;
-    }
-    default:
+    auto product = [&](const cd* X, const cd* Y, cd* Z) {
+        wave_sync();
+        for (int e = t; e < m2; e += 64) {
+            const int i = e % d, j = e / d;
+            cd s = cd{0, 0};
+            for (int l = 0; l < d; ++l) s = cfma(X[i + l * d], Y[l + j * d], s);
+            Z[e] = s;
+        }
+        wave_sync();
+    };
+    wave_sync();
+    for (int e = t; e < m2; e += 64) mq[e] = A(2)[e];
+    product(Vi, mq, tmp);
+    product(tmp, Vi, P2);
+    for (int e = t; e < m2; e += 64) mq[e] = A(3)[e];
+    product(Vi, mq, tmp);
+    for (int e = t; e < m2; e += 64) {
+        const int i = e % d, j = e / d;
+        cd s = cd{0, 0};
         for (int l = 0; l < d; ++l) s = cfma(tmp[i + l * d], Vi[l + j * d], s);
         for (int l = 0; l < d; ++l) s = cfms(P2[i + l * d], P2[l + j * d], s);
         out[e] = s;
-        break;
     }
 }
 
@@ -307,9 +319,11 @@ __global__ __launch_bounds__(kSelThreads) void k_mom_select(const double* __rest
 #pragma clang fp contract(off)
         const double* v = trace + (size_t)a * range + i;  // centre i + Nv, window [i, i + 2 Nv]
         double mean = 0.0;
+#pragma unroll 8
         for (int j = 0; j < 2 * Nv + 1; ++j) mean += v[j];
         mean /= (2 * Nv + 1);
         double ss = 0.0;
+#pragma unroll 8
         for (int j = 0; j < 2 * Nv + 1; ++j) {
             const double dv = v[j] - mean;
             ss += dv * dv;
@@ -373,6 +387,7 @@ __global__ void k_mom_final(const cd* __restrict__ mt, int d, int range, int gre
     cd* out = mom + (size_t)target * m2;
     const int al = e % d, be = e / d;
     cd s = cd{0, 0}, st = cd{0, 0};
+#pragma unroll 4
     for (int w = cen - Nv; w <= cen + Nv; ++w) {
         const cd* m = mt + ((size_t)mom_idx * range + w) * m2;
         s = cadd(s, cscale(cadd(m[al + be * d], cconj(m[be + al * d])), 0.5));
@@ -840,7 +855,7 @@ extern "C" int dmftgpu_moments(dmftgpu_handle h, int d, int n_freq, double beta,
     double4* tab = (double4*)kbase;
     double* kinv = (double*)(kbase + ((size_t)n_freq * sizeof(double4) + 255) / 256 * 256);
     size_t need = (size_t)nm * range * m2 * 16 + (size_t)nm * range * 8 +
-                  (size_t)nm * ncent * m2 * 16 + (size_t)ncent * m2 * 16 * 6 + (size_t)ncent * d * 8 * 2 + 64 * 256;
+                  (size_t)nm * ncent * m2 * 16 + (size_t)ncent * m2 * 16 * 3 + (size_t)ncent * d * 8 * 2 + 64 * 256;
     int rc = 0;
     char* base = ft_ws(h, need, &rc);
     if (!base) return rc;
@@ -851,7 +866,6 @@ extern "C" int dmftgpu_moments(dmftgpu_handle h, int d, int n_freq, double beta,
     double* w1 = cv.take<double>((size_t)ncent * d);
     cd* U1 = cv.take<cd>((size_t)ncent * m2);
     cd* T = cv.take<cd>((size_t)ncent * m2);
-    cd* scr = cv.take<cd>((size_t)ncent * m2 * 3);
     double* wT = cv.take<double>((size_t)ncent * d);
     int* cen = cv.take<int>(4);
     hipStream_t s = h->stream;
@@ -875,19 +889,20 @@ extern "C" int dmftgpu_moments(dmftgpu_handle h, int d, int n_freq, double beta,
         ent->beta = beta;
         ent->green = green_asym;
     }
-    hipLaunchKernelGGL(k_mom_fit, dim3(nblk((size_t)range * m2)), dim3(256), 0, s, (const cd*)fw, d, n_freq, range, tab,
-                       green_asym, kinv, mt);
+    const dim3 gfit(nblk((size_t)range * m2), nm);
+    if (green_asym)
+        hipLaunchKernelGGL((k_mom_fit<true>), gfit, dim3(256), 0, s, (const cd*)fw, d, n_freq, range, tab, kinv, mt);
+    else hipLaunchKernelGGL((k_mom_fit<false>), gfit, dim3(256), 0, s, (const cd*)fw, d, n_freq, range, tab, kinv, mt);
     HIPCHK(hipGetLastError());
     hipLaunchKernelGGL(k_mom_trace, dim3(nblk((size_t)range * nm)), dim3(256), 0, s, mt, d, range, nm, trace);
     HIPCHK(hipGetLastError());
     hipLaunchKernelGGL(k_mom_avg, dim3(nblk((size_t)nm * ncent * m2)), dim3(256), 0, s, mt, m2, range, nm, Nv, avg);
     HIPCHK(hipGetLastError());
     if (!green_asym) HIPCHK(dg::launch_herm_eig(avg + (size_t)1 * ncent * m2, d, 0, d, nullptr, 0, w1, U1, ncent, s));
-    for (int stage = green_asym ? -1 : 0; stage <= (green_asym ? -1 : 4); ++stage) {
-        hipLaunchKernelGGL(k_mom_posmat, dim3(nblk((size_t)ncent * m2)), dim3(256), 0, s, avg, d, ncent, stage, w1, U1,
-                           T, scr);
-        HIPCHK(hipGetLastError());
-    }
+    const int pshm = (int)(4 * (size_t)m2 * sizeof(cd));
+    HIPCHK(hipFuncSetAttribute((const void*)k_mom_posmat, hipFuncAttributeMaxDynamicSharedMemorySize, pshm));
+    hipLaunchKernelGGL(k_mom_posmat, dim3(ncent), dim3(64), pshm, s, avg, d, ncent, green_asym, w1, U1, T);
+    HIPCHK(hipGetLastError());
     HIPCHK(dg::launch_herm_eig(T, d, 0, d, nullptr, 0, wT, nullptr, ncent, s));
     // window choice and final moments on the device: no host round trip
     cd* dm = (cd*)moments;
