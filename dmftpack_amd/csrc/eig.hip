@@ -3,14 +3,15 @@
 // Replaces the per-k SelfAdjointEigenSolver calls of the static part of
 // GreenFtn_w (GreenFtn.cpp:197-215) and the small Hermitian problems of the
 // Fourier transform.  Jacobi with complex rotations in a parallel order: the
-// disjoint rotations of a round are applied together.  m <= 16: one matrix per
-// 4-, 8- or 16-lane slot of a wavefront, rows in registers (k_herm_eig_slots);
-// 17 <= m <= 32: one wavefront per matrix held in LDS (k_herm_eig).
-// Eigenvalues are returned in ascending order like Eigen.
+// disjoint rotations of a round are applied together: one matrix per 4-, 8-, 16- or
+// 32-lane slot of a wavefront, rows in registers (k_herm_eig_slots), or one wavefront
+// per matrix held in LDS (k_herm_eig).  Eigenvalues are returned in ascending order
+// like Eigen.
 #include "lattice_kernels.hpp"
 
 namespace dg {
 
+// One wavefront per matrix in LDS, for the sizes that would leave a 32-lane slot half idle
 __global__ __launch_bounds__(64) void k_herm_eig(const cd* __restrict__ X, int ldx, int off, int m,
                                                  const cd* __restrict__ add, int nadd, double* __restrict__ w,
                                                  cd* __restrict__ V, int batch)
@@ -174,7 +175,7 @@ __global__ __launch_bounds__(64) void k_herm_eig(const cd* __restrict__ X, int l
 }
 
 // ---------------------------------------------------------------------------
-// m <= 16: one matrix per M-lane slot of the wavefront (M = 4, 8 or 16), with
+// One matrix per M-lane slot of the wavefront (M = 4, 8, 16 or 32), with
 // row j of A and of V in the registers of lane j, stored in XOR order:
 // register r holds column j^r, so the diagonal is register 0 of every lane.
 // A sweep is the M-1 rounds s = 1..M-1 that pair every index j with j^s (each
@@ -185,9 +186,9 @@ __global__ __launch_bounds__(64) void k_herm_eig(const cd* __restrict__ X, int l
 //                                      registers r and r^s of the same lane);
 //   row update    A <- J^H A           one exchange with lane j^s (ds_swizzle,
 //                                      partner register r^s into register r).
-// The rotation of pair (p, q), p < q, is the one of the LDS kernel below
-// (zero A[p][q] with a real diagonal); both lanes compute it from the same
-// three inputs, so they agree bit for bit.
+// The rotation of pair (p, q), p < q, zeroes A[p][q] and keeps the diagonal real; both
+// lanes compute it from the same three inputs, so they agree bit for bit.
+// M = 32 holds 256 registers of A and V at one wavefront per SIMD.
 // ---------------------------------------------------------------------------
 
 // value of lane (lane ^ S) within each 32-lane group
@@ -213,7 +214,7 @@ __device__ __forceinline__ cd lin2c(cd al, cd x, cd be, cd y) { return cfmac(be,
 template <int S>
 constexpr int high_bit()
 {
-    return S >= 8 ? 8 : S >= 4 ? 4 : S >= 2 ? 2 : 1;
+    return S >= 16 ? 16 : S >= 8 ? 8 : S >= 4 ? 4 : S >= 2 ? 2 : 1;
 }
 
 // Round s = S of a sweep.  tab: this slot's M entries (row coefficients of
@@ -303,7 +304,7 @@ __device__ __forceinline__ double slot_sum(double x)
 }
 
 template <int M, bool WANTV>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_herm_eig_slots(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(M > 16 ? 1 : 2))) void k_herm_eig_slots(
     const cd* __restrict__ X, int ldx, int off, int m, const cd* __restrict__ add, int nadd, double* __restrict__ w,
     cd* __restrict__ V, int batch)
 {
@@ -392,7 +393,11 @@ hipError_t launch_herm_eig(const cd* X, int ldx, int off, int m, const cd* add, 
     if (m <= 4) return launch_slots<4>(X, ldx, off, m, add, nadd, w, V, batch, s);
     if (m <= 8) return launch_slots<8>(X, ldx, off, m, add, nadd, w, V, batch, s);
     if (m <= 16) return launch_slots<16>(X, ldx, off, m, add, nadd, w, V, batch, s);
-    if (m > 32) return hipErrorInvalidValue;  // the pair table holds 16 rotations
+    if (m > 32) return hipErrorInvalidValue;
+    // The 32-lane slots do the work of a 32 x 32 matrix at any m; the LDS kernel's time falls
+    // with m.  4096 matrices with V, slots against LDS: m = 32 1.93 and 6.27 ms, 28 1.88 and
+    // 2.82, 26 1.84 and 2.05, 24 1.85 and 1.87 (1728 matrices: 0.94 and 0.85), 22 1.74 and 1.14
+    if (m >= 26) return launch_slots<32>(X, ldx, off, m, add, nadd, w, V, batch, s);
     size_t shm = sizeof(cd) * 2 * (size_t)m * m + sizeof(double) * 4 * 16 + sizeof(int) * 2 * 16;
     hipLaunchKernelGGL(k_herm_eig, dim3(batch), dim3(64), shm, s, X, ldx, off, m, add, nadd, w, V, batch);
     return hipGetLastError();
