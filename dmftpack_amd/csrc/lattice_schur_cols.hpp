@@ -15,7 +15,7 @@
 // of N lanes (N = n_c rounded up to 8/10/12/16) owns one (k, iw) matrix and
 // lane c holds column c of S, then of G_cc:
 //   * S column c:  S_ic = E_ic - H_cc,ic - sum_d W_id (g_d conj(W_cd)),
-//     E = (z+mu) I - Sigma(iw) kept in registers across the k loop;
+//     E = (z+mu) I - Sigma(iw), Sigma read from the cache at each k;
 //     the g_d of the slot's frequency are computed once per slot and shared
 //     through LDS;
 //   * inversion: column-per-lane Gauss-Jordan (gj.hpp); FP32R inverts in FP32
@@ -49,16 +49,23 @@ __host__ __device__ constexpr int cols_nc_min(int N)
 // wavefronts share nothing but the cache
 __host__ __device__ constexpr int cols_wg(int, int) { return 64; }
 
-// per-slot LDS (cd units): bc 2N (GJ broadcast), gsh 32 (g_d), MA N*N, MB N*N, GB N*N.
-// The FP32R forward keeps only X0 (FP32) in MB: N*N/2 cd, so that at N = 10 a
-// wavefront needs 22.7 KB instead of 28.2 KB and 7 fit in a CU's LDS instead of 5.
+// per-slot LDS (cd units): gsh 32 - nc_min (g_d), MA N*N, MB N*N (the FP32R forward
+// keeps only X0, FP32, there: N*N/2); the elimination's broadcast buffer (2N) lies where
+// nothing is held yet, in MB (FP32R) or MA, and on its own only in the FP64 forward.
+// Sigma and gbar are read from the cache at each k and the spare lanes repeat lanes of
+// the last slot instead of writing to a slot of their own: the LDS is what decides how
+// many wavefronts of the adjoint a CU holds (N = 10: 39.5 KB each with tables of their
+// own for all of these, 4 to a CU; 21.4 KB, 7 to a CU.  With cols_waves below, FP64
+// adjoint of n = 32, n_c = 10, 1728 k x 528 points: 4.85 -> 3.28 ms, n_c = 16: 21.8 ->
+// 12.3 ms; forward 1.81 -> 1.51 ms and 6.0 -> 3.7 ms).
 // The size is odd (in 16-byte entries): the slots of a wavefront read the same entry of
 // their own matrices at once, and with a multiple of 16 entries (the adjoint at N = 10 or
 // 16, every form at N = 8) all of those fell into the same four banks.
 __host__ __device__ constexpr int cols_slot_size(int N, int mode, int prec)
 {
-    const int mb = mode == MODE_FWD ? (prec > 0 ? (N * N + 1) / 2 : 0) : N * N;
-    return (2 * N + 32 + ((prec > 0 || mode != MODE_FWD) ? N * N + mb : 0) + (mode == MODE_VJP ? N * N : 0)) | 1;
+    const int g = 32 - cols_nc_min(N);  // n_d at most
+    if (mode == MODE_FWD && prec == 0) return (g + 2 * N) | 1;
+    return (g + N * N + (mode == MODE_FWD ? (N * N + 1) / 2 : N * N)) | 1;
 }
 
 __host__ __device__ constexpr int cols_slots(int N, int mode, int prec) { return cols_wg(mode, prec) / 64 * (64 / N); }
@@ -67,8 +74,18 @@ inline size_t cols_lds_bytes(int N, int mode, int prec, int, int)
 {
     const int nwave = cols_wg(mode, prec) / 64;
     const int spw = 64 / N;
-    return sizeof(cd) * ((size_t)nwave * (spw + 1) * cols_slot_size(N, mode, prec));
+    return sizeof(cd) * ((size_t)nwave * spw * cols_slot_size(N, mode, prec));
 }
+
+// Wavefronts per SIMD the register allocator is held to: as many as fit without spilling
+// column-sized values (three at N = 10 only for the FP64 forward; the adjoint at N = 16
+// needs 356 registers, and its LDS admits four wavefronts to a CU anyway).
+__host__ __device__ constexpr int cols_waves(int N, int mode, int prec)
+{
+    return mode == MODE_FWD ? (N <= 8 || (N == 10 && prec == 0) ? 3 : 2) : N <= 12 ? 2 : 1;
+}
+
+__device__ __forceinline__ cd ld_off(const cd* base, unsigned bytes) { return *(const cd*)((const char*)base + bytes); }
 
 // One (frequency tile, k chunk) work item of one lattice: the body of the
 // per-lattice kernel and of the persistent multi-lattice kernel below.
@@ -79,26 +96,25 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
     constexpr int SPW = 64 / N;
     constexpr int SLOTS = cols_slots(N, MODE, PREC);
     constexpr int SS = cols_slot_size(N, MODE, PREC);
-    constexpr bool MATS = (PREC > 0 || MODE != MODE_FWD);
     const int n = a.n, nc = a.nc, nd = a.n - nc, m2 = nc * nc;
     constexpr int NMIN = cols_nc_min(N);
     auto inb = [nc](int i) { return i < NMIN || i < nc; };  // row / column i inside the n_c block
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int sl = lane / N;  // == SPW for the spare lanes of a wavefront
-    const int c = lane - sl * N;
-    const bool active = sl < SPW;
-    const bool live = active && c < nc;  // lanes c >= nc hold identity padding
-    const int cc = live ? c : 0;         // clamped column index for loads
-    cd* my = lds + (size_t)(wave * (SPW + 1) + sl) * SS;  // spare lanes get a scratch slot
-    cd* bc = my;
-    cd* gsh = my + 2 * N;
-    cd* MA = gsh + 32;
+    // the spare lanes of a wavefront repeat the first lanes of its last slot: the same
+    // values to the same LDS entries, and nothing stored at the end
+    const bool active = lane < SPW * N;
+    const int sl = active ? lane / N : SPW - 1;
+    const int c0 = active ? lane - sl * N : lane - SPW * N;
+    const int cc = c0 < nc ? c0 : 0;  // clamped column index for loads
+    cd* my = lds + (size_t)(wave * SPW + sl) * SS;
+    cd* gsh = my;
+    cd* MA = gsh + 32 - NMIN;
     cd* MB = MA + N * N;
-    cd* GB = MB + N * N;
+    cd* bc = PREC > 0 ? MB : MA;  // before MB (PREC 0: MA) is written
     const int npts = n_points(a);
     if (wtile * SLOTS >= npts) return;  // tile past the last frequency point
-    const int nw = wtile * SLOTS + wave * SPW + (active ? sl : 0);
-    const bool wvalid = active && nw < npts;
+    const int nw = wtile * SLOTS + wave * SPW + sl;
+    const bool wvalid = nw < npts;
     const int nwc = nw < npts ? nw : npts - 1;
     const int k0 = chunk * a.k_per_chunk;
     const int k1 = min(a.nk, k0 + a.k_per_chunk);
@@ -107,20 +123,15 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
     const bool vjp_here = (MODE == MODE_VJP) && wvalid && nw < a.n_freq;
     const double cn = (MODE == MODE_VJP) ? 2.0 * (a.nbar_dev ? *a.nbar_dev : a.nbar) / a.beta : 0.0;
 
-    // E = (z+mu) I - Sigma(iw), column c
-    cd E[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        cd v = cd{0.0, 0.0};
-        if (live && i < nc) v = cneg(sig_all[(size_t)nwc * m2 + i + cc * nc]);
-        if (live && i == c) v = cadd(v, cd{mu, w});
-        E[i] = v;
-    }
-    if (MODE == MODE_VJP) {
-#pragma unroll
-        for (int i = 0; i < N; ++i)
-            GB[i + c * N] = (vjp_here && live && i < nc) ? a.gbar[(size_t)nw * m2 + i + cc * nc] : cd{0.0, 0.0};
-    }
+    // column c of Sigma(iw) and row c of gbar, read at each k: held across the k walk
+    // they would take 8 N registers
+    // (addresses as a wave-uniform base and a 32-bit offset of the lane: kept across the
+    // walk as 64-bit addresses of single entries they spill)
+    const cd* sig = sig_all + (size_t)(wtile * SLOTS) * m2;
+    const cd* gb = MODE == MODE_VJP ? a.gbar + (size_t)min(wtile * SLOTS, a.n_freq - 1) * m2 : nullptr;
+    const unsigned sig_off = ((nwc - wtile * SLOTS) * m2 + cc * nc) * 16;
+    const unsigned gb_off = ((min(nw, a.n_freq - 1) - min(wtile * SLOTS, a.n_freq - 1)) * m2 + cc) * 16;
+    const unsigned h_off = cc * n * 16;
     cd acc[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) acc[i] = cd{0.0, 0.0};
@@ -128,9 +139,14 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
     __syncthreads();
 
     for (int k = k0; k < k1; ++k) {
+        // (hidden from the compiler at each k: what it derives from these, masks and
+        // addresses for every entry, it would hold across the walk, in scratch memory)
+        int c = c0, ncs = nc;
+        asm volatile("" : "+v"(c), "+s"(ncs)::"memory");
+        const bool live = c < nc;  // lanes c >= nc hold identity padding
         // per-k data straight from global memory through the constant address
         // space: the wave-uniform reads (W_id, e_d) become scalar loads
-        const kconst_cd* Hkk = (const kconst_cd*)(a.Hk + (size_t)k * n * n);  // H_cc(i, c) at i + c*n
+        const cd* Hkk = a.Hk + (size_t)k * n * n;  // H_cc(i, c) at i + c*n
         const kconst_cd* Wk = (const kconst_cd*)(a.W + (size_t)k * nc * nd);
         const kconst_double* ed = (const kconst_double*)(a.ed + (size_t)k * nd);
         // This k's W and e_d into the caches at once: vector loads into L1 for
@@ -165,15 +181,22 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
         // (the loads are unconditional, rows clamped in range, and pinned by an
         // empty asm so that the compiler cannot sink each into a branch of its
         // own: they issue together instead of one round trip per entry)
-        cd hcol[N];
+        {
+            cd t[N];
 #pragma unroll
-        for (int i = 0; i < N; ++i) hcol[i] = ldc(Hkk + (i < nc ? i : 0) + (size_t)cc * n);
+            for (int i = 0; i < N; ++i) t[i] = ld_off(Hkk + (inb(i) ? i : 0), h_off);
 #pragma unroll
-        for (int i = 0; i < N; ++i) asm volatile("" ::"v"(hcol[i].x), "v"(hcol[i].y));
+            for (int i = 0; i < N; ++i) asm volatile("" ::"v"(t[i].x), "v"(t[i].y));
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-            const cd pad = (i == c) ? cd{1.0, 0.0} : cd{0.0, 0.0};
-            col[i] = live ? ((i < nc) ? csub(E[i], hcol[i]) : cd{0.0, 0.0}) : pad;
+            for (int i = 0; i < N; ++i) col[i] = csub(i == c ? cd{mu, w} : cd{0.0, 0.0}, t[i]);
+#pragma unroll
+            for (int i = 0; i < N; ++i) t[i] = ld_off(sig + (inb(i) ? i : 0), sig_off);
+#pragma unroll
+            for (int i = 0; i < N; ++i) asm volatile("" ::"v"(t[i].x), "v"(t[i].y));
+#pragma unroll
+            for (int i = 0; i < N; ++i)
+                col[i] = live ? (inb(i) ? csub(col[i], t[i]) : cd{0.0, 0.0})
+                              : ((i == c) ? cd{1.0, 0.0} : cd{0.0, 0.0});
         }
         if constexpr (MODE != MODE_FWD) {
 #pragma unroll
@@ -274,18 +297,6 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
 #pragma unroll
             for (int i = 0; i < N; ++i) MA[i + c * N] = col[i];
             wave_sync();
-            // Z = G (I + Y), column c
-            cd z[N];
-#pragma unroll
-            for (int i = 0; i < N; ++i) z[i] = col[i];
-#pragma unroll
-            for (int l = 0; l < N; ++l) {
-                if (l < nc) {
-                    const cd yl = y[l];
-#pragma unroll
-                    for (int i = 0; i < N; ++i) z[i] = cfma(MA[i + l * N], yl, z[i]);
-                }
-            }
             // trace shares: tr G and tr G^2 = sum g^2 + tr(Z^2) + 2 sum g^3 M_d
             cd tg = live ? gdiag : cd{0.0, 0.0};
             cd t2 = cd{0.0, 0.0};
@@ -303,6 +314,22 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
                 if (c == 0) {
                     tg = cadd(tg, g);
                     t2 = cadd(t2, g2);
+                }
+            }
+            // row c of gbar, on its way during the product
+            cd gv[MODE == MODE_VJP ? N : 1];
+            if constexpr (MODE == MODE_VJP) {
+#pragma unroll
+                for (int j = 0; j < N; ++j) gv[j] = ld_off(gb + (inb(j) ? j : 0) * ncs, gb_off);
+            }
+            // Z = G (I + Y), column c, over column c of G
+            cd(&z)[N] = col;
+#pragma unroll
+            for (int l = 0; l < N; ++l) {
+                if (l < nc) {
+                    const cd yl = y[l];
+#pragma unroll
+                    for (int i = 0; i < N; ++i) z[i] = cfma(MA[i + l * N], yl, z[i]);
                 }
             }
 #pragma unroll
@@ -329,7 +356,7 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
 #pragma unroll
                     for (int j = 0; j < N; ++j)
                         if (j < nc)
-                            MB[c + j * N] = cadd(GB[c + j * N], cscale(cadd(cconj(y[j]), cd{j == c ? 1.0 : 0.0, 0.0}), cn));
+                            MB[c + j * N] = cadd(gv[j], cscale(cadd(cconj(y[j]), cd{j == c ? 1.0 : 0.0, 0.0}), cn));
                 }
                 wave_sync();
                 if (vjp_here && live) {
@@ -366,12 +393,14 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
         wave_sync();  // gsh of this k is read by every lane of the slot before it is rewritten
     }
 
+    const int c = c0;
+    const bool live = c < nc;
     // ---- sum the trace shares over the lanes of each slot
     my[c] = trA;
     my[N + c] = tr2A;
     my[2 * N + c] = muA;
     wave_sync();
-    if (!wvalid) return;
+    if (!wvalid || !active) return;
     const size_t ch = chunk;
     if (c == 0) {
         cd s1 = cd{0.0, 0.0}, s2 = cd{0.0, 0.0}, s3 = cd{0.0, 0.0};
@@ -396,11 +425,10 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
                 if (b < nc) a.pSb[(ch * a.n_freq + nw) * m2 + b + c * nc] = acc[b];  // column c
         }
     }
-    (void)MATS;
 }
 
 template <int N, int MODE, int PREC, bool TRACE>
-__global__ __launch_bounds__(cols_wg(MODE, PREC)) void k_lattice_schur_cols(LatArgs a, const cd* __restrict__ sig_all)
+__global__ __launch_bounds__(cols_wg(MODE, PREC)) __attribute__((amdgpu_waves_per_eu(cols_waves(N, MODE, PREC)))) void k_lattice_schur_cols(LatArgs a, const cd* __restrict__ sig_all)
 {
     extern __shared__ cd lds[];
     cols_item<N, MODE, PREC, TRACE>(a, sig_all, lattice_tile(), blockIdx.y, lds);
@@ -411,7 +439,7 @@ __global__ __launch_bounds__(cols_wg(MODE, PREC)) void k_lattice_schur_cols(LatA
 // tile, k chunk}; static striding, no atomics, so every replay does the same
 // work in the same order).  Each system's tables come from its LatArgs.
 template <int N, int MODE, int PREC, bool TRACE>
-__global__ __launch_bounds__(cols_wg(MODE, PREC)) void k_lattice_schur_cols_multi(const LatArgs* __restrict__ args,
+__global__ __launch_bounds__(cols_wg(MODE, PREC)) __attribute__((amdgpu_waves_per_eu(cols_waves(N, MODE, PREC)))) void k_lattice_schur_cols_multi(const LatArgs* __restrict__ args,
                                                                                  const int4* __restrict__ items,
                                                                                  int n_items)
 {
