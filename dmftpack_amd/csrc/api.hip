@@ -164,8 +164,8 @@ extern "C" int dmftgpu_set_option(dmftgpu_handle h, int option, int value)
     if (!h) return DMFTGPU_ERR_ARG;
     switch (option) {
         case DMFTGPU_OPT_REFINE_STEPS:
+            // accepted and checked; the elimination is FP64 and has no steps to count
             if (value < 1 || value > 2) return fail(h, DMFTGPU_ERR_ARG, "refine steps %d outside 1..2", value);
-            h->refine_steps = value;
             return DMFTGPU_OK;
         case DMFTGPU_OPT_TARGET_WORKGROUPS:
             if (value < 0) return fail(h, DMFTGPU_ERR_ARG, "target workgroups %d < 0", value);
@@ -513,7 +513,7 @@ int run_lattice(dmftgpu_handle h, int method, int mode, const double* sigma, dou
     const int n_freq = ra ? ra->n_e : L.n_freq;
     int slots;
     if (method == DMFTGPU_PLAIN_F64) slots = dg::plain_slots(n, mode);
-    else slots = dg::schur_slots(nc, mode, method == DMFTGPU_SCHUR_F32R, h->schur_layout == 1 || (ra && mode != dg::MODE_FWD));
+    else slots = dg::schur_slots(nc, h->schur_layout == 1 || (ra && mode != dg::MODE_FWD));
     const bool cols = h->schur_layout == 1 || (ra && mode != dg::MODE_FWD);
     const int nw_plan = plan_points(h, method, ra);
     Plan P = pk ? Plan{nk, 1} : make_plan(nk, nw_plan, slots, lattice_target(h, method, nc, cols, nk, nw_plan, slots));
@@ -545,7 +545,6 @@ int run_lattice(dmftgpu_handle h, int method, int mode, const double* sigma, dou
     a.ed = h->ed;
     a.W = h->W;
     a.kdata = h->kdata;
-    a.refine = h->refine_steps;
     a.want_trace = want_trace ? 1 : 0;
     if (method != DMFTGPU_PLAIN_F64 && !ra) {
         a.pt_n = h->pt_n;
@@ -588,7 +587,7 @@ int run_lattice(dmftgpu_handle h, int method, int mode, const double* sigma, dou
         HIPCHK(dg::launch_lattice_plain(a, mode, h->stream, nullptr));
     } else {
         // schur_wg 0: each launch at its default width (launch_lattice_schur)
-        HIPCHK(dg::launch_lattice_schur(a, mode, method == DMFTGPU_SCHUR_F32R, h->stream, h->schur_wg,
+        HIPCHK(dg::launch_lattice_schur(a, mode, h->stream, h->schur_wg,
                                         h->schur_layout == 1));
     }
     if (h->timing) {
@@ -618,7 +617,7 @@ size_t lattice_ws_bytes(dmftgpu_handle h, int method, int mode, const RealAxis* 
     const size_t nw_tot = ra ? (size_t)ra->n_e : (size_t)L.n_freq * L.high_freq;
     const size_t n_freq = ra ? (size_t)ra->n_e : (size_t)L.n_freq;
     int slots = method == DMFTGPU_PLAIN_F64 ? dg::plain_slots(L.n, mode)
-                                            : dg::schur_slots(nc, mode, method == DMFTGPU_SCHUR_F32R,
+                                            : dg::schur_slots(nc,
                                                               h->schur_layout == 1 || (ra && mode != dg::MODE_FWD));
     const int nw_plan = plan_points(h, method, ra);
     Plan P = make_plan(L.n_k, nw_plan, slots,

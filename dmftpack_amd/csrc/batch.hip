@@ -168,7 +168,6 @@ LatArgs make_args(const dmftgpu_batch_s* b, const Sys& s, int mode, int chunks, 
     a.ed = s.ed;
     a.W = s.W;
     a.kdata = s.kdata;
-    a.refine = b->h->refine_steps;
     a.pSigAll = s.sig_all;
     a.pt_n = s.pt_n;
     a.pt_w = s.pt_w;
@@ -209,7 +208,7 @@ int build_group(dmftgpu_batch_s* b, Group& g, int mode, int wg, double target)
         args.push_back(a);
         // (the k-pair form covers 64 frequencies per item)
         const int wf = wg == dg::SCHUR_WG_KPAIR ? 64 : wg;
-        const int per_tile = g.cols ? dg::schur_slots(s.nc, mode, b->method == DMFTGPU_SCHUR_F32R, true) : wf;
+        const int per_tile = g.cols ? dg::schur_slots(s.nc, true) : wf;
         // tiles past the planned frequency points have work only when the moments rule the
         // Gauss points out: listed last, so that the striding stays even without them
         const int nwt = (s.nw_tot + per_tile - 1) / per_tile, nwp = (s.n_plan + per_tile - 1) / per_tile;
@@ -240,10 +239,8 @@ int build_group(dmftgpu_batch_s* b, Group& g, int mode, int wg, double target)
 int launch_group(dmftgpu_batch_s* b, Group& g, int mode)
 {
     dmftgpu_handle h = b->h;
-    const bool fp32 = b->method == DMFTGPU_SCHUR_F32R;
     LatArgs proto{};
     proto.nc = g.nc;
-    proto.refine = h->refine_steps;
     proto.want_trace = 1;
     SchurMulti m;
     m.args = g.dargs[slot(mode)];
@@ -252,10 +249,10 @@ int launch_group(dmftgpu_batch_s* b, Group& g, int mode)
     m.grid = std::min(g.n_items[slot(mode)], 256 * 16);
     m.max_nd = g.max_nd;
     if (g.cols) {
-        HIPCHK(dg::launch_lattice_schur_cols_multi(proto, mode, fp32, h->stream, m));
+        HIPCHK(dg::launch_lattice_schur_cols_multi(proto, mode, h->stream, m));
         return DMFTGPU_OK;
     }
-    HIPCHK(dg::launch_lattice_schur_multi(proto, mode, fp32, h->stream, g.wg[slot(mode)], m));
+    HIPCHK(dg::launch_lattice_schur_multi(proto, mode, h->stream, g.wg[slot(mode)], m));
     return DMFTGPU_OK;
 }
 
@@ -349,10 +346,10 @@ int issue_step(dmftgpu_batch_s* b)
     return DMFTGPU_OK;
 }
 
-// the k-pair form exists for the FP32R forward of the one-matrix-per-lane kernels at n_c >= 5
-bool kpair_ok(const dmftgpu_batch_s* b, const Group& g, int mode)
+// the k-pair form exists for the forward of the one-matrix-per-lane kernels at n_c >= 3
+bool kpair_ok(const Group& g, int mode)
 {
-    return mode == MODE_FWD && b->method == DMFTGPU_SCHUR_F32R && !g.cols && g.nc >= 5;
+    return mode == MODE_FWD && !g.cols && g.nc >= 3;
 }
 
 // times one mode's group launch for each candidate and keeps the fastest
@@ -378,7 +375,7 @@ int tune_group(dmftgpu_batch_s* b, Group& g, int mode)
     for (int wg : wgs)
         for (double t : targets) {
             if (g.cols && wg != 64) continue;  // one width: a wavefront per workgroup
-            if (wg == dg::SCHUR_WG_KPAIR && !kpair_ok(b, g, mode)) continue;
+            if (wg == dg::SCHUR_WG_KPAIR && !kpair_ok(g, mode)) continue;
             int rc = build_group(b, g, mode, wg, t);
             if (rc) return rc;
             rc = launch_group(b, g, mode);  // warm-up
@@ -421,7 +418,6 @@ extern "C" int dmftgpu_batch_create(dmftgpu_handle hu, int count, const dmftgpu_
         delete b;
         return fail(hu, DMFTGPU_ERR_HIP, "batch stream: %s", hipGetErrorString(e));
     }
-    b->h->refine_steps = hu->refine_steps;
     // inputs were produced on the caller's stream
     (void)hipEventRecord(b->ev_in, hu->stream);
     (void)hipStreamWaitEvent(b->bs, b->ev_in, 0);
@@ -566,7 +562,7 @@ static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system
     for (Group& g : b->groups) {
         for (int mode : {MODE_FWD, MODE_VJP}) {
             if (mode == MODE_VJP && !b->vjp) continue;
-            const int wg0 = kpair_ok(b, g, mode) ? dg::SCHUR_WG_KPAIR : 64;  // as the single-lattice default
+            const int wg0 = kpair_ok(g, mode) && dg::schur_kpair(g.nc, g.max_nd) ? dg::SCHUR_WG_KPAIR : 64;  // as the single-lattice default
             rc = (flags & DMFTGPU_BATCH_TUNE) ? 0 : build_group(b, g, mode, wg0, 1.0e6);
             if (rc) return rc;
         }

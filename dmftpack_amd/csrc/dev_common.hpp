@@ -10,10 +10,6 @@ namespace dg {
 struct __align__(16) cd {
     double x, y;
 };
-struct __align__(8) cf {
-    float x, y;
-};
-
 // Matches the reference's pi (dmft_common.h:43).
 constexpr double kPi = 3.1415926535897932384626;
 
@@ -57,24 +53,6 @@ __device__ __forceinline__ cd crcp(cd a)
     return cd{a.x * d, -a.y * d};
 }
 __device__ __forceinline__ cd csel(bool c, cd a, cd b) { return c ? a : b; }
-
-// float complex
-__device__ __forceinline__ cf fmk(float x, float y) { return cf{x, y}; }
-__device__ __forceinline__ cf fmul(cf a, cf b) { return cf{fmaf(a.x, b.x, -a.y * b.y), fmaf(a.x, b.y, a.y * b.x)}; }
-__device__ __forceinline__ cf ffms(cf a, cf b, cf acc)
-{
-    return cf{fmaf(-a.x, b.x, fmaf(a.y, b.y, acc.x)), fmaf(-a.x, b.y, fmaf(-a.y, b.x, acc.y))};
-}
-// acc + a*b
-__device__ __forceinline__ cf ffma(cf a, cf b, cf acc)
-{
-    return cf{fmaf(a.x, b.x, fmaf(-a.y, b.y, acc.x)), fmaf(a.x, b.y, fmaf(a.y, b.x, acc.y))};
-}
-__device__ __forceinline__ cf frcp(cf a)
-{
-    float d = __frcp_rn(fmaf(a.x, a.x, a.y * a.y));
-    return cf{a.x * d, -a.y * d};
-}
 
 // Orders LDS traffic between lanes of one wavefront (lock-step execution, LDS
 // operations of a wave complete in issue order; the fences stop the compiler

@@ -232,36 +232,4 @@ __device__ __forceinline__ void gj_columns_row16(cd (&col)[N], int c, int n)
     for (int i = 0; i < N; ++i) col[i] = cmul(col[i], scl);
 }
 
-// FP32 form of the same elimination (the first solve of FP32 + FP64-residual
-// refinement).
-template <int N>
-__device__ __forceinline__ void gj_columns_f32(cf (&col)[N], cf* bc, int c, int n)
-{
-    cf scl = cf{1.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-        if (j < n) {
-            cf* buf = bc + (j & 1) * N;
-            if (c == j) {
-#pragma unroll
-                for (int i = 0; i < N; ++i) buf[i] = col[i];
-            }
-            wave_sync();
-            cf b[N];
-#pragma unroll
-            for (int i = 0; i < N; ++i) b[i] = buf[i];
-            const cf p = frcp(b[j]);
-            const bool isj = (c == j);
-            const cf t = isj ? cf{0.f, 0.f} : fmul(col[j], p);
-#pragma unroll
-            for (int i = 0; i < N; ++i)
-                if (i != j) col[i] = ffms(b[i], t, col[i]);
-            col[j] = isj ? cf{-1.f, 0.f} : t;
-            scl = isj ? cf{-p.x, -p.y} : scl;
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i) col[i] = fmul(col[i], scl);
-}
-
 }  // namespace dg

@@ -3,14 +3,14 @@
 
 namespace dg {
 
-hipError_t launch_cols_16(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s)
+hipError_t launch_cols_16(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s)
 {
-    return launch_cols_bucket<16>(a, mode, fp32, sig_all, s);
+    return launch_cols_bucket<16>(a, mode, sig_all, s);
 }
 
-hipError_t launch_cols_multi_16(const LatArgs& proto, int mode, bool fp32, hipStream_t s, const SchurMulti& m)
+hipError_t launch_cols_multi_16(const LatArgs& proto, int mode, hipStream_t s, const SchurMulti& m)
 {
-    return launch_cols_bucket<16>(proto, mode, fp32, nullptr, s, &m);
+    return launch_cols_bucket<16>(proto, mode, nullptr, s, &m);
 }
 
 }  // namespace dg

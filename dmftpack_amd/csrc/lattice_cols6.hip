@@ -3,9 +3,9 @@
 
 namespace dg {
 
-hipError_t launch_cols_6(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s)
+hipError_t launch_cols_6(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s)
 {
-    return launch_cols_bucket<6>(a, mode, fp32, sig_all, s);
+    return launch_cols_bucket<6>(a, mode, sig_all, s);
 }
 
 }  // namespace dg

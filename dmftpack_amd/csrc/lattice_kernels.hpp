@@ -128,7 +128,6 @@ struct LatArgs {
     // Schur-complement data (per k), see lattice_schur.hip
     const double* ed;  // [nk][nd]      eigenvalues of H_dd(k)
     const cd* W;       // [nk][nc][nd]  H_cd(k) V_d(k), column-major nc x nd
-    int refine;        // FP32R: number of FP64-residual refinement steps
     cd* pSigAll;       // Schur: Sigma expanded to all nw_tot frequencies [nw_tot][nc*nc]
     int want_trace;    // FWD: also accumulate tr G (total N)
     const double* nbar_dev;  // VJP: device copy of nbar (overrides nbar when set)
@@ -198,22 +197,20 @@ bool density_lr_supported(int n, int nc);
 hipError_t launch_density_matrix_lr(const LatArgs& a, const cd* W, const cd* Vd, const double* ed, const cd* U,
                                     const double* wt, cd* dens, hipStream_t s);
 
-// Schur complement (FP64 or FP32 + refinement); wg = workgroup width of the
-// one-matrix-per-lane kernels: 64 or 128 frequencies, or 0 for the default of
-// each launch (the FP32R forward at n_c >= 5 in SCHUR_WG_KPAIR form, the adjoint at
-// 128, the others at 64); cols selects the column-per-lane kernels for n_c <= 6
-// (always used above 6)
-// wg value of the FP32R forward kernel (n_c >= 5) as two wavefronts over 64
-// frequencies, each walking every other k of the chunk into shared LDS
-// accumulators (half the LDS per wavefront of the 64-lane form); its work items
-// cover 64 frequencies
+// Schur complement; wg = workgroup width of the one-matrix-per-lane kernels: 64 or 128
+// frequencies, SCHUR_WG_KPAIR (forward, n_c >= 3), or 0 for the default (the forward by
+// schur_kpair, everything else at 64); cols selects the column-per-lane kernels for
+// n_c <= 6 (always used above 6).
+// SCHUR_WG_KPAIR: two wavefronts over 64 frequencies, each walking every other k of the
+// chunk into shared LDS accumulators; its work items cover 64 frequencies
 constexpr int SCHUR_WG_KPAIR = 1;
-hipError_t launch_lattice_schur(const LatArgs& a, int mode, bool fp32, hipStream_t s, int wg = 64, bool cols = false);
+bool schur_kpair(int nc, int nd);
+hipError_t launch_lattice_schur(const LatArgs& a, int mode, hipStream_t s, int wg = 64, bool cols = false);
 // Sigma expanded over all frequency points into a.pSigAll
 hipError_t launch_sigma_all(const LatArgs& a, hipStream_t s);
-// Persistent launch over a work list of several lattices sharing n_c (and mode,
-// precision, refinement): args [systems] in device memory, items {system,
-// wtile, chunk, 0}; proto carries nc / refine / want_trace.
+// Persistent launch over a work list of several lattices sharing n_c (and mode):
+// args [systems] in device memory, items {system,
+// wtile, chunk, 0}; proto carries nc / want_trace.
 struct SchurMulti {
     const LatArgs* args;
     const int4* items;
@@ -221,42 +218,42 @@ struct SchurMulti {
     int grid;
     int max_nd;
 };
-hipError_t launch_lattice_schur_multi(const LatArgs& proto, int mode, bool fp32, hipStream_t s, int wg,
+hipError_t launch_lattice_schur_multi(const LatArgs& proto, int mode, hipStream_t s, int wg,
                                       const SchurMulti& m);
 // the same for 6 < n_c <= 16: column-per-lane kernels (MODE_FWD, MODE_VJP over every frequency)
-hipError_t launch_lattice_schur_cols_multi(const LatArgs& proto, int mode, bool fp32, hipStream_t s,
+hipError_t launch_lattice_schur_cols_multi(const LatArgs& proto, int mode, hipStream_t s,
                                            const SchurMulti& m);
 // frequencies per workgroup of the Schur kernel for n_c (grid planning)
-int schur_slots(int nc, int mode, bool fp32, bool cols);
+int schur_slots(int nc, bool cols);
 bool schur_supported(int n, int nc);
 // the persistent multi-lattice launch covers the one-matrix-per-lane kernels
 bool schur_multi_supported(int nc);
 // one-matrix-per-lane Schur kernels of one n_c (lattice_lane{1..6}.hip)
-hipError_t launch_lane_1(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s, int wg,
+hipError_t launch_lane_1(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s, int wg,
                          const SchurMulti* m);
-hipError_t launch_lane_2(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s, int wg,
+hipError_t launch_lane_2(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s, int wg,
                          const SchurMulti* m);
-hipError_t launch_lane_3(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s, int wg,
+hipError_t launch_lane_3(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s, int wg,
                          const SchurMulti* m);
-hipError_t launch_lane_4(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s, int wg,
+hipError_t launch_lane_4(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s, int wg,
                          const SchurMulti* m);
-hipError_t launch_lane_5(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s, int wg,
+hipError_t launch_lane_5(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s, int wg,
                          const SchurMulti* m);
-hipError_t launch_lane_6(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s, int wg,
+hipError_t launch_lane_6(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s, int wg,
                          const SchurMulti* m);
 // column-per-lane Schur kernels (lattice_cols{4,5,6,8,10,12,16}.hip)
-hipError_t launch_cols_4(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s);
-hipError_t launch_cols_5(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s);
-hipError_t launch_cols_6(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s);
-hipError_t launch_cols_8(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s);
+hipError_t launch_cols_4(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s);
+hipError_t launch_cols_5(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s);
+hipError_t launch_cols_6(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s);
+hipError_t launch_cols_8(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s);
 // persistent multi-lattice launches of the column-per-lane buckets for n_c > 6
-hipError_t launch_cols_multi_8(const LatArgs& proto, int mode, bool fp32, hipStream_t s, const SchurMulti& m);
-hipError_t launch_cols_multi_10(const LatArgs& proto, int mode, bool fp32, hipStream_t s, const SchurMulti& m);
-hipError_t launch_cols_multi_12(const LatArgs& proto, int mode, bool fp32, hipStream_t s, const SchurMulti& m);
-hipError_t launch_cols_multi_16(const LatArgs& proto, int mode, bool fp32, hipStream_t s, const SchurMulti& m);
-hipError_t launch_cols_10(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s);
-hipError_t launch_cols_12(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s);
-hipError_t launch_cols_16(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s);
+hipError_t launch_cols_multi_8(const LatArgs& proto, int mode, hipStream_t s, const SchurMulti& m);
+hipError_t launch_cols_multi_10(const LatArgs& proto, int mode, hipStream_t s, const SchurMulti& m);
+hipError_t launch_cols_multi_12(const LatArgs& proto, int mode, hipStream_t s, const SchurMulti& m);
+hipError_t launch_cols_multi_16(const LatArgs& proto, int mode, hipStream_t s, const SchurMulti& m);
+hipError_t launch_cols_10(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s);
+hipError_t launch_cols_12(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s);
+hipError_t launch_cols_16(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s);
 
 // W = H_cd V_d per k (Schur preparation)
 hipError_t launch_schur_prep(const cd* Hk, const cd* Vd, int n, int nc, int nk, cd* W, hipStream_t s);

@@ -3,10 +3,10 @@
 
 namespace dg {
 
-hipError_t launch_lane_5(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s, int wg,
+hipError_t launch_lane_5(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s, int wg,
                          const SchurMulti* m)
 {
-    return launch_lane_nc<5>(a, mode, fp32, sig_all, s, wg, m);
+    return launch_lane_nc<5>(a, mode, sig_all, s, wg, m);
 }
 
 }  // namespace dg

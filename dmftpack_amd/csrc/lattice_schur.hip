@@ -15,24 +15,22 @@ static int cols_bucket(int nc)
 {
     return nc <= 4 ? 4 : nc <= 6 ? nc : nc <= 8 ? 8 : nc <= 10 ? 10 : nc <= 12 ? 12 : 16;
 }
-int schur_slots(int nc, int mode, bool fp32, bool cols)
+int schur_slots(int nc, bool cols)
 {
     if (nc <= 6 && !cols) return 64;
-    (void)mode;
-    (void)fp32;
     return 64 / cols_bucket(nc);  // one wavefront of 64/N slots per workgroup
 }
 
-static hipError_t dispatch_nc(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s, int wg,
+static hipError_t dispatch_nc(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s, int wg,
                               const SchurMulti* m)
 {
     switch (a.nc) {
-        case 1: return launch_lane_1(a, mode, fp32, sig_all, s, wg, m);
-        case 2: return launch_lane_2(a, mode, fp32, sig_all, s, wg, m);
-        case 3: return launch_lane_3(a, mode, fp32, sig_all, s, wg, m);
-        case 4: return launch_lane_4(a, mode, fp32, sig_all, s, wg, m);
-        case 5: return launch_lane_5(a, mode, fp32, sig_all, s, wg, m);
-        case 6: return launch_lane_6(a, mode, fp32, sig_all, s, wg, m);
+        case 1: return launch_lane_1(a, mode, sig_all, s, wg, m);
+        case 2: return launch_lane_2(a, mode, sig_all, s, wg, m);
+        case 3: return launch_lane_3(a, mode, sig_all, s, wg, m);
+        case 4: return launch_lane_4(a, mode, sig_all, s, wg, m);
+        case 5: return launch_lane_5(a, mode, sig_all, s, wg, m);
+        case 6: return launch_lane_6(a, mode, sig_all, s, wg, m);
         default: return hipErrorInvalidValue;
     }
 }
@@ -55,48 +53,52 @@ hipError_t launch_sigma_all(const LatArgs& a, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_lattice_schur(const LatArgs& a, int mode, bool fp32, hipStream_t s, int wg, bool cols)
+// Forward as two wavefronts splitting the k walk over 64 frequencies, sums of G_cc in
+// LDS, rather than one with the sums in registers: half the registers, so at n_c = 5
+// three wavefronts per SIMD instead of two and at n_c = 6 two instead of one, against
+// two barriers and n_c^2 LDS updates per k, which a short walk over d does not cover.
+// Measured (8000 k x 1040 points, pair / single, ms): n_c = 6, n_d = 0 0.63 / 0.69, 9
+// 1.43 / 2.41; n_c = 5, n_d = 0 0.57 / 0.36, 4 0.62 / 0.58, 6 0.69 / 0.70, 9 0.80 / 0.91,
+// 16 1.27 / 1.67; n_c = 4, n_d = 4 0.38 / 0.37, 6 0.44 / 0.45, 16 0.76 / 0.87; n_c = 3,
+// n_d = 9 0.33 / 0.35.  Real axis, 32768 k x 1000 points, n_c = 5, n_d = 9: 2.84 / 3.35.
+bool schur_kpair(int nc, int nd) { return nc == 6 || (nc >= 3 && nc <= 5 && nd >= 6); }
+
+hipError_t launch_lattice_schur(const LatArgs& a, int mode, hipStream_t s, int wg, bool cols)
 {
-    // wg = 0: the adjoint call at 128 frequencies per workgroup (its one wavefront
-    // per SIMD gains from a second sharing each per-k scalar fill), the FP32R
-    // forward at n_c >= 5 as two wavefronts splitting the k walk over 64 frequencies
-    // (its LDS accumulators, n_c^2 x 1 KB per 64 frequencies, then allow the 8
-    // wavefronts per CU that its registers allow, against 6 at n_c = 5 and 4 at
-    // n_c = 6), the other launches at 64
-    const int wg_call = wg ? wg : mode == MODE_VJP ? 128 : 64;
-    const int wg_fwd = wg ? wg : mode == MODE_FWD && fp32 && a.nc >= 5 ? SCHUR_WG_KPAIR : wg_call;
+    const int wg_call = wg ? wg : 64;
+    const int wg_fwd = wg ? wg : schur_kpair(a.nc, a.n - a.nc) ? SCHUR_WG_KPAIR : 64;
     hipError_t e = launch_sigma_all(a, s);
     if (e != hipSuccess) return e;
     if (a.real_axis && mode == MODE_FWD && a.nc <= 6 && !cols)
-        return dispatch_nc(a, MODE_FWD_REAL, fp32, a.pSigAll, s, wg_call, nullptr);
+        return dispatch_nc(a, MODE_FWD_REAL, a.pSigAll, s, wg_fwd, nullptr);
     if (a.nc > 6 || cols || a.real_axis) {  // the per-lane kernels take the real axis in the forward only
         switch (cols_bucket(a.nc)) {
-            case 4: return launch_cols_4(a, mode, fp32, a.pSigAll, s);
-            case 5: return launch_cols_5(a, mode, fp32, a.pSigAll, s);
-            case 6: return launch_cols_6(a, mode, fp32, a.pSigAll, s);
-            case 8: return launch_cols_8(a, mode, fp32, a.pSigAll, s);
-            case 10: return launch_cols_10(a, mode, fp32, a.pSigAll, s);
-            case 12: return launch_cols_12(a, mode, fp32, a.pSigAll, s);
-            default: return launch_cols_16(a, mode, fp32, a.pSigAll, s);
+            case 4: return launch_cols_4(a, mode, a.pSigAll, s);
+            case 5: return launch_cols_5(a, mode, a.pSigAll, s);
+            case 6: return launch_cols_6(a, mode, a.pSigAll, s);
+            case 8: return launch_cols_8(a, mode, a.pSigAll, s);
+            case 10: return launch_cols_10(a, mode, a.pSigAll, s);
+            case 12: return launch_cols_12(a, mode, a.pSigAll, s);
+            default: return launch_cols_16(a, mode, a.pSigAll, s);
         }
     }
-    return dispatch_nc(a, mode, fp32, a.pSigAll, s, wg_fwd, nullptr);
+    return dispatch_nc(a, mode, a.pSigAll, s, mode == MODE_FWD ? wg_fwd : wg_call, nullptr);
 }
 
-hipError_t launch_lattice_schur_multi(const LatArgs& proto, int mode, bool fp32, hipStream_t s, int wg,
+hipError_t launch_lattice_schur_multi(const LatArgs& proto, int mode, hipStream_t s, int wg,
                                       const SchurMulti& m)
 {
-    return dispatch_nc(proto, mode, fp32, nullptr, s, wg, &m);
+    return dispatch_nc(proto, mode, nullptr, s, wg, &m);
 }
 
-hipError_t launch_lattice_schur_cols_multi(const LatArgs& proto, int mode, bool fp32, hipStream_t s,
+hipError_t launch_lattice_schur_cols_multi(const LatArgs& proto, int mode, hipStream_t s,
                                            const SchurMulti& m)
 {
     switch (cols_bucket(proto.nc)) {
-        case 8: return launch_cols_multi_8(proto, mode, fp32, s, m);
-        case 10: return launch_cols_multi_10(proto, mode, fp32, s, m);
-        case 12: return launch_cols_multi_12(proto, mode, fp32, s, m);
-        case 16: return launch_cols_multi_16(proto, mode, fp32, s, m);
+        case 8: return launch_cols_multi_8(proto, mode, s, m);
+        case 10: return launch_cols_multi_10(proto, mode, s, m);
+        case 12: return launch_cols_multi_12(proto, mode, s, m);
+        case 16: return launch_cols_multi_16(proto, mode, s, m);
         default: return hipErrorInvalidValue;
     }
 }

@@ -18,9 +18,9 @@
 //     E = (z+mu) I - Sigma(iw), Sigma read from the cache at each k;
 //     the g_d of the slot's frequency are computed once per slot and shared
 //     through LDS;
-//   * inversion: column-per-lane Gauss-Jordan (gj.hpp); FP32R inverts in FP32
-//     and refines each column against the FP64 S held in LDS,
-//     x_c <- x_c + X0 (e_c - S x_c);
+//   * inversion: column-per-lane Gauss-Jordan (gj.hpp), in FP64 for both Schur methods
+//     (lattice_schur_lane.hpp; n = 32, n_c = 10, 1728 k x 528 points, forward + adjoint:
+//     4.8 ms against 5.5 ms with an FP32 inverse and one FP64-residual step);
 //   * FWD accumulates column c of G_cc over the k chunk in registers; the
 //     trace terms are per-lane partials summed over the slot at the end;
 //   * DENS/VJP exchange G_cc, Z and V = gbar + cn (I + Y)^H through per-slot
@@ -47,11 +47,10 @@ __host__ __device__ constexpr int cols_nc_min(int N)
 
 // one wavefront per workgroup: the per-k data comes from global memory, so
 // wavefronts share nothing but the cache
-__host__ __device__ constexpr int cols_wg(int, int) { return 64; }
+__host__ __device__ constexpr int cols_wg() { return 64; }
 
-// per-slot LDS (cd units): gsh 32 - nc_min (g_d), MA N*N, MB N*N (the FP32R forward
-// keeps only X0, FP32, there: N*N/2); the elimination's broadcast buffer (2N) lies where
-// nothing is held yet, in MB (FP32R) or MA, and on its own only in the FP64 forward.
+// per-slot LDS (cd units): gsh 32 - nc_min (g_d), and the elimination's broadcast buffer
+// (2 N) in the forward; MA N*N and MB N*N otherwise, the buffer then lying in MA.
 // Sigma and gbar are read from the cache at each k and the spare lanes repeat lanes of
 // the last slot instead of writing to a slot of their own: the LDS is what decides how
 // many wavefronts of the adjoint a CU holds (N = 10: 39.5 KB each with tables of their
@@ -61,59 +60,56 @@ __host__ __device__ constexpr int cols_wg(int, int) { return 64; }
 // The size is odd (in 16-byte entries): the slots of a wavefront read the same entry of
 // their own matrices at once, and with a multiple of 16 entries (the adjoint at N = 10 or
 // 16, every form at N = 8) all of those fell into the same four banks.
-__host__ __device__ constexpr int cols_slot_size(int N, int mode, int prec)
+__host__ __device__ constexpr int cols_slot_size(int N, int mode)
 {
     const int g = 32 - cols_nc_min(N);  // n_d at most
-    if (mode == MODE_FWD && prec == 0) return (g + 2 * N) | 1;
-    return (g + N * N + (mode == MODE_FWD ? (N * N + 1) / 2 : N * N)) | 1;
+    return (g + (mode == MODE_FWD ? 2 * N : 2 * N * N)) | 1;
 }
 
-__host__ __device__ constexpr int cols_slots(int N, int mode, int prec) { return cols_wg(mode, prec) / 64 * (64 / N); }
+__host__ __device__ constexpr int cols_slots(int N) { return 64 / N; }
 
-inline size_t cols_lds_bytes(int N, int mode, int prec, int, int)
+inline size_t cols_lds_bytes(int N, int mode)
 {
-    const int nwave = cols_wg(mode, prec) / 64;
-    const int spw = 64 / N;
-    return sizeof(cd) * ((size_t)nwave * spw * cols_slot_size(N, mode, prec));
+    return sizeof(cd) * ((size_t)cols_slots(N) * cols_slot_size(N, mode));
 }
 
 // Wavefronts per SIMD the register allocator is held to: as many as fit without spilling
-// column-sized values (three at N = 10 only for the FP64 forward; the adjoint at N = 16
+// column-sized values (three in the forward up to N = 10; the adjoint at N = 16
 // needs 356 registers, and its LDS admits four wavefronts to a CU anyway).
-__host__ __device__ constexpr int cols_waves(int N, int mode, int prec)
+__host__ __device__ constexpr int cols_waves(int N, int mode)
 {
-    return mode == MODE_FWD ? (N <= 8 || (N == 10 && prec == 0) ? 3 : 2) : N <= 12 ? 2 : 1;
+    return mode == MODE_FWD ? (N <= 10 ? 3 : 2) : N <= 12 ? 2 : 1;
 }
 
 __device__ __forceinline__ cd ld_off(const cd* base, unsigned bytes) { return *(const cd*)((const char*)base + bytes); }
 
 // One (frequency tile, k chunk) work item of one lattice: the body of the
 // per-lattice kernel and of the persistent multi-lattice kernel below.
-template <int N, int MODE, int PREC, bool TRACE>
+template <int N, int MODE, bool TRACE>
 __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict__ sig_all, int wtile, int chunk,
                                           cd* lds)
 {
     constexpr int SPW = 64 / N;
-    constexpr int SLOTS = cols_slots(N, MODE, PREC);
-    constexpr int SS = cols_slot_size(N, MODE, PREC);
+    constexpr int SLOTS = cols_slots(N);
+    constexpr int SS = cols_slot_size(N, MODE);
     const int n = a.n, nc = a.nc, nd = a.n - nc, m2 = nc * nc;
     constexpr int NMIN = cols_nc_min(N);
     auto inb = [nc](int i) { return i < NMIN || i < nc; };  // row / column i inside the n_c block
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, lane = tid;  // one wavefront
     // the spare lanes of a wavefront repeat the first lanes of its last slot: the same
     // values to the same LDS entries, and nothing stored at the end
     const bool active = lane < SPW * N;
     const int sl = active ? lane / N : SPW - 1;
     const int c0 = active ? lane - sl * N : lane - SPW * N;
     const int cc = c0 < nc ? c0 : 0;  // clamped column index for loads
-    cd* my = lds + (size_t)(wave * SPW + sl) * SS;
+    cd* my = lds + (size_t)sl * SS;
     cd* gsh = my;
     cd* MA = gsh + 32 - NMIN;
     cd* MB = MA + N * N;
-    cd* bc = PREC > 0 ? MB : MA;  // before MB (PREC 0: MA) is written
+    cd* bc = MA;  // the elimination's buffer, before MA is written
     const int npts = n_points(a);
     if (wtile * SLOTS >= npts) return;  // tile past the last frequency point
-    const int nw = wtile * SLOTS + wave * SPW + sl;
+    const int nw = wtile * SLOTS + sl;
     const bool wvalid = nw < npts;
     const int nwc = nw < npts ? nw : npts - 1;
     const int k0 = chunk * a.k_per_chunk;
@@ -218,57 +214,7 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
         }
 
         // ---- G_cc = S^{-1}, column c
-        if constexpr (PREC == 0) {
-            gj_columns<N>(col, bc, c, nc);
-        } else {
-            cf* X0 = (cf*)MB;
-#pragma unroll
-            for (int i = 0; i < N; ++i) MA[i + c * N] = col[i];
-            cf x0[N];
-#pragma unroll
-            for (int i = 0; i < N; ++i) x0[i] = cf{(float)col[i].x, (float)col[i].y};
-            gj_columns_f32<N>(x0, (cf*)bc, c, nc);
-#pragma unroll
-            for (int i = 0; i < N; ++i) X0[i + c * N] = x0[i];
-            wave_sync();
-#pragma unroll
-            for (int i = 0; i < N; ++i) col[i] = cd{(double)x0[i].x, (double)x0[i].y};
-            const int steps = a.refine < 1 ? 1 : (a.refine > 2 ? 2 : a.refine);
-#pragma unroll 1
-            for (int it = 0; it < steps; ++it) {
-                wave_sync();  // keeps the S and X0 reads inside the step (no hoisting into registers)
-                cf r[N];  // e_c - S x_c in FP64, stored in FP32
-                // each row of S (then of X0) is read from LDS as a whole before
-                // its products, pinned by empty asm statements: left to itself the
-                // compiler issues one read, waits for it and uses it, one LDS
-                // round trip per entry
-#pragma unroll
-                for (int i = 0; i < N; ++i) {
-                    cd srow[N];
-#pragma unroll
-                    for (int l = 0; l < N; ++l) srow[l] = MA[i + l * N];
-#pragma unroll
-                    for (int l = 0; l < N; ++l) asm volatile("" ::"v"(srow[l].x), "v"(srow[l].y));
-                    cd s = (i == c) ? cd{1.0, 0.0} : cd{0.0, 0.0};
-#pragma unroll
-                    for (int l = 0; l < N; ++l) s = cfms(srow[l], col[l], s);
-                    r[i] = cf{(float)s.x, (float)s.y};
-                }
-#pragma unroll
-                for (int i = 0; i < N; ++i) {
-                    cf xrow[N];
-#pragma unroll
-                    for (int l = 0; l < N; ++l) xrow[l] = X0[i + l * N];
-#pragma unroll
-                    for (int l = 0; l < N; ++l) asm volatile("" ::"v"(xrow[l].x), "v"(xrow[l].y));
-                    cf t = cf{0.f, 0.f};
-#pragma unroll
-                    for (int l = 0; l < N; ++l) t = ffma(xrow[l], r[l], t);
-                    col[i] = cadd(col[i], cd{(double)t.x, (double)t.y});
-                }
-            }
-            wave_sync();
-        }
+        gj_columns<N>(col, bc, c, nc);
         cd gdiag = cd{0.0, 0.0};  // G_cc(c, c)
 #pragma unroll
         for (int i = 0; i < N; ++i)
@@ -427,19 +373,19 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
     }
 }
 
-template <int N, int MODE, int PREC, bool TRACE>
-__global__ __launch_bounds__(cols_wg(MODE, PREC)) __attribute__((amdgpu_waves_per_eu(cols_waves(N, MODE, PREC)))) void k_lattice_schur_cols(LatArgs a, const cd* __restrict__ sig_all)
+template <int N, int MODE, bool TRACE>
+__global__ __launch_bounds__(cols_wg()) __attribute__((amdgpu_waves_per_eu(cols_waves(N, MODE)))) void k_lattice_schur_cols(LatArgs a, const cd* __restrict__ sig_all)
 {
     extern __shared__ cd lds[];
-    cols_item<N, MODE, PREC, TRACE>(a, sig_all, lattice_tile(), blockIdx.y, lds);
+    cols_item<N, MODE, TRACE>(a, sig_all, lattice_tile(), blockIdx.y, lds);
 }
 
 // Persistent form over a work list spanning several lattices with n_c in this
 // bucket: workgroup b takes items b, b + gridDim.x, ... ({system, frequency
 // tile, k chunk}; static striding, no atomics, so every replay does the same
 // work in the same order).  Each system's tables come from its LatArgs.
-template <int N, int MODE, int PREC, bool TRACE>
-__global__ __launch_bounds__(cols_wg(MODE, PREC)) __attribute__((amdgpu_waves_per_eu(cols_waves(N, MODE, PREC)))) void k_lattice_schur_cols_multi(const LatArgs* __restrict__ args,
+template <int N, int MODE, bool TRACE>
+__global__ __launch_bounds__(cols_wg()) __attribute__((amdgpu_waves_per_eu(cols_waves(N, MODE)))) void k_lattice_schur_cols_multi(const LatArgs* __restrict__ args,
                                                                                  const int4* __restrict__ items,
                                                                                  int n_items)
 {
@@ -447,54 +393,46 @@ __global__ __launch_bounds__(cols_wg(MODE, PREC)) __attribute__((amdgpu_waves_pe
     for (int it = blockIdx.x; it < n_items; it += gridDim.x) {
         const int4 item = items[it];  // {system, wtile, chunk, -}
         const LatArgs a = args[item.x];
-        cols_item<N, MODE, PREC, TRACE>(a, a.pSigAll, item.y, item.z, lds);
+        cols_item<N, MODE, TRACE>(a, a.pSigAll, item.y, item.z, lds);
         __syncthreads();
     }
 }
 
-template <int N, int MODE, int PREC, bool TRACE>
+template <int N, int MODE, bool TRACE>
 hipError_t launch_cols_k(const LatArgs& a, const cd* sig_all, hipStream_t s, const SchurMulti* m)
 {
     if (a.nc < cols_nc_min(N) || a.nc > N) return hipErrorInvalidValue;  // the kernels assume this bucket
     const int nd = a.n - a.nc;
-    const size_t shm = cols_lds_bytes(N, MODE, PREC, a.nc, nd);
-    constexpr int SLOTS = cols_slots(N, MODE, PREC);
+    const size_t shm = cols_lds_bytes(N, MODE);
+    constexpr int SLOTS = cols_slots(N);
     if (m) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_lattice_schur_cols_multi<N, MODE, PREC, TRACE>,
+        hipError_t e = hipFuncSetAttribute((const void*)k_lattice_schur_cols_multi<N, MODE, TRACE>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((k_lattice_schur_cols_multi<N, MODE, PREC, TRACE>), dim3(m->grid),
-                           dim3(cols_wg(MODE, PREC)), shm, s, m->args, m->items, m->n_items);
+        hipLaunchKernelGGL((k_lattice_schur_cols_multi<N, MODE, TRACE>), dim3(m->grid),
+                           dim3(cols_wg()), shm, s, m->args, m->items, m->n_items);
         return hipGetLastError();
     }
-    hipError_t e = hipFuncSetAttribute((const void*)k_lattice_schur_cols<N, MODE, PREC, TRACE>,
+    hipError_t e = hipFuncSetAttribute((const void*)k_lattice_schur_cols<N, MODE, TRACE>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
     if (e != hipSuccess) return e;
     const dim3 grid = lattice_grid(a, SLOTS);
-    hipLaunchKernelGGL((k_lattice_schur_cols<N, MODE, PREC, TRACE>), grid, dim3(cols_wg(MODE, PREC)), shm, s, a,
+    hipLaunchKernelGGL((k_lattice_schur_cols<N, MODE, TRACE>), grid, dim3(cols_wg()), shm, s, a,
                        sig_all);
     return hipGetLastError();
 }
 
-template <int N, int PREC>
-hipError_t launch_cols_p(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s, const SchurMulti* m)
-{
-    if (mode == MODE_FWD)
-        return a.want_trace ? launch_cols_k<N, MODE_FWD, PREC, true>(a, sig_all, s, m)
-                            : launch_cols_k<N, MODE_FWD, PREC, false>(a, sig_all, s, m);
-    if (mode == MODE_DENS) return launch_cols_k<N, MODE_DENS, PREC, false>(a, sig_all, s, m);
-    return launch_cols_k<N, MODE_VJP, PREC, false>(a, sig_all, s, m);
-}
-
-// entry of one bucket (one translation unit each); PREC 0 = FP64, 1 = FP32 +
-// a.refine (1 or 2) FP64-residual steps; with m, the persistent multi-lattice
-// launch over m's work list (a is then only a prototype: n_c, refine, want_trace)
+// entry of one bucket (one translation unit each); with m, the persistent
+// multi-lattice launch over m's work list (a is then only a prototype: n_c, want_trace)
 template <int N>
-hipError_t launch_cols_bucket(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s,
+hipError_t launch_cols_bucket(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s,
                               const SchurMulti* m = nullptr)
 {
-    if (!fp32) return launch_cols_p<N, 0>(a, mode, sig_all, s, m);
-    return launch_cols_p<N, 1>(a, mode, sig_all, s, m);
+    if (mode == MODE_FWD)
+        return a.want_trace ? launch_cols_k<N, MODE_FWD, true>(a, sig_all, s, m)
+                            : launch_cols_k<N, MODE_FWD, false>(a, sig_all, s, m);
+    if (mode == MODE_DENS) return launch_cols_k<N, MODE_DENS, false>(a, sig_all, s, m);
+    return launch_cols_k<N, MODE_VJP, false>(a, sig_all, s, m);
 }
 
 }  // namespace dg

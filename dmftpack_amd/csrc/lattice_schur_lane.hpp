@@ -19,17 +19,19 @@
 // This header holds the kernel templates; lattice_lane{1..6}.hip instantiate
 // one n_c each (launch_lane_<n_c>), lattice_schur.hip dispatches.
 //
-// Mapping: one (k, iw) matrix per lane, everything in registers (n_c <= 6):
+// Mapping: one (k, iw) matrix per lane, in registers (n_c <= 6):
 // a wavefront owns 64 consecutive frequencies and walks a chunk of k points;
 // the per-k data (H_cc, e_d, P_d for pairs a <= b; built once by k_schur_kdata)
 // is read with wave-uniform scalar loads.  The n_c x n_c inversion is
 // Gauss-Jordan without pivoting (the Hermitian part of -iS is >= w_n I for
 // causal Sigma, so elimination without pivoting is stable).
 //
-// FP32R: the Schur complement S is formed in FP64, inverted in FP32, and the
-// FP32 inverse X0 preconditions iterative refinement with FP64 residuals
-//   X = X0 + D,  D <- D + X0 (I - S X),
-// `refine` times; the correction D is kept in FP32.
+// Both Schur methods run this FP64 elimination.  An FP32 inverse with one FP64-residual
+// step (X0 + X0 (I - S X0)) takes three times the multiply-adds, which pays only where
+// FP32 arithmetic is at least that much faster: the FP32 vector rate of gfx950 without
+// packed FP32 is the FP64 rate.  Measured in that form and in this one, 8000 k x 1040
+// points, forward + adjoint: n = 14, n_c = 5 3.33 against 2.87 ms, n = 14, n_c = 6 9.5
+// against 7.3 ms, n_c = 1 and 2 equal.
 #pragma once
 #include "lattice_kernels.hpp"
 
@@ -52,29 +54,6 @@ __device__ __forceinline__ void gj_inverse(cd (&S)[NC][NC])
             for (int c = 0; c < NC; ++c)
                 if (c != j) S[i][c] = cfms(f, S[j][c], S[i][c]);
             S[i][j] = cneg(cmul(f, p));
-        }
-        S[j][j] = p;
-    }
-}
-
-template <int NC>
-__device__ __forceinline__ void gj_inverse_f32(cf (&S)[NC][NC])
-{
-#pragma unroll
-    for (int j = 0; j < NC; ++j) {
-        const cf p = frcp(S[j][j]);
-#pragma unroll
-        for (int c = 0; c < NC; ++c)
-            if (c != j) S[j][c] = fmul(S[j][c], p);
-#pragma unroll
-        for (int i = 0; i < NC; ++i) {
-            if (i == j) continue;
-            const cf f = S[i][j];
-#pragma unroll
-            for (int c = 0; c < NC; ++c)
-                if (c != j) S[i][c] = ffms(f, S[j][c], S[i][c]);
-            const cf fp = fmul(f, p);
-            S[i][j] = cf{-fp.x, -fp.y};
         }
         S[j][j] = p;
     }
@@ -156,10 +135,10 @@ __host__ __device__ __forceinline__ int kblock_size(int nd)
 // a.kdata through the constant address space: its addresses are wave-uniform,
 // so the loads become scalar loads and the products against it take SGPR
 // operands, with no LDS traffic and no barriers in the k loop.
-// KS = 2 (the FP32R forward only): the WG lanes are KS wavefronts over the same
+// KS = 2 (the forward, schur_kpair): the WG lanes are KS wavefronts over the same
 // WG / KS frequencies, each walking every KS-th k of the chunk and adding into
-// one set of LDS accumulators, which then costs a wavefront half the LDS.
-template <int NC, int MODE, bool F32R, int WG, bool TRACE, int REFINE, int KS = 1>
+// one set of LDS accumulators.
+template <int NC, int MODE, int WG, bool TRACE, int KS = 1>
 __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restrict__ sig_all, int wtile, int chunk,
                                            cd* lds)
 {
@@ -169,9 +148,9 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
     constexpr int M2 = NC * NC;
     constexpr bool FWDLIKE = MODE == MODE_FWD || MODE == MODE_FWD_REAL;
     // accumulators that do not fit next to the working matrices live in LDS
-    constexpr bool ACC_LDS = (MODE == MODE_VJP) || (FWDLIKE && F32R);
+    constexpr bool ACC_LDS = MODE == MODE_VJP || KS > 1;
     constexpr int FW = WG / KS;       // frequencies per workgroup
-    static_assert(KS == 1 || (KS == 2 && MODE == MODE_FWD && ACC_LDS && FW % 64 == 0),
+    static_assert(KS == 1 || (KS == 2 && FWDLIKE && FW % 64 == 0),
                   "k pairs: LDS-accumulating forward, whole wavefronts per part");
     const int nd = a.n - NC;
     const int bs = kblock_size<NC>(nd);
@@ -235,7 +214,7 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
         // Sigma's loads are issued here, all together, so that they complete under
         // the d loop below instead of waiting in turn where S is combined; not in
         // the FP64 forward kernels, whose G_cc sums already fill the registers
-        constexpr bool SIG_EARLY = F32R || !FWDLIKE;
+        constexpr bool SIG_EARLY = !FWDLIKE;
         cd sg[SIG_EARLY ? NC : 1][SIG_EARLY ? NC : 1];
         if constexpr (SIG_EARLY) {
 #pragma unroll
@@ -309,101 +288,22 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                 }
             }
         // ---- G_cc = S^{-1}
-        if (!F32R) {
-            gj_inverse<NC>(G);
-        } else {
-            // G holds S (FP64); X0 = S^{-1} in FP32
-            cf X0[NC][NC];
-#pragma unroll
-            for (int i = 0; i < NC; ++i)
-#pragma unroll
-                for (int j = 0; j < NC; ++j) X0[i][j] = cf{(float)G[i][j].x, (float)G[i][j].y};
-            gj_inverse_f32<NC>(X0);
-            if constexpr (REFINE == 1) {
-                // One step: the whole residual R = I - S X0 (FP64 products,
-                // FP32 storage) is formed first, after which S is dead and
-                // G = X0 + X0 R is written over it.  Peak: S + X0 + R.
-                // R is formed row by row so that each row of S dies as soon as
-                // its row of R is done.
-                cf Rm[NC][NC];
-#pragma unroll
-                for (int i = 0; i < NC; ++i)
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) {
-                        cd s = cd{i == c ? 1.0 : 0.0, 0.0};
-#pragma unroll
-                        for (int l = 0; l < NC; ++l) s = cfms(G[i][l], cd{(double)X0[l][c].x, (double)X0[l][c].y}, s);
-                        Rm[i][c] = cf{(float)s.x, (float)s.y};
-                    }
-#pragma unroll
-                for (int c = 0; c < NC; ++c)
-#pragma unroll
-                    for (int i = 0; i < NC; ++i) {
-                        cf t = cf{0.f, 0.f};
-#pragma unroll
-                        for (int l = 0; l < NC; ++l) t = ffma(X0[i][l], Rm[l][c], t);
-                        G[i][c] = cd{(double)X0[i][c].x + (double)t.x, (double)X0[i][c].y + (double)t.y};
-                    }
-            } else {
-            // X = X0 + D with the correction D held in FP32: D is ~kappa*eps32 of
-            // |X|, so its own FP32 rounding (~kappa*eps32^2 of |X|) is the
-            // accuracy floor of the refinement, the same as adding an FP32
-            // correction into an FP64 X, at half the registers.
-            cf D[NC][NC];
-#pragma unroll
-            for (int i = 0; i < NC; ++i)
-#pragma unroll
-                for (int j = 0; j < NC; ++j) D[i][j] = cf{0.f, 0.f};
-            for (int it = 0; it < REFINE; ++it) {
-#pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    cd xc[NC];  // column c of X in FP64
-#pragma unroll
-                    for (int l = 0; l < NC; ++l)
-                        xc[l] = cd{(double)X0[l][c].x + (double)D[l][c].x, (double)X0[l][c].y + (double)D[l][c].y};
-                    cf rc[NC];  // r = e_c - S x_c, formed in FP64, stored in FP32
-#pragma unroll
-                    for (int i = 0; i < NC; ++i) {
-                        cd s = cd{i == c ? 1.0 : 0.0, 0.0};
-#pragma unroll
-                        for (int l = 0; l < NC; ++l) s = cfms(G[i][l], xc[l], s);
-                        rc[i] = cf{(float)s.x, (float)s.y};
-                    }
-#pragma unroll
-                    for (int i = 0; i < NC; ++i) {
-                        cf t = D[i][c];
-#pragma unroll
-                        for (int l = 0; l < NC; ++l) t = ffma(X0[i][l], rc[l], t);
-                        D[i][c] = t;
-                    }
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < NC; ++i)
-#pragma unroll
-                for (int j = 0; j < NC; ++j)
-                    G[i][j] = cd{(double)X0[i][j].x + (double)D[i][j].x, (double)X0[i][j].y + (double)D[i][j].y};
-            }
-        }
+        gj_inverse<NC>(G);
 
         if (FWDLIKE) {
             if constexpr (ACC_LDS) {
+                // the parts add in turn, part 0 first, so that every sum has one
+                // order and the result is the same on every run
                 auto add_g = [&]() {
 #pragma unroll
                     for (int j = 0; j < NC; ++j)
 #pragma unroll
                         for (int i = 0; i < NC; ++i) lds_add(&sAcc[(i + j * NC) * FW + lane], G[i][j]);
                 };
-                if constexpr (KS > 1) {
-                    // the parts add in turn, part 0 first, so that every sum has one
-                    // order and the result is the same on every run
-                    __syncthreads();
-                    if (part == 0) add_g();
-                    __syncthreads();
-                    if (part == 1 && kin) add_g();
-                } else {
-                    add_g();
-                }
+                __syncthreads();
+                if (part == 0) add_g();
+                __syncthreads();
+                if (part == 1 && kin) add_g();
             } else {
 #pragma unroll
                 for (int i = 0; i < (ACC_LDS ? 1 : NC); ++i)
@@ -641,26 +541,31 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
     }
 }
 
-// Waves per SIMD the register allocator is held to.  At n_c = 5 the forward and
-// density kernels (FP64, or FP32 with one refinement step) need a few registers
-// more than the 256 of two waves; two waves with a few bytes of scratch beat one.
-template <int NC, int MODE, int REFINE>
-constexpr int schur_waves() { return (NC == 5 && MODE != MODE_VJP && REFINE <= 1) ? 2 : 1; }
+// Waves per SIMD the register allocator is held to.  At n_c = 5 the density kernel
+// needs a few registers more than the 256 of two waves; two waves with a few bytes
+// of scratch beat one.  KS > 1: as many as its LDS admits, without scratch.
+template <int NC, int MODE, int KS>
+constexpr int schur_waves()
+{
+    if (MODE == MODE_VJP) return 1;
+    if (KS > 1) return NC <= 4 ? 4 : NC == 5 ? 3 : 2;
+    return NC == 5 ? 2 : 1;
+}
 
-template <int NC, int MODE, bool F32R, int WG, bool TRACE, int REFINE, int KS = 1>
-__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(schur_waves<NC, MODE, REFINE>())))
+template <int NC, int MODE, int WG, bool TRACE, int KS = 1>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(schur_waves<NC, MODE, KS>())))
 void k_lattice_schur(LatArgs a, const cd* __restrict__ sig_all)
 {
     extern __shared__ cd lds[];
-    schur_item<NC, MODE, F32R, WG, TRACE, REFINE, KS>(a, sig_all, lattice_tile(), blockIdx.y, lds);
+    schur_item<NC, MODE, WG, TRACE, KS>(a, sig_all, lattice_tile(), blockIdx.y, lds);
 }
 
 // Persistent form over a work list spanning several lattices of the same n_c:
 // workgroup b takes items b, b + gridDim.x, ... (static striding, no atomics,
 // so every replay does the same work in the same order).  Each system's per-k
 // blocks come from its LatArgs (kdata), read through the constant address space.
-template <int NC, int MODE, bool F32R, int WG, bool TRACE, int REFINE, int KS = 1>
-__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(schur_waves<NC, MODE, REFINE>())))
+template <int NC, int MODE, int WG, bool TRACE, int KS = 1>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(schur_waves<NC, MODE, KS>())))
 void k_lattice_schur_multi(const LatArgs* __restrict__ args,
                                                             const int4* __restrict__ items, int n_items)
 {
@@ -668,90 +573,62 @@ void k_lattice_schur_multi(const LatArgs* __restrict__ args,
     for (int it = blockIdx.x; it < n_items; it += gridDim.x) {
         const int4 item = items[it];  // {system, wtile, chunk, -}
         const LatArgs a = args[item.x];
-        schur_item<NC, MODE, F32R, WG, TRACE, REFINE, KS>(a, a.pSigAll, item.y, item.z, lds);
+        schur_item<NC, MODE, WG, TRACE, KS>(a, a.pSigAll, item.y, item.z, lds);
         __syncthreads();
     }
 }
 
-template <int NC, int MODE, bool F32R, int WG, int KS = 1>
+template <int NC, int MODE, int WG, int KS = 1>
 constexpr size_t schur_shm()
 {
-    constexpr bool ACC_LDS = (MODE == MODE_VJP) || ((MODE == MODE_FWD || MODE == MODE_FWD_REAL) && F32R);
+    constexpr bool ACC_LDS = MODE == MODE_VJP || KS > 1;
     // KS > 1: one accumulator set per frequency, plus the tr G sums
     return ACC_LDS ? sizeof(cd) * (size_t)(NC * NC + (KS > 1 ? 1 : 0)) * (WG / KS) : 0;
 }
 
-template <int NC, int MODE, bool F32R, bool TRACE, int REFINE, int WG, int KS = 1>
+template <int NC, int MODE, bool TRACE, int WG, int KS = 1>
 hipError_t launch_nc_w(const LatArgs& a, const cd* sig_all, hipStream_t s, const SchurMulti* multi)
 {
-    constexpr size_t shm = schur_shm<NC, MODE, F32R, WG, KS>();
+    constexpr size_t shm = schur_shm<NC, MODE, WG, KS>();
     if (multi) {
-        hipError_t e = hipFuncSetAttribute((const void*)k_lattice_schur_multi<NC, MODE, F32R, WG, TRACE, REFINE, KS>,
+        hipError_t e = hipFuncSetAttribute((const void*)k_lattice_schur_multi<NC, MODE, WG, TRACE, KS>,
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((k_lattice_schur_multi<NC, MODE, F32R, WG, TRACE, REFINE, KS>), dim3(multi->grid), dim3(WG),
+        hipLaunchKernelGGL((k_lattice_schur_multi<NC, MODE, WG, TRACE, KS>), dim3(multi->grid), dim3(WG),
                            shm, s, multi->args, multi->items, multi->n_items);
         return hipGetLastError();
     }
     constexpr int FW = WG / KS;  // frequencies per workgroup
     const dim3 grid = lattice_grid(a, FW);
-    hipError_t e = hipFuncSetAttribute((const void*)k_lattice_schur<NC, MODE, F32R, WG, TRACE, REFINE, KS>,
+    hipError_t e = hipFuncSetAttribute((const void*)k_lattice_schur<NC, MODE, WG, TRACE, KS>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_lattice_schur<NC, MODE, F32R, WG, TRACE, REFINE, KS>), grid, dim3(WG), shm, s, a, sig_all);
+    hipLaunchKernelGGL((k_lattice_schur<NC, MODE, WG, TRACE, KS>), grid, dim3(WG), shm, s, a, sig_all);
     return hipGetLastError();
 }
 
-template <int NC, int MODE, bool F32R, bool TRACE, int REFINE>
-hipError_t launch_nc_r(const LatArgs& a, const cd* sig_all, hipStream_t s, int wg, const SchurMulti* m)
-{
-    if constexpr (MODE == MODE_FWD_REAL) {  // one width on the real axis
-        (void)wg;
-        return launch_nc_w<NC, MODE, F32R, TRACE, REFINE, 128>(a, sig_all, s, m);
-    } else {
-        if constexpr (MODE == MODE_FWD && F32R && NC >= 5) {  // two wavefronts over 64 frequencies
-            if (wg == SCHUR_WG_KPAIR) return launch_nc_w<NC, MODE, F32R, TRACE, REFINE, 128, 2>(a, sig_all, s, m);
-        }
-        if (wg == 128) return launch_nc_w<NC, MODE, F32R, TRACE, REFINE, 128>(a, sig_all, s, m);
-        return launch_nc_w<NC, MODE, F32R, TRACE, REFINE, 64>(a, sig_all, s, m);
-    }
-}
-
-template <int NC, int MODE, bool F32R, bool TRACE>
+template <int NC, int MODE, bool TRACE>
 hipError_t launch_nc(const LatArgs& a, const cd* sig_all, hipStream_t s, int wg, const SchurMulti* m)
 {
-    if constexpr (!F32R) {
-        return launch_nc_r<NC, MODE, false, TRACE, 0>(a, sig_all, s, wg, m);
-    } else {
-        if (a.refine <= 1) return launch_nc_r<NC, MODE, true, TRACE, 1>(a, sig_all, s, wg, m);
-        return launch_nc_r<NC, MODE, true, TRACE, 2>(a, sig_all, s, wg, m);
+    if constexpr (NC >= 3 && (MODE == MODE_FWD || MODE == MODE_FWD_REAL)) {  // two wavefronts over 64 frequencies
+        if (wg == SCHUR_WG_KPAIR) return launch_nc_w<NC, MODE, TRACE, 128, 2>(a, sig_all, s, m);
     }
+    if (wg == 128) return launch_nc_w<NC, MODE, TRACE, 128>(a, sig_all, s, m);
+    return launch_nc_w<NC, MODE, TRACE, 64>(a, sig_all, s, m);
 }
 
-// All variants of one n_c: mode, precision, trace.
+// All variants of one n_c: mode, trace.
 template <int NC>
-hipError_t launch_lane_nc(const LatArgs& a, int mode, bool fp32, const cd* sig_all, hipStream_t s, int wg,
-                          const SchurMulti* m)
+hipError_t launch_lane_nc(const LatArgs& a, int mode, const cd* sig_all, hipStream_t s, int wg, const SchurMulti* m)
 {
-    if (mode == MODE_FWD) {
-        if (a.want_trace)
-            return fp32 ? launch_nc<NC, MODE_FWD, true, true>(a, sig_all, s, wg, m)
-                        : launch_nc<NC, MODE_FWD, false, true>(a, sig_all, s, wg, m);
-        return fp32 ? launch_nc<NC, MODE_FWD, true, false>(a, sig_all, s, wg, m)
-                    : launch_nc<NC, MODE_FWD, false, false>(a, sig_all, s, wg, m);
-    }
-    if (mode == MODE_FWD_REAL) {
-        if (a.want_trace)
-            return fp32 ? launch_nc<NC, MODE_FWD_REAL, true, true>(a, sig_all, s, wg, m)
-                        : launch_nc<NC, MODE_FWD_REAL, false, true>(a, sig_all, s, wg, m);
-        return fp32 ? launch_nc<NC, MODE_FWD_REAL, true, false>(a, sig_all, s, wg, m)
-                    : launch_nc<NC, MODE_FWD_REAL, false, false>(a, sig_all, s, wg, m);
-    }
-    if (mode == MODE_DENS)
-        return fp32 ? launch_nc<NC, MODE_DENS, true, false>(a, sig_all, s, wg, m)
-                    : launch_nc<NC, MODE_DENS, false, false>(a, sig_all, s, wg, m);
-    return fp32 ? launch_nc<NC, MODE_VJP, true, false>(a, sig_all, s, wg, m)
-                : launch_nc<NC, MODE_VJP, false, false>(a, sig_all, s, wg, m);
+    if (mode == MODE_FWD)
+        return a.want_trace ? launch_nc<NC, MODE_FWD, true>(a, sig_all, s, wg, m)
+                            : launch_nc<NC, MODE_FWD, false>(a, sig_all, s, wg, m);
+    if (mode == MODE_FWD_REAL)
+        return a.want_trace ? launch_nc<NC, MODE_FWD_REAL, true>(a, sig_all, s, wg, m)
+                            : launch_nc<NC, MODE_FWD_REAL, false>(a, sig_all, s, wg, m);
+    if (mode == MODE_DENS) return launch_nc<NC, MODE_DENS, false>(a, sig_all, s, wg, m);
+    return launch_nc<NC, MODE_VJP, false>(a, sig_all, s, wg, m);
 }
 
 }  // namespace dg

@@ -50,7 +50,9 @@ extern "C" {
  * solves every frequency. */
 #define DMFTGPU_PLAIN_F64 0  /* full n x n inverse per (k,iw) in FP64 (GreenFtn.cpp:261) */
 #define DMFTGPU_SCHUR_F64 1  /* Schur complement on the correlated block, FP64 */
-#define DMFTGPU_SCHUR_F32R 2 /* Schur complement, FP32 solve + FP64-residual refinement */
+#define DMFTGPU_SCHUR_F32R 2 /* Schur complement at FP32-with-refinement accuracy or better: runs the FP64
+                                elimination, which gfx950 does in a third of the operations (its FP32 vector
+                                rate is its FP64 rate) */
 
 typedef struct dmftgpu_lattice {
     int32_t n;          /* NBAND[k] (TB.h:29), uniform over k, 1..32 */
@@ -76,14 +78,15 @@ const char* dmftgpu_last_error(dmftgpu_handle h);
 const char* dmftgpu_version(void);
 
 /* Tuning options (no reference counterpart). */
-#define DMFTGPU_OPT_REFINE_STEPS 1      /* FP64-residual refinement steps of SCHUR_F32R (1 or 2, default 2) */
+#define DMFTGPU_OPT_REFINE_STEPS 1      /* FP64-residual refinement steps of SCHUR_F32R (1 or 2): checked and
+                                           without effect, the elimination being FP64 */
 #define DMFTGPU_OPT_TARGET_WORKGROUPS 2 /* work items per lattice launch, sets the k chunking (0 = default: up to
                                            32768 for the one-matrix-per-lane Schur kernels, keeping >= 64 k per
                                            chunk and >= 8192 items; 8192 for the others) */
 #define DMFTGPU_OPT_SCHUR_WG 3          /* frequencies per workgroup of the Schur kernels (64 or 128; default 0 =
-                                           the adjoint at 128, the FP32R forward at n_corr >= 5 as two
-                                           wavefronts over 64 frequencies splitting the k walk, the others
-                                           at 64) */
+                                           64, or, for the forward at n_corr = 6 and at n_corr 3..5 with six or
+                                           more uncorrelated orbitals, two wavefronts over 64 frequencies
+                                           splitting the k walk) */
 #define DMFTGPU_OPT_SCHUR_LAYOUT 4      /* n_c <= 6: 0 = one (k,iw) matrix per lane (default), 1 = one column
                                            per lane (always used for n_c > 6) */
 #define DMFTGPU_OPT_UPFOLD_CHUNK 5      /* k points per chunk of dmftgpu_upfold_density (0 = as many as 512 MiB of
@@ -269,7 +272,7 @@ int dmftgpu_batch_create(dmftgpu_handle h, int count, const dmftgpu_system* syst
                          dmftgpu_batch* out);
 int dmftgpu_batch_run(dmftgpu_batch b);
 /* Tuning result of n_corr group `group` (returns the number of groups when out of range):
- * wg[2], target[2], ms[2] per mode (forward, adjoint); wg = 1 is the FP32R forward's k-pair form
+ * wg[2], target[2], ms[2] per mode (forward, adjoint); wg = 1 is the forward's k-pair form
  * (two wavefronts over 64 frequencies, each taking every other k of a chunk). */
 int dmftgpu_batch_tuning(dmftgpu_batch b, int group, int* nc, int* systems, int* wg, double* target, double* ms);
 int dmftgpu_batch_destroy(dmftgpu_batch b);
