@@ -206,8 +206,8 @@ int build_group(dmftgpu_batch_s* b, Group& g, int mode, int wg, double target)
         }
         LatArgs a = make_args(b, s, mode, chunks, kpc);
         args.push_back(a);
-        // (the k-pair form covers 64 frequencies per item)
-        const int wf = wg == dg::SCHUR_WG_KPAIR ? 64 : wg;
+        // (the k-split form covers 64 frequencies per item)
+        const int wf = wg == dg::SCHUR_WG_KSPLIT ? 64 : wg;
         const int per_tile = g.cols ? dg::schur_slots(s.nc, true) : wf;
         // tiles past the planned frequency points have work only when the moments rule the
         // Gauss points out: listed last, so that the striding stays even without them
@@ -346,17 +346,17 @@ int issue_step(dmftgpu_batch_s* b)
     return DMFTGPU_OK;
 }
 
-// the k-pair form exists for the forward of the one-matrix-per-lane kernels at n_c >= 3
-bool kpair_ok(const Group& g, int mode)
+// the k-split form of the one-matrix-per-lane kernels: forward at n_c >= 3, adjoint at n_c >= 4
+bool ksplit_ok(const Group& g, int mode)
 {
-    return mode == MODE_FWD && !g.cols && g.nc >= 3;
+    return !g.cols && g.nc >= (mode == MODE_FWD ? 3 : 4);
 }
 
 // times one mode's group launch for each candidate and keeps the fastest
 int tune_group(dmftgpu_batch_s* b, Group& g, int mode)
 {
     dmftgpu_handle h = b->h;
-    const int wgs[3] = {64, 128, dg::SCHUR_WG_KPAIR};
+    const int wgs[3] = {64, 128, dg::SCHUR_WG_KSPLIT};
     const double targets[4] = {6.25e4, 2.5e5, 1.0e6, 4.0e6};
     struct Events {  // destroyed on every return path
         hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -375,7 +375,7 @@ int tune_group(dmftgpu_batch_s* b, Group& g, int mode)
     for (int wg : wgs)
         for (double t : targets) {
             if (g.cols && wg != 64) continue;  // one width: a wavefront per workgroup
-            if (wg == dg::SCHUR_WG_KPAIR && !kpair_ok(g, mode)) continue;
+            if (wg == dg::SCHUR_WG_KSPLIT && !ksplit_ok(g, mode)) continue;
             int rc = build_group(b, g, mode, wg, t);
             if (rc) return rc;
             rc = launch_group(b, g, mode);  // warm-up
@@ -562,7 +562,7 @@ static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system
     for (Group& g : b->groups) {
         for (int mode : {MODE_FWD, MODE_VJP}) {
             if (mode == MODE_VJP && !b->vjp) continue;
-            const int wg0 = kpair_ok(g, mode) && dg::schur_kpair(g.nc, g.max_nd) ? dg::SCHUR_WG_KPAIR : 64;  // as the single-lattice default
+            const int wg0 = ksplit_ok(g, mode) && dg::schur_ksplit(g.nc, g.max_nd, mode) ? dg::SCHUR_WG_KSPLIT : 64;  // as the single-lattice default
             rc = (flags & DMFTGPU_BATCH_TUNE) ? 0 : build_group(b, g, mode, wg0, 1.0e6);
             if (rc) return rc;
         }

@@ -197,14 +197,14 @@ bool density_lr_supported(int n, int nc);
 hipError_t launch_density_matrix_lr(const LatArgs& a, const cd* W, const cd* Vd, const double* ed, const cd* U,
                                     const double* wt, cd* dens, hipStream_t s);
 
-// Schur complement; wg = workgroup width of the one-matrix-per-lane kernels: 64 or 128
-// frequencies, SCHUR_WG_KPAIR (forward, n_c >= 3), or 0 for the default (the forward by
-// schur_kpair, everything else at 64); cols selects the column-per-lane kernels for
-// n_c <= 6 (always used above 6).
-// SCHUR_WG_KPAIR: two wavefronts over 64 frequencies, each walking every other k of the
-// chunk into shared LDS accumulators; its work items cover 64 frequencies
-constexpr int SCHUR_WG_KPAIR = 1;
-bool schur_kpair(int nc, int nd);
+// Schur complement; wg = width of the one-matrix-per-lane kernels: 64 or 128 frequencies
+// per workgroup, SCHUR_WG_KSPLIT (forward at n_c >= 3, adjoint at n_c >= 4), or 0 for the
+// default (schur_ksplit, else 64); cols selects the column-per-lane kernels for n_c <= 6
+// (always used above 6).
+// SCHUR_WG_KSPLIT: several wavefronts over 64 frequencies, each walking every second (or
+// fourth) k of the chunk into shared LDS sums; its work items cover 64 frequencies
+constexpr int SCHUR_WG_KSPLIT = 1;
+bool schur_ksplit(int nc, int nd, int mode);
 hipError_t launch_lattice_schur(const LatArgs& a, int mode, hipStream_t s, int wg = 64, bool cols = false);
 // Sigma expanded over all frequency points into a.pSigAll
 hipError_t launch_sigma_all(const LatArgs& a, hipStream_t s);

@@ -53,24 +53,34 @@ hipError_t launch_sigma_all(const LatArgs& a, hipStream_t s)
     return hipGetLastError();
 }
 
-// Forward as two wavefronts splitting the k walk over 64 frequencies, sums of G_cc in
-// LDS, rather than one with the sums in registers: half the registers, so at n_c = 5
-// three wavefronts per SIMD instead of two and at n_c = 6 two instead of one, against
-// two barriers and n_c^2 LDS updates per k, which a short walk over d does not cover.
-// Measured (8000 k x 1040 points, pair / single, ms): n_c = 6, n_d = 0 0.63 / 0.69, 9
-// 1.43 / 2.41; n_c = 5, n_d = 0 0.57 / 0.36, 4 0.62 / 0.58, 6 0.69 / 0.70, 9 0.80 / 0.91,
-// 16 1.27 / 1.67; n_c = 4, n_d = 4 0.38 / 0.37, 6 0.44 / 0.45, 16 0.76 / 0.87; n_c = 3,
-// n_d = 9 0.33 / 0.35.  Real axis, 32768 k x 1000 points, n_c = 5, n_d = 9: 2.84 / 3.35.
-bool schur_kpair(int nc, int nd) { return nc == 6 || (nc >= 3 && nc <= 5 && nd >= 6); }
+// Launches as wavefronts that split the k walk over the same 64 frequencies, with one
+// set of sums in LDS, rather than one wavefront per 64 frequencies.
+// Forward (two wavefronts; alone the sums are in registers): half the registers, so at
+// n_c = 5 three wavefronts per SIMD instead of two and at n_c = 6 two instead of one,
+// against two barriers and n_c^2 LDS updates per k, which a short walk over d does not
+// cover.  Measured (8000 k x 1040 points, split / alone, ms): n_c = 6, n_d = 0 0.63 /
+// 0.69, 9 1.43 / 2.41; n_c = 5, n_d = 0 0.57 / 0.36, 4 0.62 / 0.58, 6 0.69 / 0.70, 9
+// 0.80 / 0.91, 16 1.27 / 1.67; n_c = 4, n_d = 4 0.38 / 0.37, 6 0.44 / 0.45, 16 0.76 /
+// 0.87; n_c = 3, n_d = 9 0.33 / 0.35.  Real axis, 32768 k x 1000 points, n_c = 5,
+// n_d = 9: 2.84 / 3.35.
+// Adjoint (four wavefronts, at n_c = 6 two; gbar is in LDS and no longer in registers):
+// two wavefronts per SIMD at n_c = 4 and 5, no AGPR traffic at n_c = 6, against a barrier
+// per column.  n_c = 4, n_d = 0 0.55 / 0.58, 9 1.01 / 1.11, 18 1.60 / 1.89; n_c = 6, n_d =
+// 0 2.1 / 4.0, 9 3.7 / 5.5, 18 6.6 / 8.2; n_c = 5, n_d = 0 1.23 / 1.03, 9 1.79 / 1.79, 18
+// 2.68 / 3.04.
+bool schur_ksplit(int nc, int nd, int mode)
+{
+    if (mode == MODE_VJP) return nc == 4 || nc == 6 || (nc == 5 && nd >= 9);
+    return mode == MODE_FWD && (nc == 6 || (nc >= 3 && nc <= 5 && nd >= 6));
+}
 
 hipError_t launch_lattice_schur(const LatArgs& a, int mode, hipStream_t s, int wg, bool cols)
 {
-    const int wg_call = wg ? wg : 64;
-    const int wg_fwd = wg ? wg : schur_kpair(a.nc, a.n - a.nc) ? SCHUR_WG_KPAIR : 64;
+    if (wg == 0) wg = schur_ksplit(a.nc, a.n - a.nc, mode) ? SCHUR_WG_KSPLIT : 64;
     hipError_t e = launch_sigma_all(a, s);
     if (e != hipSuccess) return e;
     if (a.real_axis && mode == MODE_FWD && a.nc <= 6 && !cols)
-        return dispatch_nc(a, MODE_FWD_REAL, a.pSigAll, s, wg_fwd, nullptr);
+        return dispatch_nc(a, MODE_FWD_REAL, a.pSigAll, s, wg, nullptr);
     if (a.nc > 6 || cols || a.real_axis) {  // the per-lane kernels take the real axis in the forward only
         switch (cols_bucket(a.nc)) {
             case 4: return launch_cols_4(a, mode, a.pSigAll, s);
@@ -82,7 +92,7 @@ hipError_t launch_lattice_schur(const LatArgs& a, int mode, hipStream_t s, int w
             default: return launch_cols_16(a, mode, a.pSigAll, s);
         }
     }
-    return dispatch_nc(a, mode, a.pSigAll, s, mode == MODE_FWD ? wg_fwd : wg_call, nullptr);
+    return dispatch_nc(a, mode, a.pSigAll, s, wg, nullptr);
 }
 
 hipError_t launch_lattice_schur_multi(const LatArgs& proto, int mode, hipStream_t s, int wg,

@@ -131,13 +131,38 @@ __host__ __device__ __forceinline__ int kblock_size(int nd)
     return NC * NC + nd * NP + (nd + 1) / 2;
 }
 
+template <int NC>
+__host__ __device__ constexpr bool schur_sig_lds() { return NC <= 4; }
+
+template <int I>
+struct ColumnIndex {
+    static constexpr int value = I;
+};
+// f(0), ..., f(NC - 1), or f(b) for a wave-uniform b, with the column as a constant
+template <int NC, int B = 0, class F>
+__device__ __forceinline__ void for_columns(F&& f)
+{
+    if constexpr (B < NC) {
+        f(ColumnIndex<B>{});
+        for_columns<NC, B + 1>(f);
+    }
+}
+template <int NC, int B = 0, class F>
+__device__ __forceinline__ void pick_column(int b, F&& f)
+{
+    if constexpr (B < NC) {
+        if (b == B) f(ColumnIndex<B>{});
+        else pick_column<NC, B + 1>(b, f);
+    }
+}
+
 // One (frequency tile, k chunk) work item.  The per-k block is read from
 // a.kdata through the constant address space: its addresses are wave-uniform,
 // so the loads become scalar loads and the products against it take SGPR
 // operands, with no LDS traffic and no barriers in the k loop.
-// KS = 2 (the forward, schur_kpair): the WG lanes are KS wavefronts over the same
-// WG / KS frequencies, each walking every KS-th k of the chunk and adding into
-// one set of LDS accumulators.
+// KS > 1 (schur_ksplit): the WG lanes are KS
+// groups of wavefronts over the same WG / KS frequencies, each walking every KS-th k
+// of the chunk and adding into one set of LDS accumulators.
 template <int NC, int MODE, int WG, bool TRACE, int KS = 1>
 __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restrict__ sig_all, int wtile, int chunk,
                                            cd* lds)
@@ -150,21 +175,27 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
     // accumulators that do not fit next to the working matrices live in LDS
     constexpr bool ACC_LDS = MODE == MODE_VJP || KS > 1;
     constexpr int FW = WG / KS;       // frequencies per workgroup
-    static_assert(KS == 1 || (KS == 2 && FWDLIKE && FW % 64 == 0),
-                  "k pairs: LDS-accumulating forward, whole wavefronts per part");
+    // adjoint, KS > 1: Sigma in LDS too, where that leaves room for three workgroups to
+    // a CU (n_c = 4); at n_c = 5 it would fit twice but gained nothing at n_d = 9 and lost
+    // 14 % at n_d = 18
+    constexpr bool SIG_LDS = MODE == MODE_VJP && KS > 1 && schur_sig_lds<NC>();
+    static_assert(KS == 1 || (FW % 64 == 0 && (FWDLIKE ? KS == 2 : MODE == MODE_VJP)),
+                  "split k walk: forward pairs or the adjoint, whole wavefronts per part");
     const int nd = a.n - NC;
     const int bs = kblock_size<NC>(nd);
     cd* sAcc = lds;                   // [M2][FW] complex, frequency-contiguous
-    cd* sTr = lds + M2 * FW;          // KS > 1: [FW] sums of the tr G shares
+    cd* sTr = lds + M2 * FW;          // KS > 1: forward [FW] sums of the tr G shares
+    cd* sGb = lds + M2 * FW;          //         adjoint [M2][FW] gbar, [M2][FW] Sigma
+    cd* sSig = lds + 2 * M2 * FW;
     const int lane = KS == 1 ? (int)threadIdx.x : (int)threadIdx.x % FW;  // this lane's frequency in the tile
     // which k of every KS: wave-uniform (FW is a multiple of 64), so that the k
     // walk and the per-k block addresses stay scalar
     const int part = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / FW);
     const int nw_hi = n_points(a);
     const int nw = wtile * FW + lane;
-    // a wavefront past the last point has no work (KS > 1: both parts of a
-    // workgroup hold the same frequencies, so they leave together)
-    if (__builtin_amdgcn_readfirstlane(nw) >= nw_hi) return;
+    // a wavefront past the last point has no work (KS > 1: they meet at barriers, so
+    // only a whole workgroup leaves)
+    if ((KS > 1 ? wtile * FW : __builtin_amdgcn_readfirstlane(nw)) >= nw_hi) return;
     const bool wvalid = nw < nw_hi;
     const int nwc = wvalid ? nw : nw_hi - 1;  // clamp for loads
     const int k0 = chunk * a.k_per_chunk;
@@ -178,6 +209,7 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
         mu = a.mu;
     }
     const bool vjp_here = (MODE == MODE_VJP) && wvalid && nw < a.n_freq;
+    const bool tile_vjp = wtile * FW < a.n_freq;  // the same for the whole workgroup
     const cd* sig = sig_all + (size_t)nwc * M2;
     const cd* gb = (MODE == MODE_VJP) ? a.gbar + (size_t)(nw < a.n_freq ? nw : 0) * M2 : nullptr;
     // nbar: host value, or (batched adjoint) a device scalar written by an earlier kernel
@@ -188,7 +220,14 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
         // (KS > 1: every part clears the same entries, before the barrier below)
         for (int e = 0; e < M2; ++e) sAcc[e * FW + lane] = cd{0.0, 0.0};
         if constexpr (KS > 1) {
-            sTr[lane] = cd{0.0, 0.0};
+            if constexpr (MODE == MODE_VJP) {
+                for (int e = part; e < M2; e += KS) {
+                    sGb[e * FW + lane] = gb[e];
+                    if constexpr (SIG_LDS) sSig[e * FW + lane] = sig[e];
+                }
+            } else {
+                sTr[lane] = cd{0.0, 0.0};
+            }
             __syncthreads();
         }
     } else {
@@ -210,20 +249,20 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
         // compiler treats as invariant: those loads stay scalar despite the
         // clobber.
         __asm__ __volatile__("" ::: "memory");
-        kcache_fill(a.kdata + (size_t)k * bs);
         // Sigma's loads are issued here, all together, so that they complete under
         // the d loop below instead of waiting in turn where S is combined; not in
         // the FP64 forward kernels, whose G_cc sums already fill the registers
-        constexpr bool SIG_EARLY = !FWDLIKE;
-        cd sg[SIG_EARLY ? NC : 1][SIG_EARLY ? NC : 1];
+        constexpr bool SIG_EARLY = !FWDLIKE && !SIG_LDS, SIG_REG = SIG_EARLY || SIG_LDS;
+        cd sg[SIG_REG ? NC : 1][SIG_REG ? NC : 1];
         if constexpr (SIG_EARLY) {
 #pragma unroll
             for (int ib = 0; ib < NC; ++ib)
 #pragma unroll
                 for (int ia = 0; ia < NC; ++ia) sg[ia][ib] = sig[ia + ib * NC];
         }
+        kcache_fill(a.kdata + (size_t)k * bs);
         auto sig_at = [&](int ia, int ib) -> cd {
-            if constexpr (SIG_EARLY) return sg[ia][ib];
+            if constexpr (SIG_REG) return sg[ia][ib];
             else return sig[ia + ib * NC];
         };
         const BT* B = (const BT*)(a.kdata + (size_t)k * bs);
@@ -271,6 +310,13 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                         G[ib][ia] = cd{fma(gi, p.x, G[ib][ia].x), fma(gi, p.y, G[ib][ia].y)};
                     }
                 }
+        }
+        if constexpr (SIG_LDS) {
+#pragma unroll
+            for (int ib = 0; ib < NC; ++ib)
+#pragma unroll
+                for (int ia = 0; ia < NC; ++ia) sg[ia][ib] = sSig[(ia + ib * NC) * FW + lane];
+            __builtin_amdgcn_sched_barrier(0);  // issued together
         }
 #pragma unroll
         for (int ib = 0; ib < NC; ++ib)
@@ -354,11 +400,11 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                 if (wvalid && kin) trA = cadd(trA, t);
             }
         } else {
-            // the adjoint's cotangent, loaded all together here so that it arrives
-            // under the d loop below (it is k-invariant; keeping it across k would
-            // hold 4 NC^2 registers for the whole walk)
-            cd gbv[MODE == MODE_VJP ? NC : 1][MODE == MODE_VJP ? NC : 1];
-            if constexpr (MODE == MODE_VJP) {
+            // the adjoint's cotangent (KS > 1: in LDS), on its way during the d loop below
+            // (it is k-invariant; kept across k it would hold 4 NC^2 registers)
+            constexpr bool GB_REG = MODE == MODE_VJP && KS == 1;
+            cd gbv[GB_REG ? NC : 1][GB_REG ? NC : 1];
+            if constexpr (GB_REG) {
 #pragma unroll
                 for (int j = 0; j < NC; ++j)
 #pragma unroll
@@ -370,7 +416,7 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
             for (int i = 0; i < NC; ++i)
 #pragma unroll
                 for (int j = 0; j < NC; ++j) Y[i][j] = cd{0.0, 0.0};
-            cd sg = cd{0.0, 0.0}, sg2 = cd{0.0, 0.0}, sgM2 = cd{0.0, 0.0}, sgM3 = cd{0.0, 0.0};
+            cd trG = cd{0.0, 0.0}, tz = cd{0.0, 0.0};  // sum_d g + g^2 M_d, sum_d g^2 + 2 g^3 M_d
             // Y is accumulated as R + i J (R = sum Re(g^2) P_d, J = sum Im(g^2) P_d,
             // upper triangles in place: Y[a][b] = R_ab, Y[b][a] = J_ab), as S is
             // M_d = sum_ab conj(w_a) G_ab w_b = sum_ab G_ab P_{ba} with G folded
@@ -412,10 +458,8 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                             Md.y = fma(sm.x, p.x, fma(sm.y, p.y, Md.y));
                         }
                     }
-                sg = cadd(sg, g);
-                sg2 = cadd(sg2, g2);
-                sgM2 = cfma(g2, Md, sgM2);
-                sgM3 = cfma(cmul(g2, g), Md, sgM3);
+                trG = cfma(g2, Md, cadd(trG, g));
+                tz = cfma(cscale(cmul(g2, g), 2.0), Md, cadd(tz, g2));
             }
 #pragma unroll
             for (int ib = 0; ib < NC; ++ib)
@@ -433,13 +477,9 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                     Y[ia][ib] = cd{R.x - J.y, R.y + J.x};
                     Y[ib][ia] = cd{R.x + J.y, J.x - R.y};
                 }
-            cd trG = cadd(sg, sgM2);
 #pragma unroll
             for (int i = 0; i < NC; ++i) trG = cadd(trG, G[i][i]);
-            // Z = G S' = G + G Y.  DENS: in place of Y.  VJP: apart, as S' = I + Y
-            // is used again below.
-            cd Z[MODE == MODE_VJP ? NC : 1][MODE == MODE_VJP ? NC : 1];
-            auto Zr = [&](int i, int j) -> cd& { return MODE == MODE_VJP ? Z[i][j] : Y[i][j]; };
+            // Z = G S' = G + G Y, column by column in place of Y
 #pragma unroll
             for (int j = 0; j < NC; ++j) {
                 cd t[NC];
@@ -451,72 +491,106 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                     t[i] = s;
                 }
 #pragma unroll
-                for (int i = 0; i < NC; ++i) Zr(i, j) = t[i];
+                for (int i = 0; i < NC; ++i) Y[i][j] = t[i];
             }
+            cd(&Z)[NC][NC] = Y;
             // tr(Z^2) = sum_i Z_ii^2 + 2 sum_{i<j} Z_ij Z_ji
-            cd tzz = cd{0.0, 0.0};
             {
                 cd off = cd{0.0, 0.0};
 #pragma unroll
                 for (int i = 0; i < NC; ++i) {
-                    tzz = cfma(Zr(i, i), Zr(i, i), tzz);
+                    tz = cfma(Z[i][i], Z[i][i], tz);
 #pragma unroll
-                    for (int j = i + 1; j < NC; ++j) off = cfma(Zr(i, j), Zr(j, i), off);
+                    for (int j = i + 1; j < NC; ++j) off = cfma(Z[i][j], Z[j][i], off);
                 }
-                tzz = cadd(tzz, cscale(off, 2.0));
+                tz = cadd(tz, cscale(off, 2.0));
             }
-            const cd tz = cadd(cadd(sg2, cscale(sgM3, 2.0)), tzz);
-            if (wvalid) {
+            if (wvalid && kin) {
                 trA = cadd(trA, trG);
                 tr2A = cadd(tr2A, tz);
             }
-            if (MODE == MODE_VJP && vjp_here) {
-                // sigma_bar += G^H gbar G^H + cn ((G^2)_cc)^H with (G^2)_cc = G S' G:
-                // both terms are C = G^H V G^H, V = gbar + cn S'^H.
-                // mu term tr(gbar^H (G^2)_cc) = tr(S' G gbar^H G)
-                //   = sum_ab S'_ab conj(C_ab) - cn tr(Z^2)
-                // (G gbar^H G is (G^H gbar G^H)^H = (C - cn G^H S'^H G^H)^H, and
-                // tr(S' G S' G) = tr(Z^2)).
-                cd V[NC][NC];
+            if (MODE == MODE_VJP && tile_vjp) {
+                // sigma_bar += G^H gbar G^H + cn ((G^2)_cc)^H with (G^2)_cc = Z G: column b
+                // of both is G^H t, t_i = s_i + cn conj(Z_bi), s_i = sum_l gbar_il conj(G_bl).
+                // mu term tr(gbar^H (G^2)_cc) = tr(Z G gbar^H) = sum_bi Z_ib conj(s_i), as
+                // (G gbar^H)_bi = conj(s_i).  G and Z are all that lives here; with
+                // V = gbar + cn S'^H as a third matrix n_c = 6 spilled 0.6 KB per lane.
+                cd ms = cd{0.0, 0.0};
+                auto gbar_at = [&](int i, int l) -> cd {
+                    if constexpr (GB_REG) return gbv[i][l];
+                    else return sGb[(i + l * NC) * FW + lane];
+                };
+                auto barrier = [] {
+                    if constexpr (KS > 1) __builtin_amdgcn_sched_barrier(0);
+                };
+                auto column = [&](auto bc) {
+                    constexpr int b = decltype(bc)::value;
+                    // gbar (then the sums) come NC entries ahead, each entry's registers
+                    // loaded again as soon as it is used: left to itself the compiler
+                    // reads one entry, waits and uses it, an LDS round trip per entry
+                    cd buf[NC], t[NC];
 #pragma unroll
-                for (int j = 0; j < NC; ++j)
-#pragma unroll
-                    for (int i = 0; i < NC; ++i) {
-                        const cd gv = gbv[i][j];
-                        const double dg = i == j ? cn : 0.0;
-                        V[i][j] = cd{fma(cn, Y[j][i].x, gv.x + dg), fma(-cn, Y[j][i].y, gv.y)};
-                    }
-                cd ms = cscale(tzz, -cn);
-#pragma unroll
-                for (int b = 0; b < NC; ++b) {
-                    cd t[NC];  // column b of L = V G^H: t_i = sum_l V_il conj(G_bl)
+                    for (int l = 0; l < NC; ++l) buf[l] = gbar_at(0, l);
+                    barrier();
 #pragma unroll
                     for (int i = 0; i < NC; ++i) {
                         cd s = cd{0.0, 0.0};
 #pragma unroll
-                        for (int l = 0; l < NC; ++l) s = cfma(V[i][l], cconj(G[b][l]), s);
-                        t[i] = s;
+                        for (int l = 0; l < NC; ++l) {
+                            s = cfma(buf[l], cconj(G[b][l]), s);
+                            buf[l] = i + 1 < NC ? gbar_at(i + 1, l) : sAcc[(l + b * NC) * FW + lane];
+                            barrier();
+                        }
+                        ms = cfmac(s, Z[i][b], ms);
+                        t[i] = cd{fma(cn, Z[b][i].x, s.x), fma(-cn, Z[b][i].y, s.y)};
                     }
 #pragma unroll
                     for (int aa = 0; aa < NC; ++aa) {  // C_ab = sum_i conj(G_ia) t_i
-                        cd s = cd{0.0, 0.0};
+                        cd s = buf[aa];
 #pragma unroll
                         for (int i = 0; i < NC; ++i) s = cfmac(G[i][aa], t[i], s);
-                        lds_add(&sAcc[(aa + b * NC) * FW + lane], s);
-                        const cd sp = aa == b ? cadd(Y[aa][b], cd{1.0, 0.0}) : Y[aa][b];
-                        ms = cfmac(s, sp, ms);  // S'_ab conj(C_ab)
+                        sAcc[(aa + b * NC) * FW + lane] = s;
+                    }
+                };
+                if constexpr (KS == 1) {
+                    for_columns<NC>(column);
+                } else {
+                    // part p takes column p + step (mod the number of steps): at each step the
+                    // parts add to different columns, and every sum has one order
+                    constexpr int STEPS = NC > KS ? NC : KS;
+                    int b = part;
+#pragma unroll 1
+                    for (int st = 0; st < STEPS; ++st) {
+                        if (kin) pick_column<NC>(b, column);
+                        b = b + 1 == STEPS ? 0 : b + 1;
+                        __syncthreads();
                     }
                 }
-                muA = cadd(muA, ms);
+                if (vjp_here) muA = cadd(muA, ms);
             }
         }
     }
 
     if constexpr (KS > 1) {  // the parts' tr G shares and G_cc sums meet in LDS; part 0 writes them
-        lds_add(&sTr[lane], trA);
-        __syncthreads();
-        if (part != 0) return;
-        trA = sTr[lane];
+        if constexpr (FWDLIKE) {
+            lds_add(&sTr[lane], trA);
+            __syncthreads();
+            if (part != 0) return;
+            trA = sTr[lane];
+        } else {  // (gbar is not needed any more)
+            __syncthreads();
+            cd* share = sGb + lane;
+            share[(3 * part) * FW] = trA;
+            share[(3 * part + 1) * FW] = tr2A;
+            share[(3 * part + 2) * FW] = muA;
+            __syncthreads();
+            if (part == 0)
+                for (int p = 1; p < KS; ++p) {
+                    trA = cadd(trA, share[(3 * p) * FW]);
+                    tr2A = cadd(tr2A, share[(3 * p + 1) * FW]);
+                    muA = cadd(muA, share[(3 * p + 2) * FW]);
+                }
+        }
     }
     if (!wvalid) return;
     const size_t ch = chunk;
@@ -532,12 +606,13 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                     a.pG[(ch * a.nw_tot + nw) * M2 + i + j * NC] = acc[i][j];
         }
     } else {
-        a.pTr[ch * a.nw_tot + nw] = trA;
-        a.pTr2[ch * a.nw_tot + nw] = tr2A;
-        if (MODE == MODE_VJP && vjp_here) {
-            a.pMu[ch * a.n_freq + nw] = muA;
-            for (int e = 0; e < M2; ++e) a.pSb[(ch * a.n_freq + nw) * M2 + e] = sAcc[e * FW + lane];
+        if (part == 0) {
+            a.pTr[ch * a.nw_tot + nw] = trA;
+            a.pTr2[ch * a.nw_tot + nw] = tr2A;
+            if (MODE == MODE_VJP && vjp_here) a.pMu[ch * a.n_freq + nw] = muA;
         }
+        if (MODE == MODE_VJP && vjp_here)
+            for (int e = part; e < M2; e += KS) a.pSb[(ch * a.n_freq + nw) * M2 + e] = sAcc[e * FW + lane];
     }
 }
 
@@ -547,7 +622,7 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
 template <int NC, int MODE, int KS>
 constexpr int schur_waves()
 {
-    if (MODE == MODE_VJP) return 1;
+    if (MODE == MODE_VJP) return NC == 4 || (NC == 5 && KS > 1) ? 2 : 1;
     if (KS > 1) return NC <= 4 ? 4 : NC == 5 ? 3 : 2;
     return NC == 5 ? 2 : 1;
 }
@@ -582,8 +657,11 @@ template <int NC, int MODE, int WG, int KS = 1>
 constexpr size_t schur_shm()
 {
     constexpr bool ACC_LDS = MODE == MODE_VJP || KS > 1;
-    // KS > 1: one accumulator set per frequency, plus the tr G sums
-    return ACC_LDS ? sizeof(cd) * (size_t)(NC * NC + (KS > 1 ? 1 : 0)) * (WG / KS) : 0;
+    // KS > 1: one accumulator set per frequency, plus the tr G sums (forward) or gbar
+    // and Sigma, at the end the parts' three shares (adjoint)
+    constexpr int tables = (schur_sig_lds<NC>() ? 2 : 1) * NC * NC;
+    constexpr int extra = KS == 1 ? 0 : MODE != MODE_VJP ? 1 : tables > 3 * KS ? tables : 3 * KS;
+    return ACC_LDS ? sizeof(cd) * (size_t)(NC * NC + extra) * (WG / KS) : 0;
 }
 
 template <int NC, int MODE, bool TRACE, int WG, int KS = 1>
@@ -611,7 +689,11 @@ template <int NC, int MODE, bool TRACE>
 hipError_t launch_nc(const LatArgs& a, const cd* sig_all, hipStream_t s, int wg, const SchurMulti* m)
 {
     if constexpr (NC >= 3 && (MODE == MODE_FWD || MODE == MODE_FWD_REAL)) {  // two wavefronts over 64 frequencies
-        if (wg == SCHUR_WG_KPAIR) return launch_nc_w<NC, MODE, TRACE, 128, 2>(a, sig_all, s, m);
+        if (wg == SCHUR_WG_KSPLIT) return launch_nc_w<NC, MODE, TRACE, 128, 2>(a, sig_all, s, m);
+    }
+    if constexpr (NC >= 4 && MODE == MODE_VJP) {  // four, or at n_c = 6 two
+        constexpr int KS = NC == 6 ? 2 : 4;
+        if (wg == SCHUR_WG_KSPLIT) return launch_nc_w<NC, MODE, TRACE, 64 * KS, KS>(a, sig_all, s, m);
     }
     if (wg == 128) return launch_nc_w<NC, MODE, TRACE, 128>(a, sig_all, s, m);
     return launch_nc_w<NC, MODE, TRACE, 64>(a, sig_all, s, m);

@@ -84,9 +84,8 @@ const char* dmftgpu_version(void);
                                            32768 for the one-matrix-per-lane Schur kernels, keeping >= 64 k per
                                            chunk and >= 8192 items; 8192 for the others) */
 #define DMFTGPU_OPT_SCHUR_WG 3          /* frequencies per workgroup of the Schur kernels (64 or 128; default 0 =
-                                           64, or, for the forward at n_corr = 6 and at n_corr 3..5 with six or
-                                           more uncorrelated orbitals, two wavefronts over 64 frequencies
-                                           splitting the k walk) */
+                                           64, or two or four wavefronts over 64 frequencies splitting the k
+                                           walk where that is faster) */
 #define DMFTGPU_OPT_SCHUR_LAYOUT 4      /* n_c <= 6: 0 = one (k,iw) matrix per lane (default), 1 = one column
                                            per lane (always used for n_c > 6) */
 #define DMFTGPU_OPT_UPFOLD_CHUNK 5      /* k points per chunk of dmftgpu_upfold_density (0 = as many as 512 MiB of
@@ -272,8 +271,8 @@ int dmftgpu_batch_create(dmftgpu_handle h, int count, const dmftgpu_system* syst
                          dmftgpu_batch* out);
 int dmftgpu_batch_run(dmftgpu_batch b);
 /* Tuning result of n_corr group `group` (returns the number of groups when out of range):
- * wg[2], target[2], ms[2] per mode (forward, adjoint); wg = 1 is the forward's k-pair form
- * (two wavefronts over 64 frequencies, each taking every other k of a chunk). */
+ * wg[2], target[2], ms[2] per mode (forward, adjoint); wg = 1 is the form that splits the
+ * k walk (two or four wavefronts over 64 frequencies). */
 int dmftgpu_batch_tuning(dmftgpu_batch b, int group, int* nc, int* systems, int* wg, double* target, double* ms);
 int dmftgpu_batch_destroy(dmftgpu_batch b);
 
