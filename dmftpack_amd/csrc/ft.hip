@@ -148,61 +148,101 @@ __global__ void k_mom_kinv(int range, int green, double* __restrict__ kinv)
 // design matrix contributes sum_b Kinv[a][b] Re_b and the Im row
 // sum_b Kinv[a][b] Im_b (the rows' zero entries left out), each taken times
 // its half of g and added, Re row first, in ascending frequency order.
-// One thread per (moment, window, element): the sum is a serial chain, so the time is
-// that of the longest window, and the loads of kFitAhead frequencies are issued together
-// ahead of their use.  With one thread per (window, element) and loads at their use, d = 5
-// and N_freq = 1000 took 275 us (660 cycles a frequency, most of it load latency); this
-// form 220 us (bound by its L1 loads).
+// One thread per (moment, window, element pair al <= be): the transposed element's row
+// values are the conjugates, term by term, so its sum is the conjugate and is written with
+// it.  The sum is a serial chain, so the time is that of the longest window.  A wavefront's
+// frequencies are uniform (its windows are neighbours; each waits for its own start), so
+// the basis values come as scalar operands and a frequency costs two vector loads, those of
+// kFitAhead frequencies issued ahead of their use.  With the basis loaded by each lane and
+// an element a thread, d = 5 and N_freq = 1000 took 220 us, bound by the L1 loads; this
+// form 75 us.
 constexpr int kFitAhead = 8;
 
 template <bool GREEN>
-__global__ __launch_bounds__(256) void k_mom_fit(const cd* __restrict__ fw, int d, int n_freq, int range,
-                                                 const double4* __restrict__ tab, const double* __restrict__ kinv,
-                                                 cd* __restrict__ mt)
+__global__ __launch_bounds__(64) void k_mom_fit(const cd* __restrict__ fw, int d, int n_freq, int range,
+                                                const double* __restrict__ tab_, const double* __restrict__ kinv,
+                                                cd* __restrict__ mt)
 {
 #pragma clang fp contract(off)
-    const int m2 = d * d, a = blockIdx.y;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (size_t)range * m2) return;
-    const int w = (int)(t / m2), e = (int)(t % m2);
-    const int al = e % d, be = e / d;
+    const int m2 = d * d, np = d * (d + 1) / 2, a = blockIdx.y;
+    const kconst_double* tab = (const kconst_double*)tab_;
+    const unsigned first = blockIdx.x * 64, last = min(first + 63, (unsigned)(range * np - 1));
+    const unsigned t = min(first + threadIdx.x, last);  // spare lanes repeat the last entry
+    const int w = (int)(t / np), q = (int)(t % np);
+    int be = 0, al = q;
+    while (al > be) al -= ++be;  // pair q -> (al, be), al <= be
     const double* X = kinv + (size_t)w * 16 + a;  // Kinv(a, b) at X[4 b]
     const double x0 = X[0], x1 = X[4], x2 = GREEN ? 0.0 : X[8], x3 = GREEN ? 0.0 : X[12];
-    const cd* fa = fw + al + (size_t)be * d;
-    const cd* fb = fw + be + (size_t)al * d;
-    cd s = cd{0, 0};
-    auto add = [&](double4 c, cd fab, cd fba) {
-        // Re = (F_ab + conj(F_ba))/2 ; Im = (F_ab - conj(F_ba))/(2i)
-        const cd re = cd{0.5 * (fab.x + fba.x), 0.5 * (fab.y - fba.y)};
-        cd im = cd{0.5 * (fab.y + fba.y), -0.5 * (fab.x - fba.x)};
+    // element addresses: the frequency's uniform base and the lane's offset
+    const unsigned oa = (al + be * d) * sizeof(cd), ob = (be + al * d) * sizeof(cd);
+    auto at = [&](int wn, unsigned o) -> cd { return *(const cd*)((const char*)(fw + (size_t)wn * m2) + o); };
+    cd s = cd{0, 0};  // twice the sum: the halves of Re and Im are taken at the end (exactly)
+    // basis values {-1/z, -1/z^2, 1/z^3, 1/z} of a frequency at c
+    auto add = [&](double c0, double c1, double c2, double c3, cd fab, cd fba) {
+        // 2 Re = F_ab + conj(F_ba) ; 2 Im = (F_ab - conj(F_ba))/i
+        const cd re = cd{fab.x + fba.x, fab.y - fba.y};
+        cd im = cd{fab.y + fba.y, fba.x - fab.x};
         double kr, ki;
         if (!GREEN) {
             // Re row [1, 0, -1/z^2, 0], Im row [0, -1/z, 0, 1/z^3]   (:227-230)
-            kr = fma(x2, c.y, x0);
-            ki = fma(x3, c.z, x1 * c.x);
+            kr = fma(x2, c1, x0);
+            ki = fma(x3, c2, x1 * c0);
         } else {
             // Re row [-1/z^2, 0], Im row [0, 1/z^3]   (:366-367)
-            if (al == be) im.x += c.w;  // (:373)
-            kr = x0 * c.y;
-            ki = x1 * c.z;
+            if (al == be) im.x += 2.0 * c3;  // (:373)
+            kr = x0 * c1;
+            ki = x1 * c2;
         }
         s = cadd(s, cd{fma(ki, im.x, kr * re.x), fma(ki, im.y, kr * re.y)});
     };
-    int wn = w;
-    for (; wn + kFitAhead <= n_freq; wn += kFitAhead) {
-        double4 c[kFitAhead];
-        cd p[kFitAhead], q[kFitAhead];
+    auto add1 = [&](int wn) {
+        const kconst_double* c = tab + 4 * wn;
+        add(c[0], c[1], c[2], c[3], at(wn, oa), at(wn, ob));
+    };
+    int wn = (int)(first / np);       // the first window of the wavefront
+    const int w1 = (int)(last / np);  // and its last
+    for (; wn < w1; ++wn)
+        if (wn >= w) add1(wn);
+    if (wn + kFitAhead <= n_freq) {
+        // the next kFitAhead frequencies' loads are under way while these are added, and
+        // the scalar loads of a group are waited for together
+        cd p[2][kFitAhead], r[2][kFitAhead];
+        auto load = [&](int h, int w0) {
 #pragma unroll
-        for (int u = 0; u < kFitAhead; ++u) {
-            c[u] = tab[wn + u];
-            p[u] = fa[(size_t)(wn + u) * m2];
-            q[u] = fb[(size_t)(wn + u) * m2];
+            for (int u = 0; u < kFitAhead; ++u) {
+                const int f = min(w0 + u, n_freq - 1);
+                p[h][u] = at(f, oa);
+                r[h][u] = at(f, ob);
+            }
+        };
+        auto sum = [&](int h, int w0) {
+            double c[kFitAhead][4];
+#pragma unroll
+            for (int u = 0; u < kFitAhead; ++u)
+#pragma unroll
+                for (int x = GREEN ? 1 : 0; x < (GREEN ? 4 : 3); ++x) c[u][x] = tab[4 * (w0 + u) + x];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < kFitAhead; ++u) add(c[u][0], c[u][1], c[u][2], c[u][3], p[h][u], r[h][u]);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        load(0, wn);
+        for (; wn + 2 * kFitAhead <= n_freq; wn += 2 * kFitAhead) {
+            load(1, wn + kFitAhead);
+            sum(0, wn);
+            load(0, wn + 2 * kFitAhead);
+            sum(1, wn + kFitAhead);
         }
-#pragma unroll
-        for (int u = 0; u < kFitAhead; ++u) add(c[u], p[u], q[u]);
+        if (wn + kFitAhead <= n_freq) {
+            sum(0, wn);
+            wn += kFitAhead;
+        }
     }
-    for (; wn < n_freq; ++wn) add(tab[wn], fa[(size_t)wn * m2], fb[(size_t)wn * m2]);
-    mt[((size_t)a * range + w) * m2 + e] = s;
+    for (; wn < n_freq; ++wn) add1(wn);
+    s = cd{0.5 * s.x, 0.5 * s.y};
+    cd* out = mt + ((size_t)a * range + w) * m2;
+    out[be + al * d] = cconj(s);
+    out[al + be * d] = s;
 }
 
 // trace[a][w] = sum_alpha Re mt[a][w][alpha alpha]     (:244-247)
@@ -889,10 +929,11 @@ extern "C" int dmftgpu_moments(dmftgpu_handle h, int d, int n_freq, double beta,
         ent->beta = beta;
         ent->green = green_asym;
     }
-    const dim3 gfit(nblk((size_t)range * m2), nm);
+    const dim3 gfit((unsigned)(((size_t)range * (d * (d + 1) / 2) + 63) / 64), nm);
+    const double* dtab = (const double*)tab;
     if (green_asym)
-        hipLaunchKernelGGL((k_mom_fit<true>), gfit, dim3(256), 0, s, (const cd*)fw, d, n_freq, range, tab, kinv, mt);
-    else hipLaunchKernelGGL((k_mom_fit<false>), gfit, dim3(256), 0, s, (const cd*)fw, d, n_freq, range, tab, kinv, mt);
+        hipLaunchKernelGGL((k_mom_fit<true>), gfit, dim3(64), 0, s, (const cd*)fw, d, n_freq, range, dtab, kinv, mt);
+    else hipLaunchKernelGGL((k_mom_fit<false>), gfit, dim3(64), 0, s, (const cd*)fw, d, n_freq, range, dtab, kinv, mt);
     HIPCHK(hipGetLastError());
     hipLaunchKernelGGL(k_mom_trace, dim3(nblk((size_t)range * nm)), dim3(256), 0, s, mt, d, range, nm, trace);
     HIPCHK(hipGetLastError());
