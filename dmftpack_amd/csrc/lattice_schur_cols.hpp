@@ -37,9 +37,7 @@ namespace dg {
 // Smallest n_c the bucket of width N serves (lattice_schur.hip, cols_bucket):
 // rows i below it are inside every served block, so in the d loops the tests
 // i < n_c on them fold away at compile time and the W loads issue
-// unconditionally (a load under a uniform branch waits on its own).  The
-// adjoint's LDS products keep their tests: unconditional, their reads would
-// all be hoisted and spill.
+// unconditionally (a load under a uniform branch waits on its own).
 __host__ __device__ constexpr int cols_nc_min(int N)
 {
     return N <= 4 ? 1 : N <= 6 ? N : N == 8 ? 7 : N == 10 ? 9 : N == 12 ? 11 : 13;
@@ -49,21 +47,25 @@ __host__ __device__ constexpr int cols_nc_min(int N)
 // wavefronts share nothing but the cache
 __host__ __device__ constexpr int cols_wg() { return 64; }
 
-// per-slot LDS (cd units): gsh 32 - nc_min (g_d), and the elimination's broadcast buffer
-// (2 N) in the forward; MA N*N and MB N*N otherwise, the buffer then lying in MA.
+// per-slot LDS (cd units): gsh 32 - nc_min (g_d; in the forward then the elimination's
+// broadcast buffer, 2 N), MA N*N and, but for the forward, MB N*N.
 // Sigma and gbar are read from the cache at each k and the spare lanes repeat lanes of
 // the last slot instead of writing to a slot of their own: the LDS is what decides how
 // many wavefronts of the adjoint a CU holds (N = 10: 39.5 KB each with tables of their
-// own for all of these, 4 to a CU; 21.4 KB, 7 to a CU.  With cols_waves below, FP64
-// adjoint of n = 32, n_c = 10, 1728 k x 528 points: 4.85 -> 3.28 ms, n_c = 16: 21.8 ->
-// 12.3 ms; forward 1.81 -> 1.51 ms and 6.0 -> 3.7 ms).
+// own for all of these, 4 to a CU; 21.4 KB, 7 to a CU.  With cols_waves below, adjoint
+// of n = 32, n_c = 10, 1728 k x 528 points: 4.85 -> 3.28 ms, n_c = 16: 21.8 -> 12.3 ms;
+// forward 1.81 -> 1.51 ms and 6.0 -> 3.7 ms).
 // The size is odd (in 16-byte entries): the slots of a wavefront read the same entry of
 // their own matrices at once, and with a multiple of 16 entries (the adjoint at N = 10 or
 // 16, every form at N = 8) all of those fell into the same four banks.
-__host__ __device__ constexpr int cols_slot_size(int N, int mode)
+__host__ __device__ constexpr int cols_g_size(int N, int mode)
 {
     const int g = 32 - cols_nc_min(N);  // n_d at most
-    return (g + (mode == MODE_FWD ? 2 * N : 2 * N * N)) | 1;
+    return mode == MODE_FWD && g < 2 * N ? 2 * N : g;
+}
+__host__ __device__ constexpr int cols_slot_size(int N, int mode)
+{
+    return (cols_g_size(N, mode) + (mode == MODE_FWD ? N * N : 2 * N * N)) | 1;
 }
 
 __host__ __device__ constexpr int cols_slots(int N) { return 64 / N; }
@@ -82,6 +84,38 @@ __host__ __device__ constexpr int cols_waves(int N, int mode)
 }
 
 __device__ __forceinline__ cd ld_off(const cd* base, unsigned bytes) { return *(const cd*)((const char*)base + bytes); }
+
+// out_i += sum_l M_il x_l (ADJ: M^H), M column-major in LDS.  M's entries are read a
+// column (row) ahead of their use, four at a time, each into the registers of an entry
+// just used: left to itself the compiler reads a column, waits for it and uses it
+// (adjoint of n = 32, n_c = 10, 1728 k x 528 points: 3.32 against 2.49 ms; n_c = 16 12.3
+// against 8.5; a barrier after every entry instead of every four cost 0.5 ms, the four
+// FMAs of an entry being a chain).
+// Padding needs no test: entries of M there are finite and meet a zero.
+template <int N, bool ADJ, class X>
+__device__ __forceinline__ void lds_product(const cd* M, cd (&out)[N], X&& x)
+{
+    auto at = [M](int i, int l) -> cd { return ADJ ? M[l + i * N] : M[i + l * N]; };
+    cd buf[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) buf[i] = at(i, 0);
+    cd xn = x(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int l = 0; l < N; ++l) {
+        const cd xl = xn;
+        if (l + 1 < N) xn = x(l + 1);
+#pragma unroll
+        for (int i0 = 0; i0 < N; i0 += 4) {
+#pragma unroll
+            for (int i = i0; i < N && i < i0 + 4; ++i) {
+                out[i] = ADJ ? cfmac(buf[i], xl, out[i]) : cfma(buf[i], xl, out[i]);
+                if (l + 1 < N) buf[i] = at(i, l + 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
 
 // One (frequency tile, k chunk) work item of one lattice: the body of the
 // per-lattice kernel and of the persistent multi-lattice kernel below.
@@ -104,9 +138,12 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
     const int cc = c0 < nc ? c0 : 0;  // clamped column index for loads
     cd* my = lds + (size_t)sl * SS;
     cd* gsh = my;
-    cd* MA = gsh + 32 - NMIN;
+    cd* MA = gsh + cols_g_size(N, MODE);
     cd* MB = MA + N * N;
-    cd* bc = MA;  // the elimination's buffer, before MA is written
+    // the elimination's buffer: over g_d, which the forward needs no more by then, or in
+    // MA, not yet written; the row values kept across the inversion
+    cd* bc = MODE == MODE_FWD ? gsh : MA;
+    cd* park = MODE == MODE_FWD ? MA : MB;
     const int npts = n_points(a);
     if (wtile * SLOTS >= npts) return;  // tile past the last frequency point
     const int nw = wtile * SLOTS + sl;
@@ -164,10 +201,14 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
             asm volatile("" ::"v"(pf));
         }
         // g_d = 1/(iw + mu - e_d) of this slot's frequency, shared by its lanes
+        cd tg = cd{0.0, 0.0}, t2 = cd{0.0, 0.0};  // lane shares of tr G and tr G^2
         for (int d = c; d < nd; d += N) {
             const double x = mu - ed[d];
             const double r = rcp_pos(fma(x, x, w * w));
-            gsh[d] = cd{x * r, -w * r};
+            const cd g = cd{x * r, -w * r};
+            gsh[d] = g;
+            tg = cadd(tg, g);
+            if constexpr (MODE != MODE_FWD) t2 = cfma(g, g, t2);
         }
         wave_sync();
 
@@ -194,6 +235,16 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
                 col[i] = live ? (inb(i) ? csub(col[i], t[i]) : cd{0.0, 0.0})
                               : ((i == c) ? cd{1.0, 0.0} : cd{0.0, 0.0});
         }
+        // row c of sum_d g_d^p w_d w_d^H, p = 2 (forward) or 3: with column c of G_cc it
+        // gives the trace's sum_d g_d^p M_d as sum_i G_ic Y_ci, in this same walk over W
+        // (a walk of its own after the inversion, one dot product per d, took 1.51 ms
+        // against 1.29, forward of n = 32, n_c = 10, 1728 k x 528 points)
+        constexpr bool ROW = MODE != MODE_FWD || TRACE;
+        cd yr[ROW ? N : 1];
+        if constexpr (ROW) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) yr[i] = cd{0.0, 0.0};
+        }
         if constexpr (MODE != MODE_FWD) {
 #pragma unroll
             for (int i = 0; i < N; ++i) y[i] = cd{0.0, 0.0};
@@ -201,82 +252,72 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
         for (int d = 0; d < nd; ++d) {
             const cd g = gsh[d];
             const kconst_cd* Wd = Wk + d * nc;
-            const cd u = live ? cmulc(g, ldc(Wd + cc)) : cd{0.0, 0.0};  // g_d conj(W_cd)
+            const cd wc = live ? ldc(Wd + cc) : cd{0.0, 0.0};
+            const cd u = cmulc(g, wc);  // g_d conj(W_cd)
+            const cd g2 = cmul(g, g);
+            const cd ur = cmul(MODE == MODE_FWD ? g2 : cmul(g2, g), wc);
+            const cd u2 = cmul(g, u);
 #pragma unroll
             for (int i = 0; i < N; ++i)
-                if (inb(i)) col[i] = cfms(ldc(Wd + i), u, col[i]);
-            if constexpr (MODE != MODE_FWD) {
-                const cd u2 = cmul(g, u);
+                if (inb(i)) {
+                    const cd wi = ldc(Wd + i);
+                    col[i] = cfms(wi, u, col[i]);
+                    if constexpr (MODE != MODE_FWD) y[i] = cfma(wi, u2, y[i]);
+                    if constexpr (ROW) yr[i] = cfmac(wi, ur, yr[i]);
+                }
+        }
+        if constexpr (ROW) {  // kept in LDS during the inversion, each lane its own entries
 #pragma unroll
-                for (int i = 0; i < N; ++i)
-                    if (inb(i)) y[i] = cfma(ldc(Wd + i), u2, y[i]);
-            }
+            for (int i = 0; i < N; ++i)
+                if (nd > 0) park[c + i * N] = yr[i];
         }
 
         // ---- G_cc = S^{-1}, column c
         gj_columns<N>(col, bc, c, nc);
+        if constexpr (ROW) __builtin_amdgcn_sched_barrier(0);
         cd gdiag = cd{0.0, 0.0};  // G_cc(c, c)
 #pragma unroll
         for (int i = 0; i < N; ++i)
             if (i == c) gdiag = col[i];
 
+        cd tm = cd{0.0, 0.0};  // lane share of sum_d g_d^p M_d
+        if constexpr (ROW) {
+            if (nd > 0) {
+#pragma unroll
+                for (int i = 0; i < N; ++i) tm = cfma(col[i], park[c + i * N], tm);
+            }
+            // (each stretch between these holds one more column-sized value than fits twice)
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if constexpr (MODE == MODE_FWD) {
 #pragma unroll
             for (int i = 0; i < N; ++i) acc[i] = cadd(acc[i], col[i]);
             if constexpr (TRACE) {
-                // lane share of tr G: G_cc + sum_d g_d^2 W_cd (sum_i conj(W_id) G_ic)
-                cd t = live ? gdiag : cd{0.0, 0.0};
-                for (int d = 0; d < nd; ++d) {
-                    const cd g = gsh[d];
-                    const kconst_cd* Wd = Wk + d * nc;
-                    cd v = cd{0.0, 0.0};
-#pragma unroll
-                    for (int i = 0; i < N; ++i)
-                        if (inb(i)) v = cfmac(ldc(Wd + i), col[i], v);
-                    const cd m = live ? cmul(ldc(Wd + cc), v) : cd{0.0, 0.0};
-                    t = cfma(cmul(g, g), m, t);
-                    if (c == 0) t = cadd(t, g);
-                }
-                if (wvalid) trA = cadd(trA, t);
+                if (live) tg = cadd(tg, cadd(gdiag, tm));
+                if (wvalid) trA = cadd(trA, tg);
             }
         } else {
 #pragma unroll
             for (int i = 0; i < N; ++i) MA[i + c * N] = col[i];
             wave_sync();
-            // trace shares: tr G and tr G^2 = sum g^2 + tr(Z^2) + 2 sum g^3 M_d
-            cd tg = live ? gdiag : cd{0.0, 0.0};
-            cd t2 = cd{0.0, 0.0};
-            for (int d = 0; d < nd; ++d) {
-                const cd g = gsh[d];
-                const cd g2 = cmul(g, g);
-                const kconst_cd* Wd = Wk + d * nc;
-                cd v = cd{0.0, 0.0};
+            // Z = G (I + Y), column c, over column c of G
+            cd(&z)[N] = col;
+            lds_product<N, false>(MA, z, [&](int l) { return y[l]; });
+            // tr G = sum g + tr G_cc + tr(G Y) = sum g + tr Z,
+            // tr G^2 = sum g^2 + tr(Z^2) + 2 sum g^3 M_d
+            cd zdiag = cd{0.0, 0.0};
 #pragma unroll
-                for (int i = 0; i < N; ++i)
-                    if (inb(i)) v = cfmac(ldc(Wd + i), col[i], v);
-                const cd m = live ? cmul(ldc(Wd + cc), v) : cd{0.0, 0.0};
-                tg = cfma(g2, m, tg);
-                t2 = cfma(cscale(cmul(g2, g), 2.0), m, t2);
-                if (c == 0) {
-                    tg = cadd(tg, g);
-                    t2 = cadd(t2, g2);
-                }
+            for (int i = 0; i < N; ++i)
+                if (i == c) zdiag = z[i];
+            if (live) {
+                tg = cadd(tg, zdiag);
+                t2 = cadd(t2, cscale(tm, 2.0));
             }
-            // row c of gbar, on its way during the product
+            // row c of gbar, on its way during tr(Z^2); earlier, it would not fit beside the product
             cd gv[MODE == MODE_VJP ? N : 1];
             if constexpr (MODE == MODE_VJP) {
 #pragma unroll
                 for (int j = 0; j < N; ++j) gv[j] = ld_off(gb + (inb(j) ? j : 0) * ncs, gb_off);
-            }
-            // Z = G (I + Y), column c, over column c of G
-            cd(&z)[N] = col;
-#pragma unroll
-            for (int l = 0; l < N; ++l) {
-                if (l < nc) {
-                    const cd yl = y[l];
-#pragma unroll
-                    for (int i = 0; i < N; ++i) z[i] = cfma(MA[i + l * N], yl, z[i]);
-                }
             }
 #pragma unroll
             for (int i = 0; i < N; ++i) MB[i + c * N] = z[i];
@@ -309,28 +350,13 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
                     cd l[N];  // column c of L = V G^H: l_i = sum_j V_ij conj(G_cj)
 #pragma unroll
                     for (int i = 0; i < N; ++i) l[i] = cd{0.0, 0.0};
-#pragma unroll
-                    for (int j = 0; j < N; ++j) {
-                        if (j < nc) {
-                            const cd gc = cconj(MA[c + j * N]);
-#pragma unroll
-                            for (int i = 0; i < N; ++i)
-                                if (i < nc) l[i] = cfma(MB[i + j * N], gc, l[i]);
-                        }
-                    }
+                    lds_product<N, false>(MB, l, [&](int j) { return cconj(MA[c + j * N]); });
+                    // sum_a S'_ac conj(C_ac) = sum_i Z_ic conj(l_i), as G S' = Z
                     cd ms = cscale(zz, -cn);
 #pragma unroll
-                    for (int aa = 0; aa < N; ++aa) {
-                        if (aa < nc) {  // C_ac = sum_i conj(G_ia) l_i
-                            cd s = cd{0.0, 0.0};
-#pragma unroll
-                            for (int i = 0; i < N; ++i)
-                                if (i < nc) s = cfmac(MA[i + aa * N], l[i], s);
-                            acc[aa] = cadd(acc[aa], s);
-                            const cd sp = aa == c ? cadd(y[aa], cd{1.0, 0.0}) : y[aa];  // S'_ac
-                            ms = cfmac(s, sp, ms);
-                        }
-                    }
+                    for (int i = 0; i < N; ++i) ms = cfmac(l[i], z[i], ms);
+                    // C_ac = sum_i conj(G_ia) l_i
+                    lds_product<N, true>(MA, acc, [&](int i) { return l[i]; });
                     muA = cadd(muA, ms);
                 }
             }
