@@ -388,15 +388,15 @@ Plan make_plan(int nk, int nw_tot, int slots, int target_wg)
     return Plan{chunks, kpc};
 }
 
-// Static weights and their per-k reduction: fills st_out[m2] (complex) and
-// st_scalars[2] = {sum w, sum dN terms} (device), all unnormalised.  With
+// Static weights and their per-k reduction: *st_out [m2] (complex) and
+// *st_scalars [2] = {sum w, sum dN terms} (device), all unnormalised.  With
 // Kohn-Sham bands bound by dmftgpu_set_core_bands the scalars include the
 // core-band term of GiwToNele (GreenFtn.cpp:622-631) and its mu-derivative.
 // The result depends only on (mu, prepared lattice, core bands) and is kept
 // per handle, in the handle's workspaces; with from_ws every buffer is carved
 // from ws instead and nothing is kept.  wt_out (optional) receives the
 // per-level weights w_kl [nk][n].
-int run_static(dmftgpu_handle h, double mu, cd* st_out, double* st_scalars, char* ws, size_t& off,
+int run_static(dmftgpu_handle h, double mu, const cd** st_out, const double** st_scalars, char* ws, size_t& off,
                bool from_ws = false, const double** wt_out = nullptr, size_t cap = SIZE_MAX)
 {
     const dmftgpu_lattice& L = h->lat;
@@ -435,16 +435,19 @@ int run_static(dmftgpu_handle h, double mu, cd* st_out, double* st_scalars, char
         if (cchunks)
             HIPCHK(dg::launch_core_bands(h->core_eps, h->core_out, h->core_n_orb, nk, kpc, cchunks, L.beta, mu,
                                          pN + chunks, pdN + chunks, h->stream));
-        HIPCHK(dg::launch_reduce_chunks(pNum, chunks, m2, (cd*)cache, h->stream));
-        HIPCHK(dg::launch_reduce_chunks_d(pN, tot, 1, (double*)(cache + (size_t)m2 * sizeof(cd)), h->stream));
-        HIPCHK(dg::launch_reduce_chunks_d(pdN, tot, 1, (double*)(cache + (size_t)m2 * sizeof(cd)) + 1, h->stream));
+        dg::ReduceSet r;
+        double* scal = (double*)(cache + (size_t)m2 * sizeof(cd));
+        r.add(pNum, chunks, m2, (cd*)cache);
+        r.add(pN, tot, 1, scal);
+        r.add(pdN, tot, 1, scal + 1);
+        HIPCHK(dg::launch_reduce_set(r, h->stream));
         if (!from_ws) {
             h->static_gen = h->prep_gen;
             h->static_mu = mu;
         }
     }
-    HIPCHK(hipMemcpyAsync(st_out, cache, sizeof(cd) * m2, hipMemcpyDeviceToDevice, h->stream));
-    HIPCHK(hipMemcpyAsync(st_scalars, cache + (size_t)m2 * sizeof(cd), 2 * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
+    *st_out = (const cd*)cache;
+    *st_scalars = (const double*)(cache + (size_t)m2 * sizeof(cd));
     return DMFTGPU_OK;
 }
 
@@ -597,16 +600,16 @@ int run_lattice(dmftgpu_handle h, int method, int mode, const double* sigma, dou
     if (pk) return DMFTGPU_OK;
     S.pt_n = a.pt_n;
     S.pt_wt = a.pt_wt;
-    HIPCHK(dg::launch_reduce_chunks(a.pTr, P.n_chunks, nw_tot, S.tr, h->stream, a.pt_n));
-    if (mode == dg::MODE_FWD) {
-        HIPCHK(dg::launch_reduce_chunks(a.pG, P.n_chunks, (size_t)nw_tot * m2, S.Gsum, h->stream, a.pt_n, m2));
-    } else {
-        HIPCHK(dg::launch_reduce_chunks(a.pTr2, P.n_chunks, nw_tot, S.tr2, h->stream, a.pt_n));
-    }
+    dg::ReduceSet r;
+    const int C1 = P.n_chunks;
+    if (mode != dg::MODE_VJP) r.add(a.pTr, C1, nw_tot, S.tr, 1);
+    if (mode == dg::MODE_FWD) r.add(a.pG, C1, (size_t)nw_tot * m2, S.Gsum, m2);
+    else r.add(a.pTr2, C1, nw_tot, S.tr2, 1);
     if (mode == dg::MODE_VJP) {
-        HIPCHK(dg::launch_reduce_chunks(a.pSb, P.n_chunks, (size_t)n_freq * m2, S.Sb, h->stream));
-        HIPCHK(dg::launch_reduce_chunks(a.pMu, P.n_chunks, n_freq, S.mu, h->stream));
+        r.add(a.pSb, C1, (size_t)n_freq * m2, S.Sb);
+        r.add(a.pMu, C1, n_freq, S.mu);
     }
+    HIPCHK(dg::launch_reduce_set(r, h->stream, a.pt_n));
     return DMFTGPU_OK;
 }
 
@@ -669,43 +672,33 @@ int forward_impl(dmftgpu_handle h, int method, const double* sigma, double mu, d
     // capacity before it launches anything
     cd* tot = (cd*)(ws + off);
     off += ((size_t)(m2 + 3) * sizeof(cd) + 255) / 256 * 256;
-    cd* st = (cd*)(ws + off);
-    off += ((size_t)m2 * sizeof(cd) + 255) / 256 * 256;
-    double* sts = (double*)(ws + off);
-    off += 256;
+    const cd* st = nullptr;
+    const double* sts = nullptr;
     const size_t cap = ext_ws ? ext_cap : SIZE_MAX;
-    int rc = run_static(h, mu, st, sts, ws, off, ext_ws != nullptr, nullptr, cap);
+    int rc = run_static(h, mu, &st, &sts, ws, off, ext_ws != nullptr, nullptr, cap);
     if (rc) return rc;
     rc = run_lattice(h, method, dg::MODE_FWD, sigma, mu, nullptr, 0.0, ws, off, S, n_total != nullptr, nullptr,
                      nullptr, max_chunks, cap);
     if (rc) return rc;
-    HIPCHK(dg::launch_freq_totals(S.Gsum, m2, nc, S.tr, nullptr, nw_tot, nullptr, 0, tot, h->stream, S.pt_n,
-                                  S.pt_wt));
     const double inv_nk = 1.0 / (double)L.n_k_global;
-    HIPCHK(dg::launch_gloc_finalize(S.Gsum, L.n_freq, nc, L.n_cluster, inv_nk, (cd*)gloc, h->stream));
+    const dg::FreqScale out{S.Gsum, (cd*)gloc, (size_t)L.n_freq * m2, nc / L.n_cluster, inv_nk};
+    HIPCHK(dg::launch_freq_totals(S.Gsum, m2, nc, S.tr, nullptr, nw_tot, nullptr, 0, tot, h->stream, S.pt_n, S.pt_wt,
+                                  out));
     if (gloc_hf)
         HIPCHK(dg::launch_gloc_hf(h->ev, h->U, L.n, nc, L.n_k, L.n_freq, L.beta, mu, inv_nk, L.n_cluster, (cd*)gloc_hf,
                                   h->stream));
     // NumMatrix = [ (1/beta) sum_n sum_k (G_cc + G_cc^H) + sum_k (U w U^H)_cc ] / knum_mpiGlobal
-    // (host arrays on the stack: n_corr <= 32)
-    cd htot[32 * 32 + 3], hst[32 * 32], num[32 * 32];
-    double hsts[2];
-    HIPCHK(hipMemcpyAsync(htot, tot, sizeof(cd) * (m2 + 3), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipMemcpyAsync(hst, st, sizeof(cd) * m2, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipMemcpyAsync(hsts, sts, sizeof(double) * 2, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(dg::launch_results(tot, st, sts, m2, L.beta, (double)L.n_k_global, (cd*)num_matrix, h->stream));
+    cd res[32 * 32 + 3];  // NumMatrix, N (on the stack: n_corr <= 32)
+    HIPCHK(hipMemcpyAsync(res, tot, sizeof(cd) * (m2 + 1), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
     if (n_total) {
-        *n_total = (htot[m2].x / L.beta + hsts[0]) / (double)L.n_k_global;
+        *n_total = res[m2].x;
         if (!std::isfinite(*n_total)) return fail(h, DMFTGPU_ERR_NUMERIC, "N(mu) is not finite");
     }
-    for (int q = 0; q < m2; ++q) {
-        num[q].x = (htot[q].x / L.beta + hst[q].x) * inv_nk;
-        num[q].y = (htot[q].y / L.beta + hst[q].y) * inv_nk;
-        if (!std::isfinite(num[q].x) || !std::isfinite(num[q].y))
+    for (int q = 0; q < m2; ++q)
+        if (!std::isfinite(res[q].x) || !std::isfinite(res[q].y))
             return fail(h, DMFTGPU_ERR_NUMERIC, "NumMatrix is not finite");
-    }
-    HIPCHK(hipMemcpyAsync(num_matrix, num, sizeof(cd) * m2, hipMemcpyHostToDevice, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
     return DMFTGPU_OK;
 }
 
@@ -824,21 +817,16 @@ static int density_impl(dmftgpu_handle h, int method, const double* sigma, doubl
     if (rc) return rc;
     cd* tot = (cd*)(ws + off);
     off += ((size_t)(m2 + 3) * sizeof(cd) + 255) / 256 * 256;
-    cd* st = (cd*)(ws + off);
-    off += ((size_t)m2 * sizeof(cd) + 255) / 256 * 256;
-    double* sts = (double*)(ws + off);
-    off += 256;
-    rc = run_static(h, mu, st, sts, ws, off);
+    const cd* st = nullptr;
+    const double* sts = nullptr;
+    rc = run_static(h, mu, &st, &sts, ws, off);
     if (rc) return rc;
     HIPCHK(dg::launch_freq_totals(nullptr, m2, nc, S.tr, S.tr2, nw_tot, nullptr, 0, tot, h->stream, S.pt_n, S.pt_wt));
-    std::vector<cd> htot(m2 + 3);
-    double hsts[2];
-    HIPCHK(hipMemcpyAsync(htot.data(), tot, sizeof(cd) * (m2 + 3), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipMemcpyAsync(hsts, sts, sizeof(double) * 2, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(dg::launch_results(tot, st, sts, m2, L.beta, (double)L.n_k_global, nullptr, h->stream));
+    cd res[2];
+    HIPCHK(hipMemcpyAsync(res, tot + m2, sizeof(res), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
-    const double inv_nk = 1.0 / (double)L.n_k_global;
-    const double N = (htot[m2].x / L.beta + hsts[0]) * inv_nk;
-    const double dN = (-htot[m2 + 1].x / L.beta + hsts[1]) * inv_nk;
+    const double N = res[0].x, dN = res[1].x;
     if (!std::isfinite(N) || !std::isfinite(dN)) return fail(h, DMFTGPU_ERR_NUMERIC, "N(mu) is not finite");
     if (n_out) *n_out = N;
     if (dn_out) *dn_out = dN;
@@ -921,23 +909,20 @@ int vjp_impl(dmftgpu_handle h, int method, const double* sigma, double mu, const
     if (rc) return rc;
     cd* tot = (cd*)(ws + off);
     off += ((size_t)(m2 + 3) * sizeof(cd) + 255) / 256 * 256;
-    cd* st = (cd*)(ws + off);
-    off += ((size_t)m2 * sizeof(cd) + 255) / 256 * 256;
-    double* sts = (double*)(ws + off);
-    off += 256;
-    rc = run_static(h, mu, st, sts, ws, off);
+    const cd* st = nullptr;
+    const double* sts = nullptr;
+    rc = run_static(h, mu, &st, &sts, ws, off);
     if (rc) return rc;
     const double inv_nk = 1.0 / (double)L.n_k_global;
-    HIPCHK(dg::launch_scale(S.Sb, (size_t)L.n_freq * m2, inv_nk, (cd*)sigma_bar, h->stream));
+    const dg::FreqScale out{S.Sb, (cd*)sigma_bar, (size_t)L.n_freq * m2, nc, inv_nk};
     HIPCHK(dg::launch_freq_totals(nullptr, m2, nc, nullptr, S.tr2, nw_tot, S.mu, L.n_freq, tot, h->stream, S.pt_n,
-                                  S.pt_wt));
-    std::vector<cd> htot(m2 + 3);
-    double hsts[2];
-    HIPCHK(hipMemcpyAsync(htot.data(), tot, sizeof(cd) * (m2 + 3), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipMemcpyAsync(hsts, sts, sizeof(double) * 2, hipMemcpyDeviceToHost, h->stream));
+                                  S.pt_wt, out));
+    HIPCHK(dg::launch_results(tot, st, sts, m2, L.beta, (double)L.n_k_global, nullptr, h->stream));
+    cd res[3];
+    HIPCHK(hipMemcpyAsync(res, tot + m2, sizeof(res), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
-    const double dN = (-htot[m2 + 1].x / L.beta + hsts[1]) * inv_nk;
-    const double mub = -htot[m2 + 2].x * inv_nk + n_bar * dN;
+    const double dN = res[1].x;
+    const double mub = -res[2].x * inv_nk + n_bar * dN;
     if (!std::isfinite(mub)) return fail(h, DMFTGPU_ERR_NUMERIC, "mu_bar is not finite");
     if (mu_bar) *mu_bar = mub;
     return DMFTGPU_OK;
@@ -987,23 +972,20 @@ static int jvp_impl(dmftgpu_handle h, int method, const double* sigma, double mu
     if (rc) return rc;
     cd* tot = (cd*)(ws + off);
     off += ((size_t)(m2 + 3) * sizeof(cd) + 255) / 256 * 256;
-    cd* st = (cd*)(ws + off);
-    off += ((size_t)m2 * sizeof(cd) + 255) / 256 * 256;
-    double* sts = (double*)(ws + off);
-    off += 256;
-    rc = run_static(h, mu, st, sts, ws, off);
+    const cd* st = nullptr;
+    const double* sts = nullptr;
+    rc = run_static(h, mu, &st, &sts, ws, off);
     if (rc) return rc;
     const double inv_nk = 1.0 / (double)L.n_k_global;
     HIPCHK(dg::launch_adjoint_stack(S.Sb, (size_t)L.n_freq, nc, inv_nk, (cd*)dgloc, h->stream));
     HIPCHK(dg::launch_freq_totals(nullptr, m2, nc, nullptr, S.tr2, nw_tot, S.mu, L.n_freq, tot, h->stream, S.pt_n,
                                   S.pt_wt));
-    cd htot[32 * 32 + 3];
-    double hsts[2];
-    HIPCHK(hipMemcpyAsync(htot, tot, sizeof(cd) * (m2 + 3), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipMemcpyAsync(hsts, sts, sizeof(double) * 2, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(dg::launch_results(tot, st, sts, m2, L.beta, (double)L.n_k_global, nullptr, h->stream));
+    cd res[3];
+    HIPCHK(hipMemcpyAsync(res, tot + m2, sizeof(res), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
-    const double dNdmu = (-htot[m2 + 1].x / L.beta + hsts[1]) * inv_nk;
-    const double d = 2.0 / L.beta * htot[m2 + 2].x * inv_nk + dmu * dNdmu;
+    const double dNdmu = res[1].x;
+    const double d = 2.0 / L.beta * res[2].x * inv_nk + dmu * dNdmu;
     if (!std::isfinite(d)) return fail(h, DMFTGPU_ERR_NUMERIC, "dN is not finite");
     if (dn) *dn = d;
     return DMFTGPU_OK;
@@ -1078,14 +1060,12 @@ extern "C" int dmftgpu_density_matrix(dmftgpu_handle h, const double* sigma, dou
     char* ws = (char*)h->ws.get(need, &e);
     if (!ws) return fail(h, DMFTGPU_ERR_HIP, "workspace %zu bytes: %s", need, hipGetErrorString(e));
     size_t off = 0;
-    cd* st = (cd*)(ws + off);
-    off += ((size_t)m2 * sizeof(cd) + 255) / 256 * 256;
-    double* sts = (double*)(ws + off);
-    off += 256;
+    const cd* st = nullptr;
+    const double* sts = nullptr;
     cd* sig_all = block ? (cd*)(ws + off) : nullptr;
     off += sig_bytes;
     const double* wt = nullptr;
-    int rc = run_static(h, mu, st, sts, ws, off, false, &wt);  // the static weights for this mu
+    int rc = run_static(h, mu, &st, &sts, ws, off, false, &wt);  // the static weights for this mu
     if (rc) return rc;
     dg::LatArgs a{};
     a.Hk = h->Hk;

@@ -82,7 +82,7 @@ struct Sys {
     // lattice partials / sums (sized for the largest chunk count)
     int max_chunks;
     cd *pTrF, *pG, *pTrV, *pTr2, *pSb, *pMu;
-    cd *trF, *Gsum, *trV, *tr2, *Sb, *musum;
+    cd *trF, *Gsum, *tr2, *Sb, *musum;
     // chosen plans
     int chunks_f, kpc_f, chunks_v, kpc_v;
     // frequency points of the density sums (freq_points.hip)
@@ -299,9 +299,11 @@ int issue_step(dmftgpu_batch_s* b)
         HIPCHK(dg::launch_static_terms(s.ev, s.n, s.nk, s.nw_tot, beta, s.d.mu, s.wt, s.dt, h->stream));
         HIPCHK(dg::launch_static_reduce(s.wt, s.dt, s.U, s.n, s.nc, s.nk, s.st_kpc, s.st_chunks, s.pNum, s.pN,
                                         s.pN + s.st_chunks, h->stream));
-        HIPCHK(dg::launch_reduce_chunks(s.pNum, s.st_chunks, s.m2, s.st, h->stream));
-        HIPCHK(dg::launch_reduce_chunks_d(s.pN, s.st_chunks, 1, s.sts, h->stream));
-        HIPCHK(dg::launch_reduce_chunks_d(s.pN + s.st_chunks, s.st_chunks, 1, s.sts + 1, h->stream));
+        dg::ReduceSet r;
+        r.add(s.pNum, s.st_chunks, s.m2, s.st);
+        r.add(s.pN, s.st_chunks, 1, s.sts);
+        r.add(s.pN + s.st_chunks, s.st_chunks, 1, s.sts + 1);
+        HIPCHK(dg::launch_reduce_set(r, h->stream));
     }
     for (Group& g : b->groups) {  // forward: one persistent launch per n_c
         int rc = launch_group(b, g, MODE_FWD);
@@ -309,11 +311,13 @@ int issue_step(dmftgpu_batch_s* b)
     }
     for (Sys& s : b->sys) {
         const double inv_nk = 1.0 / (double)s.d.lat.n_k_global;
-        HIPCHK(dg::launch_reduce_chunks(s.pTrF, s.chunks_f, s.nw_tot, s.trF, h->stream, s.pt_n));
-        HIPCHK(dg::launch_reduce_chunks(s.pG, s.chunks_f, (size_t)s.nw_tot * s.m2, s.Gsum, h->stream, s.pt_n, s.m2));
+        dg::ReduceSet r;
+        r.add(s.pTrF, s.chunks_f, s.nw_tot, s.trF, 1);
+        r.add(s.pG, s.chunks_f, (size_t)s.nw_tot * s.m2, s.Gsum, s.m2);
+        HIPCHK(dg::launch_reduce_set(r, h->stream, s.pt_n));
+        const dg::FreqScale out{s.Gsum, (cd*)s.d.gloc, (size_t)s.nf * s.m2, s.nc / s.d.lat.n_cluster, inv_nk};
         HIPCHK(dg::launch_freq_totals(s.Gsum, s.m2, s.nc, s.trF, nullptr, s.nw_tot, nullptr, 0, s.tot_f, h->stream, s.pt_n,
-                                      s.pt_wt));
-        HIPCHK(dg::launch_gloc_finalize(s.Gsum, s.nf, s.nc, s.d.lat.n_cluster, inv_nk, (cd*)s.d.gloc, h->stream));
+                                      s.pt_wt, out));
         hipLaunchKernelGGL(k_fin_fwd, dim3(1), dim3(1024), 0, h->stream, s.tot_f, s.st, s.sts, s.m2, s.d.lat.beta,
                            inv_nk, (cd*)s.d.num_matrix, s.d.n_total);
         HIPCHK(hipGetLastError());
@@ -332,13 +336,14 @@ int issue_step(dmftgpu_batch_s* b)
     }
     for (Sys& s : b->sys) {
         const double inv_nk = 1.0 / (double)s.d.lat.n_k_global;
-        HIPCHK(dg::launch_reduce_chunks(s.pTrV, s.chunks_v, s.nw_tot, s.trV, h->stream, s.pt_n));
-        HIPCHK(dg::launch_reduce_chunks(s.pTr2, s.chunks_v, s.nw_tot, s.tr2, h->stream, s.pt_n));
-        HIPCHK(dg::launch_reduce_chunks(s.pSb, s.chunks_v, (size_t)s.nf * s.m2, s.Sb, h->stream));
-        HIPCHK(dg::launch_reduce_chunks(s.pMu, s.chunks_v, s.nf, s.musum, h->stream));
-        HIPCHK(dg::launch_scale(s.Sb, (size_t)s.nf * s.m2, inv_nk, (cd*)s.d.sigma_bar, h->stream));
-        HIPCHK(dg::launch_freq_totals(nullptr, s.m2, s.nc, s.trV, s.tr2, s.nw_tot, s.musum, s.nf, s.tot_v, h->stream,
-                                      s.pt_n, s.pt_wt));
+        dg::ReduceSet r;
+        r.add(s.pTr2, s.chunks_v, s.nw_tot, s.tr2, 1);
+        r.add(s.pSb, s.chunks_v, (size_t)s.nf * s.m2, s.Sb);
+        r.add(s.pMu, s.chunks_v, s.nf, s.musum);
+        HIPCHK(dg::launch_reduce_set(r, h->stream, s.pt_n));
+        const dg::FreqScale out{s.Sb, (cd*)s.d.sigma_bar, (size_t)s.nf * s.m2, s.nc, inv_nk};
+        HIPCHK(dg::launch_freq_totals(nullptr, s.m2, s.nc, nullptr, s.tr2, s.nw_tot, s.musum, s.nf, s.tot_v, h->stream,
+                                      s.pt_n, s.pt_wt, out));
         hipLaunchKernelGGL(k_fin_vjp, dim3(1), dim3(1), 0, h->stream, s.tot_v, s.sts, s.m2, s.d.lat.beta, inv_nk,
                            s.nbar, s.d.mu_bar);
         HIPCHK(hipGetLastError());
@@ -543,7 +548,6 @@ static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system
         s.pSb = (cd*)take(16 * C * s.nf * s.m2);
         s.pMu = (cd*)take(16 * C * s.nf);
         s.trF = (cd*)take(16 * (size_t)s.nw_tot);
-        s.trV = (cd*)take(16 * (size_t)s.nw_tot);
         s.tr2 = (cd*)take(16 * (size_t)s.nw_tot);
         s.Gsum = (cd*)take(16 * (size_t)s.nw_tot * s.m2);
         s.Sb = (cd*)take(16 * (size_t)s.nf * s.m2);

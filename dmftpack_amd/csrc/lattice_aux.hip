@@ -249,15 +249,12 @@ __device__ __forceinline__ cd radd(cd a, cd b) { return cadd(a, b); }
 constexpr int kRedX = 32, kRedY = 8;
 
 template <class T>
-__global__ __launch_bounds__(kRedX* kRedY) void k_reduce_chunks(const T* __restrict__ part, int n_chunks, size_t len,
-                                                                 T* __restrict__ out, const int* __restrict__ n_pts,
-                                                                 int per)
+__device__ __forceinline__ void reduce_block(const T* __restrict__ part, int n_chunks, size_t len, T* __restrict__ out,
+                                             size_t lim, size_t block, T (&red)[kRedY][kRedX])
 {
-    __shared__ T red[kRedY][kRedX];
-    const size_t lim = n_pts ? (size_t)*n_pts * per : len;
-    if ((size_t)blockIdx.x * kRedX >= lim) return;
+    if (block * kRedX >= lim) return;
     const int tx = threadIdx.x % kRedX, ty = threadIdx.x / kRedX;
-    const size_t i = (size_t)blockIdx.x * kRedX + tx;
+    const size_t i = block * kRedX + tx;
     const int c0 = (int)((long long)n_chunks * ty / kRedY);
     const int c1 = (int)((long long)n_chunks * (ty + 1) / kRedY);
     T acc{};
@@ -274,37 +271,54 @@ __global__ __launch_bounds__(kRedX* kRedY) void k_reduce_chunks(const T* __restr
     }
 }
 
-template <class T>
-static hipError_t launch_reduce(const T* part, int n_chunks, size_t len, T* out, hipStream_t s,
-                                const int* n_pts = nullptr, int per = 1)
+// the arrays of one lattice launch (or of the static part) in one launch: block b works
+// on the array whose range of blocks holds it
+__global__ __launch_bounds__(kRedX* kRedY) void k_reduce_set(ReduceSet r, const int* __restrict__ n_pts)
 {
-    if (len == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_reduce_chunks<T>, dim3((unsigned)((len + kRedX - 1) / kRedX)), dim3(kRedX * kRedY), 0, s,
-                       part, n_chunks, len, out, n_pts, per);
+    __shared__ cd red[kRedY][kRedX];
+    size_t block = blockIdx.x;
+    int q = 0;
+    for (; q < r.n - 1; ++q) {
+        const size_t nb = (r.a[q].len + kRedX - 1) / kRedX;
+        if (block < nb) break;
+        block -= nb;
+    }
+    const ReduceSet::Array& a = r.a[q];
+    const size_t lim = n_pts && a.per ? (size_t)*n_pts * a.per : a.len;
+    if (a.is_double)
+        reduce_block((const double*)a.part, a.n_chunks, a.len, (double*)a.out, lim, block,
+                     *(double(*)[kRedY][kRedX])(void*)red);
+    else reduce_block((const cd*)a.part, a.n_chunks, a.len, (cd*)a.out, lim, block, red);
+}
+
+hipError_t launch_reduce_set(const ReduceSet& r, hipStream_t s, const int* n_pts)
+{
+    size_t nb = 0;
+    for (int q = 0; q < r.n; ++q) nb += (r.a[q].len + kRedX - 1) / kRedX;
+    if (nb == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_reduce_set, dim3((unsigned)nb), dim3(kRedX * kRedY), 0, s, r, n_pts);
     return hipGetLastError();
-}
-
-hipError_t launch_reduce_chunks(const cd* part, int n_chunks, size_t len, cd* out, hipStream_t s, const int* n_pts,
-                                int per)
-{
-    return launch_reduce(part, n_chunks, len, out, s, n_pts, per);
-}
-
-hipError_t launch_reduce_chunks_d(const double* part, int n_chunks, size_t len, double* out, hipStream_t s)
-{
-    return launch_reduce(part, n_chunks, len, out, s);
 }
 
 // One workgroup per output quantity q: q < m2 -> element e=q of
 // sum_nw (G + G^H)[e]; q = m2 -> sum 2 Re tr; m2+1 -> sum 2 Re tr2;
-// m2+2 -> sum Re mu.  Fixed-order block reduction.
+// m2+2 -> sum Re mu.  Fixed-order block reduction.  The workgroups after those scale
+// the frequency-resolved sums into the call's output (npc: zero outside blocks of npc).
 __global__ __launch_bounds__(256) void k_freq_totals(const cd* __restrict__ G, int m2, int nc,
                                                      const cd* __restrict__ tr, const cd* __restrict__ tr2, int nw_tot,
                                                      const cd* __restrict__ mu, int n_mu, cd* __restrict__ out,
-                                                     const int* __restrict__ n_pts, const double* __restrict__ pt_wt)
+                                                     const int* __restrict__ n_pts, const double* __restrict__ pt_wt,
+                                                     FreqScale f)
 {
     __shared__ double rx[256], ry[256];
     const int q = blockIdx.x;
+    if (q >= m2 + 3) {
+        const size_t t = (size_t)(q - m2 - 3) * 256 + threadIdx.x;
+        if (t >= f.len) return;
+        const int e = (int)(t % m2), i = e % nc, j = e / nc;
+        f.out[t] = (i / f.npc == j / f.npc) ? cscale(f.in[t], f.scale) : cd{0.0, 0.0};
+        return;
+    }
     double ax = 0.0, ay = 0.0;
     if (n_pts) nw_tot = *n_pts;
     auto wt = [&](int nw) { return pt_wt ? pt_wt[nw] : 1.0; };
@@ -342,29 +356,40 @@ __global__ __launch_bounds__(256) void k_freq_totals(const cd* __restrict__ G, i
 }
 
 hipError_t launch_freq_totals(const cd* G, int m2, int nc, const cd* tr, const cd* tr2, int nw_tot, const cd* mu,
-                              int n_mu, cd* out, hipStream_t s, const int* n_pts, const double* pt_wt)
+                              int n_mu, cd* out, hipStream_t s, const int* n_pts, const double* pt_wt,
+                              const FreqScale& f)
 {
-    hipLaunchKernelGGL(k_freq_totals, dim3(m2 + 3), dim3(256), 0, s, G, m2, nc, tr, tr2, nw_tot, mu, n_mu, out, n_pts,
-                       pt_wt);
+    hipLaunchKernelGGL(k_freq_totals, dim3((unsigned)(m2 + 3 + (f.len + 255) / 256)), dim3(256), 0, s, G, m2, nc, tr,
+                       tr2, nw_tot, mu, n_mu, out, n_pts, pt_wt, f);
     return hipGetLastError();
 }
 
-__global__ __launch_bounds__(256) void k_gloc_finalize(const cd* __restrict__ Gsum, int n_freq, int nc, int npc,
-                                                       double scale, cd* __restrict__ gloc)
+// The call's scalars and NumMatrix from the frequency totals and the static part, over
+// the totals (so that the host copies one array): entries q < m2 (with num) NumMatrix,
+// also to num; m2 N = (tr/beta + sum w)/n_k; m2+1 dN/dmu = (-tr2/beta + sum dN)/n_k;
+// m2+2 unchanged.
+__global__ __launch_bounds__(1024) void k_results(cd* __restrict__ tot, const cd* __restrict__ st,
+                                                  const double* __restrict__ sts, int m2, double beta, double n_k,
+                                                  cd* __restrict__ num)
 {
-    const int m2 = nc * nc;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n_freq * m2) return;
-    const int e = t % m2, i = e % nc, j = e / nc;
-    gloc[t] = (i / npc == j / npc) ? cscale(Gsum[t], scale) : cd{0.0, 0.0};
+    const int q = threadIdx.x;
+    const double inv_nk = 1.0 / n_k;
+    if (q < m2 && num) {
+        const cd v = cd{(tot[q].x / beta + st[q].x) * inv_nk, (tot[q].y / beta + st[q].y) * inv_nk};
+        tot[q] = v;
+        num[q] = v;
+    }
+    if (q == 0) {
+        const double N = tot[m2].x / beta + sts[0];
+        tot[m2].x = num ? N / n_k : N * inv_nk;
+        tot[m2 + 1].x = (-tot[m2 + 1].x / beta + sts[1]) * inv_nk;
+    }
 }
 
-hipError_t launch_gloc_finalize(const cd* Gsum, int n_freq, int nc, int n_cluster, double scale, cd* gloc,
-                                hipStream_t s)
+hipError_t launch_results(cd* tot, const cd* st, const double* sts, int m2, double beta, double n_k, cd* num,
+                          hipStream_t s)
 {
-    const int total = n_freq * nc * nc;
-    hipLaunchKernelGGL(k_gloc_finalize, dim3((total + 255) / 256), dim3(256), 0, s, Gsum, n_freq, nc, nc / n_cluster,
-                       scale, gloc);
+    hipLaunchKernelGGL(k_results, dim3(1), dim3(num ? (m2 + 63) / 64 * 64 : 64), 0, s, tot, st, sts, m2, beta, n_k, num);
     return hipGetLastError();
 }
 

@@ -287,11 +287,21 @@ hipError_t launch_loss_cotangent(const cd* gloc, const cd* gtgt, int n_freq, int
 hipError_t launch_gloc_hf(const double* ev, const cd* U, int n, int nc, int nk, int n_freq, double beta, double mu,
                           double inv_nkg, int n_cluster, cd* out, hipStream_t s);
 
-// Deterministic reductions over chunks: out[i] = sum_c part[c*len + i]
-// (n_pts, optional: only the first *n_pts * per entries of each chunk are summed)
-hipError_t launch_reduce_chunks(const cd* part, int n_chunks, size_t len, cd* out, hipStream_t s,
-                                const int* n_pts = nullptr, int per = 1);
-hipError_t launch_reduce_chunks_d(const double* part, int n_chunks, size_t len, double* out, hipStream_t s);
+// Deterministic sums over chunks, out[i] = sum_c part[c*len + i], of up to four arrays in
+// one launch (each on its own took a launch, 3 to 5 us of a small call's 120).  per > 0: only the
+// first *n_pts * per entries of the array are summed.
+struct ReduceSet {
+    struct Array {
+        const void* part;
+        void* out;
+        size_t len;
+        int n_chunks, per, is_double;
+    } a[4];
+    int n = 0;
+    void add(const cd* part, int n_chunks, size_t len, cd* out, int per = 0) { a[n++] = {part, out, len, n_chunks, per, 0}; }
+    void add(const double* part, int n_chunks, size_t len, double* out) { a[n++] = {part, out, len, n_chunks, 0, 1}; }
+};
+hipError_t launch_reduce_set(const ReduceSet& r, hipStream_t s, const int* n_pts = nullptr);
 
 // Final reductions over frequency: for FWD/DENS/VJP totals.
 //   sumG[e]  = sum_nw (G[nw][e] + conj(G[nw][e^T]))        (e < m2)   if G != null
@@ -299,14 +309,22 @@ hipError_t launch_reduce_chunks_d(const double* part, int n_chunks, size_t len, 
 //   sumTr2   = sum_nw 2 Re tr2[nw]                          if tr2 != null
 //   sumMu    = sum_nw Re mu[nw] over n_mu entries           if mu != null
 // out layout: [m2 complex] [3 doubles as complex .x].  With n_pts the sums run over
-// *n_pts points, each term weighted by pt_wt[nw].
+// *n_pts points, each term weighted by pt_wt[nw].  In the same launch (FreqScale, optional):
+// out[i] = in[i] * scale for i < len (stack of nc x nc), zero outside blocks of npc orbitals
+struct FreqScale {
+    const cd* in = nullptr;
+    cd* out = nullptr;
+    size_t len = 0;
+    int npc = 1;
+    double scale = 0.0;
+};
 hipError_t launch_freq_totals(const cd* G, int m2, int nc, const cd* tr, const cd* tr2, int nw_tot, const cd* mu,
                               int n_mu, cd* out, hipStream_t s, const int* n_pts = nullptr,
-                              const double* pt_wt = nullptr);
-
-// gloc[nw][e] = Gsum[nw][e] * scale for nw < n_freq, zero outside cluster blocks
-hipError_t launch_gloc_finalize(const cd* Gsum, int n_freq, int nc, int n_cluster, double scale, cd* gloc,
-                                hipStream_t s);
+                              const double* pt_wt = nullptr, const FreqScale& f = FreqScale());
+// NumMatrix (with num: into it and tot[0..m2)), N (tot[m2].x) and dN/dmu (tot[m2+1].x)
+// from the totals and the static part
+hipError_t launch_results(cd* tot, const cd* st, const double* sts, int m2, double beta, double n_k, cd* num,
+                          hipStream_t s);
 // out[m] = scale * in[m]^H over a stack of count d x d matrices (in != out)
 hipError_t launch_adjoint_stack(const cd* in, size_t count, int d, double scale, cd* out, hipStream_t s);
 // out[i] = in[i] * scale
