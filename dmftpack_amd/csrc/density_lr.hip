@@ -156,13 +156,25 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NC <= 5 ? 2 
             const cd g = cd{md * x * rr, -md * w2 * rr};
             gsum = cd{fma(sWt[wl], g.x, gsum.x), fma(sWt[wl], g.y, gsum.y)};
             const int jc = j < NC ? j : 0;
+            // row q of G_cc (and the lane's own entry of it), read a row ahead: with each entry
+            // read where it is used, n = 14, n_c = 5 on 4096 k x 1040 points took 1556 us for
+            // the call, against 1320
+            cd row[2][NC + 1];
+            auto read = [&](int q) {
+#pragma unroll
+                for (int b = 0; b < NC; ++b) row[q & 1][b] = Gs[q + b * NC];
+                row[q & 1][NC] = Gs[q + jc * NC];
+            };
+            read(0);
 #pragma unroll
             for (int q = 0; q < NC; ++q) {
+                if (q + 1 < NC) read(q + 1);
+                __builtin_amdgcn_sched_barrier(0);
                 // R[q][j] = G_cc[q][j] (j < NC) or (G_cc W)_{q d} g_d (j = NC + d)
                 cd tq = cd{0.0, 0.0};
 #pragma unroll
-                for (int b = 0; b < NC; ++b) tq = cfma(Gs[q + b * NC], wcol[b], tq);
-                const cd gc = Gs[q + jc * NC];
+                for (int b = 0; b < NC; ++b) tq = cfma(row[q & 1][b], wcol[b], tq);
+                const cd gc = row[q & 1][NC];
                 const cd tg = cmul(tq, g);
                 const cd r = cd{fma(m1, gc.x, tg.x), fma(m1, gc.y, tg.y)};
                 // E[j][q] = delta_jq (j < NC) or g_d conj(W_qd) (j = NC + d)
