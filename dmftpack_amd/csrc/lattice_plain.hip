@@ -39,10 +39,9 @@ __device__ __forceinline__ void s2_from_lanes(const cd (&col)[N], cd (&S2)[NCR],
 {
     if constexpr (M < N) {
         if (M < n) {
-            const double mwy = -col[M].y;
 #pragma unroll
             for (int i = 0; i < NCR; ++i)
-                if (i < nc) cfma_bcast<M>(S2[i], col[i], col[M], mwy);
+                if (i < nc) cfma_bcast<M>(S2[i], col[i], col[M]);
             s2_from_lanes<N, NCR, M + 1>(col, S2, nc, n);
         }
     }
@@ -54,17 +53,33 @@ __device__ __forceinline__ void xh_from_lanes(const cd (&col)[N], const cd (&z)[
 {
     if constexpr (I < NCR) {
         if (I < nc) {
-            const double mzy = -z[I].y;
 #pragma unroll
             for (int r = 0; r < NCR; ++r)
-                if (r < nc) cfma_bcast<I>(XH[r], col[r], z[I], mzy);
+                if (r < nc) cfma_bcast<I>(XH[r], col[r], z[I]);
             xh_from_lanes<N, NCR, I + 1>(col, z, XH, nc);
         }
     }
 }
 
+// tr += sum_{I < n} G_II, lane I's entry of its own column, on every lane of the slot
+template <int N, int I>
+__device__ __forceinline__ void trace_from_lanes(const cd (&col)[N], cd& tr, double one, int n)
+{
+    if constexpr (I < N) {
+        if (I < n) {
+            cadd_bcast<I>(tr, col[I], one);
+            trace_from_lanes<N, I + 1>(col, tr, one, n);
+        }
+    }
+}
+
+// Wavefronts per SIMD the register allocator is held to (a third pays for the forward and
+// the densities; the adjoint at n = 16 is faster with one or two and no spills)
+template <int L, int N, int MODE>
+constexpr int plain_waves() { return L == 16 && N > 12 && MODE != MODE_VJP ? 3 : 1; }
+
 template <int N, int L, int MODE, int WG>
-__global__ __launch_bounds__(WG) void k_lattice_plain(LatArgs a)
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(plain_waves<L, N, MODE>()))) void k_lattice_plain(LatArgs a)
 {
     constexpr int SLOTS = WG / L;
     // 16-lane slots with n_c <= NCR keep the adjoint sums in registers: lane
@@ -90,7 +105,6 @@ __global__ __launch_bounds__(WG) void k_lattice_plain(LatArgs a)
     const int k1 = min(a.nk, k0 + a.k_per_chunk);
     double mun, wn;
     freq_point(a, nw, mun, wn);
-    const cd zmu = cd{mun, wn};
     const bool vjp_here = (MODE == MODE_VJP) && wvalid && nw < a.n_freq;
 
     for (int e = tid; e < 2 * NN; e += WG) sH[e] = cd{0.0, 0.0};
@@ -110,6 +124,28 @@ __global__ __launch_bounds__(WG) void k_lattice_plain(LatArgs a)
     cd S2[NCR], XH[NCR];
 #pragma unroll
     for (int i = 0; i < NCR; ++i) S2[i] = XH[i] = cd{0.0, 0.0};
+    // Column c of (iw + mu) I - P Sigma P^H (past n: of I).  Up to 12 orbitals it is kept in
+    // registers, so that A is one subtraction an entry; above, the diagonal is added by a
+    // product with a 0/1 factor and Sigma read from LDS, the registers deciding the number of
+    // wavefronts.  (With selections of whole entries in the set-up and in the trace, 280 of a
+    // wavefront's 1650 instructions per k at n = 14 were masks.)  Forward, 1728 k x 1024
+    // frequencies, before / now: n = 9 0.68 / 0.56 ms, 12 1.04 / 0.88, 14 1.35 / 1.16, 16
+    // 1.84 / 1.70.
+    constexpr bool KEEP = N <= 12;
+    const cd diag = cd{c < n ? mun : 1.0, c < n ? wn : 0.0};
+    cd E[KEEP ? N : 1];
+    if constexpr (KEEP) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            double x = i == c ? diag.x : 0.0, y = i == c ? diag.y : 0.0;
+            if (i < nc && c < nc) {
+                const cd v = sSig[slot * m2 + i + c * nc];
+                x -= v.x;
+                y -= v.y;
+            }
+            E[i] = cd{x, y};
+        }
+    }
     __syncthreads();
 
     for (int k = k0; k < k1; ++k) {
@@ -124,26 +160,39 @@ __global__ __launch_bounds__(WG) void k_lattice_plain(LatArgs a)
         }
         // column c of A = (iw+mu) I - H - P Sigma P^H
         cd col[N];
+        // (lanes n <= c < N read zeros; what lanes c >= N hold is never read)
         const cd* Hc = sH + cur * NN + (c < N ? c : 0) * N;
+        if constexpr (KEEP) {
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-            cd h = Hc[i];
-            col[i] = (c < n) ? cneg(h) : cd{0.0, 0.0};
-            if (i == c) col[i] = (c < n) ? cadd(col[i], zmu) : cd{1.0, 0.0};
-        }
-        if (c < nc) {
+            for (int i = 0; i < N; ++i) col[i] = csub(E[i], Hc[i]);
+        } else {
+            int ch = c;
+            // (hidden, or its N masks are held across the k walk: 32 registers at n = 16)
+            if constexpr (N > 14 && MODE != MODE_VJP) asm volatile("" : "+v"(ch));
 #pragma unroll
-            for (int i = 0; i < N; ++i)
-                if (i < nc) col[i] = csub(col[i], sSig[slot * m2 + i + c * nc]);
+            for (int i = 0; i < N; ++i) {
+                const double one = __hiloint2double(i == ch ? 0x3FF00000 : 0, 0);  // 1 on lane i, else 0
+                const cd h = Hc[i];
+                col[i] = cd{fma(one, diag.x, -h.x), fma(one, diag.y, -h.y)};
+            }
+            if (c < nc) {
+#pragma unroll
+                for (int i = 0; i < N; ++i)
+                    if (i < nc) col[i] = csub(col[i], sSig[slot * m2 + i + c * nc]);
+            }
         }
         if constexpr (L == 16) gj_columns_row16<N>(col, c, n);
         else gj_columns<N>(col, bc, c, n);
         // lane c < n now holds column c of G
-        cd gcc = cd{0.0, 0.0};
+        if constexpr (L == 16) {
+            trace_from_lanes<N, 0>(col, trA, 1.0, n);
+        } else {
+            cd gcc = cd{0.0, 0.0};
 #pragma unroll
-        for (int i = 0; i < N; ++i)
-            if (i == c) gcc = col[i];
-        if (c < n && wvalid) trA = cadd(trA, gcc);
+            for (int i = 0; i < N; ++i)
+                if (i == c) gcc = col[i];
+            if (c < n && wvalid) trA = cadd(trA, gcc);
+        }
 
         if (MODE == MODE_FWD) {
             if (c < nc) {
@@ -235,8 +284,10 @@ __global__ __launch_bounds__(WG) void k_lattice_plain(LatArgs a)
     // reduce lane partials of the slot (lanes of a slot are contiguous)
 #pragma unroll
     for (int o = L / 2; o > 0; o >>= 1) {
-        trA.x += __shfl_xor(trA.x, o);
-        trA.y += __shfl_xor(trA.y, o);
+        if (L != 16) {  // (16: every lane has the slot's)
+            trA.x += __shfl_xor(trA.x, o);
+            trA.y += __shfl_xor(trA.y, o);
+        }
         if (MODE != MODE_FWD) {
             tr2A.x += __shfl_xor(tr2A.x, o);
             tr2A.y += __shfl_xor(tr2A.y, o);
