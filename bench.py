@@ -317,11 +317,11 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f32+f64" if args.method == "schur_f32r" else "f64",
+        "dtype": "f64",
         "data": "synthetic",
         "config": {"workload": WORKLOADS[args.workload],
                    "n": n, "n_corr": nc, "n_k": nk, "n_freq": nf, "beta": beta, "method": args.method,
-                   "refine_steps": args.refine, "schur_layout": args.layout, "schur_wg": args.wg or "default (adjoint 128, forward 64, FP32R forward below N_freq in k pairs)",
+                   "refine_steps": args.refine, "schur_layout": args.layout, "schur_wg": args.wg or "default (64 frequencies, k walk split where faster)",
                    "target_workgroups": args.target or "default",
                    "units_per_step": units,
                    "step": "tail-moment fit of Sigma + static eig for the tail + GreenFtn_w forward (G_loc, NumMatrix, "
@@ -428,7 +428,7 @@ def bench_batch(args, torch, capi, G, L):
     out = {
         "metric": METRIC, "value": units / sec, "unit": "(k,w) inversions/s",
         "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "ms_per_step": sec * 1e3, "higher_is_better": True,
-        "scaling": "weak", "vs_baseline": None, "dtype": "f32+f64" if method == G.SCHUR_F32R else "f64",
+        "scaling": "weak", "vs_baseline": None, "dtype": "f64",
         "data": "synthetic",
         "config": {"workload": WORKLOADS["batch64"], "systems": len(systems), "units_per_step": units,
                    "method": args.method, "refine_steps": args.refine,
@@ -595,7 +595,7 @@ def bench_path(args, torch, capi, G, L):
             per[name] = dict(value=units / t_wall, ms_per_call=t_wall * 1e3, gpu_ms=t_gpu * 1e3)
         head = args.method
         metric, unit, value = "real-axis (k,E) inversions/s (k-summed G^R)", "(k,E) inversions/s", per[head]["value"]
-        dtype = "f32+f64" if head == "schur_f32r" else "f64"
+        dtype = "f64"
         ach = f_fwd(n) * units / (per[head]["gpu_ms"] / 1e3) / 1e12
         roof = _flop_roofline(ach, "k_lattice_schur_cols<FWD> (real axis)" if head != "plain_f64" else
                               "k_lattice_plain<FWD> (real axis)", "algorithmic 8n^3 FLOPs per (k,E) x Nk*n_E / call "

@@ -187,10 +187,14 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
     cd* sTr = lds + M2 * FW;          // KS > 1: forward [FW] sums of the tr G shares
     cd* sGb = lds + M2 * FW;          //         adjoint [M2][FW] gbar, [M2][FW] Sigma
     cd* sSig = lds + 2 * M2 * FW;
+    // adjoint, KS > 1: the parts' sums of tr G, tr G^2 and the mu term
+    constexpr bool SUM_LDS = MODE == MODE_VJP && KS > 1;
+    cd* sSum = nullptr;
     const int lane = KS == 1 ? (int)threadIdx.x : (int)threadIdx.x % FW;  // this lane's frequency in the tile
     // which k of every KS: wave-uniform (FW is a multiple of 64), so that the k
     // walk and the per-k block addresses stay scalar
     const int part = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / FW);
+    if constexpr (SUM_LDS) sSum = lds + (SIG_LDS ? 3 : 2) * M2 * FW + 3 * part * FW + lane;
     const int nw_hi = n_points(a);
     const int nw = wtile * FW + lane;
     // a wavefront past the last point has no work (KS > 1: they meet at barriers, so
@@ -221,6 +225,7 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
         for (int e = 0; e < M2; ++e) sAcc[e * FW + lane] = cd{0.0, 0.0};
         if constexpr (KS > 1) {
             if constexpr (MODE == MODE_VJP) {
+                for (int q = 0; q < 3; ++q) sSum[q * FW] = cd{0.0, 0.0};
                 for (int e = part; e < M2; e += KS) {
                     sGb[e * FW + lane] = gb[e];
                     if constexpr (SIG_LDS) sSig[e * FW + lane] = sig[e];
@@ -479,6 +484,13 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                 }
 #pragma unroll
             for (int i = 0; i < NC; ++i) trG = cadd(trG, G[i][i]);
+            if constexpr (SUM_LDS) {  // out of the registers before the product
+                if (kin) {
+                    lds_add(&sSum[0], trG);
+                    lds_add(&sSum[FW], tz);
+                }
+                tz = cd{0.0, 0.0};
+            }
             // Z = G S' = G + G Y, column by column in place of Y
 #pragma unroll
             for (int j = 0; j < NC; ++j) {
@@ -505,7 +517,9 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                 }
                 tz = cadd(tz, cscale(off, 2.0));
             }
-            if (wvalid && kin) {
+            if constexpr (SUM_LDS) {
+                if (kin) lds_add(&sSum[FW], tz);
+            } else if (wvalid && kin) {
                 trA = cadd(trA, trG);
                 tr2A = cadd(tr2A, tz);
             }
@@ -525,20 +539,25 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                 };
                 auto column = [&](auto bc) {
                     constexpr int b = decltype(bc)::value;
-                    // gbar (then the sums) come NC entries ahead, each entry's registers
-                    // loaded again as soon as it is used: left to itself the compiler
-                    // reads one entry, waits and uses it, an LDS round trip per entry
-                    cd buf[NC], t[NC];
+                    // gbar (rows in turn, then the column's sums) comes AHEAD entries early, an
+                    // entry's registers loaded again as soon as it is used: left to itself the
+                    // compiler reads one entry, waits and uses it, an LDS round trip per entry
+                    constexpr int AHEAD = 3;
+                    auto fetch = [&](int q) -> cd {
+                        return q < M2 ? gbar_at(q / NC, q % NC) : sAcc[(q - M2 + b * NC) * FW + lane];
+                    };
+                    cd buf[AHEAD], t[NC];
 #pragma unroll
-                    for (int l = 0; l < NC; ++l) buf[l] = gbar_at(0, l);
+                    for (int q = 0; q < AHEAD; ++q) buf[q] = fetch(q);
                     barrier();
 #pragma unroll
                     for (int i = 0; i < NC; ++i) {
                         cd s = cd{0.0, 0.0};
 #pragma unroll
                         for (int l = 0; l < NC; ++l) {
-                            s = cfma(buf[l], cconj(G[b][l]), s);
-                            buf[l] = i + 1 < NC ? gbar_at(i + 1, l) : sAcc[(l + b * NC) * FW + lane];
+                            const int q = i * NC + l;
+                            s = cfma(buf[q % AHEAD], cconj(G[b][l]), s);
+                            buf[q % AHEAD] = fetch(q + AHEAD);
                             barrier();
                         }
                         ms = cfmac(s, Z[i][b], ms);
@@ -546,7 +565,8 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                     }
 #pragma unroll
                     for (int aa = 0; aa < NC; ++aa) {  // C_ab = sum_i conj(G_ia) t_i
-                        cd s = buf[aa];
+                        cd s = buf[(M2 + aa) % AHEAD];
+                        if (aa + AHEAD < NC) buf[(M2 + aa) % AHEAD] = fetch(M2 + aa + AHEAD);
 #pragma unroll
                         for (int i = 0; i < NC; ++i) s = cfmac(G[i][aa], t[i], s);
                         sAcc[(aa + b * NC) * FW + lane] = s;
@@ -566,7 +586,8 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                         __syncthreads();
                     }
                 }
-                if (vjp_here) muA = cadd(muA, ms);
+                if constexpr (SUM_LDS) lds_add(&sSum[2 * FW], ms);
+                else if (vjp_here) muA = cadd(muA, ms);
             }
         }
     }
@@ -577,18 +598,13 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
             __syncthreads();
             if (part != 0) return;
             trA = sTr[lane];
-        } else {  // (gbar is not needed any more)
-            __syncthreads();
-            cd* share = sGb + lane;
-            share[(3 * part) * FW] = trA;
-            share[(3 * part + 1) * FW] = tr2A;
-            share[(3 * part + 2) * FW] = muA;
+        } else {
             __syncthreads();
             if (part == 0)
-                for (int p = 1; p < KS; ++p) {
-                    trA = cadd(trA, share[(3 * p) * FW]);
-                    tr2A = cadd(tr2A, share[(3 * p + 1) * FW]);
-                    muA = cadd(muA, share[(3 * p + 2) * FW]);
+                for (int p = 0; p < KS; ++p) {
+                    trA = cadd(trA, sSum[3 * p * FW]);
+                    tr2A = cadd(tr2A, sSum[(3 * p + 1) * FW]);
+                    muA = cadd(muA, sSum[(3 * p + 2) * FW]);
                 }
         }
     }
@@ -657,10 +673,9 @@ template <int NC, int MODE, int WG, int KS = 1>
 constexpr size_t schur_shm()
 {
     constexpr bool ACC_LDS = MODE == MODE_VJP || KS > 1;
-    // KS > 1: one accumulator set per frequency, plus the tr G sums (forward) or gbar
-    // and Sigma, at the end the parts' three shares (adjoint)
-    constexpr int tables = (schur_sig_lds<NC>() ? 2 : 1) * NC * NC;
-    constexpr int extra = KS == 1 ? 0 : MODE != MODE_VJP ? 1 : tables > 3 * KS ? tables : 3 * KS;
+    // KS > 1: one accumulator set per frequency, plus the tr G sums (forward) or gbar,
+    // Sigma and the parts' three sums (adjoint)
+    constexpr int extra = KS == 1 ? 0 : MODE != MODE_VJP ? 1 : (schur_sig_lds<NC>() ? 2 : 1) * NC * NC + 3 * KS;
     return ACC_LDS ? sizeof(cd) * (size_t)(NC * NC + extra) * (WG / KS) : 0;
 }
 
