@@ -63,14 +63,14 @@ hipError_t launch_sigma_all(const LatArgs& a, hipStream_t s)
 // 0.80 / 0.91, 16 1.27 / 1.67; n_c = 4, n_d = 4 0.38 / 0.37, 6 0.44 / 0.45, 16 0.76 /
 // 0.87; n_c = 3, n_d = 9 0.33 / 0.35.  Real axis, 32768 k x 1000 points, n_c = 5,
 // n_d = 9: 2.84 / 3.35.
-// Adjoint (four wavefronts, at n_c = 6 two; gbar is in LDS and no longer in registers):
-// two wavefronts per SIMD at n_c = 4 and 5, no AGPR traffic at n_c = 6, against a barrier
-// per column.  n_c = 4, n_d = 0 0.55 / 0.58, 9 1.01 / 1.11, 18 1.60 / 1.89; n_c = 6, n_d =
-// 0 2.1 / 4.0, 9 3.7 / 5.5, 18 6.6 / 8.2; n_c = 5, n_d = 0 1.23 / 1.03, 9 1.79 / 1.79, 18
-// 2.68 / 3.04.
+// Adjoint (four wavefronts, at n_c = 6 two; gbar and the traces' sums are in LDS and no
+// longer in registers): two wavefronts per SIMD at n_c = 4 and 5, no AGPR traffic at
+// n_c = 6, against a barrier per column.  n_c = 4, n_d = 0 0.55 / 0.58, 9 1.01 / 1.11, 18
+// 1.60 / 1.89; n_c = 5, n_d = 0 1.09 / 1.10, 4 1.36 / 1.41, 9 1.62 / 1.81, 18 2.53 / 3.06;
+// n_c = 6, n_d = 0 2.1 / 4.0, 9 3.6 / 5.5, 18 6.5 / 8.2.
 bool schur_ksplit(int nc, int nd, int mode)
 {
-    if (mode == MODE_VJP) return nc == 4 || nc == 6 || (nc == 5 && nd >= 9);
+    if (mode == MODE_VJP) return nc >= 4 && nc <= 6;
     return mode == MODE_FWD && (nc == 6 || (nc >= 3 && nc <= 5 && nd >= 6));
 }
 

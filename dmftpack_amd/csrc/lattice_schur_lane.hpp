@@ -133,6 +133,8 @@ __host__ __device__ __forceinline__ int kblock_size(int nd)
 
 template <int NC>
 __host__ __device__ constexpr bool schur_sig_lds() { return NC <= 4; }
+template <int NC, int MODE, int KS>
+__host__ __device__ constexpr bool schur_sum_lds() { return (MODE == MODE_VJP && KS > 1) || (MODE == MODE_DENS && NC == 5); }
 
 template <int I>
 struct ColumnIndex {
@@ -187,14 +189,18 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
     cd* sTr = lds + M2 * FW;          // KS > 1: forward [FW] sums of the tr G shares
     cd* sGb = lds + M2 * FW;          //         adjoint [M2][FW] gbar, [M2][FW] Sigma
     cd* sSig = lds + 2 * M2 * FW;
-    // adjoint, KS > 1: the parts' sums of tr G, tr G^2 and the mu term
-    constexpr bool SUM_LDS = MODE == MODE_VJP && KS > 1;
+    // sums of tr G, tr G^2 and the mu term in LDS where registers are short (adjoint with
+    // KS > 1: one set a part)
+    constexpr bool SUM_LDS = schur_sum_lds<NC, MODE, KS>();
     cd* sSum = nullptr;
     const int lane = KS == 1 ? (int)threadIdx.x : (int)threadIdx.x % FW;  // this lane's frequency in the tile
     // which k of every KS: wave-uniform (FW is a multiple of 64), so that the k
     // walk and the per-k block addresses stay scalar
     const int part = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / FW);
-    if constexpr (SUM_LDS) sSum = lds + (SIG_LDS ? 3 : 2) * M2 * FW + 3 * part * FW + lane;
+    if constexpr (SUM_LDS) {
+        sSum = lds + (MODE == MODE_DENS ? 0 : SIG_LDS ? 3 : 2) * M2 * FW + 3 * part * FW + lane;
+        for (int q = 0; q < 3; ++q) sSum[q * FW] = cd{0.0, 0.0};
+    }
     const int nw_hi = n_points(a);
     const int nw = wtile * FW + lane;
     // a wavefront past the last point has no work (KS > 1: they meet at barriers, so
@@ -225,7 +231,6 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
         for (int e = 0; e < M2; ++e) sAcc[e * FW + lane] = cd{0.0, 0.0};
         if constexpr (KS > 1) {
             if constexpr (MODE == MODE_VJP) {
-                for (int q = 0; q < 3; ++q) sSum[q * FW] = cd{0.0, 0.0};
                 for (int e = part; e < M2; e += KS) {
                     sGb[e * FW + lane] = gb[e];
                     if constexpr (SIG_LDS) sSig[e * FW + lane] = sig[e];
@@ -608,6 +613,10 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                 }
         }
     }
+    if constexpr (SUM_LDS && KS == 1) {
+        trA = sSum[0];
+        tr2A = sSum[FW];
+    }
     if (!wvalid) return;
     const size_t ch = chunk;
     if (MODE == MODE_FWD || MODE == MODE_FWD_REAL) {
@@ -632,9 +641,10 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
     }
 }
 
-// Waves per SIMD the register allocator is held to.  At n_c = 5 the density kernel
-// needs a few registers more than the 256 of two waves; two waves with a few bytes
-// of scratch beat one.  KS > 1: as many as its LDS admits, without scratch.
+// Waves per SIMD the register allocator is held to: as many as fit without values
+// spilled in the k walk (at these rates a spilled value a lane is gigabytes of writes:
+// with 136 B of scratch the adjoint at n_c = 5 wrote 8 GB a launch, and the loss and
+// gradient of 32^3 k x 2048 frequencies took 20.5 ms against 18.4).
 template <int NC, int MODE, int KS>
 constexpr int schur_waves()
 {
@@ -672,6 +682,7 @@ void k_lattice_schur_multi(const LatArgs* __restrict__ args,
 template <int NC, int MODE, int WG, int KS = 1>
 constexpr size_t schur_shm()
 {
+    if (MODE == MODE_DENS) return schur_sum_lds<NC, MODE, KS>() ? sizeof(cd) * 3 * (size_t)WG : 0;
     constexpr bool ACC_LDS = MODE == MODE_VJP || KS > 1;
     // KS > 1: one accumulator set per frequency, plus the tr G sums (forward) or gbar,
     // Sigma and the parts' three sums (adjoint)
