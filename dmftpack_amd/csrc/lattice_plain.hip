@@ -73,10 +73,10 @@ __device__ __forceinline__ void trace_from_lanes(const cd (&col)[N], cd& tr, dou
     }
 }
 
-// Wavefronts per SIMD the register allocator is held to (a third pays for the forward and
-// the densities; the adjoint at n = 16 is faster with one or two and no spills)
+// Wavefronts per SIMD the register allocator is held to (a third pays for the forward; for
+// the densities it spills, 1.73 ms against 1.58 at n = 14, 1728 k x 1024 frequencies)
 template <int L, int N, int MODE>
-constexpr int plain_waves() { return L == 16 && N > 12 && MODE != MODE_VJP ? 3 : 1; }
+constexpr int plain_waves() { return L == 16 && N > 12 && MODE == MODE_FWD ? 3 : 1; }
 
 template <int N, int L, int MODE, int WG>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(plain_waves<L, N, MODE>()))) void k_lattice_plain(LatArgs a)
