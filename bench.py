@@ -13,8 +13,10 @@ once, with its Schur data eig(H_dd(k)), W = H_cd V_d, before timing):
             and the static eigen-decomposition of H(k) + P m0 P^H (:197-215)
   forward   GreenFtn_w: G_loc, NumMatrix and total N over Nk x 2 N_freq (k, iw)
   adjoint   VJP of L = sum_w ||G_loc - G_tgt||_F^2 + (N - N0)^2 -> dL/dSigma, dL/dmu
-value = Nk * 2 N_freq / step time, for the FP32 + FP64-refinement Schur method;
-the plain FP64 full-inverse path runs the same step for the ratio.
+value = Nk * 2 N_freq / step time, for the Schur method schur_f32r, which computes in
+FP64 and takes the density sums beyond N_freq at 16 Gauss points (the 2 N_freq
+units are those the step answers for); the plain FP64 full-inverse path, which
+inverts all of them, runs the same step for the ratio.
 """
 import argparse
 import json
@@ -72,8 +74,8 @@ def parse():
     ap.add_argument("--refine", type=int, default=1)
     ap.add_argument("--wg", type=int, default=0, choices=[0, 64, 128],
                     help="frequencies per workgroup of the Schur kernels (DMFTGPU_OPT_SCHUR_WG; 0 = the default "
-                         "of each launch: adjoint 128, FP32R forward below N_freq as two wavefronts splitting the k "
-                         "walk over 64 frequencies, the others 64)")
+                         "of each launch: 64, or two or four wavefronts over 64 frequencies splitting the k "
+                         "walk where that is faster)")
     ap.add_argument("--target", type=int, default=0,
                     help="work items per lattice launch, sets the k chunking (DMFTGPU_OPT_TARGET_WORKGROUPS; 0 = default)")
     ap.add_argument("--layout", type=int, default=0, choices=[0, 1],
@@ -219,15 +221,13 @@ def main():
             extra["plain_fp64_executed"] = plain_executed(others["plain_f64"], args.workload)
 
     # ---- roofline of the dominant kernel --------------------------------------
-    # On the one-matrix-per-lane Schur path dmftgpu_gloc_loss_grad is fused: the
-    # forward call is two launches (forward below N_freq; Hermitian-part forward +
-    # tr G^2 above), the adjoint call one launch over the first N_freq frequencies,
-    # which is the longest single launch of the step.  The library's events time
-    # each call's main launches on its own stream.
+    # The Schur methods solve the first N_freq frequencies and 16 Gauss points; the
+    # adjoint launch is the longest of the step.  The library's events time each
+    # call's main launch on its own stream.
     t_f, t_v = float(np.mean(kf)) / 1e3, float(np.mean(kv)) / 1e3
     fused = head != G.PLAIN_F64 and nc <= 6 and args.layout == 0
     if fused or t_v >= t_f:
-        kname = "k_lattice_schur<VJP> (first N_freq)" if fused else "k_lattice_schur<VJP>"
+        kname = "k_lattice_schur<VJP>"
         t_k, flop, pkey = t_v, f_adj(n, nc), ("VJP" if fused else "VJP_CALL")
         units_k = nk * nf if fused else units
     else:
@@ -274,7 +274,7 @@ def main():
                     plain_equivalent=plain_eq,
                     note="achieved = FLOPs the dominant kernel executes per launch (hardware counters, same kernel "
                          "and workload) / its live duration (HIP events on the library's stream); the kernels are "
-                         "FP64/FP32 VALU code (no MFMA), bound by the VALU issue rate, 78.6 TFLOP/s")
+                         "FP64 VALU code (no MFMA), 78.6 TFLOP/s at the full clock")
 
     # ---- CPU baseline: the oracle's GreenFtn_w on a k subset ---------------------
     cpu = None
@@ -597,7 +597,7 @@ def bench_path(args, torch, capi, G, L):
         metric, unit, value = "real-axis (k,E) inversions/s (k-summed G^R)", "(k,E) inversions/s", per[head]["value"]
         dtype = "f64"
         ach = f_fwd(n) * units / (per[head]["gpu_ms"] / 1e3) / 1e12
-        roof = _flop_roofline(ach, "k_lattice_schur_cols<FWD> (real axis)" if head != "plain_f64" else
+        roof = _flop_roofline(ach, "k_lattice_schur<FWD_REAL>" if head != "plain_f64" else
                               "k_lattice_plain<FWD> (real axis)", "algorithmic 8n^3 FLOPs per (k,E) x Nk*n_E / call "
                               "time (events)", f_fwd(n), units, plain_equivalent=head != "plain_f64")
         extra["methods"] = per
@@ -629,14 +629,15 @@ def bench_path(args, torch, capi, G, L):
         pairs = (ntau + 1) * nf
         units = 2 * pairs
         metric, unit, value = "(tau,iw) pairs/s, iw->tau->iw round trip", "(tau,w) pairs/s", units / t_wall
-        ach = 8.0 * d * d * units / t_gpu / 1e12
-        roof = _flop_roofline(ach, "k_dft_mfma<W2Tau> + k_dft_mfma<Tau2W>",
-                              "algorithmic 8 d^2 FLOPs (one complex MAC per element) per (tau,iw) pair and direction "
-                              "/ call time (events, both calls: moment-free transform kernels, tail, causality "
-                              "eigensolves); the two transforms are FP64 MFMA complex GEMMs (4 real "
-                              "v_mfma_f64_16x16x4 per complex step, d^2 padded to 16-element tiles)",
-                              8.0 * d * d, units)
-        roof["bound"] = "mfma"
+        ach = 2.0 * (nf + ntau + 1) * d * d * 16.0 / t_gpu / 1e9
+        roof = dict(bound="hbm", achieved=ach, peak=PEAK_HBM_GBS, unit="GB/s", frac=ach / PEAK_HBM_GBS, traffic=None,
+                    kernel="k_czt", bytes_per_unit=2.0 * (nf + ntau + 1) * d * d * 16.0 / units, units_per_launch=units,
+                    plain_equivalent=dict(flop_per_unit=8.0 * d * d, units_per_launch=units,
+                                          tflops=8.0 * d * d * units / t_gpu / 1e12,
+                                          note="the dense transforms' 8 d^2 FLOPs per (tau,iw) pair and direction over "
+                                               "the same time: a speed figure, the transforms being FFTs"),
+                    note="algorithmic bytes = both functions read and written once per round trip / call time "
+                         "(events, both calls: chirp-z transforms, tail, causality tests)")
         if not args.no_cpu:
             sig_np, mom_np = sig, mom
 
@@ -672,11 +673,10 @@ def bench_path(args, torch, capi, G, L):
         nbytes = nk * n * n * 16.0
         ach = nbytes / t_gpu / 1e9
         roof = dict(bound="hbm", achieved=ach, peak=PEAK_HBM_GBS, unit="GB/s", frac=ach / PEAK_HBM_GBS,
-                    traffic=None, kernel="k_hk_from_hr", bytes_per_unit=n * n * 16.0, units_per_launch=units,
+                    traffic=None, kernel="k_hr_phases + k_hk_dense", bytes_per_unit=n * n * 16.0, units_per_launch=units,
                     hops=len(hops),
                     note="algorithmic bytes = the H(k) written once (n^2 x 16 B per k) / call time (events, incl. "
-                         "the host grouping of the hops); each element also takes one FP64 sincos per hop, "
-                         "which sets the time")
+                         "the host grouping of the hops)")
         if not args.no_cpu:
             def run(kk):
                 O.hk_from_hr(n, hops, kp_np[:kk])
@@ -711,7 +711,7 @@ def bench_path(args, torch, capi, G, L):
         fl = 8.0 * (7 * no ** 3 + 2 * n ** 3) + 24.0 * nr
         metric, unit, value = "upfolded k points/s (D_k and the three R sums)", "k points/s", units / t_wall
         ach = fl * units / t_gpu / 1e12
-        roof = _flop_roofline(ach, "k_zgemm_sq / k_gj_inverse / k_dm_r", "algorithmic FLOPs per k: 8(7 n_orb^3 + "
+        roof = _flop_roofline(ach, "k_upfold_small / k_r_sums", "algorithmic FLOPs per k: 8(7 n_orb^3 + "
                               "2 n^3) for the products and inverses + 24 n_R for the R sums (sincos not counted) / "
                               "call time (events)", fl, units)
         if not args.no_cpu:

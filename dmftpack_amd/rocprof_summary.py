@@ -84,16 +84,13 @@ def lattice_mode(name):
         return None
     args = [x.strip() for x in m.group(2).split(",")]
     idx = 2 if m.group(1) == "plain" else 1
-    return {"0": "FWD", "1": "DENS", "2": "VJP", "3": "FWD_HERM", "4": "DENS_HERM", "5": "FWD_REAL"}.get(
+    return {"0": "FWD", "1": "DENS", "2": "VJP", "5": "FWD_REAL"}.get(
         args[idx] if len(args) > idx else "")
 
 
 def add_calls(d, keys):
-    """A forward or adjoint call of the one-matrix-per-lane Schur path can be more
-    than one launch: FWD below N_freq plus FWD_HERM or DENS_HERM (fused with the
-    adjoint's tr G^2) above; VJP below N_freq plus DENS above when not fused (the
-    bench step makes no other launch of those modes).  FWD_CALL and VJP_CALL sum them."""
-    for call, parts in (("FWD_CALL", ("FWD", "FWD_HERM", "DENS_HERM")), ("VJP_CALL", ("VJP", "DENS"))):
+    """The launches of a forward or an adjoint call (one each)."""
+    for call, parts in (("FWD_CALL", ("FWD",)), ("VJP_CALL", ("VJP",))):
         have = [m for m in parts if m in d]
         if have:
             d[call] = {k: sum(d[m][k] for m in have) for k in keys}
