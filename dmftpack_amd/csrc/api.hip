@@ -688,7 +688,8 @@ int forward_impl(dmftgpu_handle h, int method, const double* sigma, double mu, d
         HIPCHK(dg::launch_gloc_hf(h->ev, h->U, L.n, nc, L.n_k, L.n_freq, L.beta, mu, inv_nk, L.n_cluster, (cd*)gloc_hf,
                                   h->stream));
     // NumMatrix = [ (1/beta) sum_n sum_k (G_cc + G_cc^H) + sum_k (U w U^H)_cc ] / knum_mpiGlobal
-    HIPCHK(dg::launch_results(tot, st, sts, m2, L.beta, (double)L.n_k_global, (cd*)num_matrix, h->stream));
+    HIPCHK(dg::launch_results(tot, st, sts, m2, L.beta, (double)L.n_k_global, (cd*)num_matrix, n_total != nullptr,
+                              h->stream));
     cd res[32 * 32 + 3];  // NumMatrix, N (on the stack: n_corr <= 32)
     HIPCHK(hipMemcpyAsync(res, tot, sizeof(cd) * (m2 + 1), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
@@ -822,7 +823,7 @@ static int density_impl(dmftgpu_handle h, int method, const double* sigma, doubl
     rc = run_static(h, mu, &st, &sts, ws, off);
     if (rc) return rc;
     HIPCHK(dg::launch_freq_totals(nullptr, m2, nc, S.tr, S.tr2, nw_tot, nullptr, 0, tot, h->stream, S.pt_n, S.pt_wt));
-    HIPCHK(dg::launch_results(tot, st, sts, m2, L.beta, (double)L.n_k_global, nullptr, h->stream));
+    HIPCHK(dg::launch_results(tot, st, sts, m2, L.beta, (double)L.n_k_global, nullptr, false, h->stream));
     cd res[2];
     HIPCHK(hipMemcpyAsync(res, tot + m2, sizeof(res), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
@@ -917,7 +918,7 @@ int vjp_impl(dmftgpu_handle h, int method, const double* sigma, double mu, const
     const dg::FreqScale out{S.Sb, (cd*)sigma_bar, (size_t)L.n_freq * m2, nc, inv_nk};
     HIPCHK(dg::launch_freq_totals(nullptr, m2, nc, nullptr, S.tr2, nw_tot, S.mu, L.n_freq, tot, h->stream, S.pt_n,
                                   S.pt_wt, out));
-    HIPCHK(dg::launch_results(tot, st, sts, m2, L.beta, (double)L.n_k_global, nullptr, h->stream));
+    HIPCHK(dg::launch_results(tot, st, sts, m2, L.beta, (double)L.n_k_global, nullptr, false, h->stream));
     cd res[3];
     HIPCHK(hipMemcpyAsync(res, tot + m2, sizeof(res), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
@@ -980,7 +981,7 @@ static int jvp_impl(dmftgpu_handle h, int method, const double* sigma, double mu
     HIPCHK(dg::launch_adjoint_stack(S.Sb, (size_t)L.n_freq, nc, inv_nk, (cd*)dgloc, h->stream));
     HIPCHK(dg::launch_freq_totals(nullptr, m2, nc, nullptr, S.tr2, nw_tot, S.mu, L.n_freq, tot, h->stream, S.pt_n,
                                   S.pt_wt));
-    HIPCHK(dg::launch_results(tot, st, sts, m2, L.beta, (double)L.n_k_global, nullptr, h->stream));
+    HIPCHK(dg::launch_results(tot, st, sts, m2, L.beta, (double)L.n_k_global, nullptr, false, h->stream));
     cd res[3];
     HIPCHK(hipMemcpyAsync(res, tot + m2, sizeof(res), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));

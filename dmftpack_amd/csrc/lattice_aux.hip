@@ -366,30 +366,35 @@ hipError_t launch_freq_totals(const cd* G, int m2, int nc, const cd* tr, const c
 
 // The call's scalars and NumMatrix from the frequency totals and the static part, over
 // the totals (so that the host copies one array): entries q < m2 (with num) NumMatrix,
-// also to num; m2 N = (tr/beta + sum w)/n_k; m2+1 dN/dmu = (-tr2/beta + sum dN)/n_k;
-// m2+2 unchanged.
+// also to num unless the call will fail, with a value (or N, with check_n) that is not
+// finite; m2 N = (tr/beta + sum w)/n_k; m2+1 dN/dmu = (-tr2/beta + sum dN)/n_k; m2+2
+// unchanged.
 __global__ __launch_bounds__(1024) void k_results(cd* __restrict__ tot, const cd* __restrict__ st,
                                                   const double* __restrict__ sts, int m2, double beta, double n_k,
-                                                  cd* __restrict__ num)
+                                                  cd* __restrict__ num, bool check_n)
 {
     const int q = threadIdx.x;
     const double inv_nk = 1.0 / n_k;
+    const double N0 = tot[m2].x / beta + sts[0], N = num ? N0 / n_k : N0 * inv_nk;
+    cd v{};
     if (q < m2 && num) {
-        const cd v = cd{(tot[q].x / beta + st[q].x) * inv_nk, (tot[q].y / beta + st[q].y) * inv_nk};
+        v = cd{(tot[q].x / beta + st[q].x) * inv_nk, (tot[q].y / beta + st[q].y) * inv_nk};
         tot[q] = v;
-        num[q] = v;
     }
+    // (also the barrier between the reads of N's total and its overwriting)
+    const int ok = __syncthreads_and(isfinite(v.x) && isfinite(v.y) && (!check_n || isfinite(N)));
+    if (q < m2 && num && ok) num[q] = v;
     if (q == 0) {
-        const double N = tot[m2].x / beta + sts[0];
-        tot[m2].x = num ? N / n_k : N * inv_nk;
+        tot[m2].x = N;
         tot[m2 + 1].x = (-tot[m2 + 1].x / beta + sts[1]) * inv_nk;
     }
 }
 
 hipError_t launch_results(cd* tot, const cd* st, const double* sts, int m2, double beta, double n_k, cd* num,
-                          hipStream_t s)
+                          bool check_n, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_results, dim3(1), dim3(num ? (m2 + 63) / 64 * 64 : 64), 0, s, tot, st, sts, m2, beta, n_k, num);
+    hipLaunchKernelGGL(k_results, dim3(1), dim3(num ? (m2 + 63) / 64 * 64 : 64), 0, s, tot, st, sts, m2, beta, n_k, num,
+                       check_n);
     return hipGetLastError();
 }
 

@@ -324,7 +324,7 @@ hipError_t launch_freq_totals(const cd* G, int m2, int nc, const cd* tr, const c
 // NumMatrix (with num: into it and tot[0..m2)), N (tot[m2].x) and dN/dmu (tot[m2+1].x)
 // from the totals and the static part
 hipError_t launch_results(cd* tot, const cd* st, const double* sts, int m2, double beta, double n_k, cd* num,
-                          hipStream_t s);
+                          bool check_n, hipStream_t s);
 // out[m] = scale * in[m]^H over a stack of count d x d matrices (in != out)
 hipError_t launch_adjoint_stack(const cd* in, size_t count, int d, double scale, cd* out, hipStream_t s);
 // out[i] = in[i] * scale

@@ -54,3 +54,22 @@ def test_schur_forms(G, nc, nd, nf, target):
     g1, t1 = lat.greenftn_real(sr, mu, -3.0, 0.09, 0.05, method=G.SCHUR_F64)
     assert rel(g1, g0) <= 1e-11 and rel(t1, t0) <= 1e-11
     lat.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nc,bad", [(5, (0, 0)), (20, (19, 19))])
+@pytest.mark.parametrize("want_n", [True, False])
+def test_failed_call_leaves_num_matrix(G, nc, bad, want_n):
+    """A result that is not finite is an error, and the caller's NumMatrix keeps what it held
+    (one element of a block of nc^2 threads is enough to refuse all of them)."""
+    import torch
+    Hk = L.random_tb_hk(nc + 2, 2, nc)
+    sig, mom = L.pole_sigma(nc, 6, 20.0, nc)
+    lat = G.LatticeGF(Hk, nc, 6, 20.0, mom)
+    sig = sig.copy()
+    sig[(3,) + bad] = np.nan
+    num = torch.full((nc, nc), 7.0, dtype=torch.complex128, device="cuda")
+    with pytest.raises(Exception, match="not finite"):
+        lat.greenftn_w_dev(lat.sigma_dev(sig), 0.1, G.PLAIN_F64, num=num, want_n=want_n)
+    assert bool((num == 7.0).all())
+    lat.close()
