@@ -29,11 +29,12 @@ namespace dg {
 namespace {
 
 // Gauss rule of the measure with unit mass at each t_n = 1/(2n+1), n0 <= n < n1:
-// x[i] = 1/node (a real-valued "2n+1"), w[i] its weight.  Stieltjes recurrence, then
-// implicit QL on the 16 x 16 Jacobi matrix (first eigenvector row only).  The sums over
-// the measure take 8 partial sums, which vectorise: 83 us of host time at 2048
-// frequencies, in dmftgpu_prepare under the eigensolvers; node and weight errors of a
-// few 1e-16.
+// x[i] = 1/node (a real-valued "2n+1"), w[i] its weight.  Stieltjes recurrence to the
+// 16 x 16 Jacobi matrix; its eigenvalues, all at once, by bisection on Sturm counts
+// (Barth, Martin and Wilkinson, Numer. Math. 9, 386 (1967)); the weights are the
+// Christoffel numbers len / sum_k p_k(node)^2 (Golub and Welsch, Math. Comp. 23, 221
+// (1969)).  The sums over the measure take 8 partial sums, which vectorise: about 80 us of
+// host time at 2048 frequencies, in dmftgpu_prepare under the eigensolvers.
 void gauss_rule(int n0, int n1, double* x, double* w)
 {
     constexpr int m = kGaussPoints, V = 8;
@@ -46,7 +47,7 @@ void gauss_rule(int n0, int n1, double* x, double* w)
         s[i] = ((t - lo) - (hi - t)) / (hi - lo);
         p1[i] = 1.0 / std::sqrt((double)len);
     }
-    double d[m], e[m], z[m], beta = 0.0;
+    double d[m], e[m], beta = 0.0;
     for (int k = 0; k < m; ++k) {
         double sa[V] = {}, sn[V] = {};
         for (int i = 0; i < lv; i += V)
@@ -63,52 +64,41 @@ void gauss_rule(int n0, int n1, double* x, double* w)
         for (int i = 0; i < lv; ++i) p1[i] /= beta;
         d[k] = al;
         e[k] = beta;
-        z[k] = k == 0 ? 1.0 : 0.0;
     }
-    e[m - 1] = 0.0;
-    for (int l = 0; l < m; ++l) {  // implicit QL, Wilkinson shift
-        for (int it = 0; it < 60; ++it) {
-            int q = l;
-            for (; q < m - 1; ++q)
-                if (std::fabs(e[q]) <= 1e-17 * (std::fabs(d[q]) + std::fabs(d[q + 1]))) break;
-            if (q == l) break;
-            double g = (d[l + 1] - d[l]) / (2.0 * e[l]);
-            double r = std::hypot(g, 1.0);
-            g = d[q] - d[l] + e[l] / (g + (g >= 0.0 ? r : -r));
-            double sn = 1.0, cs = 1.0, p = 0.0;
-            int i = q - 1;
-            for (; i >= l; --i) {
-                double f = sn * e[i];
-                const double b = cs * e[i];
-                r = std::hypot(f, g);
-                e[i + 1] = r;
-                if (r == 0.0) {
-                    d[i + 1] -= p;
-                    e[q] = 0.0;
-                    break;
-                }
-                sn = f / r;
-                cs = g / r;
-                g = d[i + 1] - p;
-                r = (d[i] - g) * sn + 2.0 * cs * b;
-                p = sn * r;
-                d[i + 1] = g + p;
-                g = cs * r - b;
-                f = z[i + 1];
-                z[i + 1] = sn * z[i] + cs * f;
-                z[i] = cs * z[i] - sn * f;
+    double lower[m], upper[m];  // node j has j eigenvalues above it
+    for (int j = 0; j < m; ++j) {
+        lower[j] = -1.0;
+        upper[j] = 1.0;
+    }
+    for (int it = 0; it < 54; ++it) {
+        double mid[m], q[m], above[m];
+        for (int j = 0; j < m; ++j) {
+            mid[j] = 0.5 * (lower[j] + upper[j]);
+            q[j] = d[0] - mid[j];
+            above[j] = q[j] > 0.0 ? 1.0 : 0.0;
+        }
+        for (int k = 1; k < m; ++k)
+            for (int j = 0; j < m; ++j) {  // pivots of T - mid; a zero one passes as +-infinity
+                q[j] = d[k] - mid[j] - e[k - 1] * e[k - 1] / q[j];
+                above[j] += q[j] > 0.0 ? 1.0 : 0.0;
             }
-            if (r == 0.0 && i >= l) continue;
-            d[l] -= p;
-            e[l] = g;
-            e[q] = 0.0;
+        for (int j = 0; j < m; ++j) {
+            const bool right = above[j] > j;
+            lower[j] = right ? mid[j] : lower[j];
+            upper[j] = right ? upper[j] : mid[j];
         }
     }
-    double zz = 0.0;
-    for (int i = 0; i < m; ++i) zz += z[i] * z[i];
-    for (int i = 0; i < m; ++i) {
-        x[i] = 2.0 / (d[i] * (hi - lo) + hi + lo);
-        w[i] = z[i] * z[i] / zz * len;
+    for (int j = 0; j < m; ++j) {
+        const double node = 0.5 * (lower[j] + upper[j]);
+        double pa = 0.0, pb = 1.0, sum = 1.0;
+        for (int k = 0; k + 1 < m; ++k) {
+            const double pc = ((node - d[k]) * pb - (k ? e[k - 1] : 0.0) * pa) / e[k];
+            pa = pb;
+            pb = pc;
+            sum += pc * pc;
+        }
+        x[j] = 2.0 / (node * (hi - lo) + hi + lo);
+        w[j] = len / sum;
     }
 }
 
