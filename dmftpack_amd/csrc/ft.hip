@@ -996,8 +996,10 @@ static void tail_setup(int d, const std::vector<hl::cx>& m1, const std::vector<h
     A2 = mul(d, VH, U);
 }
 
-// The two-pole tail on the device, one copy
+// The two-pole tail on the device, one copy from host, which the caller keeps until it has
+// waited for the stream
 struct TailDev {
+    std::vector<double> host;
     const cd *A1, *A2;
     const double *e1, *e2;
 };
@@ -1005,16 +1007,22 @@ struct TailDev {
 static TailDev tail_upload(dmftgpu_handle h, int d, const std::vector<hl::cx>& A1, const std::vector<double>& e1,
                            const std::vector<hl::cx>& A2, const std::vector<double>& e2, Carve& cv, int* rc)
 {
-    const int m2 = d * d;
-    std::vector<double> host((size_t)4 * m2 + 2 * d);
-    std::memcpy(host.data(), A1.data(), sizeof(cd) * m2);
-    std::memcpy(host.data() + 2 * m2, A2.data(), sizeof(cd) * m2);
-    std::memcpy(host.data() + 4 * m2, e1.data(), sizeof(double) * d);
-    std::memcpy(host.data() + 4 * m2 + d, e2.data(), sizeof(double) * d);
-    double* dev = cv.take<double>(host.size());
-    const hipError_t e = hipMemcpyAsync(dev, host.data(), sizeof(double) * host.size(), hipMemcpyHostToDevice, h->stream);
+    const size_t m2 = (size_t)d * d;
+    TailDev t;
+    t.host.resize(4 * m2 + 2 * d);
+    double* dev = cv.take<double>(t.host.size());
+    auto put = [&](size_t at, const void* src, size_t count) {
+        std::memcpy(t.host.data() + at, src, sizeof(double) * count);
+        return dev + at;
+    };
+    t.A1 = (const cd*)put(0, A1.data(), 2 * m2);
+    t.A2 = (const cd*)put(2 * m2, A2.data(), 2 * m2);
+    t.e1 = put(4 * m2, e1.data(), d);
+    t.e2 = put(4 * m2 + d, e2.data(), d);
+    const hipError_t e =
+        hipMemcpyAsync(dev, t.host.data(), sizeof(double) * t.host.size(), hipMemcpyHostToDevice, h->stream);
     if (e != hipSuccess) *rc = fail(h, DMFTGPU_ERR_HIP, "tail upload: %s", hipGetErrorString(e));
-    return TailDev{(const cd*)dev, (const cd*)(dev + 2 * m2), dev + 4 * m2, dev + 4 * m2 + d};
+    return t;
 }
 
 // Tables of the chirp-z form for n_tau, kept in the handle for the last n_tau
