@@ -362,12 +362,10 @@ struct Plan {
 };
 
 // Work items per lattice launch that set the k chunking: the option's value,
-// or by default 32768 for the one-matrix-per-lane Schur kernels (their
-// forward is capped by LDS or registers at 6-8 wavefronts per CU, and shorter
-// k walks over more workgroups keep the CUs fuller: 24.0 -> 21.4 ms for the
-// config-2 forward call), but no fewer than 64 k per chunk (the per-chunk
-// partial sums grow with the chunk count: with 1000 real-axis energies 16 k
-// per chunk made the call 25% slower), and 8192 for the others.
+// or by default 32768 for the one-matrix-per-lane Schur kernels (shorter k walks over
+// more workgroups leave less of a last wave), but no fewer than 64 k per chunk (the
+// per-chunk partial sums grow with the chunk count: with 1000 real-axis energies 16 k
+// per chunk made the call 25% slower) above 8192, and 8192 for the others.
 int lattice_target(dmftgpu_handle h, int method, int nc, bool cols, int nk, int nw_tot, int slots)
 {
     if (h->target_wg > 0) return h->target_wg;
@@ -377,13 +375,15 @@ int lattice_target(dmftgpu_handle h, int method, int nc, bool cols, int nk, int 
     return (int)std::max(8192L, std::min(32768L, cap));
 }
 
-Plan make_plan(int nk, int nw_tot, int slots, int target_wg)
+// parts: wavefronts that split a chunk's k walk, which k_per_chunk is a multiple of
+Plan make_plan(int nk, int nw_tot, int slots, int target_wg, int parts = 1)
 {
     const int n_wt = (nw_tot + slots - 1) / slots;
     int chunks = (target_wg + n_wt - 1) / n_wt;
     if (chunks < 1) chunks = 1;
     if (chunks > nk) chunks = nk;
     int kpc = (nk + chunks - 1) / chunks;
+    kpc = (kpc + parts - 1) / parts * parts;
     chunks = (nk + kpc - 1) / kpc;
     return Plan{chunks, kpc};
 }
@@ -519,11 +519,14 @@ int run_lattice(dmftgpu_handle h, int method, int mode, const double* sigma, dou
     else slots = dg::schur_slots(nc, h->schur_layout == 1 || (ra && mode != dg::MODE_FWD));
     const bool cols = h->schur_layout == 1 || (ra && mode != dg::MODE_FWD);
     const int nw_plan = plan_points(h, method, ra);
-    Plan P = pk ? Plan{nk, 1} : make_plan(nk, nw_plan, slots, lattice_target(h, method, nc, cols, nk, nw_plan, slots));
-    if (max_chunks > 0 && P.n_chunks > max_chunks) {  // partial sums held to a fixed scratch size
-        const int kpc = (nk + max_chunks - 1) / max_chunks;
-        P = Plan{(nk + kpc - 1) / kpc, kpc};
-    }
+    const int form = method == DMFTGPU_PLAIN_F64 || cols || nc > 6 ? 64
+                     : h->schur_wg ? h->schur_wg
+                                   : dg::schur_form(nc, n - nc, mode, ra != nullptr, pk != nullptr, nk, nw_plan);
+    const int parts = form == dg::SCHUR_WG_KSPLIT ? dg::schur_parts(nc, mode) : 1;
+    Plan P = pk ? Plan{nk, 1}
+                : make_plan(nk, nw_plan, slots, lattice_target(h, method, nc, cols, nk, nw_plan, slots), parts);
+    if (max_chunks > 0 && P.n_chunks > max_chunks)  // partial sums held to a fixed scratch size
+        P = make_plan(nk, 1, 1, max_chunks, parts);
     dg::LatArgs a{};
     a.Hk = h->Hk;
     a.sigma = (const cd*)sigma;
@@ -589,9 +592,7 @@ int run_lattice(dmftgpu_handle h, int method, int mode, const double* sigma, dou
     if (method == DMFTGPU_PLAIN_F64) {
         HIPCHK(dg::launch_lattice_plain(a, mode, h->stream, nullptr));
     } else {
-        // schur_wg 0: each launch at its default width (launch_lattice_schur)
-        HIPCHK(dg::launch_lattice_schur(a, mode, h->stream, h->schur_wg,
-                                        h->schur_layout == 1));
+        HIPCHK(dg::launch_lattice_schur(a, mode, h->stream, form, h->schur_layout == 1));
     }
     if (h->timing) {
         HIPCHK(hipEventRecord(h->ev1[mode], h->stream));

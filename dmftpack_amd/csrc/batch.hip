@@ -136,16 +136,13 @@ namespace {
 // rough per-(k, iw) cost of the Schur work, for k chunking
 double lane_cost(int nc, int nd) { return 8.0 * nd * nc * (nc + 1) / 2 + 10.0 * nc * nc * nc + 100.0; }
 
-int plan_chunks(const Sys& s, double target, int* kpc)
+// parts: wavefronts that split a chunk's k walk, which *kpc is a multiple of
+int plan_chunks(const Sys& s, double target, int parts, int* kpc)
 {
     int k = (int)std::max(1.0, std::floor(target / lane_cost(s.nc, s.nd)));
-    if (k > s.nk) k = s.nk;
-    int chunks = (s.nk + k - 1) / k;
-    if (chunks > s.max_chunks) {
-        chunks = s.max_chunks;
-        k = (s.nk + chunks - 1) / chunks;
-        chunks = (s.nk + k - 1) / k;
-    }
+    k = std::max(std::min(k, s.nk), (s.nk + s.max_chunks - 1) / s.max_chunks);
+    k = (k + parts - 1) / parts * parts;
+    const int chunks = (s.nk + k - 1) / k;
     *kpc = k;
     return chunks;
 }
@@ -196,7 +193,8 @@ int build_group(dmftgpu_batch_s* b, Group& g, int mode, int wg, double target)
     for (size_t q = 0; q < g.systems.size(); ++q) {
         Sys& s = b->sys[g.systems[q]];
         int kpc;
-        const int chunks = plan_chunks(s, target, &kpc);
+        const int chunks =
+            plan_chunks(s, target, wg == dg::SCHUR_WG_KSPLIT ? dg::schur_parts(s.nc, mode) : 1, &kpc);
         if (mode == MODE_FWD) {
             s.chunks_f = chunks;
             s.kpc_f = kpc;
@@ -566,7 +564,10 @@ static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system
     for (Group& g : b->groups) {
         for (int mode : {MODE_FWD, MODE_VJP}) {
             if (mode == MODE_VJP && !b->vjp) continue;
-            const int wg0 = ksplit_ok(g, mode) && dg::schur_ksplit(g.nc, g.max_nd, mode) ? dg::SCHUR_WG_KSPLIT : 64;  // as the single-lattice default
+            long items = 0;
+            for (int q : g.systems) items += (long)b->sys[q].nk * ((b->sys[q].n_plan + 63) / 64);
+            // as the single-lattice default
+            const int wg0 = !g.cols && dg::schur_ksplit(g.nc, g.max_nd, mode, items) ? dg::SCHUR_WG_KSPLIT : 64;
             rc = (flags & DMFTGPU_BATCH_TUNE) ? 0 : build_group(b, g, mode, wg0, 1.0e6);
             if (rc) return rc;
         }

@@ -197,14 +197,17 @@ bool density_lr_supported(int n, int nc);
 hipError_t launch_density_matrix_lr(const LatArgs& a, const cd* W, const cd* Vd, const double* ed, const cd* U,
                                     const double* wt, cd* dens, hipStream_t s);
 
-// Schur complement; wg = width of the one-matrix-per-lane kernels: 64 or 128 frequencies
-// per workgroup, SCHUR_WG_KSPLIT (forward at n_c >= 3, adjoint at n_c >= 4), or 0 for the
-// default (schur_ksplit, else 64); cols selects the column-per-lane kernels for n_c <= 6
-// (always used above 6).
-// SCHUR_WG_KSPLIT: several wavefronts over 64 frequencies, each walking every second (or
+// Schur complement; wg = form of the one-matrix-per-lane kernels (schur_form): 64 or 128
+// frequencies per workgroup or SCHUR_WG_KSPLIT (forward at n_c >= 3, adjoint at n_c >= 4); cols
+// selects the column-per-lane kernels for n_c <= 6 (always used above 6).
+// SCHUR_WG_KSPLIT: schur_parts wavefronts over 64 frequencies, each walking every second (or
 // fourth) k of the chunk into shared LDS sums; its work items cover 64 frequencies
 constexpr int SCHUR_WG_KSPLIT = 1;
-bool schur_ksplit(int nc, int nd, int mode);
+constexpr int schur_parts(int nc, int mode) { return mode == MODE_VJP && nc < 6 ? 4 : 2; }
+// whether the split form is the faster one for a launch of items (k, tile of 64 points) pairs
+bool schur_ksplit(int nc, int nd, int mode, long items);
+// the form for a launch over nk k and n_pts points (per_k: one k per workgroup)
+int schur_form(int nc, int nd, int mode, bool real_axis, bool per_k, int nk, int n_pts);
 hipError_t launch_lattice_schur(const LatArgs& a, int mode, hipStream_t s, int wg = 64, bool cols = false);
 // Sigma expanded over all frequency points into a.pSigAll
 hipError_t launch_sigma_all(const LatArgs& a, hipStream_t s);

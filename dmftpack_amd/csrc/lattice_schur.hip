@@ -41,6 +41,10 @@ __global__ void k_sigma_all(LatArgs a)
     const int m2 = a.nc * a.nc;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int nw = t / m2, e = t % m2;
+    if (nw < a.n_freq) {  // (n_freq <= *pt_n; on the real axis every point)
+        a.pSigAll[t] = a.sigma[t];
+        return;
+    }
     if (nw >= n_points(a)) return;
     const double w = a.pt_w ? a.pt_w[nw] : matsubara(nw, a.beta);
     a.pSigAll[t] = sigma_elem_at(a.sigma, a.mom, a.nc, a.n_freq, w, nw, e % a.nc, e / a.nc);
@@ -68,15 +72,40 @@ hipError_t launch_sigma_all(const LatArgs& a, hipStream_t s)
 // n_c = 6, against a barrier per column.  n_c = 4, n_d = 0 0.55 / 0.58, 9 1.01 / 1.11, 18
 // 1.60 / 1.89; n_c = 5, n_d = 0 1.09 / 1.10, 4 1.36 / 1.41, 9 1.62 / 1.81, 18 2.53 / 3.06;
 // n_c = 6, n_d = 0 2.1 / 4.0, 9 3.6 / 5.5, 18 6.5 / 8.2.
-bool schur_ksplit(int nc, int nd, int mode)
+// The figures above are for chunks of many k.  A part with no k of its own repeats one, so the
+// chunks are multiples of schur_parts (17 k in four parts, adjoint of n = 10, n_c = 4, 4096 k x
+// 1040 points: 450 us, 20 k 408; alone 395 to 406), and there must be 256 workgroups of such chunks, one
+// to a CU: below that a wavefront for each k ends sooner.  Adjoint of n = 14, n_c = 5, split at four k a
+// chunk / alone at one k, us: 64 k x 216 points 27.6 / 25.0, 343 k x 216 39.1 / 49.3, 512 k x 116
+// 30.6 / 34.8, 512 k x 272 58 / 64 (one k a chunk, split: 120); forward, two k: 64 k x 80 18.8 / 18.4,
+// 64 k x 216 19.9 / 20.1, 512 k x 116 27.7 / 30.0.
+bool schur_ksplit(int nc, int nd, int mode, long items)
 {
+    if (items < 256L * schur_parts(nc, mode)) return false;
     if (mode == MODE_VJP) return nc >= 4 && nc <= 6;
     return mode == MODE_FWD && (nc == 6 || (nc >= 3 && nc <= 5 && nd >= 6));
 }
 
+// Real axis, split or else at 128 points per workgroup (the second wavefront finds the k block in
+// the scalar cache) unless that pads a tile more than 64 does: n = 14, n_c = 5, 4096 k x 1000
+// energies, 128 / 64: 0.454 / 0.474 ms; 1728 k x 400, four tiles of 128 against seven of 64: 0.154 /
+// 0.140.  Up to 4096 wavefronts the padding costs nothing (n = 20, n_c = 5, 512 k x 300: 54 / 57 us).
+// Summed over k, 64 is no slower at n_c >= 4 (n = 5: 0.217 / 0.212 ms at 4096 k x 1000).
+// One k per workgroup (per_k: band spectra): a second part would only repeat it, which cost
+// n = 14, n_c = 5, 216 k x 1000 60.6 us against 48.5 at 128; n_c = 6 with few d orbitals alone
+// gains from the registers the split form saves (n = 6, 4096 k x 1000: 0.87 ms, 64 0.94, 128 1.00).
+int schur_form(int nc, int nd, int mode, bool real_axis, bool per_k, int nk, int n_pts)
+{
+    const long tiles = (n_pts + 63) / 64, items = nk * tiles;
+    if (per_k ? nc == 6 && nd < 2 : schur_ksplit(nc, nd, mode, items)) return SCHUR_WG_KSPLIT;
+    if (!real_axis) return 64;
+    if (items < 4096) return 128;
+    if (tiles % 2) return 64;
+    return per_k ? (nc == 6 && nd < 4 ? 64 : 128) : (nc <= 3 ? 128 : 64);
+}
+
 hipError_t launch_lattice_schur(const LatArgs& a, int mode, hipStream_t s, int wg, bool cols)
 {
-    if (wg == 0) wg = schur_ksplit(a.nc, a.n - a.nc, mode) ? SCHUR_WG_KSPLIT : 64;
     hipError_t e = launch_sigma_all(a, s);
     if (e != hipSuccess) return e;
     if (a.real_axis && mode == MODE_FWD && a.nc <= 6 && !cols)

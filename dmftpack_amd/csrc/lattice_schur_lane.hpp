@@ -718,7 +718,7 @@ hipError_t launch_nc(const LatArgs& a, const cd* sig_all, hipStream_t s, int wg,
         if (wg == SCHUR_WG_KSPLIT) return launch_nc_w<NC, MODE, TRACE, 128, 2>(a, sig_all, s, m);
     }
     if constexpr (NC >= 4 && MODE == MODE_VJP) {  // four, or at n_c = 6 two
-        constexpr int KS = NC == 6 ? 2 : 4;
+        constexpr int KS = schur_parts(NC, MODE_VJP);
         if (wg == SCHUR_WG_KSPLIT) return launch_nc_w<NC, MODE, TRACE, 64 * KS, KS>(a, sig_all, s, m);
     }
     if (wg == 128) return launch_nc_w<NC, MODE, TRACE, 128>(a, sig_all, s, m);

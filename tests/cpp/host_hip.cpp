@@ -4,6 +4,7 @@
 // freed or written before that wait is counted as stale).  Loaded with RTLD_GLOBAL before
 // libdmftgpu.so, whose HIP calls then resolve here (tests/host_hip.py).
 #include <cxxabi.h>
+#include <sys/mman.h>
 #include <sys/uio.h>
 #include <unistd.h>
 
@@ -100,12 +101,13 @@ void host_hip_reset()
 }
 void* host_hip_alloc(size_t bytes)
 {
-    char* p = (char*)calloc(1, bytes ? bytes : 1);
-    if (p) {
-        blocks[p] = bytes;
-        in_use += bytes;
-        if (in_use > peak) peak = in_use;
-    }
+    if (!bytes) bytes = 1;
+    // pages that nothing touches take no memory, so sizes of a GPU's memory can be asked for
+    void* p = mmap(nullptr, bytes, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+    if (p == MAP_FAILED) return nullptr;
+    blocks[(char*)p] = bytes;
+    in_use += bytes;
+    if (in_use > peak) peak = in_use;
     return p;
 }
 
@@ -121,8 +123,8 @@ int hipFree(void* p)
     auto it = blocks.find((const char*)p);
     if (it == blocks.end()) return p ? 1 : 0;
     in_use -= it->second;
+    munmap(p, it->second);
     blocks.erase(it);
-    free(p);
     return 0;
 }
 int hipMemcpy(void* dst, const void* src, size_t bytes, int) { return copy(dst, src, bytes, nullptr, false); }

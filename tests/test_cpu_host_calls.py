@@ -20,3 +20,51 @@ mom = rt.dev(np.stack([np.zeros((d, d)), np.eye(d), 0.1 * np.eye(d), np.eye(d)])
 ])
 def test_tail_copy_source_outlives_the_copy(call):
     assert host_hip.run(FT + f"rt.reset()\nrt.check(h, {call})\nresult = rt.stale()") == 0
+
+
+SPLIT = r"""
+import ctypes as C, re
+def forms(nk):
+    out = []
+    for name, grid, block in rt.launches():
+        m = re.match(r"void dg::k_lattice_schur<(\d+), (\d+), (\d+), \w+, (\d+)>", name)
+        if m:
+            mode, parts, chunks = int(m[2]), int(m[4]), grid[1]
+            out.append((mode, int(m[3]) // parts, parts, -(-nk // chunks), chunks * grid[0]))
+    return out
+result = []
+for nc, nd in ((3, 6), (4, 0), (4, 6), (5, 0), (5, 9), (6, 0), (6, 8)):
+    for nk, nf in ((64, 64), (512, 64), (512, 256), (1000, 512), (1728, 512), (4096, 512)):
+        h = rt.handle()
+        rt.prepare(h, nc + nd, nc, nk, nf)
+        s, g, num = rt.dev(16 * nf * nc * nc), rt.dev(16 * nf * nc * nc), rt.dev(16 * nc * nc)
+        rt.reset()
+        call
+        result.append((nc, nd, nk, nf, forms(nk)))
+        rt.lib.dmftgpu_destroy(h)
+"""
+
+
+def test_split_walk_has_a_k_for_every_wavefront():
+    """Matsubara forward and adjoint, real axis summed: where wavefronts split a chunk's k walk, the
+    chunks are multiples of their number and there are 256 workgroups of them"""
+    calls = ["rt.check(h, rt.lib.dmftgpu_gloc_loss_grad(h, 1, s, 0.1, g, 1.0, g, num, None, None, s, None))",
+             "rt.check(h, rt.lib.dmftgpu_greenftn_real(h, 1, nf, -1.0, 0.01, 0.05, s, 0.1, g, None))"]
+    seen = set()
+    for call in calls:
+        for nc, nd, nk, nf, forms in host_hip.run(SPLIT.replace("call", call)):
+            assert forms, (nc, nd, nk, nf)
+            for mode, width, parts, per_chunk, groups in forms:
+                assert width in (64, 128)
+                if parts > 1:
+                    assert per_chunk % parts == 0 and groups >= 256, (nc, nd, nk, nf, mode, parts, per_chunk, groups)
+                seen.add((mode, parts))
+    # adjoint in four, in two (n_c = 6) and alone, forward and real axis in two and alone
+    assert seen >= {(2, 4), (2, 2), (2, 1), (0, 2), (0, 1), (5, 2), (5, 1)}
+
+
+def test_band_spectra_do_no_k_twice():
+    """one k per workgroup: no split walk, but for n_c = 6 without (many) d orbitals, which gains from it"""
+    call = "rt.check(h, rt.lib.dmftgpu_greenftn_real_k(h, 1, nf, -1.0, 0.01, 0.05, s, 0.1, rt.dev(16 * nk * nf * nc * nc), None))"
+    for nc, nd, nk, nf, forms in host_hip.run(SPLIT.replace("call", call)):
+        assert [f[2] for f in forms] == [2 if nc == 6 and nd < 2 else 1], (nc, nd, nk, nf, forms)
