@@ -117,7 +117,6 @@ extern "C" int dmftgpu_destroy(dmftgpu_handle h)
     h->prep.release();
     h->stat.release();
     h->static_cache.release();
-    h->tail_dev.release();
     h->cot.release();
     h->core.release();
     delete h;
@@ -128,8 +127,9 @@ extern "C" int dmftgpu_set_stream(dmftgpu_handle h, void* stream)
 {
     (void)hipGetLastError();  // drop an error left by an earlier failed call
     if (!h) return DMFTGPU_ERR_ARG;
+    // the transforms' tables were formed on the previous stream
+    if (h->stream != (hipStream_t)stream) h->czt_n = 0;
     h->stream = (hipStream_t)stream;
-    h->czt_n = 0;  // formed on the previous stream
     return DMFTGPU_OK;
 }
 
@@ -211,10 +211,10 @@ static int check_lattice(dmftgpu_handle h, const dmftgpu_lattice* L)
 static int set_points(dmftgpu_handle h)
 {
     const dmftgpu_lattice& L = h->lat;
-    const int nw_tot = L.n_freq * L.high_freq, n_tail = (int)h->tail.size() / 2;
-    h->n_plan = n_tail ? L.n_freq + n_tail : nw_tot;
-    HIPCHK(dg::launch_freq_points(h->mom, L.n_corr, L.n_freq, nw_tot, n_tail, (const double*)h->tail_dev.ptr, L.beta,
-                                  h->pt_n, h->pt_w, h->pt_wt, h->stream));
+    const int nw_tot = L.n_freq * L.high_freq;
+    h->n_plan = h->tail->empty() ? nw_tot : L.n_freq + (int)h->tail->size() / 2;
+    HIPCHK(dg::launch_freq_points(h->mom, L.n_corr, L.n_freq, nw_tot, *h->tail, L.beta, h->pt_n, h->pt_w, h->pt_wt,
+                                  h->stream));
     return DMFTGPU_OK;
 }
 
@@ -267,18 +267,8 @@ extern "C" int dmftgpu_prepare(dmftgpu_handle h, const dmftgpu_lattice* L, const
         if (lane_kernels) HIPCHK(dg::launch_schur_kdata(h->Hk, h->W, h->ed, n, nc, nk, h->kdata, h->stream));
         h->schur_ready = true;
     }
-    // (after the launches above: the host forms the rule while they run)
-    if (h->tail_nf != L->n_freq || h->tail_tot != (int)nw_tot) {
-        h->tail_nf = 0;  // valid again once the copy below is in place
-        h->tail = dg::freq_tail(L->n_freq, (int)nw_tot);
-        if (!h->tail.empty()) {
-            void* t = h->tail_dev.get(h->tail.size() * sizeof(double), &e);
-            if (!t) return fail(h, DMFTGPU_ERR_HIP, "frequency rule: %s", hipGetErrorString(e));
-            HIPCHK(hipMemcpyAsync(t, h->tail.data(), h->tail.size() * sizeof(double), hipMemcpyHostToDevice, h->stream));
-        }
-        h->tail_nf = L->n_freq;
-        h->tail_tot = (int)nw_tot;
-    }
+    // (after the launches above: where the host has to form the rule, it does so while they run)
+    h->tail = dg::freq_tail(L->n_freq, (int)nw_tot);
     if ((rc = set_points(h))) return rc;
     h->core_n_orb = 0;  // Kohn-Sham bands belong to the previous H(k)
     h->prepared = true;

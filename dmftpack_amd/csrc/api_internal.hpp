@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -45,11 +46,9 @@ struct dmftgpu_handle_s {
     dg::cd* Vd = nullptr;    // [nk][nd][nd]
     dg::cd* W = nullptr;     // [nk][nc][nd] H_cd V_d
     dg::cd* kdata = nullptr; // [nk][H_cc | P_d pairs | e_d] of the one-matrix-per-lane Schur kernels
-    // frequency points of the density sums (freq_points.hip): the rule beyond n_freq for
-    // the last (n_freq, high_freq n_freq), and the table for the bound moments
-    int tail_nf = 0, tail_tot = 0;
-    std::vector<double> tail;  // [x..., weight...]
-    dgi::Workspace tail_dev;
+    // frequency points of the density sums (freq_points.hip): the rule beyond n_freq of the
+    // bound lattice, and the table for the bound moments
+    std::shared_ptr<const std::vector<double>> tail;
     int n_plan = 0;            // points of the table when the rule applies
     int* pt_n = nullptr;
     double *pt_w = nullptr, *pt_wt = nullptr;

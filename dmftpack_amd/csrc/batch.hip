@@ -86,8 +86,9 @@ struct Sys {
     // chosen plans
     int chunks_f, kpc_f, chunks_v, kpc_v;
     // frequency points of the density sums (freq_points.hip)
-    int n_plan, n_tail;
-    double *tail, *pt_w, *pt_wt;
+    dg::FreqTail tail;
+    int n_plan;
+    double *pt_w, *pt_wt;
     int* pt_n;
 };
 
@@ -260,7 +261,7 @@ int issue_prepare(dmftgpu_batch_s* b)
     dmftgpu_handle h = b->h;
     for (Sys& s : b->sys) {
         HIPCHK(hipMemcpyAsync(s.mom, s.d.moments, sizeof(cd) * 4 * s.m2, hipMemcpyDeviceToDevice, h->stream));
-        HIPCHK(dg::launch_freq_points(s.mom, s.nc, s.nf, s.nw_tot, s.n_tail, s.tail, s.d.lat.beta, s.pt_n, s.pt_w, s.pt_wt,
+        HIPCHK(dg::launch_freq_points(s.mom, s.nc, s.nf, s.nw_tot, *s.tail, s.d.lat.beta, s.pt_n, s.pt_w, s.pt_wt,
                                       h->stream));
         HIPCHK(dg::launch_herm_eig((const cd*)s.d.Hk, s.n, 0, s.n, s.mom, s.nc, s.ev, s.U, s.nk, h->stream));
         if (s.nd > 0) {
@@ -441,7 +442,6 @@ static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system
     b->flags = flags;
     b->sys.resize(count);
     std::map<int, int> gidx;
-    std::vector<std::vector<double>> tails(count);  // frequency rules (freq_points.hip)
     size_t total = 0;
     for (int i = 0; i < count; ++i) {
         Sys& s = b->sys[i];
@@ -465,9 +465,8 @@ static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system
         s.nf = L.n_freq;
         s.nw_tot = L.n_freq * L.high_freq;
         s.m2 = s.nc * s.nc;
-        tails[i] = dg::freq_tail(s.nf, s.nw_tot);
-        s.n_tail = (int)tails[i].size() / 2;
-        s.n_plan = s.n_tail ? s.nf + s.n_tail : s.nw_tot;
+        s.tail = dg::freq_tail(s.nf, s.nw_tot);
+        s.n_plan = s.tail->empty() ? s.nw_tot : s.nf + (int)s.tail->size() / 2;
         s.max_chunks = std::max(1, std::min(s.nk, 128));
         s.st_kpc = (s.nk + 255) / 256;
         s.st_chunks = (s.nk + s.st_kpc - 1) / s.st_kpc;
@@ -503,7 +502,7 @@ static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system
         t += rnd(16 * C * s.nf * s.m2) + rnd(16 * C * s.nf);
         t += 3 * rnd(16 * (size_t)s.nw_tot) + rnd(16 * (size_t)s.nw_tot * s.m2) + rnd(16 * (size_t)s.nf * s.m2) +
              rnd(16 * (size_t)s.nf);
-        t += rnd(8 * tails[i].size()) + 2 * rnd(8 * (size_t)s.nw_tot) + rnd(4);
+        t += 2 * rnd(8 * (size_t)s.nw_tot) + rnd(4);
         need[i] = t;
         total += t;
     }
@@ -550,14 +549,10 @@ static int batch_create_impl(dmftgpu_batch_s* b, int count, const dmftgpu_system
         s.Gsum = (cd*)take(16 * (size_t)s.nw_tot * s.m2);
         s.Sb = (cd*)take(16 * (size_t)s.nf * s.m2);
         s.musum = (cd*)take(16 * (size_t)s.nf);
-        s.tail = (double*)take(8 * tails[i].size());
         s.pt_w = (double*)take(8 * (size_t)s.nw_tot);
         s.pt_wt = (double*)take(8 * (size_t)s.nw_tot);
         s.pt_n = (int*)take(4);
-        if (s.n_tail)
-            HIPCHK(hipMemcpyAsync(s.tail, tails[i].data(), 8 * tails[i].size(), hipMemcpyHostToDevice, h->stream));
     }
-    HIPCHK(hipStreamSynchronize(h->stream));  // the rules are host temporaries
     int rc = issue_prepare(b);
     if (!rc) rc = issue_sigma_tables(b);
     if (rc) return rc;

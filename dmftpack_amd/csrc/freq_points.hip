@@ -19,7 +19,9 @@
 //
 // What it gives: the kernels solve N_freq + 16 frequencies instead of 2 N_freq.
 // The plain method keeps every frequency (the reference's algorithm as it stands).
+#include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <vector>
 
 #include "lattice_kernels.hpp"
@@ -33,8 +35,8 @@ namespace {
 // 16 x 16 Jacobi matrix; its eigenvalues, all at once, by bisection on Sturm counts
 // (Barth, Martin and Wilkinson, Numer. Math. 9, 386 (1967)); the weights are the
 // Christoffel numbers len / sum_k p_k(node)^2 (Golub and Welsch, Math. Comp. 23, 221
-// (1969)).  The sums over the measure take 8 partial sums, which vectorise: about 80 us of
-// host time at 2048 frequencies, in dmftgpu_prepare under the eigensolvers.
+// (1969)).  The sums over the measure take 8 partial sums, which vectorise: about 70 us of
+// host time at 2048 frequencies, 20 at 64 (freq_tail keeps the rules).
 void gauss_rule(int n0, int n1, double* x, double* w)
 {
     constexpr int m = kGaussPoints, V = 8;
@@ -102,17 +104,26 @@ void gauss_rule(int n0, int n1, double* x, double* w)
     }
 }
 
-// The point table: the first n_freq Matsubara frequencies, then the Gauss points
-// (rule) or the remaining frequencies.  One workgroup; n_pts, pt_w, pt_wt as in LatArgs.
+// The point table: the first n_freq Matsubara frequencies, then the Gauss points (rule) or the
+// remaining frequencies; n_pts, pt_w, pt_wt as in LatArgs.  The rule comes as a kernel
+// argument, tail points t0 .. t0 + kTailBlock - 1: no device copy that a stream would have to wait
+// for.  Every workgroup forms the decision, of 4 n_c^2 entries, and writes its 256 points (one
+// workgroup for the whole table took 12 us at 16384 points, a third of preparing a lattice of
+// 64 k; 3 to 4 us now).
+constexpr int kTailBlock = 64;
+struct TailBlock {
+    double x[kTailBlock], w[kTailBlock];
+};
+
 __global__ __launch_bounds__(256) void k_freq_points(const cd* __restrict__ mom, int nc, int n_freq, int nw_tot,
-                                                     int n_tail, const double* __restrict__ tail, double beta,
+                                                     int n_tail, TailBlock tail, int t0, double beta,
                                                      int* __restrict__ n_pts, double* __restrict__ pt_w,
                                                      double* __restrict__ pt_wt)
 {
-    __shared__ double red[4][256];
-    const int m2 = nc * nc, t0 = threadIdx.x;
+    __shared__ double red[4][4];
+    const int m2 = nc * nc, t = threadIdx.x;
     double nrm[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int e = t0; e < m2; e += 256) {
+    for (int e = t; e < m2; e += 256) {
         const cd a = mom[e], b = mom[e / nc + (e % nc) * nc];
         const double ax = 0.5 * (a.x - b.x), ay = 0.5 * (a.y + b.y);  // anti-Hermitian part of m0
         nrm[0] += ax * ax + ay * ay;
@@ -121,28 +132,34 @@ __global__ __launch_bounds__(256) void k_freq_points(const cd* __restrict__ mom,
             nrm[q] += m.x * m.x + m.y * m.y;
         }
     }
-    for (int q = 0; q < 4; ++q) red[q][t0] = nrm[q];
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (t0 < o)
-            for (int q = 0; q < 4; ++q) red[q][t0] += red[q][t0 + o];
-        __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) nrm[q] += __shfl_xor(nrm[q], o);
+        if ((t & 63) == 0) red[q][t >> 6] = nrm[q];
     }
+    __syncthreads();
+    for (int q = 0; q < 4; ++q) nrm[q] = (red[q][0] + red[q][1]) + (red[q][2] + red[q][3]);
     const double r = 0.746 * matsubara(n_freq, beta), ir = 1.0 / r;
-    const double s = sqrt(red[0][0]) + ir * (sqrt(red[1][0]) + ir * (sqrt(red[2][0]) + ir * sqrt(red[3][0])));
+    const double s = sqrt(nrm[0]) + ir * (sqrt(nrm[1]) + ir * (sqrt(nrm[2]) + ir * sqrt(nrm[3])));
     const bool rule = n_tail > 0 && s <= 0.5 * r;  // false for NaN
     const int np = rule ? n_freq + n_tail : nw_tot;
-    if (t0 == 0) *n_pts = np;
-    for (int i = t0; i < np; i += 256) {
-        const bool node = rule && i >= n_freq;
-        pt_w[i] = node ? kPi * tail[i - n_freq] / beta : matsubara(i, beta);
-        pt_wt[i] = node ? tail[n_tail + i - n_freq] : 1.0;
+    // t0 = 0: the table from 0, with the first tail points; else tail points alone
+    const int i = (t0 ? n_freq + t0 : 0) + blockIdx.x * 256 + t, q = i - n_freq - t0;
+    if (t0 == 0 && i == 0) *n_pts = np;
+    if (i >= np) return;
+    if (rule && i >= n_freq) {
+        if (q < kTailBlock) {
+            pt_w[i] = kPi * tail.x[q] / beta;
+            pt_wt[i] = tail.w[q];
+        }
+    } else if (t0 == 0) {
+        pt_w[i] = matsubara(i, beta);
+        pt_wt[i] = 1.0;
     }
 }
 
-}  // namespace
-
-std::vector<double> freq_tail(int n_freq, int nw_tot)
+std::vector<double> form_tail(int n_freq, int nw_tot)
 {
     std::vector<double> x, w;
     bool any = false;
@@ -167,11 +184,47 @@ std::vector<double> freq_tail(int n_freq, int nw_tot)
     return x;
 }
 
-hipError_t launch_freq_points(const cd* mom, int nc, int n_freq, int nw_tot, int n_tail, const double* tail,
+}  // namespace
+
+FreqTail freq_tail(int n_freq, int nw_tot)
+{
+    // The last kKept rules formed, for every handle of the process: each is some tens of us of
+    // host time (12 lattices on one grid formed it 12 times: creating their batch took 2.41 ms, from
+    // 2.11 without a rule) and at most a few hundred doubles.
+    struct Kept {
+        int n_freq, nw_tot;
+        FreqTail tail;
+    };
+    constexpr size_t kKept = 16;
+    static std::mutex lock;
+    static std::vector<Kept> kept;  // most recent first
+    {
+        std::lock_guard<std::mutex> lk(lock);
+        for (size_t q = 0; q < kept.size(); ++q)
+            if (kept[q].n_freq == n_freq && kept[q].nw_tot == nw_tot) {
+                std::rotate(kept.begin(), kept.begin() + q, kept.begin() + q + 1);
+                return kept[0].tail;
+            }
+    }
+    FreqTail t = std::make_shared<const std::vector<double>>(form_tail(n_freq, nw_tot));
+    std::lock_guard<std::mutex> lk(lock);
+    if (kept.size() == kKept) kept.pop_back();
+    kept.insert(kept.begin(), Kept{n_freq, nw_tot, t});
+    return t;
+}
+
+hipError_t launch_freq_points(const cd* mom, int nc, int n_freq, int nw_tot, const std::vector<double>& tail,
                               double beta, int* n_pts, double* pt_w, double* pt_wt, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_freq_points, dim3(1), dim3(256), 0, s, mom, nc, n_freq, nw_tot, n_tail, tail, beta, n_pts,
-                       pt_w, pt_wt);
+    const int n_tail = (int)tail.size() / 2;
+    for (int t0 = 0; t0 == 0 || t0 < n_tail; t0 += kTailBlock) {
+        TailBlock b{};
+        const int count = std::min(kTailBlock, n_tail - t0);
+        std::copy_n(tail.data() + t0, count, b.x);
+        std::copy_n(tail.data() + n_tail + t0, count, b.w);
+        hipLaunchKernelGGL(k_freq_points, dim3(t0 ? 1 : (nw_tot + 255) / 256), dim3(256), 0, s, mom, nc, n_freq, nw_tot,
+                           n_tail, b, t0, beta, n_pts, pt_w, pt_wt);
+    }
     return hipGetLastError();
 }
 

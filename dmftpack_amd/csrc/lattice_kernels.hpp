@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <memory>
 #include <vector>
 
 #include "dev_common.hpp"
@@ -180,11 +181,12 @@ __device__ __forceinline__ void freq_point(const LatArgs& a, int nw, double& mu,
 constexpr int kGaussPoints = 16;
 constexpr int kGaussMin = 32;
 // The rule for n_freq <= n < nw_tot: [x..., weight...] with frequency pi x / beta, or
-// empty where no run is long enough.  Depends on the two counts only.
-std::vector<double> freq_tail(int n_freq, int nw_tot);
-// Point table (pt_n, pt_w, pt_wt of LatArgs; pt_w and pt_wt hold nw_tot entries) from
-// the tail rule (n_tail points, device copy) and Sigma's tail moments
-hipError_t launch_freq_points(const cd* mom, int nc, int n_freq, int nw_tot, int n_tail, const double* tail,
+// empty where no run is long enough.  Depends on the two counts only; safe from any thread.
+using FreqTail = std::shared_ptr<const std::vector<double>>;
+FreqTail freq_tail(int n_freq, int nw_tot);
+// Point table (pt_n, pt_w, pt_wt of LatArgs; pt_w and pt_wt hold nw_tot entries) from the
+// rule (a freq_tail, read before the call returns) and Sigma's tail moments
+hipError_t launch_freq_points(const cd* mom, int nc, int n_freq, int nw_tot, const std::vector<double>& tail,
                               double beta, int* n_pts, double* pt_w, double* pt_wt, hipStream_t s);
 
 // plain FP64 full inverse; returns 0 or a HIP error

@@ -68,3 +68,47 @@ def test_band_spectra_do_no_k_twice():
     call = "rt.check(h, rt.lib.dmftgpu_greenftn_real_k(h, 1, nf, -1.0, 0.01, 0.05, s, 0.1, rt.dev(16 * nk * nf * nc * nc), None))"
     for nc, nd, nk, nf, forms in host_hip.run(SPLIT.replace("call", call)):
         assert [f[2] for f in forms] == [2 if nc == 6 and nd < 2 else 1], (nc, nd, nk, nf, forms)
+
+
+def test_frequency_rule_needs_no_host_memory_after_the_call():
+    """two grids one after the other with no wait between: the second preparation must not take the
+    first one's rule from under its copy"""
+    assert host_hip.run("""
+        h = rt.handle()
+        rt.reset()
+        for nf in (4000, 200, 100):
+            rt.prepare(h, 5, 3, 8, nf)
+        result = rt.stale()
+    """) == 0
+
+
+def test_preparation_reads_only_what_it_queued_on_its_own_stream():
+    """the same grid prepared on one stream and then on another queues the same work: nothing that
+    the first stream may still be writing is read by the second"""
+    work = host_hip.run("""
+        import ctypes as C
+        h = rt.handle(C.c_void_p(0x1000))
+        result = []
+        for stream in (0x1000, 0x2000):
+            rt.check(h, rt.lib.dmftgpu_set_stream(h, C.c_void_p(stream)))
+            rt.reset()
+            rt.prepare(h, 5, 3, 8, 100)
+            result.append([e.replace(str(stream), "S") for e in rt.events() if not e.startswith("malloc")])
+    """)
+    assert work[0] == work[1] and len(work[0]) > 3
+
+
+def test_transform_tables_are_kept_while_the_stream_is():
+    counts = host_hip.run("""
+        import ctypes as C
+        h = rt.handle(C.c_void_p(0x1000))
+        d, nf, nt = 2, 40, 64
+        f, g = rt.dev(16 * nf * d * d), rt.dev(16 * (nt + 1) * d * d)
+        result = []
+        for stream in (0x1000, 0x1000, 0x2000):
+            rt.check(h, rt.lib.dmftgpu_set_stream(h, C.c_void_p(stream)))
+            rt.reset()
+            rt.check(h, rt.lib.dmftgpu_ft_tau2w(h, d, nf, nt, 20.0, g, f, None))
+            result.append(sum("k_czt_phases" in name for name, _, _ in rt.launches()))
+    """)
+    assert counts == [1, 0, 1]

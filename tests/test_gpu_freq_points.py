@@ -111,3 +111,13 @@ def test_batch_with_and_without_the_rule(G):
             assert abs(got["mu_bar"] - mb) <= 1e-10 * max(1.0, abs(mb))
     b.close()
     h.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,nc", [(6, 3), (9, 8)])
+def test_rule_longer_than_one_kernel_argument(G, n, nc):
+    """40 x 50 frequencies: six octaves, 96 points, which reach the table in blocks of 64"""
+    Hk, sig, mom = case(n, nc, 40)
+    lat = G.LatticeGF(Hk, nc, 40, BETA, mom, high_freq=50)
+    check(G, lat, Hk, sig, mom, 50, 1, 1e-12)
+    lat.close()
