@@ -182,56 +182,78 @@ __global__ __launch_bounds__(256) void k_czt(CztPlan p, int m2, const cd* __rest
 }
 
 // Definiteness of M_b = -X_b, or of -(X_b - X_b^H)/2i (ANTI), by the pivots of its elimination: a
-// slot of N lanes per matrix, lane c holds column c, the pivot column is read from its lane.
+// slot of N lanes (a power of two, N >= d) per matrix, lane c holds column c in LDS.
 // M_b counts as positive definite only by a margin of 1e-13 of its trace (>= its largest
-// eigenvalue), a hundred times the rounding of an eigenvalue.
-template <int N, bool ANTI>
-__global__ __launch_bounds__(64) void k_not_posdef(const cd* __restrict__ X, int d, int count, int* __restrict__ bad)
+// eigenvalue), a hundred times the rounding of an eigenvalue.  ANTI: the others are eliminated
+// again with 1e-12 of the largest entry added to the diagonal; a pivot below zero after positive
+// ones shows a negative eigenvalue of that matrix up to the rounding of the elimination
+// (Higham, Accuracy and Stability of Numerical Algorithms, sec. 10.1: some N^2 eps of the
+// diagonal, 1e-13 at N = 32), hence one of M_b.
+// A matrix is read once and its elimination is a chain, so the loops are rolled: with the columns
+// in registers the straight-line code of the steps ran once per launch, and fetching it
+// (12 KB at d = 16, 24 with the second elimination) was most of the time.  A call with every matrix
+// below, d = 10, 64 frequencies: 76 us in registers, 42 so; with every matrix sent to the eigensolver 202.
+template <bool ANTI>
+__global__ __launch_bounds__(64) void k_not_posdef(const cd* __restrict__ X, int d, int N, int count,
+                                                   int* __restrict__ bad)
 {
-    const int lane = threadIdx.x, c = lane % N, sl = lane / N;
-    const int b = blockIdx.x * (64 / N) + sl;
-    const bool live = b < count && c < d;
-    const cd* M = X + (size_t)(b < count ? b : count - 1) * d * d;
-    cd col[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        cd v = cd{i == c ? 1.0 : 0.0, 0.0};
-        if (live && i < d) {
-            if (ANTI) {  // -(x - conj(y))/2i
-                const cd x = M[i + c * d], y = M[c + i * d];
-                v = cd{-0.5 * (x.y + y.y), 0.5 * (x.x - y.x)};
-            } else {  // Hermitian to the last bit: the lower triangle
-                const cd m = i >= c ? M[i + c * d] : cconj(M[c + i * d]);
-                v = cd{-m.x, i == c ? 0.0 : -m.y};
-            }
-        }
-        col[i] = v;
-    }
-    double tr = 0.0;
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-        if (i == c && live) tr = col[i].x;
-#pragma unroll
-    for (int o = N / 2; o > 0; o >>= 1) tr += __shfl_xor(tr, o, N);
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-        if (i == c && live) col[i].x -= 1e-13 * tr;
+    extern __shared__ cd sm[];
+    const int lane = threadIdx.x, c = lane & (N - 1), slots = 64 / N, sl = lane / N, ld = N + 1;
+    const int b = blockIdx.x * slots + sl;
+    const bool mine = b < count, live = mine && c < d;
+    const cd* M = X + (size_t)(mine ? b : count - 1) * d * d;
+    cd *A = sm + sl * N * ld, *col = A + c * ld;  // columns of this slot's matrix, this lane's
+    // one addition a wavefront, of its matrices for which `which` holds
+    auto add = [&](int* to, bool which) {
+        const int n = __popcll(__ballot(live && c == 0 && which));
+        if (lane == 0 && n) atomicAdd(to, n);
+    };
     bool ok = true;
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-        if (j < d) {
-            const double p = __shfl(col[j].x, j, N);
-            ok = ok && p > 0.0 && p < 1e300;  // false for NaN and infinities
-            const cd f = cscale(col[j], 1.0 / p);  // A_jc / p
-#pragma unroll
-            for (int i = j + 1; i < N; ++i) {
-                if (i >= d) continue;
-                const cd l = cd{__shfl(col[i].x, j, N), __shfl(col[i].y, j, N)};
-                col[i] = cfms(l, f, col[i]);
+    for (int pass = 0; pass < (ANTI ? 2 : 1); ++pass) {
+        double diag = 0.0, top = 0.0;
+        if (c < d) {
+#pragma unroll 4
+            for (int i = 0; i < d; ++i) {
+                cd v;
+                if (ANTI) {  // -(x - conj(y))/2i
+                    const cd x = M[i + c * d], y = M[c + i * d];
+                    v = cd{-0.5 * (x.y + y.y), 0.5 * (x.x - y.x)};
+                } else {  // Hermitian to the last bit: the lower triangle
+                    const cd m = i >= c ? M[i + c * d] : cconj(M[c + i * d]);
+                    v = cd{-m.x, i == c ? 0.0 : -m.y};
+                }
+                col[i] = v;
+                if (i == c) diag = v.x;
+                top = fmax(top, fmax(fabs(v.x), fabs(v.y)));
             }
         }
+        double tr = diag;
+        for (int o = N / 2; o > 0; o >>= 1) {
+            tr += __shfl_xor(tr, o);
+            top = fmax(top, __shfl_xor(top, o));
+        }
+        if (c < d) col[c].x = diag + (pass ? 1e-12 * top : -1e-13 * tr);
+        wave_sync();
+        int sign = 1;  // 1: every pivot positive and finite; -1: a negative one after such; 0: neither
+        for (int j = 0; j < d; ++j) {
+            const double p = A[j * ld + j].x;
+            if (sign == 1 && !(p > 0.0 && p < 1e300)) sign = p < 0.0 && p > -1e300 ? -1 : 0;  // (NaN: 0)
+            if (c > j && c < d) {
+                const cd f = cscale(col[j], 1.0 / p);  // A_jc / p
+#pragma unroll 4
+                for (int i = j + 1; i < d; ++i) col[i] = cfms(A[j * ld + i], f, col[i]);
+            }
+            wave_sync();
+        }
+        if (pass == 0) {
+            ok = sign == 1;
+            if (!ANTI) add(bad, !ok);
+            if (!__any(live && !ok)) return;
+        } else {
+            add(bad, !ok && sign >= 0);
+            add(bad + 1, !ok && sign < 0);
+        }
     }
-    if (live && c == 0 && !ok) atomicAdd(bad, 1);
 }
 
 }  // namespace
@@ -279,18 +301,12 @@ hipError_t launch_czt(const CztPlan& p, bool to_w, int m2, const cd* tab, const 
 
 hipError_t launch_not_posdef(const cd* X, int d, int count, bool anti, int* bad, hipStream_t s)
 {
-#define P_(N)                                                                                                       \
-    {                                                                                                               \
-        const dim3 grid((count + 64 / N - 1) / (64 / N));                                                           \
-        if (anti) hipLaunchKernelGGL((k_not_posdef<N, true>), grid, dim3(64), 0, s, X, d, count, bad);              \
-        else hipLaunchKernelGGL((k_not_posdef<N, false>), grid, dim3(64), 0, s, X, d, count, bad);                  \
-        return hipGetLastError();                                                                                   \
-    }
-    if (d <= 4) P_(4)
-    if (d <= 8) P_(8)
-    if (d <= 16) P_(16)
-    P_(32)
-#undef P_
+    const int N = d <= 4 ? 4 : d <= 8 ? 8 : d <= 16 ? 16 : 32, slots = 64 / N;
+    const dim3 grid((count + slots - 1) / slots);
+    const size_t shm = sizeof(cd) * 64 * (N + 1);
+    if (anti) hipLaunchKernelGGL((k_not_posdef<true>), grid, dim3(64), shm, s, X, d, N, count, bad);
+    else hipLaunchKernelGGL((k_not_posdef<false>), grid, dim3(64), shm, s, X, d, N, count, bad);
+    return hipGetLastError();
 }
 
 }  // namespace dg

@@ -23,8 +23,9 @@ CztPlan czt_plan(int n_tau, int n_in, int n_out);
 // to_w false: i = frequency f, output t = tau index; true: i = t, output f (phase +)
 hipError_t launch_czt(const CztPlan& p, bool to_w, int m2, const cd* tab, const cd* in, cd* parts, hipStream_t s);
 
-// *bad += number of matrices X_b (d x d, count of them) for which -X_b (X_b Hermitian), or with
-// anti -(X_b - X_b^H)/2i, is not positive definite by a margin; *bad preset by the caller
+// bad[0] += number of matrices X_b (d x d, count of them) for which -X_b (X_b Hermitian), or with
+// anti -(X_b - X_b^H)/2i, is not positive definite by a margin; with anti, those that have a
+// negative eigenvalue by a margin are counted in bad[1] instead; bad preset by the caller
 hipError_t launch_not_posdef(const cd* X, int d, int count, bool anti, int* bad, hipStream_t s);
 
 }  // namespace dg

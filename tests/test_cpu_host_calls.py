@@ -112,3 +112,19 @@ def test_transform_tables_are_kept_while_the_stream_is():
             result.append(sum("k_czt_phases" in name for name, _, _ in rt.launches()))
     """)
     assert counts == [1, 0, 1]
+
+
+def test_small_tau_transforms_take_one_launch_and_the_causality_test():
+    """a tau -> iw transform of a few hundred points: no FFTs, whose launches cost more than its sums"""
+    names = host_hip.run("""
+        h = rt.handle()
+        result = []
+        for d, nf, nt in ((1, 64, 128), (5, 200, 400), (5, 1000, 2000)):
+            f, g = rt.dev(16 * nf * d * d), rt.dev(16 * (nt + 1) * d * d)
+            for _ in range(2):  # the tables are kept
+                rt.reset()
+                rt.check(h, rt.lib.dmftgpu_ft_tau2w(h, d, nf, nt, 20.0, g, f, None))
+            result.append([name for name, _, _ in rt.launches()])
+    """)
+    assert [len(n) for n in names] == [2, 2, 4]
+    assert all("k_not_posdef" in n[-1] for n in names)
