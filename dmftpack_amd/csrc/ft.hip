@@ -1115,8 +1115,8 @@ extern "C" int dmftgpu_ft_w2tau(dmftgpu_handle h, int d, int n_freq, int n_tau, 
     std::vector<hl::cx> A1, A2;
     std::vector<double> e1, e2;
     tail_setup(d, m1, mm2, m3, A1, e1, A2, e2);
-    const dg::CztPlan cp = dg::czt_plan(n_tau, n_freq, n_tau);
-    const size_t npart = (size_t)cp.in_tiles * m2 * n_tau;
+    const dg::CztPlan cp = dg::czt_plan(n_tau, n_freq, n_tau, m2);
+    const size_t npart = (size_t)cp.in_groups * m2 * n_tau;
     size_t need = (size_t)n_freq * m2 * 16 + 4 * (size_t)m2 * 16 + 4 * (size_t)d * 8 +
                   (size_t)ntau1 * d * 8 + npart * 16 + 16 * 256;
     int rc = 0;
@@ -1136,7 +1136,7 @@ extern "C" int dmftgpu_ft_w2tau(dmftgpu_handle h, int d, int n_freq, int n_tau, 
                        D, (size_t)1, (size_t)n_freq, bad);
     HIPCHK(hipGetLastError());
     HIPCHK(dg::launch_czt(cp, false, m2, tab, D, parts, s));
-    const FtSums xs{parts, cp.in_tiles, (size_t)m2 * n_tau, 1, (size_t)n_tau, n_tau};
+    const FtSums xs{parts, cp.in_groups, (size_t)m2 * n_tau, 1, (size_t)n_tau, n_tau};
     cd* out = (cd*)gtau;
     hipLaunchKernelGGL(k_ft_finish, dim3((ntau1 + kTile - 1) / kTile, (m2 + kTile - 1) / kTile), dim3(256), 0, s, xs, d,
                        ntau1, beta, beta / n_tau, (const double*)nullptr, tl.A1, tl.e1, tl.A2, tl.e2, out);
@@ -1207,8 +1207,8 @@ extern "C" int dmftgpu_ft_tau2w(dmftgpu_handle h, int d, int n_freq, int n_tau, 
     const cd *g0 = (const cd*)gtau, *g1 = g0 + (size_t)(n_tau + 1) * m2;
     const bool apart = (const cd*)fw >= g1 || (const cd*)fw + (size_t)n_freq * m2 <= g0;
     const bool direct = apart && tau2w_direct(n_freq, n_tau, m2);
-    const dg::CztPlan cp = dg::czt_plan(n_tau, n_tau, n_freq);
-    const size_t npart = direct ? 0 : (size_t)cp.in_tiles * m2 * n_freq, ngin = direct ? 0 : (size_t)n_tau * m2;
+    const dg::CztPlan cp = dg::czt_plan(n_tau, n_tau, n_freq, m2);
+    const size_t npart = direct ? 0 : (size_t)cp.in_groups * m2 * n_freq, ngin = direct ? 0 : (size_t)n_tau * m2;
     size_t need = (ngin + npart + 2 * m2 + (size_t)n_freq * m2) * 16 + (size_t)n_freq * d * 8 + 9 * 256;
     int rc = 0;
     char* base = ft_ws(h, need, &rc);
@@ -1231,7 +1231,7 @@ extern "C" int dmftgpu_ft_tau2w(dmftgpu_handle h, int d, int n_freq, int n_tau, 
         HIPCHK(hipGetLastError());
         HIPCHK(dg::launch_czt(cp, true, m2, tab, gin, parts, s));
         hipLaunchKernelGGL(k_ft_w_finish, dim3((n_freq + kTile - 1) / kTile, (m2 + kTile - 1) / kTile), dim3(256), 0, s,
-                           parts, cp.in_tiles, ends, m2, n_freq, n_tau, dt, (cd*)fw);
+                           parts, cp.in_groups, ends, m2, n_freq, n_tau, dt, (cd*)fw);
     }
     HIPCHK(hipGetLastError());
     // causality test (:551-558): a frequency violates it where (F - F^H)/2i has a positive

@@ -22,6 +22,8 @@
 // the second FFT follow in registers.
 #include "ft_czt.hpp"
 
+#include <algorithm>
+
 namespace dg {
 
 namespace {
@@ -136,48 +138,64 @@ __global__ __launch_bounds__(256) void k_czt_filter(int n_tau, cd* __restrict__ 
     for (int r = 0; r < 16; ++r) tab[n2 + kCztM + t + 256 * r] = cscale(v[r], 1.0 / kCztM);
 }
 
-// One tile: inputs a0..a0+2047 of element e, outputs b0..b0+2047 (grid: element, output
-// tile, input tile).  Phase -+ pi (2f+1) t/N with (f, t) = (input, output) for iw -> tau and
-// (output, input) for tau -> iw; the + sign by conjugating input and output.
-template <bool TO_W>
+// One output tile, b0..b0+2047, of element e: the sum of this group's input tiles a0..a0+2047
+// (grid: element, output tile, group).  Phase -+ pi (2f+1) t/N with (f, t) = (input, output) for
+// iw -> tau and (output, input) for tau -> iw; the + sign by conjugating input and output.
+// ONE: a group is one tile, whose results go straight out (with the sums in registers d = 10, 4096 x
+// 8192 took 20 us more either way).
+template <bool TO_W, bool ONE>
 __global__ __launch_bounds__(256) void k_czt(CztPlan p, int m2, const cd* __restrict__ tab, const cd* __restrict__ in,
                                              cd* __restrict__ parts)
 {
     extern __shared__ cd sm[];
     const int t = threadIdx.x, e = blockIdx.x, n2 = 2 * p.n_tau;
-    const long long b0 = (long long)blockIdx.y * kCztTile, a0 = (long long)blockIdx.z * kCztTile;
+    const long long b0 = (long long)blockIdx.y * kCztTile;
     const cd *tw = tab + n2, *filt = tw + kCztM;
     const double inv = 1.0 / n2;
-    const cd* x = in + (size_t)e * p.ld_in + a0;
-    const int na = min(kCztTile, p.n_in - (int)a0), nb = min(kCztTile, p.n_out - (int)b0);
-    cd v[16];
+    const int nb = min(kCztTile, p.n_out - (int)b0);
+    cd* out = parts + ((size_t)blockIdx.z * m2 + e) * p.ld_out + b0;
+    cd y[ONE ? 1 : 8];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int a = t + 256 * r;
-        v[r] = cd{0.0, 0.0};
-        if (r < 8 && a < na) {
-            cd g = x[a];
-            if (TO_W) g.y = -g.y;
-            // 2 a b0 + a^2, and the half step (2f+1) t: + t for the tau index on the input side
-            const long long m = 2 * (long long)a * b0 + (long long)a * a + (TO_W ? a0 + a : 0);
-            v[r] = cmulc(g, tab[mod2n(m, n2, inv)]);
+    for (int r = 0; r < (ONE ? 1 : 8); ++r) y[r] = cd{0.0, 0.0};
+    for (int tile = blockIdx.z; tile < p.in_tiles; tile += p.in_groups) {
+        const long long a0 = (long long)tile * kCztTile;
+        const cd* x = in + (size_t)e * p.ld_in + a0;
+        const int na = min(kCztTile, p.n_in - (int)a0);
+        cd v[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int a = t + 256 * r;
+            v[r] = cd{0.0, 0.0};
+            if (r < 8 && a < na) {
+                cd g = x[a];
+                if (TO_W) g.y = -g.y;
+                // 2 a b0 + a^2, and the half step (2f+1) t: + t for the tau index on the input side
+                const long long m = 2 * (long long)a * b0 + (long long)a * a + (TO_W ? a0 + a : 0);
+                v[r] = cmulc(g, tab[mod2n(m, n2, inv)]);
+            }
         }
+        fft4096(v, sm, tw, t);
+        // inverse FFT as conj(FFT(conj(.)))
+#pragma unroll
+        for (int r = 0; r < 16; ++r) v[r] = cconj(cmul(v[r], filt[t + 256 * r]));
+        fft4096(v, sm, tw, t);
+        const long long ab = mod2n(2 * a0 * b0, n2, inv);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const int b = t + 256 * r;
+            if (b < nb) {
+                const long long m = ab + 2 * (long long)b * a0 + (long long)b * b + (TO_W ? 0 : b0 + b);
+                const cd w = cmulc(cconj(v[r]), tab[mod2n(m, n2, inv)]);
+                if constexpr (ONE) out[b] = TO_W ? cconj(w) : w;
+                else y[r] = cadd(y[r], w);
+            }
+        }
+        if constexpr (ONE) return;
     }
-    fft4096(v, sm, tw, t);
-    // inverse FFT as conj(FFT(conj(.)))
+    if constexpr (!ONE) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) v[r] = cconj(cmul(v[r], filt[t + 256 * r]));
-    fft4096(v, sm, tw, t);
-    cd* y = parts + ((size_t)blockIdx.z * m2 + e) * p.ld_out + b0;
-    const long long ab = mod2n(2 * a0 * b0, n2, inv);
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-        const int b = t + 256 * r;
-        if (b < nb) {
-            const long long m = ab + 2 * (long long)b * a0 + (long long)b * b + (TO_W ? 0 : b0 + b);
-            const cd w = cmulc(cconj(v[r]), tab[mod2n(m, n2, inv)]);
-            y[b] = TO_W ? cconj(w) : w;
-        }
+        for (int r = 0; r < 8; ++r)
+            if (t + 256 * r < nb) out[t + 256 * r] = TO_W ? cconj(y[r]) : y[r];
     }
 }
 
@@ -269,13 +287,15 @@ hipError_t launch_czt_tables(int n_tau, cd* tab, hipStream_t s)
     return hipGetLastError();
 }
 
-CztPlan czt_plan(int n_tau, int n_in, int n_out)
+CztPlan czt_plan(int n_tau, int n_in, int n_out, int m2)
 {
     CztPlan p;
     p.n_tau = n_tau;
     p.n_in = n_in;
     p.n_out = n_out;
     p.in_tiles = (n_in + kCztTile - 1) / kCztTile;
+    const size_t fit = kCztPartBytes / ((size_t)m2 * n_out * sizeof(cd));
+    p.in_groups = (int)std::max<size_t>(1, std::min<size_t>(p.in_tiles, fit));
     p.out_tiles = (n_out + kCztTile - 1) / kCztTile;
     p.ld_in = n_in;
     p.ld_out = n_out;
@@ -285,17 +305,12 @@ CztPlan czt_plan(int n_tau, int n_in, int n_out)
 hipError_t launch_czt(const CztPlan& p, bool to_w, int m2, const cd* tab, const cd* in, cd* parts, hipStream_t s)
 {
     const int shm = (int)(sizeof(cd) * kFftLds);
-    const dim3 grid(m2, p.out_tiles, p.in_tiles);
-    hipError_t e;
-    if (to_w) {
-        e = hipFuncSetAttribute((const void*)k_czt<true>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((k_czt<true>), grid, dim3(256), shm, s, p, m2, tab, in, parts);
-    } else {
-        e = hipFuncSetAttribute((const void*)k_czt<false>, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((k_czt<false>), grid, dim3(256), shm, s, p, m2, tab, in, parts);
-    }
+    const dim3 grid(m2, p.out_tiles, p.in_groups);
+    const bool one = p.in_groups == p.in_tiles;
+    auto kernel = to_w ? one ? k_czt<true, true> : k_czt<true, false> : one ? k_czt<false, true> : k_czt<false, false>;
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, shm);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kernel, grid, dim3(256), shm, s, p, m2, tab, in, parts);
     return hipGetLastError();
 }
 

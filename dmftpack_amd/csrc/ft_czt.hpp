@@ -14,12 +14,15 @@ constexpr int kCztTile = kCztM / 2; // inputs and outputs of a tile
 inline size_t czt_table_count(int n_tau) { return 2 * (size_t)n_tau + 2 * kCztM; }
 hipError_t launch_czt_tables(int n_tau, cd* tab, hipStream_t s);
 
+// in_tiles are shared out over in_groups workgroups, each adding its tiles, as many groups as there
+// are tiles while their partial sums, m2 n_out each, fit kCztPartBytes
 struct CztPlan {
-    int n_tau, n_in, n_out, in_tiles, out_tiles, ld_in, ld_out;
+    int n_tau, n_in, n_out, in_tiles, in_groups, out_tiles, ld_in, ld_out;
 };
-CztPlan czt_plan(int n_tau, int n_in, int n_out);
+constexpr size_t kCztPartBytes = (size_t)512 << 20;
+CztPlan czt_plan(int n_tau, int n_in, int n_out, int m2);
 
-// parts [in_tile][e][n_out] of sum_i exp(-+ i pi (2f+1) t / n_tau) in[e][i]:
+// parts [in_group][e][n_out] of sum_i exp(-+ i pi (2f+1) t / n_tau) in[e][i]:
 // to_w false: i = frequency f, output t = tau index; true: i = t, output f (phase +)
 hipError_t launch_czt(const CztPlan& p, bool to_w, int m2, const cd* tab, const cd* in, cd* parts, hipStream_t s);
 

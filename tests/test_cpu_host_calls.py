@@ -128,3 +128,29 @@ def test_small_tau_transforms_take_one_launch_and_the_causality_test():
     """)
     assert [len(n) for n in names] == [2, 2, 4]
     assert all("k_not_posdef" in n[-1] for n in names)
+
+
+@pytest.mark.parametrize("d,nf,nt", [(32, 65536, 131072), (10, 65536, 131072), (4, 100000, 3000), (32, 3000, 100000)])
+def test_scratch_of_the_tau_transforms(d, nf, nt):
+    """a copy of each grid and a bounded number of partial sums: not a partial sum of the whole
+    output for every 2048 inputs (69 GB at the first of these sizes)"""
+    to_tau, to_w = host_hip.run(f"""
+        import ctypes as C
+        d, nf, nt = {d}, {nf}, {nt}
+        f, g = rt.dev(16 * nf * d * d), rt.dev(16 * (nt + 1) * d * d)
+        mom = rt.dev(np.stack([np.zeros((d, d)), np.eye(d), 0.1 * np.eye(d), np.eye(d)]).astype(np.complex128))
+        result = []
+        for call in ("w2tau", "tau2w"):
+            h = rt.handle()
+            rt.reset()
+            before = rt.peak()
+            if call == "w2tau":
+                rt.check(h, rt.lib.dmftgpu_ft_w2tau(h, d, nf, nt, 20.0, f, mom, g, None))
+            else:
+                rt.check(h, rt.lib.dmftgpu_ft_tau2w(h, d, nf, nt, 20.0, g, f, None))
+            result.append(rt.peak() - before)
+            rt.lib.dmftgpu_destroy(h)
+    """)
+    grids = 16 * d * d * (nf + nt + 1)
+    eig = 16 * d * d * nf  # tau -> iw: (F - F^H)/2i for the eigensolver
+    assert to_tau <= grids + 2 ** 30 and to_w <= grids + eig + 2 ** 30, (to_tau, to_w, grids)
