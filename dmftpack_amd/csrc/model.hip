@@ -252,9 +252,9 @@ extern "C" int dmftgpu_hk_from_hr(dmftgpu_handle h, int n, int n_hop, const int*
     }
     // Dense lists (at least half of all (R, element) pairs present; below that the zeros cost
     // more than the per-hop phases): one matrix per distinct R
-    const RIndex ri = index_r(n_hop, hop_idx);
+    const RIndex ri = index_r(n_hop, hop_idx, 2 * (size_t)n_hop / nn);
     const int n_r = (int)ri.R.size();
-    if (n_hop > 0 && (double)n_r * nn <= 2.0 * n_hop) {
+    if (n_r > 0) {
         std::vector<cd> T((size_t)n_r * nn, cd{0.0, 0.0});
         for (int q = 0; q < n_hop; ++q) {
             cd& t = T[(size_t)ri.of[q] * nn + hop_idx[5 * q + 3] + (size_t)hop_idx[5 * q + 4] * n];

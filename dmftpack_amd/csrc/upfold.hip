@@ -449,10 +449,10 @@ extern "C" int dmftgpu_upfold_density(dmftgpu_handle h, int n, int n_orb, int n_
     }
     // at least half of all (R, element) pairs listed: a sum per distinct R and element, then a
     // gather (below that the unlisted sums cost more than the per-entry phases)
-    const RIndex ri = index_r(n_r, r_idx);
+    const RIndex ri = index_r(n_r, r_idx, 2 * (size_t)n_r / oo);
     const int n_rv = (int)ri.R.size();
     const int nx = overlap ? 3 : 1;
-    const bool dense = n_r > 0 && (double)n_rv * oo <= 2.0 * n_r && (size_t)dg::rs_pad(n_rv) * nx <= 65535;
+    const bool dense = n_rv > 0 && (size_t)dg::rs_pad(n_rv) * nx <= 65535;
     std::vector<int> order(dense ? 0 : n_r);
     for (size_t r = 0; r < order.size(); ++r) order[r] = (int)r;
     const int n_ent = (int)order.size();  // entries of the per-entry R sums (0 for dense lists)

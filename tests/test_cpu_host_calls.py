@@ -154,3 +154,36 @@ def test_scratch_of_the_tau_transforms(d, nf, nt):
     grids = 16 * d * d * (nf + nt + 1)
     eig = 16 * d * d * nf  # tau -> iw: (F - F^H)/2i for the eigensolver
     assert to_tau <= grids + 2 ** 30 and to_w <= grids + eig + 2 ** 30, (to_tau, to_w, grids)
+
+
+def test_dense_hopping_lists_are_told_from_sparse_ones_in_any_order():
+    """H(k) takes the dense sums exactly where at least half of all (R, element) pairs are listed:
+    lists around that line, grouped by R, shuffled, element by element, with R far apart, with
+    pairs listed twice"""
+    cases = host_hip.run("""
+        import ctypes as C
+        rng = np.random.default_rng(5)
+        h = rt.handle()
+        result = []
+        for n, n_r in ((1, 1), (1, 40), (3, 7), (6, 19), (6, 130), (2, 1000)):
+            R = np.unique(rng.integers(-6, 7, size=(4 * n_r, 3)), axis=0)[:n_r]
+            for scale in (1, 1, 40000000):
+                pairs = np.array([(*(scale * r), i, j) for r in R for i in range(n) for j in range(n)], np.int32)
+                full = len(pairs)
+                for keep in {1, full // 4, (full + 1) // 2 - 1, (full + 1) // 2, (full + 1) // 2 + 1, full}:
+                    if keep < 1: continue
+                    pick = np.sort(rng.permutation(full)[:keep])
+                    by_element = pick[np.lexsort((pick, pairs[pick, 3], pairs[pick, 4]))]
+                    for rows in (pick, rng.permutation(pick), by_element, np.repeat(pick, 2)):
+                        idx = np.ascontiguousarray(pairs[rows])
+                        t = np.ones(2 * len(idx))
+                        distinct = len(np.unique(idx[:, :3], axis=0))
+                        rt.reset()
+                        rt.check(h, rt.lib.dmftgpu_hk_from_hr(h, n, len(idx), idx.ctypes.data_as(C.POINTER(C.c_int)),
+                                                              t.ctypes.data_as(C.POINTER(C.c_double)), 4,
+                                                              rt.dev(96), rt.dev(64 * n * n)))
+                        dense = any("k_hk_dense" in name for name, _, _ in rt.launches())
+                        result.append([bool(distinct * n * n <= 2 * len(idx)), dense, rt.stale()])
+    """)
+    assert all(want == got and not stale for want, got, stale in cases)
+    assert {want for want, _, _ in cases} == {True, False} and len(cases) > 300
