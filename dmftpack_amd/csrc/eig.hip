@@ -386,6 +386,24 @@ static hipError_t launch_slots(const cd* X, int ldx, int off, int m, const cd* a
     return hipGetLastError();
 }
 
+// The 32-lane slots do the work of a 32 x 32 matrix at any m, two matrices a wavefront, 2048 on the
+// chip at once, in 0.77 ms (one) to 0.95 ms (2048); the LDS kernel's time falls with m, and its LDS
+// admits 160 KB / shm matrices to a CU.  us, slots / LDS, with V: m = 32 769 / 1092 (1 matrix), 1879 / 6195
+// (4096); m = 30 871 / 898 (64); m = 29 885 / 841 (512), 902 / 1050 (1210); m = 28 882 / 800 (512),
+// 898 / 1024 (1210), 1857 / 2831 (4096); m = 27 897 / 851 (1210), 939 / 1347 (1728, a second round);
+// m = 26 878 / 641 (512), 939 / 830 (1728), 945 / 1279 (2028), 1736 / 1439 (2744), 1857 / 2062 (4096);
+// m = 24 1850 / 1870 (4096), 940 / 850 (1728).  Eigenvalues alone are half the work in slots: moments of a
+// Green function with d = 28, 100 frequencies 686 / 826, d = 24 as fast either way.
+static bool lds_is_faster(int m, int batch, bool vectors, size_t shm)
+{
+    if (m < 26) return true;
+    if (!vectors) return false;
+    if (m > 29) return false;
+    if (batch <= 1024) return true;
+    const int lds_round = 256 * (int)(160 * 1024 / shm), slot_round = 2048;
+    return m <= 27 && (batch + lds_round - 1) / lds_round <= (batch + slot_round - 1) / slot_round;
+}
+
 hipError_t launch_herm_eig(const cd* X, int ldx, int off, int m, const cd* add, int nadd, double* w, cd* V, int batch,
                            hipStream_t s)
 {
@@ -394,11 +412,8 @@ hipError_t launch_herm_eig(const cd* X, int ldx, int off, int m, const cd* add, 
     if (m <= 8) return launch_slots<8>(X, ldx, off, m, add, nadd, w, V, batch, s);
     if (m <= 16) return launch_slots<16>(X, ldx, off, m, add, nadd, w, V, batch, s);
     if (m > 32) return hipErrorInvalidValue;
-    // The 32-lane slots do the work of a 32 x 32 matrix at any m; the LDS kernel's time falls
-    // with m.  4096 matrices with V, slots against LDS: m = 32 1.93 and 6.27 ms, 28 1.88 and
-    // 2.82, 26 1.84 and 2.05, 24 1.85 and 1.87 (1728 matrices: 0.94 and 0.85), 22 1.74 and 1.14
-    if (m >= 26) return launch_slots<32>(X, ldx, off, m, add, nadd, w, V, batch, s);
     size_t shm = sizeof(cd) * 2 * (size_t)m * m + sizeof(double) * 4 * 16 + sizeof(int) * 2 * 16;
+    if (!lds_is_faster(m, batch, V != nullptr, shm)) return launch_slots<32>(X, ldx, off, m, add, nadd, w, V, batch, s);
     hipLaunchKernelGGL(k_herm_eig, dim3(batch), dim3(64), shm, s, X, ldx, off, m, add, nadd, w, V, batch);
     return hipGetLastError();
 }

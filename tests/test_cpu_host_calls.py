@@ -187,3 +187,21 @@ def test_dense_hopping_lists_are_told_from_sparse_ones_in_any_order():
     """)
     assert all(want == got and not stale for want, got, stale in cases)
     assert {want for want, _, _ in cases} == {True, False} and len(cases) > 300
+
+
+def test_eigensolver_form_by_size_and_count():
+    """17 to 29 rows: the LDS kernel where one round of it ends before a round of the 32-lane slots
+    (or needs no more rounds); from 30 on, for many matrices, and without vectors the slots"""
+    names = host_hip.run("""
+        result = []
+        for n, nk in ((17, 5000), (25, 5000), (26, 1), (26, 1700), (26, 2000), (26, 2700), (26, 4096), (27, 1200),
+                      (27, 1700), (28, 1024), (28, 1100), (29, 512), (29, 2000), (30, 64), (32, 1)):
+            h = rt.handle()
+            rt.prepare(h, n, 5, nk, 8)
+            rt.reset()
+            rt.check(h, rt.lib.dmftgpu_update_moments(h, rt.dev(16 * 4 * 25)))
+            result.append([n, nk, any("k_herm_eig(" in name for name, _, _ in rt.launches())])
+            rt.lib.dmftgpu_destroy(h)
+    """)
+    slots = {(26, 2000), (26, 4096), (27, 1700), (28, 1100), (29, 2000), (30, 64), (32, 1)}
+    assert {(n, nk) for n, nk, lds in names if not lds} == slots

@@ -42,3 +42,20 @@ def test_static_eig_sizes(G, n, kind):
     assert np.abs(ev - np.linalg.eigvalsh(H)).max() <= 1e-13 * scale
     assert np.abs(U.conj().transpose(0, 2, 1) @ U - np.eye(n)).max() <= 1e-13
     assert np.abs(U * ev[:, None, :] @ U.conj().transpose(0, 2, 1) - H).max() <= 1e-13 * scale
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,nk", [(26, 2000), (27, 1600), (28, 1025), (29, 1300)])
+def test_many_matrices(G, n, nk):
+    """counts at which these sizes take the 32-lane slots"""
+    rng = np.random.default_rng(n)
+    X = rng.normal(size=(nk, n, n)) + 1j * rng.normal(size=(nk, n, n))
+    H = 0.5 * (X + X.conj().transpose(0, 2, 1))
+    sig, mom = L.pole_sigma(2, 4, 10.0, n)
+    mom[0] = 0.0
+    lat = G.LatticeGF(H, 2, 4, 10.0, mom)
+    ev, U = lat.static_eig()
+    lat.close()
+    scale = np.linalg.norm(H, axis=(1, 2)).max()
+    assert np.abs(ev - np.linalg.eigvalsh(H)).max() <= 1e-13 * scale
+    assert np.abs(U * ev[:, None, :] @ U.conj().transpose(0, 2, 1) - H).max() <= 1e-13 * scale
