@@ -155,45 +155,60 @@ __global__ void k_mom_kinv(int range, int green, double* __restrict__ kinv)
 // the basis values come as scalar operands and a frequency costs two vector loads, those of
 // kFitAhead frequencies issued ahead of their use.  With the basis loaded by each lane and
 // an element a thread, d = 5 and N_freq = 1000 took 220 us, bound by the L1 loads; this
-// form 75 us.
+// form 75 us.  From kFitAll (window, pair) fits on, a thread takes all NA moments: the data
+// are read once instead of once a moment, which counts where they leave the caches.  us of the
+// call, one moment / all a thread: d = 5, 1000 frequencies (15000 fits) 193 / 238, 2500 (37500)
+// 489 / 506, d = 10, 1000 (55000) 499 / 464, d = 28, 1500 (609000) 7475 / 3177 (an element a
+// thread: 7057), d = 32, 2500 (1.32e6) 38950 / 12920 (25420).
 constexpr int kFitAhead = 8;
+constexpr size_t kFitAll = 40960;
 
-template <bool GREEN>
+template <bool GREEN, int NA>
 __global__ __launch_bounds__(64) void k_mom_fit(const cd* __restrict__ fw, int d, int n_freq, int range,
                                                 const double* __restrict__ tab_, const double* __restrict__ kinv,
                                                 cd* __restrict__ mt)
 {
 #pragma clang fp contract(off)
-    const int m2 = d * d, np = d * (d + 1) / 2, a = blockIdx.y;
+    const int m2 = d * d, np = d * (d + 1) / 2, a0 = blockIdx.y * NA;
     const kconst_double* tab = (const kconst_double*)tab_;
     const unsigned first = blockIdx.x * 64, last = min(first + 63, (unsigned)(range * np - 1));
     const unsigned t = min(first + threadIdx.x, last);  // spare lanes repeat the last entry
     const int w = (int)(t / np), q = (int)(t % np);
     int be = 0, al = q;
     while (al > be) al -= ++be;  // pair q -> (al, be), al <= be
-    const double* X = kinv + (size_t)w * 16 + a;  // Kinv(a, b) at X[4 b]
-    const double x0 = X[0], x1 = X[4], x2 = GREEN ? 0.0 : X[8], x3 = GREEN ? 0.0 : X[12];
+    double x[NA][4];
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
+        const double* X = kinv + (size_t)w * 16 + a0 + a;  // Kinv(a, b) at X[4 b]
+#pragma unroll
+        for (int b = 0; b < 4; ++b) x[a][b] = GREEN && b > 1 ? 0.0 : X[4 * b];
+    }
     // element addresses: the frequency's uniform base and the lane's offset
     const unsigned oa = (al + be * d) * sizeof(cd), ob = (be + al * d) * sizeof(cd);
     auto at = [&](int wn, unsigned o) -> cd { return *(const cd*)((const char*)(fw + (size_t)wn * m2) + o); };
-    cd s = cd{0, 0};  // twice the sum: the halves of Re and Im are taken at the end (exactly)
+    cd s[NA];  // twice the sums: the halves of Re and Im are taken at the end (exactly)
+#pragma unroll
+    for (int a = 0; a < NA; ++a) s[a] = cd{0, 0};
     // basis values {-1/z, -1/z^2, 1/z^3, 1/z} of a frequency at c
     auto add = [&](double c0, double c1, double c2, double c3, cd fab, cd fba) {
         // 2 Re = F_ab + conj(F_ba) ; 2 Im = (F_ab - conj(F_ba))/i
         const cd re = cd{fab.x + fba.x, fab.y - fba.y};
         cd im = cd{fab.y + fba.y, fba.x - fab.x};
-        double kr, ki;
-        if (!GREEN) {
-            // Re row [1, 0, -1/z^2, 0], Im row [0, -1/z, 0, 1/z^3]   (:227-230)
-            kr = fma(x2, c1, x0);
-            ki = fma(x3, c2, x1 * c0);
-        } else {
-            // Re row [-1/z^2, 0], Im row [0, 1/z^3]   (:366-367)
-            if (al == be) im.x += 2.0 * c3;  // (:373)
-            kr = x0 * c1;
-            ki = x1 * c2;
+        if (GREEN && al == be) im.x += 2.0 * c3;  // (:373)
+#pragma unroll
+        for (int a = 0; a < NA; ++a) {
+            double kr, ki;
+            if (!GREEN) {
+                // Re row [1, 0, -1/z^2, 0], Im row [0, -1/z, 0, 1/z^3]   (:227-230)
+                kr = fma(x[a][2], c1, x[a][0]);
+                ki = fma(x[a][3], c2, x[a][1] * c0);
+            } else {
+                // Re row [-1/z^2, 0], Im row [0, 1/z^3]   (:366-367)
+                kr = x[a][0] * c1;
+                ki = x[a][1] * c2;
+            }
+            s[a] = cadd(s[a], cd{fma(ki, im.x, kr * re.x), fma(ki, im.y, kr * re.y)});
         }
-        s = cadd(s, cd{fma(ki, im.x, kr * re.x), fma(ki, im.y, kr * re.y)});
     };
     auto add1 = [&](int wn) {
         const kconst_double* c = tab + 4 * wn;
@@ -239,10 +254,13 @@ __global__ __launch_bounds__(64) void k_mom_fit(const cd* __restrict__ fw, int d
         }
     }
     for (; wn < n_freq; ++wn) add1(wn);
-    s = cd{0.5 * s.x, 0.5 * s.y};
-    cd* out = mt + ((size_t)a * range + w) * m2;
-    out[be + al * d] = cconj(s);
-    out[al + be * d] = s;
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
+        const cd v = cd{0.5 * s[a].x, 0.5 * s[a].y};
+        cd* out = mt + ((size_t)(a0 + a) * range + w) * m2;
+        out[be + al * d] = cconj(v);
+        out[al + be * d] = v;
+    }
 }
 
 // trace[a][w] = sum_alpha Re mt[a][w][alpha alpha]     (:244-247)
@@ -984,11 +1002,11 @@ extern "C" int dmftgpu_moments(dmftgpu_handle h, int d, int n_freq, double beta,
         ent->beta = beta;
         ent->green = green_asym;
     }
-    const dim3 gfit((unsigned)(((size_t)range * (d * (d + 1) / 2) + 63) / 64), nm);
-    const double* dtab = (const double*)tab;
-    if (green_asym)
-        hipLaunchKernelGGL((k_mom_fit<true>), gfit, dim3(64), 0, s, (const cd*)fw, d, n_freq, range, dtab, kinv, mt);
-    else hipLaunchKernelGGL((k_mom_fit<false>), gfit, dim3(64), 0, s, (const cd*)fw, d, n_freq, range, dtab, kinv, mt);
+    const size_t fits = (size_t)range * (d * (d + 1) / 2);
+    const bool all = fits >= kFitAll;
+    const dim3 gfit((unsigned)((fits + 63) / 64), all ? 1 : nm);
+    auto fit = green_asym ? all ? k_mom_fit<true, 2> : k_mom_fit<true, 1> : all ? k_mom_fit<false, 4> : k_mom_fit<false, 1>;
+    hipLaunchKernelGGL(fit, gfit, dim3(64), 0, s, (const cd*)fw, d, n_freq, range, (const double*)tab, kinv, mt);
     HIPCHK(hipGetLastError());
     hipLaunchKernelGGL(k_mom_trace, dim3(nblk((size_t)range * nm)), dim3(256), 0, s, mt, d, range, nm, trace);
     HIPCHK(hipGetLastError());
