@@ -549,6 +549,7 @@ __device__ __forceinline__ void schur_item(const LatArgs& a, const cd* __restric
                     // compiler reads one entry, waits and uses it, an LDS round trip per entry
                     constexpr int AHEAD = 3;
                     auto fetch = [&](int q) -> cd {
+                        if (q >= M2 + NC) return cd{0.0, 0.0};  // past the last (n_c < AHEAD), not used
                         return q < M2 ? gbar_at(q / NC, q % NC) : sAcc[(q - M2 + b * NC) * FW + lane];
                     };
                     cd buf[AHEAD], t[NC];
