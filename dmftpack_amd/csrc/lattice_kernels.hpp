@@ -225,7 +225,7 @@ struct SchurMulti {
 };
 hipError_t launch_lattice_schur_multi(const LatArgs& proto, int mode, hipStream_t s, int wg,
                                       const SchurMulti& m);
-// the same for 6 < n_c <= 16: column-per-lane kernels (MODE_FWD, MODE_VJP over every frequency)
+// the same for 6 < n_c <= 16: column-per-lane kernels (MODE_FWD, MODE_VJP), work items as above
 hipError_t launch_lattice_schur_cols_multi(const LatArgs& proto, int mode, hipStream_t s,
                                            const SchurMulti& m);
 // frequencies per workgroup of the Schur kernel for n_c (grid planning)

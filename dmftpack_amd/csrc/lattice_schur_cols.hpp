@@ -336,8 +336,8 @@ __device__ __forceinline__ void cols_item(const LatArgs& a, const cd* __restrict
             if constexpr (MODE == MODE_VJP) {
                 // sigma_bar += G^H gbar G^H + cn ((G^2)_cc)^H = C = G^H V G^H with
                 // V = gbar + cn S'^H, S' = I + Y ((G^2)_cc = G S' G); lane c forms
-                // column c of C.  mu term tr(gbar^H (G^2)_cc) = sum_ab S'_ab conj(C_ab)
-                // - cn tr(Z^2) (as in lattice_schur.hip).
+                // column c of C.  mu term tr(gbar^H (G^2)_cc) = sum_ij Z_ij conj(L_ij)
+                // - cn tr(Z^2) with L = V G^H, as G S' = Z.
                 wave_sync();  // every lane has read Z from MB
                 if (live) {  // row c of V into MB
 #pragma unroll

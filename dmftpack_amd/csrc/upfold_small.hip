@@ -6,15 +6,17 @@
 // inputs are read and the results written once (the batched kernels of upfold.hip pass
 // every intermediate through memory: 13 launches per chunk of k).
 //   * Wavefront 0 inverts T, wavefront 1 S, at the same time, in registers: lane r + 16 g holds
-//     rows r and r + 16 of columns 8 g .. 8 g + 7.  Gauss-Jordan with partial pivoting, rows not
+//     rows r and r + 16 of columns 8 g .. 8 g + 7.  Gauss-Jordan with row pivoting (to 15 bits of
+//     |a|^2: pivots within 2^-16 of the largest, so entries grow at most as with the largest
+//     times 1 + 2^-16 a step), rows not
 //     exchanged but marked used (A^-1(j, p_c) is left in row p_j, column c, p_j the pivot row of
 //     step j); per step the pivot row and column pass through LDS, and a row entry read
 //     there serves two rows' products.
 //   * The products E = T^-H K_o, X C, C^H (X C), E K, (E K) E^H, S^-1 D, (S^-1 D) S^-1 on FP64
 //     MFMA (v_mfma_f64_16x16x4, complex as four real products), a wavefront taking 16 rows.
 // At n_orb = 28, 32^3 k it takes 2.3 ms (the batched kernels: 5.2 ms): 39 KB of LDS per k leave
-// two wavefronts per SIMD, whose vector work (7200 instructions) and MFMAs (0.18 of the SIMD
-// cycles) share the SIMD, with a third of the time waiting on LDS, barriers and loads.  The
+// two wavefronts per SIMD, whose vector work (7200 instructions each, 0.35 of the SIMD cycles)
+// and MFMAs (0.23) share the SIMD, the rest waiting on LDS, barriers and loads.  The
 // pivot search by shuffles of (|a|^2, row) pairs and divisions in the copy loops cost 2.7 ms.
 #include "upfold_small.hpp"
 

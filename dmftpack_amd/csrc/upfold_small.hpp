@@ -22,6 +22,10 @@ hipError_t launch_upfold_small(const UpfoldArgs& a, hipStream_t s);
 
 // R sums of nx matrices per k: part [seg][x][R][e] = sum over the segment's k of
 // ph(k, R) Y_x(k)(e), ph [nk][n_r padded to kRsTile] from launch_r_phases (phase +)
+// (14: the 27 R of the first shell of neighbours are two tiles with one column of padding; 14
+// sums take 66 vector registers, seven wavefronts per SIMD, and a tile's phases 84 scalar ones.
+// NumOrbit = 28, 12^3 k, the whole call, a workgroup per run of entries -> tiles, ms: 125 R
+// (126 padded) 6.8 -> 0.75, 343 R (350) 20.4 -> 1.72)
 constexpr int kRsTile = 14;
 inline int rs_pad(int n_r) { return (n_r + kRsTile - 1) / kRsTile * kRsTile; }
 hipError_t launch_r_phases(const int4* R, int n_r, const double* kphase, int nk, cd* ph, hipStream_t s);

@@ -73,6 +73,9 @@ typedef struct dmftgpu_handle_s* dmftgpu_handle;
  * and its static eigen-decomposition; hip_stream NULL = the default stream. */
 int dmftgpu_create(dmftgpu_handle* h, void* hip_stream);
 int dmftgpu_destroy(dmftgpu_handle h);
+/* Later calls queue their work on hip_stream.  Work on the previous stream is not waited
+ * for: it uses the handle's workspaces, so drain that stream first if calls that do not
+ * wait for their results (the transforms, the hybridisation) may still run on it. */
 int dmftgpu_set_stream(dmftgpu_handle h, void* hip_stream);
 const char* dmftgpu_last_error(dmftgpu_handle h);
 const char* dmftgpu_version(void);
@@ -84,8 +87,9 @@ const char* dmftgpu_version(void);
                                            32768 for the one-matrix-per-lane Schur kernels, keeping >= 64 k per
                                            chunk and >= 8192 items; 8192 for the others) */
 #define DMFTGPU_OPT_SCHUR_WG 3          /* frequencies per workgroup of the Schur kernels (64 or 128; default 0 =
-                                           64, or two or four wavefronts over 64 frequencies splitting the k
-                                           walk where that is faster) */
+                                           chosen by n_corr, n, n_k and the frequency count: 64, 128 on the
+                                           real axis, or two or four wavefronts over 64 frequencies that split
+                                           a chunk's k walk) */
 #define DMFTGPU_OPT_SCHUR_LAYOUT 4      /* n_c <= 6: 0 = one (k,iw) matrix per lane (default), 1 = one column
                                            per lane (always used for n_c > 6) */
 #define DMFTGPU_OPT_UPFOLD_CHUNK 5      /* k points per chunk of dmftgpu_upfold_density (0 = as many as 512 MiB of
@@ -302,7 +306,8 @@ int dmftgpu_ft_w2tau_points(dmftgpu_handle h, int d, int n_freq, double beta, co
 
 /* FT_t_to_w (FourierTransform.cpp:521-561): exact transform of the piecewise
  * linear interpolant of G(tau).  violations HOST (optional) counts frequencies
- * failing the causality test of :551-558 (the reference asserts). */
+ * failing the causality test of :551-558 (the reference asserts).  fw may overlap
+ * gtau (which is then overwritten). */
 int dmftgpu_ft_tau2w(dmftgpu_handle h, int d, int n_freq, int n_tau, double beta, const double* gtau, double* fw,
                      int* violations);
 
@@ -358,7 +363,9 @@ int dmftgpu_hk_from_hr(dmftgpu_handle h, int n, int n_hop, const int* hop_idx, c
  *   kphase     [n_k][3]             k_x a_x, k_y a_y, k_z a_z
  *   dm_k       [n_k][n_orb][n_orb]  output D_k (densityMatDFT[k] after upfolding_k), or NULL
  *   dmr        [3][n_r] complex     output (n_r = 0: dm_k only)
- * Inverses are Gauss-Jordan with partial pivoting; a singular T_k or S_k
+ * Inverses are Gauss-Jordan with row pivoting: the largest |a| of the column, up to
+ * n_orb = 32 compared as |a|^2 to 15 bits (the pivot is within 2^-16 of the largest),
+ * exactly above; a singular T_k or S_k
  * returns DMFTGPU_ERR_NUMERIC.  With k split over ranks the R sums are the
  * rank's share (the operands of the reference's MPI_Allreduce, :80-82). */
 int dmftgpu_upfold_density(dmftgpu_handle h, int n, int n_orb, int n_k, int n_k_global, double beta, double mu,
