@@ -16,7 +16,9 @@ once, with its Schur data eig(H_dd(k)), W = H_cd V_d, before timing):
 value = Nk * 2 N_freq / step time, for the Schur method schur_f32r, which computes in
 FP64 and takes the density sums beyond N_freq at 16 Gauss points (the 2 N_freq
 units are those the step answers for); the plain FP64 full-inverse path, which
-inverts all of them, runs the same step for the ratio.
+inverts all of them, runs the same step for the ratio.  "inversions" in the metric's name and
+unit are these units; matrices_inverted_per_step in the line counts the solves, so the ratio
+holds both the fewer solves and the cheaper ones.
 """
 import argparse
 import json
@@ -225,14 +227,12 @@ def main():
     # adjoint launch is the longest of the step.  The library's events time each
     # call's main launch on its own stream.
     t_f, t_v = float(np.mean(kf)) / 1e3, float(np.mean(kv)) / 1e3
-    fused = head != G.PLAIN_F64 and nc <= 6 and args.layout == 0
-    if fused or t_v >= t_f:
-        kname = "k_lattice_schur<VJP>"
-        t_k, flop, pkey = t_v, f_adj(n, nc), ("VJP" if fused else "VJP_CALL")
-        units_k = nk * nf if fused else units
+    # units_k: the (k, iw) the launch answers for, 2 N_freq per k in every method
+    if t_v >= t_f:
+        kname, t_k, flop, pkey = "k_lattice_schur<VJP>", t_v, f_adj(n, nc), "VJP"
     else:
-        kname = "k_lattice_schur<FWD>"
-        t_k, flop, pkey, units_k = t_f, f_fwd(n), "FWD_CALL", units
+        kname, t_k, flop, pkey = "k_lattice_schur<FWD>", t_f, f_fwd(n), "FWD"
+    units_k = units
     if head == G.PLAIN_F64:
         kname = kname.replace("schur", "plain")
     # HBM bytes per launch: FETCH_SIZE / WRITE_SIZE counters of the same kernel,
@@ -324,6 +324,7 @@ def main():
                    "refine_steps": args.refine, "schur_layout": args.layout, "schur_wg": args.wg or "default (64 frequencies, k walk split where faster)",
                    "target_workgroups": args.target or "default",
                    "units_per_step": units,
+                   "matrices_inverted_per_step": 2 * (units if head == G.PLAIN_F64 else nk * (nf + 16)),
                    "step": "tail-moment fit of Sigma + static eig for the tail + GreenFtn_w forward (G_loc, NumMatrix, "
                            "N) + loss cotangents + VJP (dL/dSigma, dL/dmu): dmftgpu_moments, dmftgpu_update_moments, "
                            "one dmftgpu_gloc_loss_grad call"},
