@@ -20,6 +20,10 @@
   python -m dmftpack_amd.rocprof_summary mfma --run <dir> [--command "..."]
       FP64 MFMA and VALU FLOPs per launch and MFMA busy cycles, from one --pmc
       pass of MFMA_COUNTERS.
+
+  python -m dmftpack_amd.rocprof_summary busy --run <dir> [--command "..."]
+      clock, VALU-busy share and instruction mix per launch, from one --pmc pass
+      of BUSY_COUNTERS.
 """
 import argparse
 import csv
@@ -248,8 +252,53 @@ def mfma(argv):
               f"{c.get('SQ_INSTS_VALU_MFMA_F64', 0) / 1e6:>10.2f} {busy:>9.3f}  {name[:100]}")
 
 
+BUSY_COUNTERS = ("SQ_ACTIVE_INST_VALU SQ_ACTIVE_INST_LDS SQ_INSTS_VALU SQ_INSTS_LDS SQ_LDS_BANK_CONFLICT SQ_WAVES "
+                 "SQ_WAVE_CYCLES GRBM_GUI_ACTIVE")
+
+
+def busy(argv):
+    """What a launch's cycles went to, from one --pmc pass of BUSY_COUNTERS.
+    Cycles = GRBM_GUI_ACTIVE / 8 (summed over the XCDs), clock = cycles / launch time;
+    VALU busy = 4 SQ_ACTIVE_INST_VALU (quad cycles) / (cycles x 1024 SIMDs), LDS busy
+    the same of SQ_ACTIVE_INST_LDS per CU, waves = 4 SQ_WAVE_CYCLES / (cycles x 1024).
+    Launches under 50 us are left out: their cycles are the command processor's."""
+    ap = argparse.ArgumentParser(prog="rocprof_summary busy")
+    ap.add_argument("--run", required=True)
+    ap.add_argument("--command", default="")
+    a = ap.parse_args(argv)
+    rows = defaultdict(lambda: defaultdict(float))
+    dur = defaultdict(dict)
+    for f in glob.glob(os.path.join(a.run, "**", "*results.db"), recursive=True):
+        db = sqlite3.connect(f)
+        for name, did, cn, v, d in db.execute("select kernel_name, dispatch_id, counter_name, value, duration "
+                                              "from counters_collection"):
+            rows[name][cn] += v
+            dur[name][(f, did)] = d
+    print(f"# clock and busy shares per launch from rocprofv3 --pmc {BUSY_COUNTERS}")
+    if a.command:
+        print(f"# command: {a.command}")
+    print("# clock = GRBM_GUI_ACTIVE / 8 / time; valu = 4 SQ_ACTIVE_INST_VALU / (GRBM_GUI_ACTIVE/8 x 1024 SIMDs); lds = 4 "
+          "SQ_ACTIVE_INST_LDS / (GRBM_GUI_ACTIVE/8 x 256 CUs); waves per SIMD = 4 SQ_WAVE_CYCLES / (GRBM_GUI_ACTIVE/8 x 1024); "
+          "conflict = SQ_LDS_BANK_CONFLICT / (GRBM_GUI_ACTIVE/8 x 256)")
+    print(f"{'launch_ms':>9} {'GHz':>5} {'valu':>6} {'lds':>6} {'conflict':>8} {'waves':>6} {'valu_Minst':>10} "
+          f"{'lds_Minst':>9}  kernel")
+    for name in sorted(rows):
+        nd = len(dur[name])
+        t = sum(dur[name].values()) / nd * 1e-9
+        if not is_ours(name) or t < 50e-6:
+            continue
+        c = {k: v / nd for k, v in rows[name].items()}
+        cyc = c.get("GRBM_GUI_ACTIVE", 0.0) / 8.0
+        if cyc <= 0:
+            continue
+        print(f"{t * 1e3:>9.3f} {cyc / t / 1e9:>5.2f} {4 * c.get('SQ_ACTIVE_INST_VALU', 0) / (cyc * 1024):>6.3f} "
+              f"{4 * c.get('SQ_ACTIVE_INST_LDS', 0) / (cyc * 256):>6.3f} {c.get('SQ_LDS_BANK_CONFLICT', 0) / (cyc * 256):>8.3f} "
+              f"{4 * c.get('SQ_WAVE_CYCLES', 0) / (cyc * 1024):>6.2f} {c.get('SQ_INSTS_VALU', 0) / 1e6:>10.1f} "
+              f"{c.get('SQ_INSTS_LDS', 0) / 1e6:>9.1f}  {name[:100]}")
+
+
 def main():
-    if len(sys.argv) < 2 or sys.argv[1] not in ("trace", "pmc", "sq", "mfma"):
+    if len(sys.argv) < 2 or sys.argv[1] not in ("trace", "pmc", "sq", "mfma", "busy"):
         sys.exit(__doc__)
     if sys.argv[1] == "trace":
         trace(sys.argv[2], sys.argv[3] if len(sys.argv) > 3 else "")
@@ -257,6 +306,8 @@ def main():
         sq(sys.argv[2:])
     elif sys.argv[1] == "mfma":
         mfma(sys.argv[2:])
+    elif sys.argv[1] == "busy":
+        busy(sys.argv[2:])
     else:
         pmc(sys.argv[2:])
 
